@@ -105,13 +105,13 @@ struct EcbArgs {
 };
 
 template <bool PRG>
-__global__ __launch_bounds__(256) void aes_stream_kernel(EcbArgs a) {
-  __shared__ uint32_t tab[CUOT_AES_LDS_WORDS];
-  aes_stage_table(tab, a.T0, threadIdx.x, 256);
+__global__ __launch_bounds__(CUOT_AES_WG) void aes_stream_kernel(EcbArgs a) {
+  __shared__ __align__(16) uint32_t tab[CUOT_AES_LDS_WORDS];
+  aes_stage_table(tab, a.T0, threadIdx.x, CUOT_AES_WG);
   __syncthreads();
   const AesLds aes = aes_lds(tab);
-  const int64_t stride = (int64_t)gridDim.x * 256;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < a.n; i += stride) {
+  const int64_t stride = (int64_t)gridDim.x * CUOT_AES_WG;
+  for (int64_t i = (int64_t)blockIdx.x * CUOT_AES_WG + threadIdx.x; i < a.n; i += stride) {
     blk x;
     if (PRG) {
       const uint64_t c = a.start + (uint64_t)i;
@@ -121,13 +121,6 @@ __global__ __launch_bounds__(256) void aes_stream_kernel(EcbArgs a) {
     }
     a.out[i] = aes_enc(aes, a.rk, x);
   }
-}
-
-static unsigned stream_grid(int64_t n) {
-  int64_t g = (n + 255) / 256;
-  if (g > 4096) g = 4096;
-  if (g < 1) g = 1;
-  return (unsigned)g;
 }
 
 hipError_t cuot_launch_aes_ecb(const uint32_t rk[44], const blk* in, blk* out, int64_t n, hipStream_t st) {
@@ -141,7 +134,7 @@ hipError_t cuot_launch_aes_ecb(const uint32_t rk[44], const blk* in, blk* out, i
   a.n = n;
   a.stream = a.start = 0;
   cuot_rec_begin(st, "aes_stream", 32.0 * (double)n);
-  hipLaunchKernelGGL(aes_stream_kernel<false>, dim3(stream_grid(n)), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(aes_stream_kernel<false>, dim3(cuot_aes_grid(n)), dim3(CUOT_AES_WG), 0, st, a);
   cuot_rec_end(st);
   return hipGetLastError();
 }
@@ -159,7 +152,7 @@ hipError_t cuot_launch_prg(const uint32_t rk[44], uint64_t stream, uint64_t star
   a.stream = stream;
   a.start = start;
   cuot_rec_begin(st, "aes_stream", 16.0 * (double)n);
-  hipLaunchKernelGGL(aes_stream_kernel<true>, dim3(stream_grid(n)), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(aes_stream_kernel<true>, dim3(cuot_aes_grid(n)), dim3(CUOT_AES_WG), 0, st, a);
   cuot_rec_end(st);
   return hipGetLastError();
 }

@@ -1,10 +1,24 @@
-// aes_dev.h -- AES-128 encryption on gfx950 with an LDS-resident T-table.
+// aes_dev.h -- AES-128 encryption on gfx950 with LDS-resident T-tables.
 //
-// CDNA4 has no AES instructions.  Each round is done with one 256-entry
-// 32-bit table T0 (SubBytes+MixColumns of a row-0 byte); the row-1..3 tables
-// are byte rotations of T0, applied with a rotate after the lookup.  The table
-// is replicated CUOT_AES_REP times in LDS so that lanes with different
-// (lane % REP) hit different banks: entry x of copy r is at word x*REP + r.
+// CDNA4 has no AES instructions.  Each round is done with the 256-entry 32-bit
+// table T0 (SubBytes + MixColumns of a row-0 byte) and T1 = T0 rotated by a
+// byte; the tables of rows 2 and 3 are T0 and T1 rotated by 16, applied to the
+// XOR of both lookups with one rotate.
+//
+// Layout: entry x is 256 bytes of LDS, 32 copies of T0[x] then 32 copies of
+// T1[x]; lane l reads copy l % 32.  What bounds AES here is VALU issue, then
+// the LDS: 160 dword reads per block at two cycles per wavefront allow 1.2e11
+// AES/s.  The 256-byte entry makes a lookup address one v_perm_b32 (byte k of
+// the state word over the lane's byte offset, for any k, with T1 behind the
+// instruction's immediate offset), where 128-byte entries take a bit-field
+// extract and a multiply-add; T1 saves two of three rotates per column; and
+// the 32 copies keep each half wavefront on 32 distinct banks.  A round's
+// column is 8 VALU operations (4 v_perm, XOR, rotate, three-input XOR, key)
+// instead of 14, a block ~340 instead of 577.  Measured for pairs of AES on
+// one input: 32 copies of T0 alone 5.0e10 AES/s, this form 8.3e10 with two
+// 512-lane workgroups per CU (64 KB each) and 9.3e10 with two of 1024; 64
+// copies of T0 7.6e10; four tables of 32 copies (128 KB, one 1024-lane
+// workgroup per CU) 9.4e10, which leaves no room for tree nodes.
 //
 // The tables are computed on the host from the FIPS-197 definition of the
 // S-box (multiplicative inverse + affine map) and uploaded at init.
@@ -15,42 +29,53 @@
 
 #include "common.h"
 
-#ifndef CUOT_AES_REP
-#define CUOT_AES_REP 32
-#endif
+#define CUOT_AES_LDS_WORDS (256 * 64)
+// lanes of a workgroup that shares one table (two such workgroups per CU)
+#define CUOT_AES_WG 512
 
-#define CUOT_AES_LDS_WORDS (256 * CUOT_AES_REP)
+// Grid of a kernel that streams n blocks through such workgroups: four rounds
+// of the chip's 512 resident ones balance the tail and still spread each table
+// fill over many blocks.
+inline unsigned cuot_aes_grid(int64_t n) {
+  int64_t g = (n + CUOT_AES_WG - 1) / CUOT_AES_WG;
+  if (g > 2048) g = 2048;
+  return g < 1 ? 1u : (unsigned)g;
+}
 
+typedef __attribute__((address_space(3))) const char* lds_cptr;
 
 struct AesLds {
-  const uint32_t* base;  // LDS table, replicated
-  uint32_t lane_off;     // (lane % REP) * 4 bytes
+  lds_cptr base;      // the table (first in the kernel's LDS, so that it folds into the offset)
+  uint32_t lane_off;  // (lane % 32) * 4 bytes, below 256
 };
 
-// Fill the replicated table.  Call from all threads of the block, then sync.
+// Fill the table.  Call from all threads of the block, then sync.
 // T0g: the 256-word table in global memory (uploaded by cuot_init).
+// 16-byte chunk i of the table belongs to entry i / 16, its chunks 8..15 to T1.
 CUOT_DEV void aes_stage_table(uint32_t* lds, const uint32_t* __restrict__ T0g, int tid, int nthreads) {
-  for (int i = tid; i < CUOT_AES_LDS_WORDS; i += nthreads) lds[i] = T0g[i / CUOT_AES_REP];
+#pragma unroll 8
+  for (int i = tid; i < CUOT_AES_LDS_WORDS / 4; i += nthreads) {
+    const uint32_t t = T0g[i >> 4];
+    const uint32_t v = (i & 8) ? (t << 8) | (t >> 24) : t;
+    ((uint4*)lds)[i] = make_uint4(v, v, v, v);
+  }
 }
 
 CUOT_DEV AesLds aes_lds(const uint32_t* lds) {
   AesLds a;
-  a.base = lds;
-  a.lane_off = (threadIdx.x % CUOT_AES_REP) * 4u;
+  a.base = (lds_cptr)lds;
+  a.lane_off = (threadIdx.x & 31u) * 4u;
   return a;
 }
 
-// Table lookup of byte value b (0..255).
-CUOT_DEV uint32_t tlook(const AesLds& a, uint32_t b) {
-  uint32_t off = (b * (CUOT_AES_REP * 4u)) + a.lane_off;
-  return *(const uint32_t*)((const char*)a.base + off);
+// T0 (T = 0) or T1 (T = 1) at byte K of w
+template <int K, int T>
+CUOT_DEV uint32_t tlook(const AesLds& a, uint32_t w) {
+  const uint32_t off = __builtin_amdgcn_perm(w, a.lane_off, 0x0c0c0000u | ((4u + K) << 8));
+  return *(const __attribute__((address_space(3))) uint32_t*)(a.base + off + 128 * T);
 }
 
-CUOT_DEV uint32_t rotl32(uint32_t x, int s) { return (x << s) | (x >> (32 - s)); }
-
-// a ^ b ^ c as one three-input bit operation (table 0x96) on VGPR operands;
-// the round key (uniform in some kernels, per lane in others) is added by a
-// plain XOR, which takes it from either register file
+// a ^ b ^ c as one three-input bit operation (table 0x96)
 CUOT_DEV uint32_t aes_x3(uint32_t a, uint32_t b, uint32_t c) {
   uint32_t r;
   asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0x96" : "=v"(r) : "v"(a), "v"(b), "v"(c));
@@ -58,21 +83,20 @@ CUOT_DEV uint32_t aes_x3(uint32_t a, uint32_t b, uint32_t c) {
 }
 
 CUOT_DEV uint32_t aes_col(const AesLds& a, uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3, uint32_t k) {
-  uint32_t t0 = tlook(a, w0 & 0xffu);
-  uint32_t t1 = tlook(a, (w1 >> 8) & 0xffu);
-  uint32_t t2 = tlook(a, (w2 >> 16) & 0xffu);
-  uint32_t t3 = tlook(a, w3 >> 24);
-  return aes_x3(t0, rotl32(t1, 8), rotl32(t2, 16)) ^ rotl32(t3, 24) ^ k;
+  const uint32_t t0 = tlook<0, 0>(a, w0), t1 = tlook<1, 1>(a, w1);
+  const uint32_t u = tlook<2, 0>(a, w2) ^ tlook<3, 1>(a, w3);
+  return aes_x3(t0, t1, __builtin_amdgcn_alignbit(u, u, 16)) ^ k;
 }
 
-// Last round: S-box bytes recovered from T0 (T0[x] bytes are 2s, s, s, 3s).
+// Last round: S-box bytes recovered from the tables (bytes of T0[x]: 2s, s, s,
+// 3s; of T1[x]: 3s, 2s, s, s)
 CUOT_DEV uint32_t aes_col_last(const AesLds& a, uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3,
                                uint32_t k) {
-  uint32_t t0 = tlook(a, w0 & 0xffu);
-  uint32_t t1 = tlook(a, (w1 >> 8) & 0xffu);
-  uint32_t t2 = tlook(a, (w2 >> 16) & 0xffu);
-  uint32_t t3 = tlook(a, w3 >> 24);
-  return (((t0 >> 8) & 0x000000ffu) | (t1 & 0x0000ff00u) | (t2 & 0x00ff0000u) | ((t3 << 8) & 0xff000000u)) ^ k;
+  const uint32_t t0 = tlook<0, 0>(a, w0), t1 = tlook<1, 1>(a, w1);
+  const uint32_t t2 = tlook<2, 0>(a, w2), t3 = tlook<3, 1>(a, w3);
+  const uint32_t lo = __builtin_amdgcn_perm(t0, t1, 0x0c0c0205u);  // byte 1 of t0, byte 2 of t1
+  const uint32_t hi = __builtin_amdgcn_perm(t2, t3, 0x02060c0cu);  // byte 2 of t2, byte 2 of t3
+  return (lo | hi) ^ k;
 }
 
 // rk: 44 little-endian round-key words (FIPS w[0..43] in memory order).

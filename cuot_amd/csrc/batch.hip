@@ -3,7 +3,7 @@
 // Every instance keeps its own workspace carve (the SotPlan / FerretPlan of a
 // single run), so its stage outputs are the same bytes as a plain run.  What
 // is shared is the launches:
-//   * GGM: one launch per (role, subtree split L) over the trees of all
+//   * GGM: one launch per (role, kernel form) over the trees of all
 //     instances (instance tables + tree prefix in HBM);
 //   * A^ prepare: one launch sequence per transform length 2^m;
 //   * QC encode: one launch sequence per 2^m and scratch chunk, both parties of
@@ -29,7 +29,7 @@ constexpr size_t kDefaultQcChunk = (size_t)4 << 30;
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 struct GgmGroup {
-  int L = 0;
+  int form = 0;  // cuot_ggm_form
   bool recv = false;
   std::vector<int> members;
   int64_t total = 0;  // trees
@@ -127,19 +127,19 @@ int plan_batch(cuot_batch* b) {
     }
   }
   // ---- groups ------------------------------------------------------------
-  std::map<int, int> ggm_s, ggm_r;  // L -> group index
+  std::map<int, int> ggm_s, ggm_r;  // form -> group index
   std::map<int, std::vector<int>> by_m;
   for (int i = 0; i < count; i++) {
-    const int L = cuot_ggm_split(b->inst[i].h);
+    const int form = cuot_ggm_form(b->inst[i].h);
     for (int r = 0; r < 2; r++) {
       std::map<int, int>& mp = r ? ggm_r : ggm_s;
-      auto it = mp.find(L);
+      auto it = mp.find(form);
       if (it == mp.end()) {
         GgmGroup g;
-        g.L = L;
+        g.form = form;
         g.recv = r == 1;
         b->ggm.push_back(g);
-        it = mp.emplace(L, (int)b->ggm.size() - 1).first;
+        it = mp.emplace(form, (int)b->ggm.size() - 1).first;
       }
       GgmGroup& g = b->ggm[it->second];
       g.members.push_back(i);
@@ -149,7 +149,7 @@ int plan_batch(cuot_batch* b) {
   }
   // senders before receivers
   std::stable_sort(b->ggm.begin(), b->ggm.end(), [](const GgmGroup& x, const GgmGroup& y) {
-    return x.recv != y.recv ? !x.recv : x.L < y.L;
+    return x.recv != y.recv ? !x.recv : x.form < y.form;
   });
   for (auto& kv : by_m) {
     PrepGroup pg;
@@ -370,7 +370,7 @@ hipError_t launch_all(cuot_batch* b, uint32_t stages, hipStream_t st, hipStream_
     for (const GgmGroup& g : b->ggm) {
       if (g.recv != (r == 1)) continue;
       if ((e = cuot_launch_ggm_batch((const GgmKArgs*)(ws + g.tab_off), (const int64_t*)(ws + g.start_off),
-                                     (int)g.members.size(), g.total, g.L, g.recv, st)))
+                                     (int)g.members.size(), g.total, g.form, g.recv, st)))
         return e;
     }
     if (r == 0) {

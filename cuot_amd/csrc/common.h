@@ -18,9 +18,17 @@ CUOT_DEV blk bxor(blk a, blk b) { return make_uint4(a.x ^ b.x, a.y ^ b.y, a.z ^ 
 CUOT_DEV blk bzero() { return make_uint4(0u, 0u, 0u, 0u); }
 CUOT_DEV blk bsel(bool c, blk a) { return c ? a : bzero(); }
 
-// Non-temporal-free plain 16-byte global accessors (vector memory path).
-CUOT_DEV blk ldb(const blk* p) { return *p; }
-CUOT_DEV void stb(blk* p, blk v) { *p = v; }
+// Plain 16-byte global accessors.  The address space is spelled out: through a
+// pointer read from an argument table the compiler would use flat accesses,
+// which also count as LDS operations.
+typedef uint32_t blk_vec __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) blk_vec* blk_gptr;
+typedef const __attribute__((address_space(1))) blk_vec* blk_cgptr;
+CUOT_DEV blk ldb(const blk* p) {
+  const blk_vec v = *(blk_cgptr)p;
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+CUOT_DEV void stb(blk* p, blk v) { *(blk_gptr)p = blk_vec{v.x, v.y, v.z, v.w}; }
 
 // ---------------------------------------------------------------------------
 // Host-side error plumbing: every extern "C" entry point returns an int status.

@@ -20,12 +20,12 @@
 
 namespace {
 
-// S-box byte x from the T-table (T0[x] bytes are 2s, s, s, 3s)
-CUOT_DEV uint32_t sbox(const AesLds& a, uint32_t x) { return (tlook(a, x) >> 8) & 0xffu; }
-
-CUOT_DEV uint32_t sub_word(const AesLds& a, uint32_t w) {
-  return sbox(a, w & 0xffu) | (sbox(a, (w >> 8) & 0xffu) << 8) | (sbox(a, (w >> 16) & 0xffu) << 16) |
-         (sbox(a, w >> 24) << 24);
+// SubWord(RotWord(w)): S-box bytes from the tables (byte 1 of T0, byte 2 of
+// either, byte 3 of T1)
+CUOT_DEV uint32_t sub_rot_word(const AesLds& a, uint32_t w) {
+  const uint32_t t0 = tlook<1, 0>(a, w), t1 = tlook<2, 0>(a, w);
+  const uint32_t t2 = tlook<3, 0>(a, w), t3 = tlook<0, 1>(a, w);
+  return __builtin_amdgcn_perm(t0, t1, 0x0c0c0105u) | __builtin_amdgcn_perm(t2, t3, 0x03060c0cu);
 }
 
 // FIPS-197 key expansion on little-endian words (word i = bytes 4i..4i+3)
@@ -39,7 +39,7 @@ CUOT_DEV void expand_key(const AesLds& a, blk key, uint32_t rk[44]) {
   for (int i = 4; i < 44; i++) {
     uint32_t t = rk[i - 1];
     if ((i & 3) == 0) {
-      t = sub_word(a, (t >> 8) | (t << 24)) ^ rcon;  // RotWord, SubWord, Rcon on byte 0
+      t = sub_rot_word(a, t) ^ rcon;  // Rcon on byte 0
       rcon = (rcon << 1) ^ ((rcon & 0x80u) ? 0x11bu : 0u);
     }
     rk[i] = rk[i - 4] ^ t;
@@ -74,13 +74,14 @@ __global__ __launch_bounds__(256) void cot_online_kernel(DerandArgs a) {
 }
 
 template <bool ROT>
-__global__ __launch_bounds__(256) void cot_hash_kernel(DerandArgs a) {
-  __shared__ uint32_t tab[CUOT_AES_LDS_WORDS];
-  aes_stage_table(tab, a.T0, threadIdx.x, 256);
+__global__ __launch_bounds__(CUOT_AES_WG) void cot_hash_kernel(DerandArgs a) {
+  __shared__ __align__(16) uint32_t tab[CUOT_AES_LDS_WORDS];
+  aes_stage_table(tab, a.T0, threadIdx.x, CUOT_AES_WG);
   __syncthreads();
   const AesLds aes = aes_lds(tab);
   const blk D = *a.delta;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < a.n; i += (int64_t)gridDim.x * 256) {
+  for (int64_t i = (int64_t)blockIdx.x * CUOT_AES_WG + threadIdx.x; i < a.n;
+       i += (int64_t)gridDim.x * CUOT_AES_WG) {
     const uint64_t g = a.g0 + (uint64_t)i;  // makeBlock(g, 0): hi = g, lo = 0
     const blk key = make_uint4(a.s.x, a.s.y, a.s.z ^ (uint32_t)g, a.s.w ^ (uint32_t)(g >> 32));
     uint32_t rk[44];
@@ -150,9 +151,9 @@ hipError_t cuot_launch_cot_hash(const blk* ks, const blk* mr, const blk* delta, 
   // three AES (and one key expansion) per COT; 16 B in, 48 B (OT) out per party pair
   cuot_rec_begin(st, rot ? "cot_hash_kernel<rot>" : "cot_hash_kernel<ot>", 80.0 * (double)n);
   if (rot)
-    hipLaunchKernelGGL(cot_hash_kernel<true>, dim3(grid_of(n)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(cot_hash_kernel<true>, dim3(cuot_aes_grid(n)), dim3(CUOT_AES_WG), 0, st, a);
   else
-    hipLaunchKernelGGL(cot_hash_kernel<false>, dim3(grid_of(n)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(cot_hash_kernel<false>, dim3(cuot_aes_grid(n)), dim3(CUOT_AES_WG), 0, st, a);
   cuot_rec_end(st);
   return hipGetLastError();
 }

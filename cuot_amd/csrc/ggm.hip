@@ -2,135 +2,159 @@
 // sender (full trees) and the receiver (punctured trees rebuilt from its own
 // view: chosen level sums + choice bits), in SOT and Ferret flavours.
 //
-// One workgroup of 256 lanes owns one tree (the reference launches one kernel
+// One workgroup of 512 lanes owns one tree (the reference launches one kernel
 // per level plus a multi-pass reduction per level; gpu/aes_op.cu:176-266,
 // gpu/gpu_matrix.cu:155-169).  Per tree:
-//   A. top levels 0..top breadth-first in LDS (top = h for h <= 8, else
-//      top = h - L with L = min(h - 8, 6), so 2^top is 256..1024 nodes), level
-//      sums by a workgroup XOR reduction; the receiver resolves the sibling of
-//      its punctured path at every level (silent/recver.cu:98-115,
-//      spcot_recver.h:66-95).
-//   B. (h > 8) every lane expands 2^top/256 depth-`top` nodes depth-first for
+//   A. top levels 0..top breadth-first in LDS, one parent per lane (top = h
+//      for h <= 9, else top = h - L with L = min(h - 9, 6), so 2^top is 512 or
+//      1024 nodes), level sums by a workgroup XOR reduction; the receiver
+//      resolves the sibling of its punctured path at every level
+//      (silent/recver.cu:98-115, spcot_recver.h:66-95).
+//   B. (h > 9) every lane expands 2^top/512 depth-`top` nodes depth-first for
 //      L levels, with a fully unrolled path stack in registers; leaves go
 //      straight to HBM, per-depth left/right sums are reduced over the
 //      workgroup.  The punctured depth-`top` node contributes nothing.
-//   C. (receiver, h > 8) the punctured depth-`top` subtree is rebuilt level
+//   C. (receiver, h > 9) the punctured depth-`top` subtree is rebuilt level
 //      by level in LDS from the chosen sums and the workgroup sums of phase B.
 // Child rule: left = AES_k0(p) ^ p, right = AES_k1(p) ^ p (twokeyprp.h:7-23).
+//
+// Bound by the AES (aes_dev.h): the 64 KB table is shared by 512 lanes so that
+// two workgroups fit a CU, one's breadth-first levels (a serial chain of AES
+// latencies) running beside the other's subtrees.  Sender / receiver: 1024
+// trees of depth 15 1.35 / 1.41 -> 0.81 / 0.90 ms (8.3e10 AES/s), 1270 of depth
+// 13 0.48 / 0.54 -> 0.31 / 0.33 ms (256 lanes and a 32 KB table before).
 #include "aes_dev.h"
 #include "kernels.h"
 
 namespace {
 
-constexpr int WG = 256;
+constexpr int WG = CUOT_AES_WG;
+constexpr int NWAVE = WG / 64;
 constexpr int LMAX = 6;      // deepest per-lane DFS (register budget)
 constexpr int MAXTOP = 10;   // deepest LDS breadth-first level (h <= 16)
 
-CUOT_DEV uint32_t wave_xor(uint32_t v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v ^= (uint32_t)__shfl_xor((int)v, o, 64);
-  return v;
+// value of the lane XOR_MASK away (1, 2, 8: DPP; 4, 16: swizzle; 32: permute)
+template <int XOR_MASK>
+CUOT_DEV uint32_t lane_xor(uint32_t v) {
+  if constexpr (XOR_MASK == 1)
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xb1, 0xf, 0xf, true);  // quad [1,0,3,2]
+  else if constexpr (XOR_MASK == 2)
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4e, 0xf, 0xf, true);  // quad [2,3,0,1]
+  else if constexpr (XOR_MASK == 8)
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, true);  // row rotate by 8 of 16
+  else if constexpr (XOR_MASK == 32)
+    return (uint32_t)__shfl_xor((int)v, 32, 64);
+  else
+    return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, (XOR_MASK << 10) | 0x1f);
 }
 
-// XOR-reduce two blocks over the 256-lane workgroup; result in every lane.
-// red: LDS scratch of 4 waves x 8 words.  Contains two barriers.
-CUOT_DEV void wg_xor2(blk& a, blk& b, uint32_t* red) {
+// XOR of two blocks over a wavefront, scattered: lane l returns word
+// bitreverse3(l & 7) of the eight words (a, b).  Each exchange halves the words
+// a lane still owns, so 10 exchanges do what 48 would for all words in every
+// lane.
+CUOT_DEV uint32_t wave_xor2(blk a, blk b) {
+  const uint32_t lane = threadIdx.x;
   uint32_t v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  uint32_t k4[4], k2[2];
 #pragma unroll
-  for (int i = 0; i < 8; i++) v[i] = wave_xor(v[i]);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  __syncthreads();
-  if (lane == 0) {
-#pragma unroll
-    for (int i = 0; i < 8; i++) red[wave * 8 + i] = v[i];
+  for (int i = 0; i < 4; i++) {
+    const uint32_t keep = (lane & 1) ? v[i + 4] : v[i], send = (lane & 1) ? v[i] : v[i + 4];
+    k4[i] = keep ^ lane_xor<1>(send);
   }
-  __syncthreads();
-  uint32_t r[8];
 #pragma unroll
-  for (int i = 0; i < 8; i++) r[i] = red[i] ^ red[8 + i] ^ red[16 + i] ^ red[24 + i];
-  a = make_uint4(r[0], r[1], r[2], r[3]);
-  b = make_uint4(r[4], r[5], r[6], r[7]);
+  for (int i = 0; i < 2; i++) {
+    const uint32_t keep = (lane & 2) ? k4[i + 2] : k4[i], send = (lane & 2) ? k4[i] : k4[i + 2];
+    k2[i] = keep ^ lane_xor<2>(send);
+  }
+  uint32_t r = ((lane & 4) ? k2[1] : k2[0]) ^ lane_xor<4>((lane & 4) ? k2[0] : k2[1]);
+  r ^= lane_xor<8>(r);
+  r ^= lane_xor<16>(r);
+  return r ^ lane_xor<32>(r);
 }
+
+CUOT_DEV int bitrev3(int i) { return ((i & 1) << 2) | (i & 2) | ((i >> 2) & 1); }
 
 CUOT_DEV blk clear_lsb(blk v) {
   v.x &= ~1u;
   return v;
 }
 
+// NB: breadth-first nodes held (2^9, or 2^10 for trees of depth 16)
+template <int NB>
 struct Lds {
-  uint32_t aes[CUOT_AES_LDS_WORDS];
-  blk nodes[1 << MAXTOP];
-  blk sums[2 * 16];  // [depth][L,R] for depths 1..16 (index depth-1)
-  uint32_t red[32];
+  uint32_t aes[CUOT_AES_LDS_WORDS];  // first: the table's LDS address folds into the lookups' offsets
+  blk nodes[NB];
+  blk sums[2 * 16];                // [depth][L,R] for depths 1..16 (index depth-1)
+  uint32_t red[LMAX][NWAVE][8];    // per-wave XORs
+  blk csum[16];                    // receiver: the tree's chosen sums
+  uint8_t choice[16];              // receiver: the tree's choice bits
 };
+
+// word i of the workgroup XOR parked in red[slot]
+template <int NB>
+CUOT_DEV uint32_t red_word(const Lds<NB>& s, int slot, int i) {
+  uint32_t r = 0;
+#pragma unroll
+  for (int w = 0; w < NWAVE; w++) r ^= s.red[slot][w][i];
+  return r;
+}
+
+CUOT_DEV uint32_t* words(blk* b) { return (uint32_t*)b; }
 
 // Breadth-first expansion in LDS of `nlev` levels below nodes[0].
 // Receiver mode resolves the sibling on the punctured path at each level
 // using chosen sums csum[d0 + r] and external (outside-LDS) side sums ext.
 // Returns the punctured index at the last level (receiver) in *punct_out.
 // `final_rule`: apply the punctured-leaf rule at the last level.
-template <bool RECV>
-CUOT_DEV void bfs_levels(const AesLds& aes, const GgmKArgs& a, Lds& s, int64_t tree, int d0, int nlev,
+template <bool RECV, int NB>
+CUOT_DEV void bfs_levels(const AesLds& aes, const GgmKArgs& a, Lds<NB>& s, int64_t tree, int d0, int nlev,
                          const blk* ext, bool final_rule, int* punct_out) {
   const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
   int punct = 0;
   for (int r = 0; r < nlev; r++) {
-    const int w = 1 << r;
-    // each lane expands parents tid, tid+256, ... (at most 2 for 2^10 children)
-    blk lc[2], rc[2];
-    blk L = bzero(), R = bzero();
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const int j = tid + q * WG;
-      lc[q] = bzero();
-      rc[q] = bzero();
-      if (j < w) {
-        blk p = s.nodes[j];
-        ggm_expand(aes, a.rk, p, lc[q], rc[q]);
-        if (RECV && j == punct) {
-          lc[q] = bzero();
-          rc[q] = bzero();
-        }
-      }
-      L = bxor(L, lc[q]);
-      R = bxor(R, rc[q]);
-    }
-    wg_xor2(L, R, s.red);  // barrier inside: all reads of nodes[] are done
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const int j = tid + q * WG;
-      if (j < w) {
-        s.nodes[2 * j] = lc[q];
-        s.nodes[2 * j + 1] = rc[q];
-      }
-    }
+    const int w = 1 << r;  // at most WG parents (nlev <= MAXTOP)
     const int d = d0 + r;  // sum index: depth d+1
+    blk lc = bzero(), rc = bzero();
+    const bool own = tid < w && !(RECV && tid == punct);
+    if (own) ggm_expand(aes, a.rk, s.nodes[tid], lc, rc);
+    const uint32_t x = wave_xor2(lc, rc);
+    if (lane < 8) s.red[0][wave][bitrev3(lane)] = x;
+    __syncthreads();  // all reads of nodes[] are done
+    if (own) {
+      s.nodes[2 * tid] = lc;
+      s.nodes[2 * tid + 1] = rc;
+    }
     if (!RECV) {
-      if (tid == 0) {
-        s.sums[2 * d] = L;
-        s.sums[2 * d + 1] = R;
-      }
+      if (tid < 8) words(&s.sums[2 * d])[tid] = red_word(s, 0, tid);
     } else {
-      if (ext) {
-        L = bxor(L, ext[2 * r]);
-        R = bxor(R, ext[2 * r + 1]);
-      }
-      const int c = a.choice[tree * a.h + d] ? 1 : 0;
+      const int c = s.choice[d] ? 1 : 0;
       const int sib = 2 * punct + c;
       const int np = 2 * punct + (1 - c);
-      blk sibv = bxor(a.csum[tree * a.h + d], c ? R : L);
-      __syncthreads();
-      if (tid == 0) {
-        s.nodes[sib] = sibv;
-        if (final_rule && r == nlev - 1) {
-          blk f = a.fin[tree];
-          if (a.mode == CUOT_MODE_SOT) {
-            // silent/recver.cu:106-112 final layer: opposite-side sum
-            s.nodes[np] = bxor(f, c ? L : R);
-          } else {
-            // spcot_recver.h:56-63: all other leaves, LSB cleared, xor secret
-            s.nodes[np] = bxor(f, clear_lsb(bxor(bxor(L, R), sibv)));
+      if (tid < 8) {
+        // lanes 0..3: the sibling from the chosen side's sum; 4..7: the
+        // punctured node, zero until the last level closes it
+        const int i = tid & 3;
+        const int side = tid < 4 ? c : 1 - c;
+        uint32_t v = red_word(s, 0, 4 * side + i);
+        if (ext) v ^= ((const uint32_t*)&ext[2 * r + side])[i];
+        if (tid < 4) {
+          words(&s.nodes[sib])[i] = v ^ words(&s.csum[d])[i];
+        } else {
+          uint32_t f = 0;
+          if (final_rule && r == nlev - 1) {
+            f = ((const uint32_t*)&a.fin[tree])[i];
+            if (a.mode == CUOT_MODE_SOT) {
+              f ^= v;  // silent/recver.cu:106-112 final layer: opposite-side sum
+            } else {
+              // spcot_recver.h:56-63: all other leaves, LSB cleared, xor secret;
+              // the chosen side with the sibling is its chosen sum
+              uint32_t o = v ^ words(&s.csum[d])[i];
+              if (i == 0) o &= ~1u;
+              f ^= o;
+            }
           }
+          words(&s.nodes[np])[i] = f;
         }
       }
       punct = np;
@@ -147,10 +171,10 @@ CUOT_DEV void bfs_levels(const AesLds& aes, const GgmKArgs& a, Lds& s, int64_t t
 // node below it is a left child expanded on the spot.  All branches depend on
 // jj only, so they are uniform across the wave and every array index is
 // static after unrolling (no scratch).
-// Sums of this subtree are xored into sl/sr[1..L] only when `active`.
+// Sums of this subtree are xored into sl/sr[1..L].
 template <int L>
-CUOT_DEV void dfs_subtree(const AesLds& aes, const uint32_t* rk, blk root, bool active, blk* leaves,
-                          int64_t leaf0, int64_t n_out, bool ferret, blk* sl, blk* sr) {
+CUOT_DEV void dfs_subtree(const AesLds& aes, const uint32_t* rk, blk root, blk* leaves, int64_t leaf0,
+                          int64_t n_out, bool ferret, blk* sl, blk* sr) {
   blk rightc[L > 1 ? L : 1];
   const uint32_t npairs = 1u << (L - 1);
   for (uint32_t jj = 0; jj < npairs; jj++) {
@@ -165,46 +189,48 @@ CUOT_DEV void dfs_subtree(const AesLds& aes, const uint32_t* rk, blk root, bool 
         ggm_expand(aes, rk, cur, lc, rc);
         cur = lc;
         rightc[r] = rc;
-        sl[r] = bxor(sl[r], bsel(active, lc));
-        sr[r] = bxor(sr[r], bsel(active, rc));
+        sl[r] = bxor(sl[r], lc);
+        sr[r] = bxor(sr[r], rc);
       }
     }
     blk lf, rf;
     ggm_expand(aes, rk, cur, lf, rf);
-    sl[L] = bxor(sl[L], bsel(active, lf));
-    sr[L] = bxor(sr[L], bsel(active, rf));
-    if (active) {
-      const int64_t g = leaf0 + 2 * (int64_t)jj;
-      if (ferret) {
-        lf = clear_lsb(lf);
-        rf = clear_lsb(rf);
-      }
-      if (g < n_out) stb(leaves + g, lf);
-      if (g + 1 < n_out) stb(leaves + g + 1, rf);
+    sl[L] = bxor(sl[L], lf);
+    sr[L] = bxor(sr[L], rf);
+    const int64_t g = leaf0 + 2 * (int64_t)jj;
+    if (ferret) {
+      lf = clear_lsb(lf);
+      rf = clear_lsb(rf);
     }
+    if (g < n_out) stb(leaves + g, lf);
+    if (g + 1 < n_out) stb(leaves + g + 1, rf);
   }
 }
 
-template <int L, bool RECV>
-CUOT_DEV void ggm_tree(const GgmKArgs& a, Lds& s, int64_t tree) {
+template <int L, bool RECV, int NB>
+CUOT_DEV void ggm_tree(const GgmKArgs& a, Lds<NB>& s, int64_t tree) {
   const int tid = threadIdx.x;
+  const int h = a.h;
   aes_stage_table(s.aes, a.T0, tid, WG);
-  if (tid == 0) s.nodes[0] = RECV ? bzero() : a.roots[tree];
+  if (tid == 0) s.nodes[0] = RECV ? bzero() : ldb(a.roots + tree);
+  if (RECV && tid < h) {
+    s.csum[tid] = ldb(a.csum + tree * h + tid);
+    s.choice[tid] = a.choice[tree * h + tid];
+  }
   __syncthreads();
   const AesLds aes = aes_lds(s.aes);
-  const int h = a.h;
   const bool ferret = a.mode == CUOT_MODE_FERRET;
-  const int top = h - L;  // L == 0 iff h <= 8
+  const int top = h - L;
   int punct = 0;
   bfs_levels<RECV>(aes, a, s, tree, 0, top, nullptr, L == 0, &punct);
   const int64_t tree0 = tree << h;
 
   if constexpr (L == 0) {
     // whole tree fits the top phase: write leaves from LDS
-    if (tid < (1 << h)) {
-      blk v = s.nodes[tid];
-      if (ferret && !(RECV && tid == punct)) v = clear_lsb(v);
-      const int64_t g = tree0 + tid;
+    for (int f = tid; f < (1 << h); f += WG) {
+      blk v = s.nodes[f];
+      if (ferret && !(RECV && f == punct)) v = clear_lsb(v);
+      const int64_t g = tree0 + f;
       if (g < a.n_out) stb(a.leaves + g, v);
     }
   } else {
@@ -215,21 +241,16 @@ CUOT_DEV void ggm_tree(const GgmKArgs& a, Lds& s, int64_t tree) {
       tl[r] = bzero();
       tr[r] = bzero();
     }
-    const int nf = 1 << (top - 8);  // frontier nodes per lane: 1, 2 or 4
-    for (int q = 0; q < nf; q++) {
-      const int f = tid + q * WG;
-      const bool active = !(RECV && f == punct);
-      dfs_subtree<L>(aes, a.rk, s.nodes[f], active, a.leaves, tree0 + ((int64_t)f << L), a.n_out, ferret, tl,
-                     tr);
-    }
+    for (int f = tid; f < (1 << top); f += WG)
+      if (!(RECV && f == punct))
+        dfs_subtree<L>(aes, a.rk, s.nodes[f], a.leaves, tree0 + ((int64_t)f << L), a.n_out, ferret, tl, tr);
 #pragma unroll
     for (int r = 1; r <= L; r++) {
-      wg_xor2(tl[r], tr[r], s.red);
-      if (tid == 0) {
-        s.sums[2 * (top + r - 1)] = tl[r];
-        s.sums[2 * (top + r - 1) + 1] = tr[r];
-      }
+      const uint32_t x = wave_xor2(tl[r], tr[r]);
+      if ((tid & 63) < 8) s.red[r - 1][tid >> 6][bitrev3(tid & 63)] = x;
     }
+    __syncthreads();
+    if (tid < 8 * L) words(&s.sums[2 * (top + (tid >> 3))])[tid & 7] = red_word(s, tid >> 3, tid & 7);
     __syncthreads();
     if constexpr (RECV) {
       // ---- phase C: rebuild the punctured depth-`top` subtree -------------
@@ -249,22 +270,28 @@ CUOT_DEV void ggm_tree(const GgmKArgs& a, Lds& s, int64_t tree) {
   }
   if constexpr (!RECV) {
     __syncthreads();
-    if (tid < 2 * h) a.sums[tree * 2 * h + tid] = s.sums[tid];
+    if (tid < 2 * h) stb(a.sums + tree * 2 * h + tid, s.sums[tid]);
   }
 }
 
-template <int L, bool RECV>
-__global__ __launch_bounds__(WG) void ggm_kernel(GgmKArgs a) {
-  __shared__ Lds s;
-  ggm_tree<L, RECV>(a, s, blockIdx.x);
+// nodes to hold: 2^10 only where the breadth-first top can reach it (h = 16
+// with L = 6, or a smaller L by the knob); the smaller form lets two
+// workgroups share a CU
+template <int L, bool RECV, int NB>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void ggm_kernel(GgmKArgs) {
+  __shared__ __align__(16) Lds<NB> s;
+  // the argument block read through its pointer: as a value the 88 round-key
+  // words are held across the subtree loop and spill
+  ggm_tree<L, RECV>(*(const GgmKArgs*)__builtin_amdgcn_kernarg_segment_ptr(), s, blockIdx.x);
 }
 
 // Batch: one WG per tree of every instance in the table; start[i] is the first
-// global tree of instance i (start[ninst] = total).  All instances share L.
-template <int L, bool RECV>
-__global__ __launch_bounds__(WG) void ggm_batch_kernel(const GgmKArgs* __restrict__ tab,
-                                                       const int64_t* __restrict__ start, int ninst) {
-  __shared__ Lds s;
+// global tree of instance i (start[ninst] = total).  All instances share the
+// form (L and the node array's size).
+template <int L, bool RECV, int NB>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void ggm_batch_kernel(
+    const GgmKArgs* __restrict__ tab, const int64_t* __restrict__ start, int ninst) {
+  __shared__ __align__(16) Lds<NB> s;
   const int64_t g = blockIdx.x;
   int lo = 0, hi = ninst - 1;  // last i with start[i] <= g
   while (lo < hi) {
@@ -277,32 +304,48 @@ __global__ __launch_bounds__(WG) void ggm_batch_kernel(const GgmKArgs* __restric
   ggm_tree<L, RECV>(tab[lo], s, g - start[lo]);
 }
 
+// Depth-first levels L per lane.  Every lane of the workgroup has a subtree from
+// depth 9 on, so L = h - 9 (the knob may ask for the neighbouring splits);
+// depth 16 keeps L = 6 for the registers and puts two subtrees on a lane.
 int ggm_split(int h) {
-  if (h <= 8) return 0;
   const int k = cuot_knobs().ggm_dfs;
   const int hi = h - 8 < LMAX ? h - 8 : LMAX;
   if (k >= 1 && k <= hi && h - k <= MAXTOP) return k;
-  return hi;
+  if (h <= 9) return 0;
+  return h - 9 < LMAX ? h - 9 : LMAX;
+}
+
+// L, plus 16 when the breadth-first top is deeper than 2^9 nodes
+int ggm_form(int h) {
+  const int L = ggm_split(h);
+  return L + (h - L > 9 ? 16 : 0);
 }
 
 template <bool RECV>
 hipError_t launch_ggm(const GgmKArgs& a, hipStream_t st) {
-  const int L = ggm_split(a.h);
   dim3 grid((unsigned)a.t), block(WG);
   const int64_t nl = (a.t << a.h) < a.n_out ? (a.t << a.h) : a.n_out;
   cuot_rec_begin(st, RECV ? "ggm_kernel<recv>" : "ggm_kernel<send>", 16.0 * (double)nl);
-  switch (L) {
-#define CUOT_GGM_CASE(X) \
-  case X:                \
-    hipLaunchKernelGGL((ggm_kernel<X, RECV>), grid, block, 0, st, a); \
+  switch (ggm_form(a.h)) {
+#define CUOT_GGM_CASE(X, NB)                                              \
+  case X + (NB > 512 ? 16 : 0):                                           \
+    hipLaunchKernelGGL((ggm_kernel<X, RECV, NB>), grid, block, 0, st, a); \
     break;
-    CUOT_GGM_CASE(0)
-    CUOT_GGM_CASE(1)
-    CUOT_GGM_CASE(2)
-    CUOT_GGM_CASE(3)
-    CUOT_GGM_CASE(4)
-    CUOT_GGM_CASE(5)
-    CUOT_GGM_CASE(6)
+#define CUOT_GGM_CASES   \
+  CUOT_GGM_CASE(0, 512)  \
+  CUOT_GGM_CASE(1, 512)  \
+  CUOT_GGM_CASE(2, 512)  \
+  CUOT_GGM_CASE(3, 512)  \
+  CUOT_GGM_CASE(4, 512)  \
+  CUOT_GGM_CASE(5, 512)  \
+  CUOT_GGM_CASE(6, 512)  \
+  CUOT_GGM_CASE(1, 1024) \
+  CUOT_GGM_CASE(2, 1024) \
+  CUOT_GGM_CASE(3, 1024) \
+  CUOT_GGM_CASE(4, 1024) \
+  CUOT_GGM_CASE(5, 1024) \
+  CUOT_GGM_CASE(6, 1024)
+    CUOT_GGM_CASES
 #undef CUOT_GGM_CASE
     default:
       cuot_rec_end(st);
@@ -313,22 +356,17 @@ hipError_t launch_ggm(const GgmKArgs& a, hipStream_t st) {
 }
 
 template <bool RECV>
-hipError_t launch_ggm_batch(const GgmKArgs* tab, const int64_t* start, int ninst, int64_t total, int L,
+hipError_t launch_ggm_batch(const GgmKArgs* tab, const int64_t* start, int ninst, int64_t total, int form,
                             hipStream_t st) {
   dim3 grid((unsigned)total), block(WG);
-  switch (L) {
-#define CUOT_GGM_CASE(X) \
-  case X:                \
-    hipLaunchKernelGGL((ggm_batch_kernel<X, RECV>), grid, block, 0, st, tab, start, ninst); \
+  switch (form) {
+#define CUOT_GGM_CASE(X, NB)                                                                    \
+  case X + (NB > 512 ? 16 : 0):                                                                 \
+    hipLaunchKernelGGL((ggm_batch_kernel<X, RECV, NB>), grid, block, 0, st, tab, start, ninst); \
     break;
-    CUOT_GGM_CASE(0)
-    CUOT_GGM_CASE(1)
-    CUOT_GGM_CASE(2)
-    CUOT_GGM_CASE(3)
-    CUOT_GGM_CASE(4)
-    CUOT_GGM_CASE(5)
-    CUOT_GGM_CASE(6)
+    CUOT_GGM_CASES
 #undef CUOT_GGM_CASE
+#undef CUOT_GGM_CASES
     default:
       return hipErrorInvalidValue;
   }
@@ -337,15 +375,15 @@ hipError_t launch_ggm_batch(const GgmKArgs* tab, const int64_t* start, int ninst
 
 }  // namespace
 
-int cuot_ggm_split(int h) { return ggm_split(h); }
+int cuot_ggm_form(int h) { return ggm_form(h); }
 
 hipError_t cuot_launch_ggm(const GgmKArgs& a, bool receiver, hipStream_t st) {
   return receiver ? launch_ggm<true>(a, st) : launch_ggm<false>(a, st);
 }
 
 hipError_t cuot_launch_ggm_batch(const GgmKArgs* tab_d, const int64_t* start_d, int ninst, int64_t total_trees,
-                                 int L, bool receiver, hipStream_t st) {
+                                 int form, bool receiver, hipStream_t st) {
   if (ninst < 1 || total_trees < 1 || total_trees > 0x7fffffff) return hipErrorInvalidValue;
-  return receiver ? launch_ggm_batch<true>(tab_d, start_d, ninst, total_trees, L, st)
-                  : launch_ggm_batch<false>(tab_d, start_d, ninst, total_trees, L, st);
+  return receiver ? launch_ggm_batch<true>(tab_d, start_d, ninst, total_trees, form, st)
+                  : launch_ggm_batch<false>(tab_d, start_d, ninst, total_trees, form, st);
 }

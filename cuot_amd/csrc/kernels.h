@@ -5,7 +5,7 @@
 
 #include "common.h"
 
-// GGM expansion of t trees of depth h (one 256-lane workgroup per tree).
+// GGM expansion of t trees of depth h (one 512-lane workgroup per tree).
 struct GgmKArgs {
   const uint32_t* T0;    // AES T-table in global memory
   uint32_t rk[88];       // key-0 then key-1 AES-128 schedules (little-endian words)
@@ -21,12 +21,12 @@ struct GgmKArgs {
   const blk* fin;        // receiver: [t] SOT final-row value / Ferret secret sum
 };
 hipError_t cuot_launch_ggm(const GgmKArgs& a, bool receiver, hipStream_t st);
-// depth handled per lane below the shared top levels (trees of depth h)
-int cuot_ggm_split(int h);
-// batch of instances with the same cuot_ggm_split(h) == L and role; tab_d and
+// kernel form of trees of depth h (instances of one form share a launch)
+int cuot_ggm_form(int h);
+// batch of instances with the same cuot_ggm_form(h) and role; tab_d and
 // start_d (ninst + 1 prefix of tree counts) in device memory
 hipError_t cuot_launch_ggm_batch(const GgmKArgs* tab_d, const int64_t* start_d, int ninst, int64_t total_trees,
-                                 int L, bool receiver, hipStream_t st);
+                                 int form, bool receiver, hipStream_t st);
 
 // AES-128 ECB / CTR streams.  T0: device AES table (cuot_device_T0()).
 const uint32_t* cuot_device_T0();

@@ -23,11 +23,15 @@ namespace {
 
 constexpr int D = 10;
 
-// The gathers miss L2 and wait on the last-level cache, so residency
-// matters: computing each index AES block just before the first row that
-// reads it brought the kernel from 256 VGPRs (one wave per SIMD) to ~157
-// (three).
-
+// Two lanes share a __compute4 group: with both roles in one launch the lane's
+// parity is its role, each lane computes five of the group's ten AES blocks and
+// takes the other's index words from its neighbour; with one role the parity
+// picks two of the four rows.  The gathers miss L2 and wait on the last-level
+// cache, so what counts is how many are in flight and how many cache lines an
+// instruction touches: a pair's two 16-byte reads of the interleaved table fall
+// into one line of one instruction (a lane reading both took two instructions
+// per line), and at ~110 registers four waves fit a SIMD (three at ~157).
+// n = 10,168,320, both roles: 1.68 -> 1.31 ms.
 struct LpnKArgs {
   const uint32_t* T0;
   uint32_t rk[44];
@@ -37,6 +41,7 @@ struct LpnKArgs {
   int ntasks;
   int64_t units_per_task;  // units of a full-width task
   int64_t units_total;
+  int64_t wg_units;  // batch: units per workgroup
   const blk* noise[2];
   const blk* kk[2];
   const blk* kkp;  // both roles' kk interleaved (kkp[2j], kkp[2j+1]) or NULL
@@ -44,116 +49,131 @@ struct LpnKArgs {
   int nroles;
 };
 
-// kk gathers: with the interleaved table one 32-byte read serves both roles
-template <int NR>
-CUOT_DEV void gather_kk(const LpnKArgs& a, uint32_t idx, blk* acc) {
-  if (NR == 2 && a.kkp) {
-    const blk* p = a.kkp + 2 * (int64_t)idx;
-    acc[0] = bxor(acc[0], p[0]);
-    acc[NR - 1] = bxor(acc[NR - 1], p[1]);
-  } else {
-#pragma unroll
-    for (int rr = 0; rr < NR; rr++) acc[rr] = bxor(acc[rr], a.kk[rr][idx]);
-  }
-}
-
 // number of __compute4 groups and __compute1 rows of a task of `rows` rows
 CUOT_DEV void task_shape(int64_t rows, int64_t& g4, int64_t& t1) {
   g4 = rows > 4 ? (rows - 4 + 3) / 4 : 0;
   t1 = rows - 4 * g4;
 }
 
+// One role's view of the table: block idx of the lane's role is p[idx << sh].
+struct KkView {
+  const blk* p;
+  int sh;
+};
+
+CUOT_DEV void lpn_gather(const KkView& v, uint32_t idx, blk& acc) {
+  acc = bxor(acc, ldb(v.p + ((uint64_t)idx << v.sh)));
+}
+
+// w & mask, minus k if >= k (mask < 2k, so one subtraction is enough and the
+// wrapped difference of a smaller value is the larger number)
+CUOT_DEV uint32_t lpn_idx(const LpnKArgs& a, uint32_t w) {
+  const uint32_t x = w & a.mask, y = x - (uint32_t)a.k;
+  return x < y ? x : y;
+}
+
+// the word of the pair's lane SRC (0 or 1), in both lanes
+template <int SRC>
+CUOT_DEV uint32_t pair_word(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, SRC ? 0xf5 : 0xa0, 0xf, 0xf, true);  // quad [0,0,2,2] or [1,1,3,3]
+}
+
+// unit u on the lane pair (lane & 1 = par): a __compute4 group of four rows or
+// one __compute1 row.  Both lanes of a pair take the same branches.
 template <int NR>
-CUOT_DEV void lpn_unit(const AesLds& aes, const LpnKArgs& a, int64_t u) {
+CUOT_DEV void lpn_unit(const AesLds& aes, const LpnKArgs& a, int64_t u, int par) {
   // locate the task and the unit inside it
-  int64_t task = u / a.units_per_task;
-  if (task >= a.ntasks) task = a.ntasks - 1;
+  int64_t task = 0;
+  if (a.ntasks > 1) {
+    task = u / a.units_per_task;
+    if (task >= a.ntasks) task = a.ntasks - 1;
+  }
   const int64_t start = task * a.width;
   const int64_t end = (task == a.ntasks - 1) ? a.n : start + a.width;
   const int64_t lu = u - task * a.units_per_task;
   int64_t g4, t1;
   task_shape(end - start, g4, t1);
+  const int role = NR == 2 ? par : 0;
+  KkView kk;
+  if (NR == 2 && a.kkp) {
+    kk.p = a.kkp + role;
+    kk.sh = 1;
+  } else {
+    kk.p = a.kk[role];
+    kk.sh = 0;
+  }
+  const blk* noise = a.noise[role];
+  blk* out = a.out[role];
   if (lu < g4) {
     const int64_t i = start + 4 * lu;
-    uint32_t w[4 * D];
-    // row q takes words 10q..10q+9, i.e. AES blocks 10q/4 .. (10q+9)/4: each
-    // block is computed just before the first row that reads it
-    auto block = [&](int m) {
-      blk c = make_uint4((uint32_t)m, 0u, (uint32_t)i, (uint32_t)((uint64_t)i >> 32));
-      blk e = aes_enc(aes, a.rk, c);
-      w[4 * m + 0] = e.x;
-      w[4 * m + 1] = e.y;
-      w[4 * m + 2] = e.z;
-      w[4 * m + 3] = e.w;
-    };
-    auto row = [&](int q) {
-      blk acc[NR];
+    // this lane's five blocks: words 20 par .. 20 par + 19 of the group, the
+    // indices of rows 2 par and 2 par + 1
+    uint32_t w[2 * D];
 #pragma unroll
-      for (int rr = 0; rr < NR; rr++) acc[rr] = a.noise[rr][i + q];
+    for (int m = 0; m < 5; m++) {
+      const blk c = make_uint4((uint32_t)(m + 5 * par), 0u, (uint32_t)i, (uint32_t)((uint64_t)i >> 32));
+      const blk e = aes_enc(aes, a.rk, c);
+      w[4 * m + 0] = lpn_idx(a, e.x);
+      w[4 * m + 1] = lpn_idx(a, e.y);
+      w[4 * m + 2] = lpn_idx(a, e.z);
+      w[4 * m + 3] = lpn_idx(a, e.w);
+    }
+    constexpr int NROW = NR == 2 ? 4 : 2;
+    const int64_t r0 = NR == 2 ? i : i + 2 * par;
+    blk acc[NROW];
+#pragma unroll
+    for (int q = 0; q < NROW; q++) acc[q] = ldb(noise + r0 + q);
+#pragma unroll
+    for (int q = 0; q < NROW; q++) {
 #pragma unroll
       for (int j = 0; j < D; j++) {
-        uint32_t idx = w[q * D + j] & a.mask;
-        if (idx >= (uint32_t)a.k) idx -= (uint32_t)a.k;
-        gather_kk<NR>(a, idx, acc);
+        const uint32_t v = w[(q & 1) * D + j];
+        lpn_gather(kk, NR == 1 ? v : (q < 2 ? pair_word<0>(v) : pair_word<1>(v)), acc[q]);
       }
+    }
 #pragma unroll
-      for (int rr = 0; rr < NR; rr++) a.out[rr][i + q] = acc[rr];
-    };
-    block(0);
-    block(1);
-    block(2);
-    row(0);
-    block(3);
-    block(4);
-    row(1);
-    block(5);
-    block(6);
-    block(7);
-    row(2);
-    block(8);
-    block(9);
-    row(3);
+    for (int q = 0; q < NROW; q++) stb(out + r0 + q, acc[q]);
   } else if (lu - g4 < t1) {
     const int64_t i = start + 4 * g4 + (lu - g4);
     uint32_t w[12];
 #pragma unroll
     for (int m = 0; m < 3; m++) {
-      blk c = make_uint4((uint32_t)m, 0u, (uint32_t)i, (uint32_t)((uint64_t)i >> 32));
-      blk e = aes_enc(aes, a.rk, c);
+      const blk c = make_uint4((uint32_t)m, 0u, (uint32_t)i, (uint32_t)((uint64_t)i >> 32));
+      const blk e = aes_enc(aes, a.rk, c);
       w[4 * m + 0] = e.x;
       w[4 * m + 1] = e.y;
       w[4 * m + 2] = e.z;
       w[4 * m + 3] = e.w;
     }
-    blk acc[NR];
+    if (NR == 1 && par) return;  // one row, one role: the even lane's
+    blk acc = ldb(noise + i);
 #pragma unroll
-    for (int rr = 0; rr < NR; rr++) acc[rr] = a.noise[rr][i];
-#pragma unroll
-    for (int j = 0; j < D; j++) {
-      const uint32_t idx = w[j] % (uint32_t)a.k;
-      gather_kk<NR>(a, idx, acc);
-    }
-#pragma unroll
-    for (int rr = 0; rr < NR; rr++) a.out[rr][i] = acc[rr];
+    for (int j = 0; j < D; j++) lpn_gather(kk, w[j] % (uint32_t)a.k, acc);
+    stb(out + i, acc);
   }
 }
 
+constexpr int LPN_UNITS = CUOT_AES_WG / 2;  // units per workgroup pass
+constexpr int LPN_BATCH_PASSES = 4;         // batch: passes per workgroup (one table fill for all)
+
 template <int NR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void lpn_kernel(LpnKArgs a) {
-  __shared__ uint32_t tab[CUOT_AES_LDS_WORDS];
-  aes_stage_table(tab, a.T0, threadIdx.x, 256);
+__global__ __launch_bounds__(CUOT_AES_WG) __attribute__((amdgpu_waves_per_eu(4))) void lpn_kernel(LpnKArgs a) {
+  __shared__ __align__(16) uint32_t tab[CUOT_AES_LDS_WORDS];
+  aes_stage_table(tab, a.T0, threadIdx.x, CUOT_AES_WG);
   __syncthreads();
   const AesLds aes = aes_lds(tab);
-  const int64_t stride = (int64_t)gridDim.x * 256;
-  for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < a.units_total; u += stride) lpn_unit<NR>(aes, a, u);
+  const int64_t stride = (int64_t)gridDim.x * LPN_UNITS;
+  for (int64_t u = (int64_t)blockIdx.x * LPN_UNITS + (threadIdx.x >> 1); u < a.units_total; u += stride)
+    lpn_unit<NR>(aes, a, u, threadIdx.x & 1);
 }
 
-// Batch: wg_start[i] = first WG of instance i (prefix of ceil(units / 256));
-// one WG covers 256 units of a single instance, so the round keys stay uniform.
+// Batch: wg_start[i] = first WG of instance i (prefix of ceil(units / wg_units));
+// one WG covers wg_units units of a single instance, so the round keys stay
+// uniform.
 template <int NR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void lpn_batch_kernel(const LpnKArgs* __restrict__ tabs,
-                                                        const int64_t* __restrict__ wg_start, int ninst) {
-  __shared__ uint32_t tab[CUOT_AES_LDS_WORDS];
+__global__ __launch_bounds__(CUOT_AES_WG) __attribute__((amdgpu_waves_per_eu(4))) void lpn_batch_kernel(
+    const LpnKArgs* __restrict__ tabs, const int64_t* __restrict__ wg_start, int ninst) {
+  __shared__ __align__(16) uint32_t tab[CUOT_AES_LDS_WORDS];
   const int64_t g = blockIdx.x;
   int lo = 0, hi = ninst - 1;
   while (lo < hi) {
@@ -164,11 +184,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void l
       hi = mid - 1;
   }
   const LpnKArgs& a = tabs[lo];
-  aes_stage_table(tab, a.T0, threadIdx.x, 256);
+  aes_stage_table(tab, a.T0, threadIdx.x, CUOT_AES_WG);
   __syncthreads();
   const AesLds aes = aes_lds(tab);
-  const int64_t u = (g - wg_start[lo]) * 256 + threadIdx.x;
-  if (u < a.units_total) lpn_unit<NR>(aes, a, u);
+  const int64_t u0 = (g - wg_start[lo]) * a.wg_units;
+  const int64_t u1 = u0 + a.wg_units < a.units_total ? u0 + a.wg_units : a.units_total;
+  for (int64_t u = u0 + (threadIdx.x >> 1); u < u1; u += LPN_UNITS) lpn_unit<NR>(aes, a, u, threadIdx.x & 1);
 }
 
 int64_t units_of(int64_t rows) {
@@ -198,6 +219,9 @@ bool fill_args(const LpnLaunch& l, LpnKArgs& a) {
   // full-width tasks then the last one; the kernel maps u -> task by division,
   // so the last task's units start at (ntasks-1)*units_per_task
   a.units_total = (int64_t)(a.ntasks - 1) * a.units_per_task + units_of(last_rows);
+  // batch: several passes per table fill once an instance has work for many
+  // workgroups; a small one spreads its units over as many as it can
+  a.wg_units = a.units_total >= (int64_t)512 * LPN_UNITS * LPN_BATCH_PASSES ? LPN_UNITS * LPN_BATCH_PASSES : LPN_UNITS;
   a.nroles = l.nroles;
   for (int r = 0; r < l.nroles; r++) {
     a.noise[r] = l.noise[r];
@@ -214,16 +238,16 @@ hipError_t cuot_launch_lpn(const LpnLaunch& l, hipStream_t st) {
   if (l.n <= 0) return hipSuccess;
   LpnKArgs a;
   if (!fill_args(l, a)) return hipErrorInvalidValue;
-  int64_t g = (a.units_total + 255) / 256;
-  const int64_t cap = cuot_knobs().lpn_wgs > 0 ? cuot_knobs().lpn_wgs : 8192;
+  int64_t g = (a.units_total + LPN_UNITS - 1) / LPN_UNITS;
+  const int64_t cap = cuot_knobs().lpn_wgs > 0 ? cuot_knobs().lpn_wgs : 2048;
   if (g > cap) g = cap;
   if (g < 1) g = 1;
   // algorithmic bytes per role and row: noise in, d gathers, row out
   cuot_rec_begin(st, "lpn_kernel", 16.0 * (D + 2) * (double)l.n * l.nroles);
   if (l.nroles == 2)
-    hipLaunchKernelGGL(lpn_kernel<2>, dim3((unsigned)g), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(lpn_kernel<2>, dim3((unsigned)g), dim3(CUOT_AES_WG), 0, st, a);
   else
-    hipLaunchKernelGGL(lpn_kernel<1>, dim3((unsigned)g), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(lpn_kernel<1>, dim3((unsigned)g), dim3(CUOT_AES_WG), 0, st, a);
   cuot_rec_end(st);
   return hipGetLastError();
 }
@@ -234,17 +258,17 @@ int64_t cuot_lpn_args_fill(const LpnLaunch& l, void* out) {
   LpnKArgs a;
   if (!fill_args(l, a)) return -1;
   memcpy(out, &a, sizeof(a));
-  return (a.units_total + 255) / 256;
+  return (a.units_total + a.wg_units - 1) / a.wg_units;
 }
 
 hipError_t cuot_launch_lpn_batch(const void* tabs_d, const int64_t* wg_start_d, int ninst, int64_t total_wgs,
                                  int nroles, hipStream_t st) {
   if (ninst < 1 || total_wgs < 1 || total_wgs > 0x7fffffff) return hipErrorInvalidValue;
   if (nroles == 2)
-    hipLaunchKernelGGL(lpn_batch_kernel<2>, dim3((unsigned)total_wgs), dim3(256), 0, st, (const LpnKArgs*)tabs_d,
+    hipLaunchKernelGGL(lpn_batch_kernel<2>, dim3((unsigned)total_wgs), dim3(CUOT_AES_WG), 0, st, (const LpnKArgs*)tabs_d,
                        wg_start_d, ninst);
   else
-    hipLaunchKernelGGL(lpn_batch_kernel<1>, dim3((unsigned)total_wgs), dim3(256), 0, st, (const LpnKArgs*)tabs_d,
+    hipLaunchKernelGGL(lpn_batch_kernel<1>, dim3((unsigned)total_wgs), dim3(CUOT_AES_WG), 0, st, (const LpnKArgs*)tabs_d,
                        wg_start_d, ninst);
   return hipGetLastError();
 }

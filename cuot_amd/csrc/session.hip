@@ -48,9 +48,9 @@ CUOT_DEV blk ccrh(const AesLds& aes, const uint32_t* rk, blk x) {
   return bxor(aes_enc(aes, rk, s), s);
 }
 
-__global__ __launch_bounds__(256) void ccrh_pre_kernel(CcrhArgs a) {
-  __shared__ uint32_t tab[CUOT_AES_LDS_WORDS];
-  aes_stage_table(tab, a.T0, threadIdx.x, 256);
+__global__ __launch_bounds__(CUOT_AES_WG) void ccrh_pre_kernel(CcrhArgs a) {
+  __shared__ __align__(16) uint32_t tab[CUOT_AES_LDS_WORDS];
+  aes_stage_table(tab, a.T0, threadIdx.x, CUOT_AES_WG);
   __syncthreads();
   const AesLds aes = aes_lds(tab);
   const blk D = *a.delta;
@@ -155,13 +155,13 @@ hipError_t extend_seed(cuot_ferret_session* s, blk* out_s, blk* out_r, hipStream
   c.boot = s->boot_s;
   c.out0 = s->P0;
   c.out1 = s->P1;
-  hipLaunchKernelGGL(ccrh_pre_kernel, dim3(grid_of(s->npre)), dim3(256), 0, st, c);
+  hipLaunchKernelGGL(ccrh_pre_kernel, dim3(cuot_aes_grid(s->npre)), dim3(CUOT_AES_WG), 0, st, c);
   c.recv = 1;
   c.boot = s->boot_r;
   c.out0 = s->Pr;
   c.out1 = nullptr;
   c.bits = s->bits;
-  hipLaunchKernelGGL(ccrh_pre_kernel, dim3(grid_of(s->npre)), dim3(256), 0, st, c);
+  hipLaunchKernelGGL(ccrh_pre_kernel, dim3(cuot_aes_grid(s->npre)), dim3(CUOT_AES_WG), 0, st, c);
   if ((e = hipGetLastError())) return e;
   // 2. sender MPCOT
   uint32_t rk_seed[44];
