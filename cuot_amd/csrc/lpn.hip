@@ -23,6 +23,7 @@ namespace {
 
 constexpr int D = 10;
 
+
 // Two lanes share a __compute4 group: with both roles in one launch the lane's
 // parity is its role, each lane computes five of the group's ten AES blocks and
 // takes the other's index words from its neighbour; with one role the parity
@@ -42,6 +43,7 @@ struct LpnKArgs {
   int64_t units_per_task;  // units of a full-width task
   int64_t units_total;
   int64_t wg_units;  // batch: units per workgroup
+  uint32_t lo, cnt;  // rows of the table this launch covers (cnt = 0: all, through pointers)
   const blk* noise[2];
   const blk* kk[2];
   const blk* kkp;  // both roles' kk interleaved (kkp[2j], kkp[2j+1]) or NULL
@@ -55,14 +57,26 @@ CUOT_DEV void task_shape(int64_t rows, int64_t& g4, int64_t& t1) {
   t1 = rows - 4 * g4;
 }
 
-// One role's view of the table: block idx of the lane's role is p[idx << sh].
+// One role's view of a slice of the table.  With a uniform base (BUF) the slice
+// is a buffer descriptor: a row outside it reads as zero, so a launch that
+// covers part of the table takes no branch per gather.  Else block idx of the
+// lane's role is p[idx].
+template <bool BUF>
 struct KkView {
   const blk* p;
+  __amdgpu_buffer_rsrc_t rs;
+  uint32_t add;  // byte offset (idx << sh) + add, modulo 2^32
   int sh;
 };
 
-CUOT_DEV void lpn_gather(const KkView& v, uint32_t idx, blk& acc) {
-  acc = bxor(acc, ldb(v.p + ((uint64_t)idx << v.sh)));
+template <bool BUF>
+CUOT_DEV void lpn_gather(const KkView<BUF>& v, uint32_t idx, blk& acc) {
+  if constexpr (BUF) {
+    const blk_vec x = __builtin_amdgcn_raw_buffer_load_b128(v.rs, (int)((idx << v.sh) + v.add), 0, 0);
+    acc = bxor(acc, make_uint4(x.x, x.y, x.z, x.w));
+  } else {
+    acc = bxor(acc, ldb(v.p + idx));
+  }
 }
 
 // w & mask, minus k if >= k (mask < 2k, so one subtraction is enough and the
@@ -80,7 +94,7 @@ CUOT_DEV uint32_t pair_word(uint32_t v) {
 
 // unit u on the lane pair (lane & 1 = par): a __compute4 group of four rows or
 // one __compute1 row.  Both lanes of a pair take the same branches.
-template <int NR>
+template <int NR, bool BUF>
 CUOT_DEV void lpn_unit(const AesLds& aes, const LpnKArgs& a, int64_t u, int par) {
   // locate the task and the unit inside it
   int64_t task = 0;
@@ -94,13 +108,16 @@ CUOT_DEV void lpn_unit(const AesLds& aes, const LpnKArgs& a, int64_t u, int par)
   int64_t g4, t1;
   task_shape(end - start, g4, t1);
   const int role = NR == 2 ? par : 0;
-  KkView kk;
-  if (NR == 2 && a.kkp) {
-    kk.p = a.kkp + role;
-    kk.sh = 1;
+  KkView<BUF> kk;
+  if constexpr (BUF) {
+    // kkp (two roles interleaved) or kk[0] (one role), rows [lo, lo + cnt)
+    const int rb = NR == 2 ? 32 : 16;
+    const char* base = (const char*)(NR == 2 ? a.kkp : a.kk[0]);
+    kk.rs = __builtin_amdgcn_make_buffer_rsrc((void*)(base + (int64_t)a.lo * rb), 0, (int)(a.cnt * rb), 0x00020000);
+    kk.sh = NR == 2 ? 5 : 4;
+    kk.add = (uint32_t)(16 * role) - a.lo * (uint32_t)rb;
   } else {
     kk.p = a.kk[role];
-    kk.sh = 0;
   }
   const blk* noise = a.noise[role];
   blk* out = a.out[role];
@@ -156,7 +173,7 @@ CUOT_DEV void lpn_unit(const AesLds& aes, const LpnKArgs& a, int64_t u, int par)
 constexpr int LPN_UNITS = CUOT_AES_WG / 2;  // units per workgroup pass
 constexpr int LPN_BATCH_PASSES = 4;         // batch: passes per workgroup (one table fill for all)
 
-template <int NR>
+template <int NR, bool BUF>
 __global__ __launch_bounds__(CUOT_AES_WG) __attribute__((amdgpu_waves_per_eu(4))) void lpn_kernel(LpnKArgs a) {
   __shared__ __align__(16) uint32_t tab[CUOT_AES_LDS_WORDS];
   aes_stage_table(tab, a.T0, threadIdx.x, CUOT_AES_WG);
@@ -164,7 +181,7 @@ __global__ __launch_bounds__(CUOT_AES_WG) __attribute__((amdgpu_waves_per_eu(4))
   const AesLds aes = aes_lds(tab);
   const int64_t stride = (int64_t)gridDim.x * LPN_UNITS;
   for (int64_t u = (int64_t)blockIdx.x * LPN_UNITS + (threadIdx.x >> 1); u < a.units_total; u += stride)
-    lpn_unit<NR>(aes, a, u, threadIdx.x & 1);
+    lpn_unit<NR, BUF>(aes, a, u, threadIdx.x & 1);
 }
 
 // Batch: wg_start[i] = first WG of instance i (prefix of ceil(units / wg_units));
@@ -189,7 +206,11 @@ __global__ __launch_bounds__(CUOT_AES_WG) __attribute__((amdgpu_waves_per_eu(4))
   const AesLds aes = aes_lds(tab);
   const int64_t u0 = (g - wg_start[lo]) * a.wg_units;
   const int64_t u1 = u0 + a.wg_units < a.units_total ? u0 + a.wg_units : a.units_total;
-  for (int64_t u = u0 + (threadIdx.x >> 1); u < u1; u += LPN_UNITS) lpn_unit<NR>(aes, a, u, threadIdx.x & 1);
+  if (a.cnt) {
+    for (int64_t u = u0 + (threadIdx.x >> 1); u < u1; u += LPN_UNITS) lpn_unit<NR, true>(aes, a, u, threadIdx.x & 1);
+  } else {
+    for (int64_t u = u0 + (threadIdx.x >> 1); u < u1; u += LPN_UNITS) lpn_unit<NR, false>(aes, a, u, threadIdx.x & 1);
+  }
 }
 
 int64_t units_of(int64_t rows) {
@@ -223,6 +244,11 @@ bool fill_args(const LpnLaunch& l, LpnKArgs& a) {
   // workgroups; a small one spreads its units over as many as it can
   a.wg_units = a.units_total >= (int64_t)512 * LPN_UNITS * LPN_BATCH_PASSES ? LPN_UNITS * LPN_BATCH_PASSES : LPN_UNITS;
   a.nroles = l.nroles;
+  // a slice is addressed by 32-bit byte offsets from a uniform base: one role's
+  // table, or both interleaved; other tables go through the lanes' pointers
+  a.lo = 0;
+  a.cnt = 0;
+  if ((l.nroles == 2 ? l.kkp != nullptr : true) && l.k * 16 * l.nroles < ((int64_t)1 << 32)) a.cnt = (uint32_t)l.k;
   for (int r = 0; r < l.nroles; r++) {
     a.noise[r] = l.noise[r];
     a.kk[r] = l.kk[r];
@@ -230,6 +256,18 @@ bool fill_args(const LpnLaunch& l, LpnKArgs& a) {
     a.out[r] = l.out[r];
   }
   return true;
+}
+
+// Launches that each gather from one slice of the table, adding to what the
+// one before left in out.  The gathers are bound by their L2 misses: whatever
+// the issue rate, ~57e9 lines/s arrive from the last-level cache, and a table
+// of T MB hits an XCD's 4 MB L2 about 4/T of the time.  Halving the table takes
+// the index AES twice (0.4 ms at n = 10,168,320, both roles) and pays from
+// about 11 MB on: k = 262,144 (8 MB) 1.03 ms whole, 1.07 in two; 327,680 (10 MB)
+// 1.14 / 1.13; 393,216 (12 MB) 1.24 / 1.16; 452,160 (14 MB) 1.32 / 1.22;
+// three slices lose everywhere (1.58 at 452,160).
+int lpn_slices(const LpnKArgs& a) {
+  return a.cnt && (int64_t)a.cnt * 16 * a.nroles > (11ll << 20) ? 2 : 1;
 }
 
 }  // namespace
@@ -244,10 +282,23 @@ hipError_t cuot_launch_lpn(const LpnLaunch& l, hipStream_t st) {
   if (g < 1) g = 1;
   // algorithmic bytes per role and row: noise in, d gathers, row out
   cuot_rec_begin(st, "lpn_kernel", 16.0 * (D + 2) * (double)l.n * l.nroles);
-  if (l.nroles == 2)
-    hipLaunchKernelGGL(lpn_kernel<2>, dim3((unsigned)g), dim3(CUOT_AES_WG), 0, st, a);
-  else
-    hipLaunchKernelGGL(lpn_kernel<1>, dim3((unsigned)g), dim3(CUOT_AES_WG), 0, st, a);
+  const int ns = lpn_slices(a);
+  for (int q = 0; q < ns; q++) {
+    if (a.cnt) {
+      a.lo = (uint32_t)(l.k * q / ns);
+      a.cnt = (uint32_t)(l.k * (q + 1) / ns) - a.lo;
+    }
+    if (q)
+      for (int r = 0; r < l.nroles; r++) a.noise[r] = l.out[r];
+    if (l.nroles == 2 && a.cnt)
+      hipLaunchKernelGGL((lpn_kernel<2, true>), dim3((unsigned)g), dim3(CUOT_AES_WG), 0, st, a);
+    else if (l.nroles == 2)
+      hipLaunchKernelGGL((lpn_kernel<2, false>), dim3((unsigned)g), dim3(CUOT_AES_WG), 0, st, a);
+    else if (a.cnt)
+      hipLaunchKernelGGL((lpn_kernel<1, true>), dim3((unsigned)g), dim3(CUOT_AES_WG), 0, st, a);
+    else
+      hipLaunchKernelGGL((lpn_kernel<1, false>), dim3((unsigned)g), dim3(CUOT_AES_WG), 0, st, a);
+  }
   cuot_rec_end(st);
   return hipGetLastError();
 }

@@ -32,3 +32,33 @@ def test_lpn_single_and_dual(ctx, n, k, ntasks):
     ctx.lpn_dual(_p(n, k, seed, ntasks), a, to_dev(kk), a, b, to_dev(kk2), b)
     assert np.array_equal(to_np(a)[:n], ref)
     assert np.array_equal(to_np(b)[:n], ref2)
+
+
+# tables above 11 MB are gathered in two slices (rows of the other slice read as
+# zero): one role at the limit and past it, both roles interleaved past it
+@pytest.mark.parametrize("n,k", [(4099, 720896), (4099, 720897), (3, 720897)])
+def test_lpn_table_slices_one_role(ctx, n, k):
+    print(f"lpn slices n={n} k={k}", flush=True)
+    r = rng(n + k)
+    seed = rand_blocks(r, 1)[0]
+    noise, kk = rand_blocks(r, n), rand_blocks(r, k)
+    ref = po.ferret_lpn(noise, kk, seed, ntasks=1, nthreads=4)
+    a = to_dev(noise)
+    ctx.lpn(_p(n, k, seed), a, to_dev(kk), a)
+    assert np.array_equal(to_np(a)[:n], ref)
+
+
+def test_lpn_table_slices_both_roles(ctx):
+    import torch
+
+    import cuot_amd
+
+    n, k, t, h = 380003, 370003, 47, 13
+    seed = np.array([77, 78], dtype=np.uint64)
+    cfg = cuot_amd.FerretConfig(n=n, k=k, t=t, h=h, ntasks=3, seed=cuot_amd.to_block(seed))
+    ws = torch.empty(ctx.ferret_workspace_bytes(cfg), dtype=torch.uint8, device="cuda")
+    s, w = dev_blocks(n), dev_blocks(n)
+    ctx.ferret_run(cfg, ws, s, w)
+    os_, or_, _ = po.ferret_run(n, k, t, h, seed, ntasks=3, nthreads=4)
+    assert np.array_equal(to_np(s), os_)
+    assert np.array_equal(to_np(w), or_)
