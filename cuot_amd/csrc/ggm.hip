@@ -72,6 +72,18 @@ CUOT_DEV uint32_t wave_xor2(blk a, blk b) {
   return r ^ lane_xor<32>(r);
 }
 
+// XOR of one block over a wavefront: lane l returns word bitreverse2(l & 3)
+CUOT_DEV uint32_t wave_xor1(blk a) {
+  const uint32_t lane = threadIdx.x;
+  const uint32_t k0 = ((lane & 1) ? a.z : a.x) ^ lane_xor<1>((lane & 1) ? a.x : a.z);
+  const uint32_t k1 = ((lane & 1) ? a.w : a.y) ^ lane_xor<1>((lane & 1) ? a.y : a.w);
+  uint32_t r = ((lane & 2) ? k1 : k0) ^ lane_xor<2>((lane & 2) ? k0 : k1);
+  r ^= lane_xor<4>(r);
+  r ^= lane_xor<8>(r);
+  r ^= lane_xor<16>(r);
+  return r ^ lane_xor<32>(r);
+}
+
 CUOT_DEV int bitrev3(int i) { return ((i & 1) << 2) | (i & 2) | ((i >> 2) & 1); }
 
 CUOT_DEV blk clear_lsb(blk v) {
@@ -101,7 +113,21 @@ CUOT_DEV uint32_t red_word(const Lds<NB>& s, int slot, int i) {
 
 CUOT_DEV uint32_t* words(blk* b) { return (uint32_t*)b; }
 
-// Breadth-first expansion in LDS of `nlev` levels below nodes[0].
+// word i (0..3) of one side's sum in a breadth-first level: waves 0..3 hold the
+// left children's XORs in red[0][wave][0..3], waves 4..7 the right ones'
+template <int NB>
+CUOT_DEV uint32_t side_word(const Lds<NB>& s, int side, int i) {
+  const int w0 = side * (NWAVE / 2);
+  uint32_t r = 0;
+#pragma unroll
+  for (int w = 0; w < NWAVE / 2; w++) r ^= s.red[0][w0 + w][i];
+  return r;
+}
+
+// Breadth-first expansion in LDS of `nlev` levels below nodes[0].  The lower
+// half of the workgroup computes left children (k0), the upper half right ones
+// (k1): a level is a serial chain of one AES and the LDS reads of a second one
+// on the same lane would lengthen every round of it.
 // Receiver mode resolves the sibling on the punctured path at each level
 // using chosen sums csum[d0 + r] and external (outside-LDS) side sums ext.
 // Returns the punctured index at the last level (receiver) in *punct_out.
@@ -109,24 +135,38 @@ CUOT_DEV uint32_t* words(blk* b) { return (uint32_t*)b; }
 template <bool RECV, int NB>
 CUOT_DEV void bfs_levels(const AesLds& aes, const GgmKArgs& a, Lds<NB>& s, int64_t tree, int d0, int nlev,
                          const blk* ext, bool final_rule, int* punct_out) {
+  constexpr int HALF = WG / 2;
+  constexpr int Q = NB / WG;  // parents per lane: at most NB / 2 parents in a level
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
+  const int side = __builtin_amdgcn_readfirstlane(tid / HALF);
+  const int j0 = tid % HALF;
+  const uint32_t* rk = a.rk + 44 * side;
   int punct = 0;
   for (int r = 0; r < nlev; r++) {
-    const int w = 1 << r;  // at most WG parents (nlev <= MAXTOP)
+    const int w = 1 << r;
     const int d = d0 + r;  // sum index: depth d+1
-    blk lc = bzero(), rc = bzero();
-    const bool own = tid < w && !(RECV && tid == punct);
-    if (own) ggm_expand(aes, a.rk, s.nodes[tid], lc, rc);
-    const uint32_t x = wave_xor2(lc, rc);
-    if (lane < 8) s.red[0][wave][bitrev3(lane)] = x;
+    blk ch[Q], sum = bzero();
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      const int j = j0 + q * HALF;
+      ch[q] = bzero();
+      if (j < w && !(RECV && j == punct)) {
+        const blk p = s.nodes[j];
+        ch[q] = bxor(aes_enc(aes, rk, p), p);
+      }
+      sum = bxor(sum, ch[q]);
+    }
+    const uint32_t x = wave_xor1(sum);
+    if (lane < 4) s.red[0][wave][((lane & 1) << 1) | (lane >> 1)] = x;
     __syncthreads();  // all reads of nodes[] are done
-    if (own) {
-      s.nodes[2 * tid] = lc;
-      s.nodes[2 * tid + 1] = rc;
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      const int j = j0 + q * HALF;
+      if (j < w && !(RECV && j == punct)) s.nodes[2 * j + side] = ch[q];
     }
     if (!RECV) {
-      if (tid < 8) words(&s.sums[2 * d])[tid] = red_word(s, 0, tid);
+      if (tid < 8) words(&s.sums[2 * d])[tid] = side_word(s, tid >> 2, tid & 3);
     } else {
       const int c = s.choice[d] ? 1 : 0;
       const int sib = 2 * punct + c;
@@ -135,9 +175,9 @@ CUOT_DEV void bfs_levels(const AesLds& aes, const GgmKArgs& a, Lds<NB>& s, int64
         // lanes 0..3: the sibling from the chosen side's sum; 4..7: the
         // punctured node, zero until the last level closes it
         const int i = tid & 3;
-        const int side = tid < 4 ? c : 1 - c;
-        uint32_t v = red_word(s, 0, 4 * side + i);
-        if (ext) v ^= ((const uint32_t*)&ext[2 * r + side])[i];
+        const int sd = tid < 4 ? c : 1 - c;
+        uint32_t v = side_word(s, sd, i);
+        if (ext) v ^= ((const uint32_t*)&ext[2 * r + sd])[i];
         if (tid < 4) {
           words(&s.nodes[sib])[i] = v ^ words(&s.csum[d])[i];
         } else {
