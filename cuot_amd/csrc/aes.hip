@@ -18,7 +18,7 @@ static uint8_t gf8_mul(uint8_t a, uint8_t b) {
   return r;
 }
 
-static void sbox_host(uint8_t S[256]) {
+static void sbox_compute(uint8_t S[256]) {
   for (int x = 0; x < 256; x++) {
     uint8_t inv = 0;
     if (x) {
@@ -35,9 +35,22 @@ static void sbox_host(uint8_t S[256]) {
   }
 }
 
-void cuot_aes_T0_host(uint32_t T0[256]) {
+// The table is built once: the key schedules of one instance (seed, both tree
+// keys per role, LPN seed) each need it, and building it for every one of them
+// cost more than the work of a small instance (32 us a table, eight schedules in a
+// Ferret instance of 200 us).
+struct SboxTable {
   uint8_t S[256];
-  sbox_host(S);
+  SboxTable() { sbox_compute(S); }
+};
+
+static const uint8_t* sbox_host() {
+  static const SboxTable t;
+  return t.S;
+}
+
+void cuot_aes_T0_host(uint32_t T0[256]) {
+  const uint8_t* S = sbox_host();
   for (int x = 0; x < 256; x++) {
     uint8_t s = S[x];
     T0[x] = (uint32_t)gf8_mul(s, 2) | ((uint32_t)s << 8) | ((uint32_t)s << 16) | ((uint32_t)gf8_mul(s, 3) << 24);
@@ -45,8 +58,7 @@ void cuot_aes_T0_host(uint32_t T0[256]) {
 }
 
 void cuot_aes_expand_host(const uint8_t key[16], uint32_t rk[44]) {
-  uint8_t S[256];
-  sbox_host(S);
+  const uint8_t* S = sbox_host();
   uint8_t w[176];
   memcpy(w, key, 16);
   uint8_t rcon = 1;
@@ -158,8 +170,7 @@ hipError_t cuot_launch_prg(const uint32_t rk[44], uint64_t stream, uint64_t star
 }
 
 void cuot_aes_encrypt_host(const uint32_t rk[44], const uint8_t in[16], uint8_t out[16]) {
-  uint8_t S[256];
-  sbox_host(S);
+  const uint8_t* S = sbox_host();
   const uint8_t* k = (const uint8_t*)rk;
   uint8_t s[16], u[16];
   for (int i = 0; i < 16; i++) s[i] = in[i] ^ k[i];
