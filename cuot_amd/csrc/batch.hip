@@ -107,10 +107,12 @@ int plan_batch(cuot_batch* b) {
       p.cfg.k1 = in.k1;
       p.cfg.seed = in.seed;
       p.shared_qc = true;
+      p.split = false;
       int rc = p.validate();
       if (rc) return rc;
     } else if (in.kind == CUOT_MODE_FERRET) {
       FerretPlan& p = b->fer[i];
+      p.split = false;
       memset(&p.cfg, 0, sizeof(p.cfg));
       p.cfg.n = in.n;
       p.cfg.k = in.k;

@@ -106,6 +106,9 @@ extern "C" int cuot_mpcot_recver(cuot_ctx* ctx, cuot_block* const* expanded_d, c
   a.choice = choice;
   a.csum = csum;
   a.fin = fin;
+  // split trees where the caller's scratch holds their sums
+  const size_t part = cuot_ggm_part_bytes(T, depth);
+  if (part && ((size_t)(T << depth) - (size_t)(T * depth + T)) * sizeof(blk) >= part) a.part = fin + T;
   CUOT_HIP_TRY(cuot_launch_ggm(a, true, st));
   CUOT_HIP_TRY(hipStreamSynchronize(st));
   return CUOT_OK;

@@ -17,6 +17,8 @@ struct SotPlan {
   char* qc_scratch;
   char* qc_scratch2;       // second encode's scratch (both parties' encodes overlap)
   bool shared_qc = false;  // batch: the QC scratch lives outside the instance
+  bool split = true;       // carve scratch for the receiver's split trees (batches keep one workgroup per tree)
+  blk* part;               // that scratch, or NULL
 
   size_t carve(void* ws);  // returns bytes needed; fills pointers if ws != NULL
   int validate() const;
@@ -36,6 +38,8 @@ struct FerretPlan {
   uint8_t* choice;
   blk *sums, *csum, *ssum, *lpn_seed, *K, *Mr, *cbits;
   blk* kkp;  // K and Mr interleaved for the LPN gathers
+  bool split = true;  // as in SotPlan
+  blk* part;
 
   size_t carve(void* ws);
   int validate() const;

@@ -31,6 +31,11 @@ struct Carve {
   }
 };
 
+blk* carve_part(Carve& c, bool split, int64_t t, int h) {
+  const size_t bytes = split ? cuot_ggm_part_bytes(t, h) : 0;
+  return bytes ? c.take<blk>(bytes / sizeof(blk)) : nullptr;
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -56,6 +61,7 @@ size_t SotPlan::carve(void* ws) {
   ahat = c.take<uint32_t>(cuot_qc_log_len(n) <= 30 ? (size_t)cuot_qc_ahat_words(n) : 0);
   leaves_s = c.take<blk>(2 * n);
   leaves_r = c.take<blk>(2 * n);
+  part = carve_part(c, split, t, (int)h);
   qc_scratch = shared_qc ? nullptr : c.take<char>(cuot_qc_scratch_bytes_for(n));
   qc_scratch2 = shared_qc ? nullptr : c.take<char>(cuot_qc_scratch_bytes_for(n));
   return c.off + 256;
@@ -123,6 +129,7 @@ hipError_t SotPlan::run_expand_recver(hipStream_t st) {
   a.choice = choice;
   a.csum = csum;
   a.fin = fin;
+  a.part = part;
   return cuot_launch_ggm(a, true, st);
 }
 
@@ -156,6 +163,7 @@ size_t FerretPlan::carve(void* ws) {
   Mr = c.take<blk>(k);
   cbits = c.take<blk>((k + 127) / 128);
   kkp = c.take<blk>(2 * k);
+  part = carve_part(c, split, t, (int)h);
   return c.off + 256;
 }
 
@@ -218,6 +226,7 @@ hipError_t FerretPlan::run_mpcot_recver(blk* out_r, hipStream_t st) {
   a.choice = choice;
   a.csum = csum;
   a.fin = ssum;
+  a.part = part;
   return cuot_launch_ggm(a, true, st);
 }
 
@@ -281,6 +290,7 @@ extern "C" int cuot_sot_run_stages(cuot_ctx* ctx, const cuot_sot_config* cfg, vo
   int rc = p.validate();
   if (rc) return rc;
   CUOT_CHECK_ARG(ws_d && v_d && w_d && b_d, "buffer is NULL");
+  if (ws_bytes < p.carve(nullptr)) p.split = false;  // a workspace without the split trees' scratch will do
   CUOT_CHECK_ARG(ws_bytes >= p.carve(nullptr), "workspace too small (cuot_sot_workspace_bytes)");
   p.carve(ws_d);
   CUOT_HIP_TRY(hipSetDevice(ctx->device));
@@ -313,6 +323,7 @@ extern "C" int cuot_sot_run(cuot_ctx* ctx, const cuot_sot_config* cfg, void* ws_
   int rc = p.validate();
   if (rc) return rc;
   CUOT_CHECK_ARG(ws_d && v_d && w_d && b_d, "buffer is NULL");
+  if (ws_bytes < p.carve(nullptr)) p.split = false;  // a workspace without the split trees' scratch will do
   CUOT_CHECK_ARG(ws_bytes >= p.carve(nullptr), "workspace too small (cuot_sot_workspace_bytes)");
   p.carve(ws_d);
   CUOT_HIP_TRY(hipSetDevice(ctx->device));
@@ -356,6 +367,7 @@ extern "C" int cuot_ferret_run_stages(cuot_ctx* ctx, const cuot_ferret_config* c
   int rc = p.validate();
   if (rc) return rc;
   CUOT_CHECK_ARG(ws_d && out_s_d && out_r_d, "buffer is NULL");
+  if (ws_bytes < p.carve(nullptr)) p.split = false;  // a workspace without the split trees' scratch will do
   CUOT_CHECK_ARG(ws_bytes >= p.carve(nullptr), "workspace too small (cuot_ferret_workspace_bytes)");
   p.carve(ws_d);
   CUOT_HIP_TRY(hipSetDevice(ctx->device));
@@ -408,6 +420,7 @@ extern "C" int cuot_ferret_run_noalloc(cuot_ctx* ctx, const cuot_ferret_config* 
   p.cfg = *cfg;
   const int rc = p.validate();
   if (rc) return rc;
+  p.split = false;  // a config fits if it fits without the split trees' scratch
   CUOT_CHECK_ARG(p.carve(nullptr) <= (size_t)CUOT_FERRET_NOALLOC_WORKSPACE,
                  "workspace of this config (cuot_ferret_workspace_bytes) exceeds the library scratch of "
                  "CUOT_FERRET_NOALLOC_WORKSPACE bytes");

@@ -100,6 +100,7 @@ struct Lds {
   uint32_t red[LMAX][NWAVE][8];    // per-wave XORs
   blk csum[16];                    // receiver: the tree's chosen sums
   uint8_t choice[16];              // receiver: the tree's choice bits
+  blk ext[2 * 16];                 // receiver: level sums of the tree's other subtrees
 };
 
 // word i of the workgroup XOR parked in red[slot]
@@ -247,10 +248,23 @@ CUOT_DEV void dfs_subtree(const AesLds& aes, const uint32_t* rk, blk root, blk* 
   }
 }
 
-template <int L, bool RECV, int NB>
-CUOT_DEV void ggm_tree(const GgmKArgs& a, Lds<NB>& s, int64_t tree) {
+// What a workgroup does with its tree:
+//   SEND   the sender's subtree p of 2^s (the whole tree when s = 0)
+//   PUNCT  the receiver's punctured subtree at depth s (the whole tree when s = 0)
+//   KNOWN  the receiver's subtree p of 2^s, unless it is the punctured one
+// With s > 0 every workgroup of a tree repeats the top s levels.  SEND adds its
+// level sums below depth s to the zeroed output with XOR atomics; KNOWN parks
+// them in its own slot of a.part, and PUNCT, the next launch, combines the
+// slots of the tree's other subtrees into the sums it rebuilds from.
+enum { SEND, PUNCT, KNOWN };
+
+template <int L, int WHAT, int NB>
+CUOT_DEV void ggm_tree(const GgmKArgs& a, Lds<NB>& s, int64_t tree, int p) {
+  constexpr bool RECV = WHAT != SEND;
+  constexpr bool P = WHAT == PUNCT;
   const int tid = threadIdx.x;
   const int h = a.h;
+  const int sp = a.s;
   aes_stage_table(s.aes, a.T0, tid, WG);
   if (tid == 0) s.nodes[0] = RECV ? bzero() : ldb(a.roots + tree);
   if (RECV && tid < h) {
@@ -260,16 +274,41 @@ CUOT_DEV void ggm_tree(const GgmKArgs& a, Lds<NB>& s, int64_t tree) {
   __syncthreads();
   const AesLds aes = aes_lds(s.aes);
   const bool ferret = a.mode == CUOT_MODE_FERRET;
-  const int top = h - L;
+  const int top = h - sp - L;
   int punct = 0;
-  bfs_levels<RECV>(aes, a, s, tree, 0, top, nullptr, L == 0, &punct);
-  const int64_t tree0 = tree << h;
+  if constexpr (P) {
+    // the punctured prefix follows the sides not chosen
+    for (int d = 0; d < sp; d++) punct = 2 * punct + (s.choice[d] ? 0 : 1);
+    p = punct;
+    // sums of the other subtrees, depths sp + 1 .. h (s.sums from index 2 sp)
+    if (sp > 0) {
+      const int nw = (h - sp) * 8;  // words
+      const uint32_t* slots = (const uint32_t*)(a.part + ((tree << sp) * (h - sp)) * 2);
+      for (int i = tid; i < nw; i += WG) {
+        uint32_t v = 0;
+        for (int q = 0; q < (1 << sp); q++)
+          if (q != punct) v ^= slots[q * nw + i];
+        words(&s.ext[0])[i] = v;
+      }
+      __syncthreads();
+    }
+  } else if (sp > 0) {
+    bfs_levels<RECV>(aes, a, s, tree, 0, sp, nullptr, false, &punct);
+    if (RECV && p == punct) return;  // uniform over the workgroup
+    const blk root = s.nodes[p];
+    __syncthreads();
+    if (tid == 0) s.nodes[0] = root;
+    __syncthreads();
+  }
+  punct = 0;
+  bfs_levels<P>(aes, a, s, tree, sp, top, sp > 0 ? s.ext : nullptr, L == 0, &punct);
+  const int64_t tree0 = (tree << h) + ((int64_t)p << (h - sp));
 
   if constexpr (L == 0) {
     // whole tree fits the top phase: write leaves from LDS
-    for (int f = tid; f < (1 << h); f += WG) {
+    for (int f = tid; f < (1 << top); f += WG) {
       blk v = s.nodes[f];
-      if (ferret && !(RECV && f == punct)) v = clear_lsb(v);
+      if (ferret && !(P && f == punct)) v = clear_lsb(v);
       const int64_t g = tree0 + f;
       if (g < a.n_out) stb(a.leaves + g, v);
     }
@@ -282,7 +321,7 @@ CUOT_DEV void ggm_tree(const GgmKArgs& a, Lds<NB>& s, int64_t tree) {
       tr[r] = bzero();
     }
     for (int f = tid; f < (1 << top); f += WG)
-      if (!(RECV && f == punct))
+      if (!(P && f == punct))
         dfs_subtree<L>(aes, a.rk, s.nodes[f], a.leaves, tree0 + ((int64_t)f << L), a.n_out, ferret, tl, tr);
 #pragma unroll
     for (int r = 1; r <= L; r++) {
@@ -290,15 +329,20 @@ CUOT_DEV void ggm_tree(const GgmKArgs& a, Lds<NB>& s, int64_t tree) {
       if ((tid & 63) < 8) s.red[r - 1][tid >> 6][bitrev3(tid & 63)] = x;
     }
     __syncthreads();
-    if (tid < 8 * L) words(&s.sums[2 * (top + (tid >> 3))])[tid & 7] = red_word(s, tid >> 3, tid & 7);
+    if (tid < 8 * L) {
+      const int d = top + (tid >> 3);  // below depth sp
+      uint32_t v = red_word(s, tid >> 3, tid & 7);
+      if (P && sp > 0) v ^= words(&s.ext[2 * d])[tid & 7];
+      words(&s.sums[2 * (sp + d)])[tid & 7] = v;
+    }
     __syncthreads();
-    if constexpr (RECV) {
+    if constexpr (P) {
       // ---- phase C: rebuild the punctured depth-`top` subtree -------------
       const int pt = punct;
       if (tid == 0) s.nodes[0] = bzero();
       __syncthreads();
       int pl = 0;
-      bfs_levels<true>(aes, a, s, tree, top, L, &s.sums[2 * top], true, &pl);
+      bfs_levels<true>(aes, a, s, tree, sp + top, L, &s.sums[2 * (sp + top)], true, &pl);
       const int64_t base = tree0 + ((int64_t)pt << L);
       if (tid < (1 << L)) {
         blk v = s.nodes[tid];
@@ -308,21 +352,43 @@ CUOT_DEV void ggm_tree(const GgmKArgs& a, Lds<NB>& s, int64_t tree) {
       }
     }
   }
-  if constexpr (!RECV) {
+  if constexpr (WHAT == SEND) {
     __syncthreads();
-    if (tid < 2 * h) stb(a.sums + tree * 2 * h + tid, s.sums[tid]);
+    blk* out = a.sums + tree * 2 * h;
+    if (sp == 0) {
+      if (tid < 2 * h) stb(out + tid, s.sums[tid]);
+    } else {
+      if (p == 0 && tid < 2 * sp) stb(out + tid, s.sums[tid]);
+      const int nw = (h - sp) * 4;  // 64-bit words below depth sp
+      if (tid < nw)
+        atomicXor((unsigned long long*)(out + 2 * sp) + tid, ((const unsigned long long*)(s.sums + 2 * sp))[tid]);
+    }
+  }
+  if constexpr (WHAT == KNOWN) {
+    __syncthreads();
+    if (tid < 2 * (h - sp)) stb(a.part + ((tree << sp) + p) * (h - sp) * 2 + tid, s.sums[2 * sp + tid]);
   }
 }
 
 // nodes to hold: 2^10 only where the breadth-first top can reach it (h = 16
 // with L = 6, or a smaller L by the knob); the smaller form lets two
 // workgroups share a CU
-template <int L, bool RECV, int NB>
+template <int L, int WHAT, int NB>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void ggm_kernel(GgmKArgs) {
   __shared__ __align__(16) Lds<NB> s;
   // the argument block read through its pointer: as a value the 88 round-key
   // words are held across the subtree loop and spill
-  ggm_tree<L, RECV>(*(const GgmKArgs*)__builtin_amdgcn_kernarg_segment_ptr(), s, blockIdx.x);
+  const GgmKArgs& a = *(const GgmKArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  if (WHAT == PUNCT)
+    ggm_tree<L, WHAT>(a, s, blockIdx.x, 0);
+  else
+    ggm_tree<L, WHAT>(a, s, blockIdx.x >> a.s, (int)(blockIdx.x & ((1u << a.s) - 1)));
+}
+
+// zero level sums for the workgroups that add to them
+__global__ __launch_bounds__(256) void ggm_zero_kernel(blk* p, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) stb(p + i, bzero());
 }
 
 // Batch: one WG per tree of every instance in the table; start[i] is the first
@@ -341,7 +407,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void gg
     else
       hi = mid - 1;
   }
-  ggm_tree<L, RECV>(tab[lo], s, g - start[lo]);
+  ggm_tree<L, RECV ? PUNCT : SEND>(tab[lo], s, g - start[lo], 0);
 }
 
 // Depth-first levels L per lane.  Every lane of the workgroup has a subtree from
@@ -356,20 +422,31 @@ int ggm_split(int h) {
 }
 
 // L, plus 16 when the breadth-first top is deeper than 2^9 nodes
-int ggm_form(int h) {
-  const int L = ggm_split(h);
-  return L + (h - L > 9 ? 16 : 0);
+int ggm_form(int h, int L) { return L + (h - L > 9 ? 16 : 0); }
+
+// log2 of the workgroups per tree.  With few trees one workgroup each leaves
+// most CUs idle, and a tree takes as long as one CU's AES rate allows.  The
+// split aims at two workgroups per CU; a subtree keeps at least 8 levels, and
+// trees stay whole where the repeated top and the second launch (zeroed sums,
+// or the receiver's punctured subtrees) cost what the split saves.  Whole ->
+// split, us: sender depth 12: 64 trees 48 -> 36; 13: 3 trees 75 -> 33, 64
+// 76 -> 43, 128 77 -> 53; 14: 100 130 -> 75; 15: 40 237 -> 78; 16: 16 449 -> 58.
+// Receiver depth 12: 50 -> 50 (whole); 13: 3 81 -> 54, 64 80 -> 63, 65 80 -> 78
+// (whole from there); 14: 100 137 -> 118; 15: 40 246 -> 122; 16: 16 458 -> 94.
+int ggm_wg_split(int64_t t, int h, bool recv) {
+  if (h < (recv ? 13 : 12) || t > (recv && h == 13 ? 64 : 128)) return 0;
+  int s = 0;
+  while ((t << (s + 1)) <= 512 && s + 1 <= h - 8) s++;
+  return s;
 }
 
-template <bool RECV>
-hipError_t launch_ggm(const GgmKArgs& a, hipStream_t st) {
-  dim3 grid((unsigned)a.t), block(WG);
-  const int64_t nl = (a.t << a.h) < a.n_out ? (a.t << a.h) : a.n_out;
-  cuot_rec_begin(st, RECV ? "ggm_kernel<recv>" : "ggm_kernel<send>", 16.0 * (double)nl);
-  switch (ggm_form(a.h)) {
+template <int WHAT>
+hipError_t launch_form(const GgmKArgs& a, int L, int64_t wgs, hipStream_t st) {
+  dim3 grid((unsigned)wgs), block(WG);
+  switch (ggm_form(a.h - a.s, L)) {
 #define CUOT_GGM_CASE(X, NB)                                              \
   case X + (NB > 512 ? 16 : 0):                                           \
-    hipLaunchKernelGGL((ggm_kernel<X, RECV, NB>), grid, block, 0, st, a); \
+    hipLaunchKernelGGL((ggm_kernel<X, WHAT, NB>), grid, block, 0, st, a); \
     break;
 #define CUOT_GGM_CASES   \
   CUOT_GGM_CASE(0, 512)  \
@@ -388,11 +465,30 @@ hipError_t launch_ggm(const GgmKArgs& a, hipStream_t st) {
     CUOT_GGM_CASES
 #undef CUOT_GGM_CASE
     default:
-      cuot_rec_end(st);
       return hipErrorInvalidValue;
   }
-  cuot_rec_end(st);
   return hipGetLastError();
+}
+
+hipError_t launch_ggm(GgmKArgs a, bool recv, hipStream_t st) {
+  const int64_t nl = (a.t << a.h) < a.n_out ? (a.t << a.h) : a.n_out;
+  a.s = ggm_wg_split(a.t, a.h, recv);
+  if ((recv && a.part == nullptr) || cuot_knobs().ggm_dfs) a.s = 0;  // the knob picks a split of whole trees
+  const int L = ggm_split(a.h - a.s);
+  hipError_t e = hipSuccess;
+  cuot_rec_begin(st, recv ? "ggm_kernel<recv>" : "ggm_kernel<send>", 16.0 * (double)nl);
+  if (!recv) {
+    if (a.s > 0) {
+      const int64_t nz = a.t * 2 * a.h;
+      hipLaunchKernelGGL(ggm_zero_kernel, dim3((unsigned)((nz + 255) / 256)), dim3(256), 0, st, a.sums, nz);
+    }
+    e = launch_form<SEND>(a, L, a.t << a.s, st);
+  } else {
+    if (a.s > 0) e = launch_form<KNOWN>(a, L, a.t << a.s, st);
+    if (!e) e = launch_form<PUNCT>(a, L, a.t, st);
+  }
+  cuot_rec_end(st);
+  return e;
 }
 
 template <bool RECV>
@@ -415,11 +511,14 @@ hipError_t launch_ggm_batch(const GgmKArgs* tab, const int64_t* start, int ninst
 
 }  // namespace
 
-int cuot_ggm_form(int h) { return ggm_form(h); }
+int cuot_ggm_form(int h) { return ggm_form(h, ggm_split(h)); }
 
-hipError_t cuot_launch_ggm(const GgmKArgs& a, bool receiver, hipStream_t st) {
-  return receiver ? launch_ggm<true>(a, st) : launch_ggm<false>(a, st);
+size_t cuot_ggm_part_bytes(int64_t t, int h) {
+  const int s = ggm_wg_split(t, h, true);
+  return s > 0 ? (size_t)(t << s) * (h - s) * 2 * sizeof(blk) : 0;
 }
+
+hipError_t cuot_launch_ggm(const GgmKArgs& a, bool receiver, hipStream_t st) { return launch_ggm(a, receiver, st); }
 
 hipError_t cuot_launch_ggm_batch(const GgmKArgs* tab_d, const int64_t* start_d, int ninst, int64_t total_trees,
                                  int form, bool receiver, hipStream_t st) {

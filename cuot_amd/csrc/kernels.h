@@ -5,7 +5,8 @@
 
 #include "common.h"
 
-// GGM expansion of t trees of depth h (one 512-lane workgroup per tree).
+// GGM expansion of t trees of depth h (one 512-lane workgroup per tree, or
+// 2^s of them when there are few trees).
 struct GgmKArgs {
   const uint32_t* T0;    // AES T-table in global memory
   uint32_t rk[88];       // key-0 then key-1 AES-128 schedules (little-endian words)
@@ -19,8 +20,12 @@ struct GgmKArgs {
   const uint8_t* choice; // receiver: [t][h], 1 = chose the right (odd) side
   const blk* csum;       // receiver: [t][h] chosen level sums
   const blk* fin;        // receiver: [t] SOT final-row value / Ferret secret sum
+  int s;                 // log2 workgroups per tree (set by cuot_launch_ggm)
+  blk* part;             // receiver: scratch of cuot_ggm_part_bytes(t, h) bytes, or NULL (one workgroup per tree)
 };
 hipError_t cuot_launch_ggm(const GgmKArgs& a, bool receiver, hipStream_t st);
+// scratch for the level sums of a receiver's split trees (0: never split)
+size_t cuot_ggm_part_bytes(int64_t t, int h);
 // kernel form of trees of depth h (instances of one form share a launch)
 int cuot_ggm_form(int h);
 // batch of instances with the same cuot_ggm_form(h) and role; tab_d and

@@ -98,6 +98,7 @@ struct cuot_ferret_session {
   uint8_t* chk = nullptr;  // x' (128), digests (2 x 32), ok (int32)
   char* mem = nullptr;
   blk *delta, *boot_s, *boot_r, *P0, *P1, *Pr, *roots, *sums, *csum, *ssum, *cbits, *kkp;
+  blk* part;  // scratch of the receiver's split trees, or NULL
   uint8_t* bits;
 };
 
@@ -127,6 +128,8 @@ size_t carve_session(cuot_ferret_session* s, char* base) {
   s->kkp = (blk*)take((size_t)2 * s->plan.cfg.k * 16);
   s->vwc = (blk*)take((size_t)3 * t * 16);
   s->chk = (uint8_t*)take(256);
+  const size_t part = cuot_ggm_part_bytes(t, (int)h);
+  s->part = part ? (blk*)take(part) : nullptr;
   return off + 256;
 }
 
@@ -185,6 +188,7 @@ hipError_t extend_seed(cuot_ferret_session* s, blk* out_s, blk* out_r, hipStream
   r.choice = s->bits;
   r.csum = s->csum;
   r.fin = s->ssum;
+  r.part = s->part;
   if ((e = cuot_launch_ggm(r, true, st))) return e;
   if (s->malicious) return consistency(s, out_s, out_r, st);
   return hipSuccess;

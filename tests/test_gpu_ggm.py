@@ -197,3 +197,42 @@ def test_ggm_sender_bitsliced_matches_ttable(ctx, h, t, mode):
     rwork = torch.empty(ctx.ggm_recver_bs_work_bytes(p), dtype=torch.uint8, device="cuda")
     ctx.ggm_recver_bs(p, cd, to_dev(csum), to_dev(fin), wb, rwork)
     assert np.array_equal(to_np(wb)[:n_out], to_np(wa)[:n_out])
+
+
+# few deep trees: several workgroups per tree (sender from depth 12, receiver
+# from 13 where the instance workspace holds the partial sums), at the ends of
+# the split's range, with a truncated last tree, and just past its limits
+@pytest.mark.parametrize("t,h,cut", [(1, 13, 0), (3, 13, 4577), (64, 13, 1), (65, 13, 8191), (2, 12, 100), (9, 14, 12001),
+                                     (3, 15, 32767), (2, 16, 40000)])
+def test_split_trees_match_oracle(ctx, t, h, cut):
+    import torch
+
+    import cuot_amd
+
+    n = (t << h) - cut
+    print(f"split trees t={t} h={h} n={n}", flush=True)
+    seed = np.array([t, 1000 + h], dtype=np.uint64)
+    k = 50
+    cfg = cuot_amd.FerretConfig(n=n, k=k, t=t, h=h, ntasks=1, seed=cuot_amd.to_block(seed))
+    os_, or_, _ = po.ferret_run(n, k, t, h, seed, nthreads=4)
+    full = ctx.ferret_workspace_bytes(cfg)
+    s, w = dev_blocks(n), dev_blocks(n)
+    ws = torch.full((full,), 0xA5, dtype=torch.uint8, device="cuda")
+    for _ in range(2):  # stale partial sums of the first pass
+        ctx.ferret_run(cfg, ws, s, w)
+        assert np.array_equal(to_np(s), os_)
+        assert np.array_equal(to_np(w), or_)
+    ctx.ferret_run_noalloc(cfg, s.zero_(), w.zero_())
+    assert np.array_equal(to_np(s), os_) and np.array_equal(to_np(w), or_)
+    if n % 2 == 0:
+        k0, k1 = np.array([3242342, 0], np.uint64), np.array([8993849, 0], np.uint64)
+        m = n // 2
+        scfg = cuot_amd.SotConfig(n=m, t=t, h=h, reserved=0, k0=cuot_amd.to_block(k0), k1=cuot_amd.to_block(k1),
+                                  seed=cuot_amd.to_block(seed))
+        ws = torch.full((ctx.sot_workspace_bytes(scfg),), 0x5A, dtype=torch.uint8, device="cuda")
+        v, u, d = dev_blocks(m), dev_blocks(m), dev_blocks(1)
+        b = torch.zeros(((m + 31) // 32) * 4, dtype=torch.uint8, device="cuda")
+        ctx.sot_run(scfg, ws, v, u, b, d)
+        ov, ow, ob, od = po.sot_run(m, t, h, k0, k1, seed, nthreads=4)
+        assert np.array_equal(to_np(v), ov) and np.array_equal(to_np(u), ow)
+        assert np.array_equal(b.cpu().numpy()[: (m + 7) // 8], ob[: (m + 7) // 8])
