@@ -341,11 +341,7 @@ hipError_t launch_all(cuot_batch* b, uint32_t stages, hipStream_t st, hipStream_
   hipEvent_t* ev = b->ctx->ev;
   if (stages & CUOT_BATCH_STAGE_SETUP) {
     for (int i = 0; i < count; i++) {
-      if ((e = b->is_sot(i) ? b->sot[i].run_setup(st) : b->fer[i].run_setup(st))) return e;
-      if (b->delta[i]) {
-        const blk* d = b->is_sot(i) ? b->sot[i].delta : b->fer[i].delta;
-        if ((e = hipMemcpyAsync(b->delta[i], d, 16, hipMemcpyDeviceToDevice, st))) return e;
-      }
+      if ((e = b->is_sot(i) ? b->sot[i].run_setup(b->delta[i], st) : b->fer[i].run_setup(b->delta[i], st))) return e;
     }
   }
   hipStream_t sp = st;  // preparation, sparse encodes, LPN
@@ -355,9 +351,16 @@ hipError_t launch_all(cuot_batch* b, uint32_t stages, hipStream_t st, hipStream_
     sp = ax;
   }
   if (stages & CUOT_BATCH_STAGE_QC_PREPARE)
-    for (const PrepGroup& pg : b->prep)
-      if ((e = cuot_launch_qc_prepare_batch((const QcPrep*)(ws + pg.off), (int)pg.members.size(), pg.m, sp)))
+    for (const PrepGroup& pg : b->prep) {
+      // a whole run whose encodes of this length all take the matrix cores
+      // needs only the bits of a
+      int64_t nmax = 0;
+      for (int i : pg.members) nmax = std::max(nmax, b->inst[i].n);
+      const bool transform = stages != CUOT_BATCH_STAGE_ALL || !cuot_qc_mfma_selected(nmax);
+      if ((e = cuot_launch_qc_prepare_batch((const QcPrep*)(ws + pg.off), (int)pg.members.size(), pg.m, transform,
+                                            sp)))
         return e;
+    }
   if (two) {
     if ((e = hipEventRecord(ev[1], sp))) return e;
   }
@@ -391,8 +394,6 @@ hipError_t launch_all(cuot_batch* b, uint32_t stages, hipStream_t st, hipStream_
     if ((e = hipStreamWaitEvent(st, ev[1], 0))) return e;
   }
   if ((stages & CUOT_BATCH_STAGE_LPN) && !b->ferret_ids.empty()) {
-    for (int i : b->ferret_ids)
-      if ((e = b->fer[i].fill_kkp(sp))) return e;
     if ((e = cuot_launch_lpn_batch(ws + b->lpn_tab_off, (const int64_t*)(ws + b->lpn_start_off),
                                    (int)b->ferret_ids.size(), b->lpn_wgs, 2, sp)))
       return e;

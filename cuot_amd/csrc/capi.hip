@@ -257,7 +257,7 @@ extern "C" int cuot_qc_prepare(cuot_ctx* ctx, int64_t n, const uint8_t* a_bits_d
   if (rc) return rc;
   CUOT_CHECK_ARG(a_bits_d && ahat_d && scratch_d, "buffer is NULL");
   CUOT_HIP_TRY(hipSetDevice(ctx->device));
-  CUOT_HIP_TRY(cuot_launch_qc_prepare(a_bits_d, n, ahat_d, scratch_d, ctx->st(stream)));
+  CUOT_HIP_TRY(cuot_launch_qc_prepare(a_bits_d, n, ahat_d, scratch_d, true, ctx->st(stream)));
   return CUOT_OK;
 }
 

@@ -229,8 +229,8 @@ extern "C" int cuot_sot_base_ot(cuot_sot_role* r) {
   CUOT_CHECK_ARG(r, "role NULL");
   CUOT_HIP_TRY(hipSetDevice(r->ctx->device));
   hipStream_t st = r->ctx->stream;
-  CUOT_HIP_TRY(r->plan.run_setup(st));
-  CUOT_HIP_TRY(r->plan.run_prepare(st));
+  CUOT_HIP_TRY(r->plan.run_setup(nullptr, st));
+  CUOT_HIP_TRY(r->plan.run_prepare(true, st));
   CUOT_HIP_TRY(hipStreamSynchronize(st));
   r->stage = 1;
   return CUOT_OK;

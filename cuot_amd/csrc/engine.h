@@ -6,7 +6,7 @@
 
 struct SotPlan {
   cuot_sot_config cfg;
-  blk *delta, *roots, *alpha;
+  blk *delta, *roots;
   uint8_t* choice;
   int64_t* pos;
   uint32_t* a_words;
@@ -22,8 +22,8 @@ struct SotPlan {
 
   size_t carve(void* ws);  // returns bytes needed; fills pointers if ws != NULL
   int validate() const;
-  hipError_t run_setup(hipStream_t st);
-  hipError_t run_prepare(hipStream_t st);
+  hipError_t run_setup(blk* delta_out, hipStream_t st);  // delta_out: a copy of Delta, or NULL
+  hipError_t run_prepare(bool transform, hipStream_t st);
   void ggm_args(GgmKArgs& a) const;
   hipError_t run_expand_sender(hipStream_t st);
   hipError_t run_sender_msgs(hipStream_t st);  // masked rows + receiver's view
@@ -34,23 +34,22 @@ struct SotPlan {
 
 struct FerretPlan {
   cuot_ferret_config cfg;
-  blk *delta, *roots, *alpha;
+  blk *delta, *roots;
   uint8_t* choice;
-  blk *sums, *csum, *ssum, *lpn_seed, *K, *Mr, *cbits;
+  blk *sums, *csum, *ssum, *K, *Mr;
   blk* kkp;  // K and Mr interleaved for the LPN gathers
   bool split = true;  // as in SotPlan
   blk* part;
 
   size_t carve(void* ws);
   int validate() const;
-  hipError_t run_setup(hipStream_t st);
+  hipError_t run_setup(blk* delta_out, hipStream_t st);  // delta_out: a copy of Delta, or NULL
   void ggm_args(GgmKArgs& a) const;
   hipError_t run_mpcot_sender(blk* out_s, hipStream_t st);
   hipError_t run_sender_sums(hipStream_t st);  // secret sum + receiver's chosen sums
   hipError_t run_mpcot_recver(blk* out_r, hipStream_t st);
   hipError_t run_mpcot(blk* out_s, blk* out_r, hipStream_t st);
-  void lpn_launch(blk* out_s, blk* out_r, LpnLaunch& l) const;  // gathers from kkp (fill it first)
-  hipError_t fill_kkp(hipStream_t st);
+  void lpn_launch(blk* out_s, blk* out_r, LpnLaunch& l) const;  // gathers from kkp (written by the setup)
   hipError_t run_lpn(blk* out_s, blk* out_r, hipStream_t st);
 };
 

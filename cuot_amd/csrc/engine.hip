@@ -46,7 +46,6 @@ size_t SotPlan::carve(void* ws) {
   const int64_t t = cfg.t, h = cfg.h, n = cfg.n;
   delta = c.take<blk>(1);
   roots = c.take<blk>(t);
-  alpha = c.take<blk>(t);
   choice = c.take<uint8_t>(t * h);
   pos = c.take<int64_t>(t);
   a_words_total = ((n + 127) / 128) * 4 + 4;  // PRG blocks as words + padding
@@ -76,22 +75,27 @@ int SotPlan::validate() const {
   return CUOT_OK;
 }
 
-hipError_t SotPlan::run_setup(hipStream_t st) {
-  const int64_t t = cfg.t, h = cfg.h, n = cfg.n;
+hipError_t SotPlan::run_setup(blk* delta_out, hipStream_t st) {
   uint32_t rk[44];
   cuot_aes_expand_host((const uint8_t*)&cfg.seed, rk);
-  hipError_t e;
-  if ((e = cuot_launch_prg(rk, 0, 0, 1, delta, st))) return e;
-  if ((e = cuot_launch_prg(rk, 1, 0, t, roots, st))) return e;
-  if ((e = cuot_launch_prg(rk, 2, 0, t, alpha, st))) return e;
-  if ((e = cuot_launch_prg(rk, 3, 0, (n + 127) / 128, (blk*)a_words, st))) return e;
-  if ((e = cuot_launch_prg(rk, 4, 0, h * t, m0b, st))) return e;
-  if ((e = cuot_launch_prg(rk, 5, 0, h * t, m1b, st))) return e;
-  return cuot_launch_setup_fix(delta, alpha, t, (int)h, choice, pos, a_words, n, a_words_total, st);
+  SetupArgs p;
+  memset(&p, 0, sizeof(p));
+  p.delta = delta;
+  p.delta_out = delta_out;
+  p.t = cfg.t;
+  p.h = cfg.h;
+  p.roots = roots;
+  p.choice = choice;
+  p.pos = pos;
+  p.a_words = a_words;
+  p.n = cfg.n;
+  p.m0b = m0b;
+  p.m1b = m1b;
+  return cuot_launch_setup(rk, p, st);
 }
 
-hipError_t SotPlan::run_prepare(hipStream_t st) {
-  return cuot_launch_qc_prepare((const uint8_t*)a_words, cfg.n, ahat, qc_scratch, st);
+hipError_t SotPlan::run_prepare(bool transform, hipStream_t st) {
+  return cuot_launch_qc_prepare((const uint8_t*)a_words, cfg.n, ahat, qc_scratch, transform, st);
 }
 
 void SotPlan::ggm_args(GgmKArgs& a) const {
@@ -117,9 +121,7 @@ hipError_t SotPlan::run_expand_sender(hipStream_t st) {
 }
 
 hipError_t SotPlan::run_sender_msgs(hipStream_t st) {
-  hipError_t e;
-  if ((e = cuot_launch_sot_msgs(sums, m0b, m1b, delta, cfg.t, cfg.h, M0, M1, st))) return e;
-  return cuot_launch_sot_recv_prep(choice, M0, M1, m0b, m1b, cfg.t, cfg.h, csum, fin, st);
+  return cuot_launch_sot_msgs(sums, m0b, m1b, delta, cfg.t, cfg.h, M0, M1, choice, csum, fin, st);
 }
 
 hipError_t SotPlan::run_expand_recver(hipStream_t st) {
@@ -153,15 +155,12 @@ size_t FerretPlan::carve(void* ws) {
   const int64_t t = cfg.t, h = cfg.h, k = cfg.k;
   delta = c.take<blk>(1);
   roots = c.take<blk>(t);
-  alpha = c.take<blk>(t);
   choice = c.take<uint8_t>(t * h);
   sums = c.take<blk>(2 * t * h);
   csum = c.take<blk>(t * h);
   ssum = c.take<blk>(t);
-  lpn_seed = c.take<blk>(1);
   K = c.take<blk>(k);
   Mr = c.take<blk>(k);
-  cbits = c.take<blk>((k + 127) / 128);
   kkp = c.take<blk>(2 * k);
   part = carve_part(c, split, t, (int)h);
   return c.off + 256;
@@ -178,18 +177,22 @@ int FerretPlan::validate() const {
   return CUOT_OK;
 }
 
-hipError_t FerretPlan::run_setup(hipStream_t st) {
+hipError_t FerretPlan::run_setup(blk* delta_out, hipStream_t st) {
   uint32_t rk[44];
   cuot_aes_expand_host((const uint8_t*)&cfg.seed, rk);
-  hipError_t e;
-  if ((e = cuot_launch_prg(rk, 0, 0, 1, delta, st))) return e;
-  if ((e = cuot_launch_prg(rk, 1, 0, cfg.t, roots, st))) return e;
-  if ((e = cuot_launch_prg(rk, 2, 0, cfg.t, alpha, st))) return e;
-  if ((e = cuot_launch_prg(rk, 6, 0, 1, lpn_seed, st))) return e;
-  if ((e = cuot_launch_prg(rk, 7, 0, cfg.k, K, st))) return e;
-  if ((e = cuot_launch_prg(rk, 8, 0, (cfg.k + 127) / 128, cbits, st))) return e;
-  if ((e = cuot_launch_setup_fix(delta, alpha, cfg.t, cfg.h, choice, nullptr, nullptr, 0, 0, st))) return e;
-  return cuot_launch_ferret_boot(K, Mr, (const uint8_t*)cbits, delta, cfg.k, st);
+  SetupArgs p;
+  memset(&p, 0, sizeof(p));
+  p.delta = delta;
+  p.delta_out = delta_out;
+  p.t = cfg.t;
+  p.h = cfg.h;
+  p.roots = roots;
+  p.choice = choice;
+  p.k = cfg.k;
+  p.K = K;
+  p.Mr = Mr;
+  p.kkp = kkp;
+  return cuot_launch_setup(rk, p, st);
 }
 
 void FerretPlan::ggm_args(GgmKArgs& a) const {
@@ -240,7 +243,7 @@ hipError_t FerretPlan::run_mpcot(blk* out_s, blk* out_r, hipStream_t st) {
 void FerretPlan::lpn_launch(blk* out_s, blk* out_r, LpnLaunch& l) const {
   uint32_t rk_seed[44];
   cuot_aes_expand_host((const uint8_t*)&cfg.seed, rk_seed);
-  // LPN seed = AES_seed({0, 6}) computed on the host (identical to stream 6)
+  // LPN seed = AES_seed({0, 6}) computed on the host
   uint8_t ctr[16] = {0};
   ctr[8] = 6;
   uint8_t seed6[16];
@@ -260,11 +263,7 @@ void FerretPlan::lpn_launch(blk* out_s, blk* out_r, LpnLaunch& l) const {
   l.kkp = kkp;
 }
 
-hipError_t FerretPlan::fill_kkp(hipStream_t st) { return cuot_launch_interleave(K, Mr, cfg.k, kkp, st); }
-
 hipError_t FerretPlan::run_lpn(blk* out_s, blk* out_r, hipStream_t st) {
-  hipError_t e = fill_kkp(st);
-  if (e) return e;
   LpnLaunch l;
   lpn_launch(out_s, out_r, l);
   return cuot_launch_lpn(l, st);
@@ -295,8 +294,8 @@ extern "C" int cuot_sot_run_stages(cuot_ctx* ctx, const cuot_sot_config* cfg, vo
   p.carve(ws_d);
   CUOT_HIP_TRY(hipSetDevice(ctx->device));
   hipStream_t st = ctx->st(stream);
-  if (stages & CUOT_SOT_STAGE_SETUP) CUOT_HIP_TRY(p.run_setup(st));
-  if (stages & CUOT_SOT_STAGE_QC_PREPARE) CUOT_HIP_TRY(p.run_prepare(st));
+  if (stages & CUOT_SOT_STAGE_SETUP) CUOT_HIP_TRY(p.run_setup((blk*)delta_d, st));
+  if (stages & CUOT_SOT_STAGE_QC_PREPARE) CUOT_HIP_TRY(p.run_prepare(true, st));
   if (stages & CUOT_SOT_STAGE_GGM_SENDER) CUOT_HIP_TRY(p.run_expand_sender(st));
   if (stages & CUOT_SOT_STAGE_GGM_RECVER) CUOT_HIP_TRY(p.run_expand_recver(st));
   if (stages & CUOT_SOT_STAGE_QC_SENDER)
@@ -305,8 +304,6 @@ extern "C" int cuot_sot_run_stages(cuot_ctx* ctx, const cuot_sot_config* cfg, vo
     CUOT_HIP_TRY(cuot_launch_qc_encode(p.ahat, p.cfg.n, p.leaves_r, (blk*)w_d, p.qc_scratch, st));
   if (stages & CUOT_SOT_STAGE_SPARSE)
     CUOT_HIP_TRY(cuot_launch_sparse(p.a_words, p.cfg.n, p.pos, (int)p.cfg.t, (uint32_t*)b_d, st));
-  if (delta_d && (stages & CUOT_SOT_STAGE_SETUP))
-    CUOT_HIP_TRY(hipMemcpyAsync(delta_d, p.delta, 16, hipMemcpyDeviceToDevice, st));
   return CUOT_OK;
 }
 
@@ -331,11 +328,12 @@ extern "C" int cuot_sot_run(cuot_ctx* ctx, const cuot_sot_config* cfg, void* ws_
   CUOT_HIP_TRY(cuot_qc_configure());
   hipStream_t st = ctx->st(stream), ax = ctx->aux;
   hipEvent_t e_setup = ctx->ev[0], e_prep = ctx->ev[1], e_rows = ctx->ev[2], e_done = ctx->ev[3];
-  CUOT_HIP_TRY(p.run_setup(st));
-  if (delta_d) CUOT_HIP_TRY(hipMemcpyAsync(delta_d, p.delta, 16, hipMemcpyDeviceToDevice, st));
+  CUOT_HIP_TRY(p.run_setup((blk*)delta_d, st));
   CUOT_HIP_TRY(hipEventRecord(e_setup, st));
   CUOT_HIP_TRY(hipStreamWaitEvent(ax, e_setup, 0));
-  CUOT_HIP_TRY(p.run_prepare(ax));
+  // both encodes follow in this call: when they take the matrix cores, A^ is
+  // not needed (its 33 small launches took 95 us beside n = 2^14's 45 us encodes)
+  CUOT_HIP_TRY(p.run_prepare(!cuot_qc_mfma_selected(p.cfg.n), ax));
   CUOT_HIP_TRY(hipEventRecord(e_prep, ax));
   CUOT_HIP_TRY(cuot_launch_sparse(p.a_words, p.cfg.n, p.pos, (int)p.cfg.t, (uint32_t*)b_d, ax));
   CUOT_HIP_TRY(p.run_expand_sender(st));
@@ -372,12 +370,10 @@ extern "C" int cuot_ferret_run_stages(cuot_ctx* ctx, const cuot_ferret_config* c
   p.carve(ws_d);
   CUOT_HIP_TRY(hipSetDevice(ctx->device));
   hipStream_t st = ctx->st(stream);
-  if (stages & CUOT_FERRET_STAGE_SETUP) CUOT_HIP_TRY(p.run_setup(st));
+  if (stages & CUOT_FERRET_STAGE_SETUP) CUOT_HIP_TRY(p.run_setup((blk*)delta_d, st));
   if (stages & CUOT_FERRET_STAGE_GGM_SENDER) CUOT_HIP_TRY(p.run_mpcot_sender((blk*)out_s_d, st));
   if (stages & CUOT_FERRET_STAGE_GGM_RECVER) CUOT_HIP_TRY(p.run_mpcot_recver((blk*)out_r_d, st));
   if (stages & CUOT_FERRET_STAGE_LPN) CUOT_HIP_TRY(p.run_lpn((blk*)out_s_d, (blk*)out_r_d, st));
-  if (delta_d && (stages & CUOT_FERRET_STAGE_SETUP))
-    CUOT_HIP_TRY(hipMemcpyAsync(delta_d, p.delta, 16, hipMemcpyDeviceToDevice, st));
   return CUOT_OK;
 }
 

@@ -83,7 +83,10 @@ hipError_t cuot_launch_lpn_batch(const void* tabs_d, const int64_t* wg_start_d, 
 // Quasi-cyclic encoder (qc.hip).
 int cuot_qc_log_len(int64_t n);
 size_t cuot_qc_scratch_bytes_for(int64_t n);
-hipError_t cuot_launch_qc_prepare(const uint8_t* a_bits, int64_t n, uint32_t* ahat, void* scratch, hipStream_t st);
+// transform = false: only a's bits for the matrix-core encoder, for callers
+// whose encodes run in the same call and take it (cuot_qc_mfma_selected)
+hipError_t cuot_launch_qc_prepare(const uint8_t* a_bits, int64_t n, uint32_t* ahat, void* scratch, bool transform,
+                                  hipStream_t st);
 hipError_t cuot_launch_qc_encode(const uint32_t* ahat, int64_t n, const void* x, void* y, void* scratch,
                                  hipStream_t st);
 // Batches of instances with the same transform length 2^m (one launch per
@@ -101,7 +104,7 @@ struct QcPrep {
 size_t cuot_qc_batch_scratch_bytes(int m, int B);
 bool cuot_qc_batchable(int m);   // B > 1 allowed for transform length 2^m
 hipError_t cuot_qc_configure();  // one-time device set-up (outside graph capture)
-hipError_t cuot_launch_qc_prepare_batch(const QcPrep* prep_d, int B, int m, hipStream_t st);
+hipError_t cuot_launch_qc_prepare_batch(const QcPrep* prep_d, int B, int m, bool transform, hipStream_t st);
 // nmax: the largest n of the batch (host side)
 hipError_t cuot_launch_qc_encode_batch(const QcIo* io_d, const uint32_t* const* ahats_d, int B, int m, int64_t nmax,
                                        void* scratch, hipStream_t st);
@@ -157,17 +160,31 @@ struct CuotKnobs {
 const CuotKnobs& cuot_knobs();
 
 // Protocol glue (proto.hip).
-hipError_t cuot_launch_setup_fix(blk* delta, const blk* alpha_blocks, int64_t t, int h, uint8_t* choice,
-                                 int64_t* pos, uint32_t* a_words, int64_t n, int64_t a_words_total,
-                                 hipStream_t st);
+// What an instance derives from its seed (rk), one launch.  NULL parts are
+// left out: pos, a_words (n bits, padded to ((n + 127) / 128 + 1) blocks) and
+// m0b / m1b (SOT), K / Mr / kkp (Ferret); t may be 0 (no trees).
+struct SetupArgs {
+  blk* delta;
+  blk* delta_out;  // a second copy for the caller, or NULL
+  int64_t t;
+  int h;
+  blk* roots;
+  uint8_t* choice;
+  int64_t* pos;
+  uint32_t* a_words;
+  int64_t n;
+  blk *m0b, *m1b;
+  int64_t k;
+  blk *K, *Mr, *kkp;
+};
+hipError_t cuot_launch_setup(const uint32_t rk[44], const SetupArgs& p, hipStream_t st);
+// csum / fin NULL: the masked rows only
 hipError_t cuot_launch_sot_msgs(const blk* sums, const blk* m0b, const blk* m1b, const blk* delta, int64_t t,
-                                int h, blk* M0, blk* M1, hipStream_t st);
+                                int h, blk* M0, blk* M1, const uint8_t* choice, blk* csum, blk* fin, hipStream_t st);
 hipError_t cuot_launch_sot_recv_prep(const uint8_t* choice, const blk* M0, const blk* M1, const blk* m0b,
                                      const blk* m1b, int64_t t, int h, blk* csum, blk* fin, hipStream_t st);
 hipError_t cuot_launch_ferret_sums(const blk* sums, const blk* delta, const uint8_t* choice, int64_t t, int h,
                                    blk* ssum, blk* csum, blk* lsum, blk* rsum, hipStream_t st);
-hipError_t cuot_launch_ferret_boot(blk* K, blk* Mr, const uint8_t* cbits, const blk* delta, int64_t k,
-                                   hipStream_t st);
 
 // Malicious-security consistency check of a Ferret MPCOT (consist.hip):
 // per-tree V, W, chi_alpha into vwc (3 t blocks), then both parties' check

@@ -1587,22 +1587,23 @@ size_t cuot_qc_batch_scratch_bytes(int m, int B) {
   return ((size_t)B * 64 + CONV_G) * ((size_t)1 << m) * 16;
 }
 
-hipError_t cuot_launch_qc_prepare(const uint8_t* a_bits, int64_t n, uint32_t* ahat, void* scratch, hipStream_t st) {
+hipError_t cuot_launch_qc_prepare(const uint8_t* a_bits, int64_t n, uint32_t* ahat, void* scratch, bool transform,
+                                  hipStream_t st) {
   (void)scratch;
   QcPrep p1;
   p1.a_bits = a_bits;
   p1.ahat = ahat;
   p1.n = n;
   const int m = cuot_qc_log_len(n);
-  hipError_t e = prepare_batch(nullptr, p1, 1, m, st);
+  hipError_t e = transform ? prepare_batch(nullptr, p1, 1, m, st) : hipSuccess;
   if (e == hipSuccess && cuot_qc_mfma_eligible(n)) e = cuot_launch_qc_keep_bits(nullptr, p1, 1, m, n, st);
   return e;
 }
 
-hipError_t cuot_launch_qc_prepare_batch(const QcPrep* prep_d, int B, int m, hipStream_t st) {
+hipError_t cuot_launch_qc_prepare_batch(const QcPrep* prep_d, int B, int m, bool transform, hipStream_t st) {
   QcPrep p1;
   memset(&p1, 0, sizeof(p1));
-  hipError_t e = prepare_batch(prep_d, p1, B, m, st);
+  hipError_t e = transform ? prepare_batch(prep_d, p1, B, m, st) : hipSuccess;
   // members small enough for the matrix-core encoder also keep a's bits
   const int64_t nlo = ((int64_t)1 << (m + 2)) + 1, nhi = (int64_t)1 << (m + 3);
   if (e == hipSuccess && cuot_qc_mfma_eligible(nlo))

@@ -97,7 +97,7 @@ struct cuot_ferret_session {
   blk* vwc = nullptr;      // per-tree V, W, chi_alpha (3 t blocks)
   uint8_t* chk = nullptr;  // x' (128), digests (2 x 32), ok (int32)
   char* mem = nullptr;
-  blk *delta, *boot_s, *boot_r, *P0, *P1, *Pr, *roots, *sums, *csum, *ssum, *cbits, *kkp;
+  blk *delta, *boot_s, *boot_r, *P0, *P1, *Pr, *roots, *sums, *csum, *ssum, *kkp;
   blk* part;  // scratch of the receiver's split trees, or NULL
   uint8_t* bits;
 };
@@ -124,7 +124,6 @@ size_t carve_session(cuot_ferret_session* s, char* base) {
   s->sums = (blk*)take((size_t)2 * t * h * 16);
   s->csum = (blk*)take((size_t)t * h * 16);
   s->ssum = (blk*)take((size_t)t * 16);
-  s->cbits = (blk*)take((size_t)((s->M + 127) / 128) * 16);
   s->kkp = (blk*)take((size_t)2 * s->plan.cfg.k * 16);
   s->vwc = (blk*)take((size_t)3 * t * 16);
   s->chk = (uint8_t*)take(256);
@@ -325,11 +324,13 @@ extern "C" int cuot_ferret_session_new(cuot_ctx* ctx, const cuot_ferret_config* 
   uint32_t rk[44];
   cuot_aes_expand_host((const uint8_t*)&cfg->seed, rk);
   hipStream_t st = ctx->stream;
-  hipError_t e = cuot_launch_prg(rk, 0, 0, 1, s->delta, st);
-  if (!e) e = cuot_launch_setup_fix(s->delta, nullptr, 0, cfg->h, nullptr, nullptr, nullptr, 0, 0, st);
-  if (!e) e = cuot_launch_prg(rk, 7, 0, s->M, s->boot_s, st);
-  if (!e) e = cuot_launch_prg(rk, 8, 0, (s->M + 127) / 128, s->cbits, st);
-  if (!e) e = cuot_launch_ferret_boot(s->boot_s, s->boot_r, (const uint8_t*)s->cbits, s->delta, s->M, st);
+  SetupArgs p;
+  memset(&p, 0, sizeof(p));
+  p.delta = s->delta;
+  p.k = s->M;
+  p.K = s->boot_s;
+  p.Mr = s->boot_r;
+  hipError_t e = cuot_launch_setup(rk, p, st);
   if (!e) e = hipStreamSynchronize(st);
   if (e) {
     session_destroy(s);
