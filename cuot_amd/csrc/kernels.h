@@ -108,6 +108,18 @@ hipError_t cuot_launch_qc_prepare_batch(const QcPrep* prep_d, int B, int m, bool
 // nmax: the largest n of the batch (host side)
 hipError_t cuot_launch_qc_encode_batch(const QcIo* io_d, const uint32_t* const* ahats_d, int B, int m, int64_t nmax,
                                        void* scratch, hipStream_t st);
+// The product on Frobenius orbits (qc_fa.hip), 2^12 < n <= 2^24: K = log2 of the
+// product's padded length (m + 4 for the transform length 2^m).
+bool cuot_qc_fa_selected(int64_t n);
+hipError_t cuot_qc_fa_configure();
+size_t cuot_qc_fa_scratch_bytes(int64_t n, int B);
+hipError_t cuot_launch_qc_fa_prepare(const QcPrep* pr, QcPrep pr1, int B, int K, hipStream_t st);
+hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ahat1, const uint32_t* const* ahats, int B,
+                                    int K, int64_t nmax, void* scratch, hipStream_t st);
+// novel-basis conversion of ntiles row strings of 2^mp bits in place (qc.hip);
+// tpi strings per instance, instances inst_words apart
+hipError_t cuot_launch_conv_rows(unsigned cap, hipStream_t st, uint32_t* Bw, int64_t tile_words, int64_t ntiles,
+                                 int64_t tpi, int64_t inst_words, int mp, int inverse);
 // Small codes on the matrix cores (qc_mfma.hip).  For 17 <= n <= 2^16 the
 // prepared words are the 2^m transform words followed by a's n bits, so either
 // encoder can run on them; the encode picks by cuot_qc_mfma_selected.

@@ -4,6 +4,10 @@
 // reference computes a float32 cuFFT convolution instead,
 // silent/quasi_cyclic.cu:11-49,118-128, whose parity is inexact at this size).
 //
+// This file holds the form for n <= 2^12 and n > 2^24; in between the product on
+// Frobenius orbits (qc_fa.hip) takes half the field elements (its points run
+// out above 2^26, its row strings at 2^24; n = 2^24 8.8 -> 7.3 ms a party).
+//
 // Algorithm: binary polynomial product a(x) * e1(x) by an additive FFT over
 // GF(2^32) (Lin-Chung-Han novel-basis FFT on a Cantor basis), then the fold
 // mod x^n - 1.  Bits are packed 16 per field element (chunk polynomials of
@@ -232,11 +236,6 @@ struct BarrierSync {
   __device__ void operator()() const { __syncthreads(); }
 };
 
-// fold (inverse mode, odd tiles = the upper half q of a row): after the
-// conversion, q is replaced by q ^ XOR_{e in E} rot(q, e), E = the lower terms
-// of s_mp, rotations cyclic over the 2^mp-bit string.  The lower half r then
-// satisfies r ^ T(q) = (F mod X^(2^mp) + 1) for F = r + s_mp q, the product
-// folded at half its length (s_mp = X^(2^mp) + sum_E X^e).
 // PAD (strings of >= 2^10 coefficients): the string sits in LDS with four pad
 // words after every 32, and levels 9..0 run per 1024-bit block in registers.
 // MULTI (PAD, strings shorter than 2^20): a workgroup converts S = 1024 /
@@ -279,49 +278,10 @@ __device__ __forceinline__ void rows_load(const uint32_t* g, uint32_t* sw, int64
   }
 }
 
-// fold (inverse, odd tiles): the terms e = 2^j (j a proper submask of mp) are
-// enumerated in the loop; tile_words is a power of two and a multiple of 4
 template <bool PAD, bool INW>
-__device__ __forceinline__ void rows_store(uint32_t* g, const uint32_t* sw, int64_t tile_words, int mp, bool fold_q,
-                                           int lt, int tps) {
+__device__ __forceinline__ void rows_store(uint32_t* g, const uint32_t* sw, int64_t tile_words, int lt, int tps) {
   const int n4 = (int)(tile_words >> 2);
-  if (fold_q) {
-    const int64_t wm = tile_words - 1;
-    uint4* g4 = (uint4*)g;
-    auto word = [&](int64_t i) { return sw[cbp_at<PAD>(i & wm)]; };
-    auto quad = [&](int64_t i) { return *(const uint4*)(sw + cbp_at<PAD>(i & wm)); };
-    for (int f = lt; f < n4; f += tps) {
-      const int64_t w = 4 * (int64_t)f;
-      // the terms below one word (e < 32) all shift the quad at w with the
-      // word before it: both are read once
-      const uint4 q0 = quad(w);
-      const uint32_t pv0 = word(w - 1);
-      uint4 acc = q0;
-      for (int j = 0; j < mp; j++) {
-        if (j & ~mp) continue;
-        const int64_t eo = ((int64_t)1 << j) >> 5;
-        const int eb = j < 5 ? 1 << j : 0;
-        uint4 c4;
-        if (eo == 0) {
-          c4 = q0;
-        } else if ((eo & 3) == 0) {
-          c4 = quad(w - eo);
-        } else {
-          c4 = make_uint4(word(w - eo), word(w - eo + 1), word(w - eo + 2), word(w - eo + 3));
-        }
-        if (eb) {
-          const uint32_t pv = pv0;  // eb != 0 only for j < 5, where eo = 0
-          acc.x ^= (c4.x << eb) | (pv >> (32 - eb));
-          acc.y ^= (c4.y << eb) | (c4.x >> (32 - eb));
-          acc.z ^= (c4.z << eb) | (c4.y >> (32 - eb));
-          acc.w ^= (c4.w << eb) | (c4.z >> (32 - eb));
-        } else {
-          acc = x4(acc, c4);
-        }
-      }
-      g4[f] = acc;
-    }
-  } else if ((tile_words & 3) == 0) {
+  if ((tile_words & 3) == 0) {
     uint4* g4 = (uint4*)g;
     for (int f = lt; f < n4; f += tps) {
       const uint4 v = *(const uint4*)(sw + cbp_at<PAD>(4 * (int64_t)f));
@@ -334,8 +294,7 @@ __device__ __forceinline__ void rows_store(uint32_t* g, const uint32_t* sw, int6
 
 template <bool PAD, bool INV, bool MULTI>
 __global__ __launch_bounds__(1024) void qc_conv_rows(uint32_t* __restrict__ Bw, int64_t tile_words, int64_t ntiles,
-                                                     int64_t tiles_per_inst, int64_t inst_words, int mp,
-                                                     int fold) {
+                                                     int64_t tiles_per_inst, int64_t inst_words, int mp) {
   static_assert(PAD || !MULTI, "several strings per workgroup need the blocked form");
   extern __shared__ uint32_t sw_all[];
   if constexpr (!MULTI) {
@@ -347,8 +306,7 @@ __global__ __launch_bounds__(1024) void qc_conv_rows(uint32_t* __restrict__ Bw, 
         cbp_convert<true, INV>(sw_all, 0, mp, threadIdx.x, blockDim.x, BarrierSync());
       else
         cbt_convert(sw_all, mp, INV, threadIdx.x, blockDim.x, BarrierSync());
-      rows_store<PAD, false>(g, sw_all, tile_words, mp, fold && ((tile % tiles_per_inst) & 1), threadIdx.x,
-                             blockDim.x);
+      rows_store<PAD, false>(g, sw_all, tile_words, threadIdx.x, blockDim.x);
       __syncthreads();
     }
   } else {
@@ -374,7 +332,7 @@ __global__ __launch_bounds__(1024) void qc_conv_rows(uint32_t* __restrict__ Bw, 
       cbp_convert<true, INV, false>(sw_all, base, mp, lt, tps, BarrierSync());
       if (live)
         rows_store<true, !INV>(Bw + (int64_t)(tile / tpi) * inst_words + (int64_t)(tile % tpi) * tile_words, sw,
-                               tile_words, mp, fold && ((tile % tpi) & 1), lt, tps);
+                               tile_words, lt, tps);
       __syncthreads();
     }
   }
@@ -388,7 +346,7 @@ size_t row_lds_bytes(int64_t tile_words, int mp) {
 }
 
 hipError_t launch_conv_rows(unsigned cap, hipStream_t st, uint32_t* Bw, int64_t tile_words, int64_t ntiles,
-                            int64_t tpi, int64_t inst_words, int mp, int inverse, int fold) {
+                            int64_t tpi, int64_t inst_words, int mp, int inverse) {
   if (row_pad(mp) && (tile_words < 32 || tile_words > 32 * 1024)) return hipErrorInvalidValue;
   const size_t lds = row_lds_bytes(tile_words, mp);
   const bool multi = row_pad(mp) && tile_words < 32 * 1024;
@@ -397,7 +355,7 @@ hipError_t launch_conv_rows(unsigned cap, hipStream_t st, uint32_t* Bw, int64_t 
   const unsigned grid = (unsigned)(need < (int64_t)cap ? (need < 1 ? 1 : need) : cap);
 #define CONV_ROWS_LAUNCH(PAD, INV, MULTI)                                                                    \
   hipLaunchKernelGGL((qc_conv_rows<PAD, INV, MULTI>), dim3(grid), dim3(1024), lds, st, Bw, tile_words, ntiles, \
-                     tpi, inst_words, mp, fold)
+                     tpi, inst_words, mp)
   if (multi) {
     if (inverse)
       CONV_ROWS_LAUNCH(true, true, true);
@@ -1050,86 +1008,6 @@ __global__ void qc_output(const uint4* __restrict__ X, int64_t M, int m, int64_t
   }
 }
 
-// Output from the row layout after the folded inverse conversion (n = 16 h
-// chunks, h = M/2): G_p = r_p ^ T(q_p) is the product folded mod x^n - 1 for
-// coefficient plane p, and
-//   y[16c + b] = x0[16c + b] ^ G_b[c] ^ G_{b+16}[(c - 1) mod h]   (G_31 = 0),
-// the second term being the overlap of chunk c-1's upper 15 planes.
-// Step 1 (qc_rows_fold): per plane pair b and a tile of 32 words (1024
-// chunks) of every row, combine the four row strings in LDS and bit-transpose
-// them into the element layout D[b][c] (16 planes of h elements).
-// Step 2 (qc_output_planes): y[16c + b] = x0[16c + b] ^ D[b][c], interleaving
-// the 16 planes through LDS so that both sides are contiguous.
-__global__ __launch_bounds__(256) void qc_rows_fold(const uint32_t* __restrict__ Bw, int64_t hw, int64_t inst_words,
-                                                    uint4* __restrict__ D, int64_t dps) {
-  __shared__ uint32_t sm[128][33];
-  const int b = (int)blockIdx.y;
-  const uint32_t* rb = Bw + (int64_t)b * 128 * (2 * hw);
-  const uint32_t* rh = Bw + (int64_t)(b + 16) * 128 * (2 * hw);
-  D += (int64_t)b * dps;
-  const int lane = threadIdx.x & 31;
-  const int grp = threadIdx.x >> 5;
-  const int64_t ntile = hw / 32;
-  for (int64_t t = blockIdx.x; t < ntile; t += gridDim.x) {
-    const int64_t w0 = t * 32;
-    // 128 rows x 32 words: thread f -> row f >> 3, words 4 (f & 7) .. + 3
-    for (int f = threadIdx.x; f < 128 * 8; f += 256) {
-      const int row = f >> 3, wq = (f & 7) * 4;
-      const int64_t ro = (int64_t)row * (2 * hw) + w0 + wq;
-      const uint4 a = x4(*(const uint4*)(rb + ro), *(const uint4*)(rb + ro + hw));
-      uint4 h = z4();
-      uint32_t hp = 0;
-      if (b < 15) {
-        h = x4(*(const uint4*)(rh + ro), *(const uint4*)(rh + ro + hw));
-        const int64_t rp = (int64_t)row * (2 * hw) + ((w0 + wq - 1) & (hw - 1));
-        hp = rh[rp] ^ rh[rp + hw];
-      }
-      uint32_t* S = &sm[row][wq];
-      S[0] = a.x ^ (h.x << 1) ^ (hp >> 31);
-      S[1] = a.y ^ (h.y << 1) ^ (h.x >> 31);
-      S[2] = a.z ^ (h.z << 1) ^ (h.y >> 31);
-      S[3] = a.w ^ (h.w << 1) ^ (h.z >> 31);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int tl = grp * 4 + r;
-      uint4 v;
-      v.x = cuot_transpose32(sm[0 * 32 + lane][tl], lane);
-      v.y = cuot_transpose32(sm[1 * 32 + lane][tl], lane);
-      v.z = cuot_transpose32(sm[2 * 32 + lane][tl], lane);
-      v.w = cuot_transpose32(sm[3 * 32 + lane][tl], lane);
-      D[(w0 + tl) * 32 + lane] = v;
-    }
-    __syncthreads();
-  }
-}
-
-__global__ __launch_bounds__(256) void qc_output_planes(const uint4* __restrict__ D, int64_t dps, int64_t h,
-                                                        const QcIo* __restrict__ io, QcIo io1) {
-  __shared__ uint4 sm[16][65];
-  const QcIo q = io ? io[blockIdx.y] : io1;
-  const int64_t ntile = h / 64;
-  for (int64_t t = blockIdx.x; t < ntile; t += gridDim.x) {
-    const int64_t c0 = t * 64;
-    // D[b][c0 .. c0 + 64) for 16 planes: 1024 elements, 4 per thread
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int f = (int)threadIdx.x + u * 256;
-      const int bb = f >> 6, cc = f & 63;
-      sm[bb][cc] = D[(int64_t)bb * dps + c0 + cc];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int f = (int)threadIdx.x + u * 256;  // block 16 c0 + f: chunk f >> 4, plane f & 15
-      const int64_t i = 16 * c0 + f;
-      q.y[i] = x4(q.x[i], sm[f & 15][f >> 4]);
-    }
-    __syncthreads();
-  }
-}
-
 unsigned grid_for(int64_t total, int64_t cap = 1 << 16) {
   int64_t g = (total + 255) / 256;
   if (g > cap) g = cap;
@@ -1267,7 +1145,7 @@ hipError_t conv_forward(Bufs b, int64_t M, int P, int mp, hipStream_t st) {
   if (e != hipSuccess) return e;
   const int64_t tpi = (int64_t)P * 128;
   cuot_rec_begin(st, "qc_conv_rows", 2.0 * (double)tpi * b.B * row_words * 4);
-  e = launch_conv_rows(4096, st, b.Bw, row_words, tpi * b.B, tpi, inst_words, mp, 0, 0);
+  e = launch_conv_rows(4096, st, b.Bw, row_words, tpi * b.B, tpi, inst_words, mp, 0);
   cuot_rec_end(st);
   if (e != hipSuccess) return e;
   return cuot_launch_transpose_planes2(b.Bw, Mp, b.X, true, b.B * P, P, inst_words, 128 * row_words, b.XS, M, st);
@@ -1275,7 +1153,7 @@ hipError_t conv_forward(Bufs b, int64_t M, int P, int mp, hipStream_t st) {
 
 // inverse conversion levels 0..mtop-1 of planes [0, P) of the full polynomial
 // (2^(mtop+1) elements): each half string is converted on its own
-hipError_t conv_inverse(Bufs b, int64_t M, int P, int mtop, bool fold, hipStream_t st) {
+hipError_t conv_inverse(Bufs b, int64_t M, int P, int mtop, hipStream_t st) {
   if (!row_path(mtop)) return conv_inverse_elem(b, M, P, mtop, st);
   const int64_t row_words = M / 32;
   const int64_t inst_words = b.XS * 4;
@@ -1285,9 +1163,9 @@ hipError_t conv_inverse(Bufs b, int64_t M, int P, int mtop, bool fold, hipStream
   const int64_t tile_words = row_words / 2;
   const int64_t tpi = (int64_t)P * 128 * 2;
   cuot_rec_begin(st, "qc_conv_rows", 2.0 * (double)tpi * b.B * tile_words * 4);
-  e = launch_conv_rows(8192, st, b.Bw, tile_words, tpi * b.B, tpi, inst_words, mtop, 1, fold ? 1 : 0);
+  e = launch_conv_rows(8192, st, b.Bw, tile_words, tpi * b.B, tpi, inst_words, mtop, 1);
   cuot_rec_end(st);
-  if (e != hipSuccess || fold) return e;  // folded: the output is read from the row layout
+  if (e != hipSuccess) return e;
   return cuot_launch_transpose_planes2(b.Bw, M, b.X, true, b.B * P, P, inst_words, 128 * row_words, b.XS, M, st);
 }
 
@@ -1483,6 +1361,8 @@ hipError_t encode_batch(const QcIo* io, QcIo io1, const uint32_t* ahat1, const u
   hipError_t e = configure_lds();
   if (e != hipSuccess) return e;
   if (B > 1 && !row_path(m - 1)) return hipErrorInvalidValue;
+  if (cuot_qc_fa_selected(((int64_t)1 << (m + 2)) + 1))
+    return cuot_launch_qc_fa_encode(io, io1, ahat1, ahats, B, m + 4, io ? (int64_t)1 << (m + 3) : io1.n, scratch, st);
   const int64_t M = (int64_t)1 << m;
   Bufs b = bufs(scratch, M, B);
   cuot_rec_begin(st, "qc_pack_x", 2.0 * 16.0 * (double)(M >> 1) * 16 * B);
@@ -1502,21 +1382,7 @@ hipError_t encode_batch(const QcIo* io, QcIo io1, const uint32_t* ahat1, const u
     b.X = b.Bw;
     b.Bw = t;
   }
-  // n = 16 * M/2 (n a power of two): fold in the row layout and write y from it
-  const bool fold = !io && io1.n == 8 * M && m >= 11 && row_path(m - 1) && B == 1;
-  if ((e = conv_inverse(b, M, 31, m - 1, fold, st))) return e;
-  if (fold) {
-    const int64_t h = M >> 1, hw = h / 32;
-    cuot_rec_begin(st, "qc_rows_fold", 31.0 * 16.0 * (double)M + 16.0 * 16.0 * (double)h);
-    hipLaunchKernelGGL(qc_rows_fold, dim3(capg(hw / 32, 1024), 16), dim3(256), 0, st, (const uint32_t*)b.Bw, hw,
-                       b.XS * 4, (uint4*)b.X, M);
-    cuot_rec_end(st);
-    cuot_rec_begin(st, "qc_output_planes", 48.0 * (double)io1.n);
-    hipLaunchKernelGGL(qc_output_planes, dim3(capg(h / 64, 8192), 1), dim3(256), 0, st, (const uint4*)b.X, M, h, io,
-                       io1);
-    cuot_rec_end(st);
-    return hipGetLastError();
-  }
+  if ((e = conv_inverse(b, M, 31, m - 1, st))) return e;
   const int64_t nmax = io ? (M / 2) * 16 : io1.n;  // grid covers the largest n of the class
   cuot_rec_begin(st, "qc_output", 32.0 * (double)nmax * B);
     hipLaunchKernelGGL(qc_output, dim3(grid_for(nmax), (unsigned)B), dim3(256), 0, st, (const uint4*)b.X, M, m, b.XS,
@@ -1528,6 +1394,7 @@ hipError_t encode_batch(const QcIo* io, QcIo io1, const uint32_t* ahat1, const u
 hipError_t prepare_batch(const QcPrep* pr, QcPrep pr1, int B, int m, hipStream_t st) {
   hipError_t e = configure_lds();
   if (e != hipSuccess) return e;
+  if (cuot_qc_fa_selected(((int64_t)1 << (m + 2)) + 1)) return cuot_launch_qc_fa_prepare(pr, pr1, B, m + 4, st);
   const int64_t M = (int64_t)1 << m;
   const int64_t Mh = M >> 1;
   // several polynomials: one workgroup each; a single one keeps the
@@ -1570,6 +1437,16 @@ hipError_t prepare_batch(const QcPrep* pr, QcPrep pr1, int B, int m, hipStream_t
 
 }  // namespace
 
+hipError_t cuot_launch_conv_rows(unsigned cap, hipStream_t st, uint32_t* Bw, int64_t tile_words, int64_t ntiles,
+                                 int64_t tpi, int64_t inst_words, int mp, int inverse) {
+  hipError_t e = configure_lds();
+  if (e != hipSuccess) return e;
+  cuot_rec_begin(st, "qc_conv_rows", 2.0 * (double)ntiles * tile_words * 4);
+  e = launch_conv_rows(cap, st, Bw, tile_words, ntiles, tpi, inst_words, mp, inverse);
+  cuot_rec_end(st);
+  return e;
+}
+
 int cuot_qc_log_len(int64_t n) {
   const int64_t nc = (n + 15) / 16;
   int m = 1;
@@ -1581,9 +1458,15 @@ size_t cuot_qc_scratch_bytes_for(int64_t n) { return cuot_qc_batch_scratch_bytes
 
 bool cuot_qc_batchable(int m) { return row_path(m - 1); }
 
-hipError_t cuot_qc_configure() { return configure_lds(); }
+hipError_t cuot_qc_configure() {
+  hipError_t e = configure_lds();
+  return e ? e : cuot_qc_fa_configure();
+}
 
+// the transform length 2^m holds the n of (2^(m+2), 2^(m+3)]
 size_t cuot_qc_batch_scratch_bytes(int m, int B) {
+  const int64_t nlo = ((int64_t)1 << (m + 2)) + 1;
+  if (cuot_qc_fa_selected(nlo)) return cuot_qc_fa_scratch_bytes(nlo, B);
   return ((size_t)B * 64 + CONV_G) * ((size_t)1 << m) * 16;
 }
 

@@ -1,0 +1,925 @@
+// qc_fa.hip -- the quasi-cyclic encoder's product for 2^12 < n <= 2^24: an
+// additive FFT over GF(2^32) on one point per Frobenius orbit.
+//
+//     y_i = x_i ^ XOR_{k < n} a_{(i-k) mod n} x_{n+k},   i < n
+//
+// (the same map as qc.hip; the reference's float cuFFT version is
+// silent/quasi_cyclic.cu:118-128), for all 128 bit-rows at once.
+//
+// The operands have coefficients in GF(2), so their values at the 32 conjugates
+// of a point of GF(2^32) are conjugates of each other: a product of 2^K
+// coefficients is fixed by its values at 2^(K-5) points, one per orbit, 32 bits
+// each.  Packing 16 coefficients per GF(2^32) element instead (qc.hip) spends
+// twice the elements, half of every element being room for the chunk products.
+// The idea is the Frobenius additive FFT of Li, Chen, Kuo, Cheng and Yang
+// (ISSAC 2018); the points and the bitsliced form are chosen here:
+//
+//   points  beta_a + span{beta_i : i < c or c < i <= K-5},  c = min(K-5, 15),
+//           a = 16 + c, on the Cantor basis of qc_fa.h.  Their images under
+//           s_c are beta_16 + span{beta_1, ...}, of degree 32 and pairwise not
+//           conjugate for K <= 27, so the orbits are full and distinct.
+//   layers  index bit k of a polynomial in the novel basis is evaluated with
+//           s_k(point) = beta_{a-k} + C(bits above k), C(g) = sum g_b beta_{b+1}:
+//     k = K-2 .. K-4   the same constant at every point: eight coefficients
+//                      become one GF(2^16) value (a fixed 16 x 8 map; 16 x 16
+//                      for the full product's four bits)
+//     k = K-5 .. c+1   butterflies over GF(2^16) (K > 20)
+//     k = c            the constant has a theta part of 1 and no free bit: two
+//                      GF(2^16) values u, v become u + delta v + theta v
+//     k = c-1 .. 0     butterflies over GF(2^32)
+//
+// Encode (per party), blocks x_{n+i} being coefficient i of all 128 rows:
+//   128-row bit transpose, novel-basis conversion of every row string in LDS
+//   (conv_fast.h), transpose back (levels of 2^20 coefficients and more act on
+//   the blocks before that); a first pass (GF(2^16) layers, halves of the
+//   elements apart), passes of GF(2^32) layers, the lowest of them with the
+//   product by A^ and the inverse layers; the mirror image back; y.
+// Between passes the data is element major: element e is 32 planes x 16 bytes
+// in one run, so that every tile reads and writes whole lines.
+#include <string.h>
+
+#include "conv_fast.h"
+#include "kernels.h"
+#include "qc_fa.h"
+#include "transpose32.h"
+
+namespace {
+
+__constant__ uint32_t c_fa_beta[32];
+__constant__ uint32_t c_fa_pack[FA_KC_MAX + 1][8];
+
+constexpr int FA_KMIN = 14, FA_KMAX = 25;
+constexpr int FA_STR = 20;  // longest row string converted in LDS (128 KB, 144 KB padded)
+
+CUOT_DEV uint4 x4(uint4 a, uint4 b) { return make_uint4(a.x ^ b.x, a.y ^ b.y, a.z ^ b.z, a.w ^ b.w); }
+CUOT_DEV uint4 z4() { return make_uint4(0, 0, 0, 0); }
+
+// ---- twiddles -----------------------------------------------------------------
+// C(g) from three 256-entry tables of the low 24 bits of g
+constexpr int FA_CTAB = 3 * 256;
+
+CUOT_DEV void fa_ctab_fill(uint32_t* tab, int tid, int nth) {
+  for (int i = tid; i < FA_CTAB; i += nth) {
+    const int q = i >> 8, v = i & 255;
+    uint32_t c = 0;
+    for (int b = 0; b < 8; b++)
+      if ((v >> b) & 1) c ^= c_fa_beta[8 * q + b + 1];
+    tab[i] = c;
+  }
+}
+
+CUOT_DEV uint32_t fa_ctab(const uint32_t* tab, uint32_t g) {
+  return tab[g & 255] ^ tab[256 + ((g >> 8) & 255)] ^ tab[512 + ((g >> 16) & 255)];
+}
+
+// ---- passes ---------------------------------------------------------------------
+// LDS tile: TC = 2^R * C elements (2^R of them 2^lo apart times C consecutive
+// ones) of NP planes x 4 words, 4 pad words per element.  NP = 32: whole
+// elements, layers k < c.  NP = 16: one half (blockIdx.z) of the elements, the
+// layers above c, where the halves transform apart under GF(2^16) constants.
+enum { FA_FWD = 0, FA_INV = 1, FA_FUSED = 2 };
+
+struct FaArgs {
+  const uint4* nat_in;  // natural order coefficients (first pass)
+  uint4* nat_out;       // natural order coefficients (last inverse pass)
+  uint4* E;             // element-major data
+  const uint32_t* ahat;
+  const uint32_t* const* ahats;  // per-instance A^ (batch) or NULL
+  int64_t XS;                    // instance stride of all three buffers in blocks
+  int K, c, a;
+  int lo, R, lgC;
+  int mode;
+  int first, last;  // reads nat_in / writes nat_out
+  int contract;     // the layer k = c before the forward or after the inverse layers
+};
+
+template <int NP>
+constexpr int fa_stride() {
+  return NP * 4 + 4;
+}
+template <int NP>
+constexpr int fa_tile() {
+  return 4096 / NP;  // elements per tile: 64 KB of data, two workgroups per CU
+}
+template <int NP>
+constexpr int fa_threads() {
+  return NP == 16 ? 512 : 256;  // one (butterfly, word) task per lane and layer
+}
+template <int NP>
+constexpr int fa_ld() {
+  return 4096 / fa_threads<NP>();  // staged 16-byte words per lane
+}
+
+// LDS slot of tile element e: the butterflies of the lowest tile layers touch
+// elements whose slots share their residue mod 8 (the element stride is 4 mod
+// 64 banks); reflecting every odd group of eight spreads them
+CUOT_DEV int fa_slot(int e) { return e ^ (((e >> 3) & 1) * 7); }
+
+template <int NP>
+__device__ __forceinline__ void fa_mul(uint32_t cst_lane, bool uniform, const uint32_t* xv, uint32_t* acc) {
+  const uint32_t cst = uniform ? __builtin_amdgcn_readfirstlane(cst_lane) : cst_lane;
+  if constexpr (NP == 16)
+    gf16_mulc(xv, cst, acc);
+  else
+    gf32_mulc<false>(xv, cst, acc);
+}
+
+template <int NP>
+__device__ __forceinline__ void fa_layer(const FaArgs& a, uint32_t* lds, const uint32_t* ctab, int64_t ebase, int s,
+                                         bool inv) {
+  constexpr int ST = fa_stride<NP>();
+  const int C = 1 << a.lgC;
+  const int k = NP == 16 ? a.c + 1 + s : a.lo + s;  // coefficient index bit
+  const uint32_t off = c_fa_beta[a.a - k];
+  const int ntask = (1 << (a.R - 1)) * C * 4;
+  for (int tau = threadIdx.x; tau < ntask; tau += fa_threads<NP>()) {
+    const int w = tau & 3;
+    const int cc = (tau >> 2) & (C - 1);
+    const int bp = (tau >> 2) >> a.lgC;
+    const int tu = ((bp >> s) << (s + 1)) | (bp & ((1 << s) - 1));
+    const int tv = tu | (1 << s);
+    uint32_t g;
+    if constexpr (NP == 16) {
+      g = (uint32_t)(tu >> (s + 1));
+    } else {
+      const uint32_t e = (uint32_t)ebase | (uint32_t)(tu << a.lo);  // columns lie below bit k
+      g = ((e >> a.c) << (a.c - k)) | ((e & ((1u << a.c) - 1)) >> (k + 1));
+    }
+    uint32_t* pu = lds + fa_slot(tu * C + cc) * ST + w;
+    uint32_t* pv = lds + fa_slot(tv * C + cc) * ST + w;
+    uint32_t xv[NP], acc[NP];
+    if (inv) {
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        xv[p] = pv[4 * p] ^ pu[4 * p];
+        pv[4 * p] = xv[p];
+      }
+    } else {
+#pragma unroll
+      for (int p = 0; p < NP; p++) xv[p] = pv[4 * p];
+    }
+    const uint32_t g0 = __builtin_amdgcn_readfirstlane(g);
+    if (__all(g == g0))
+      fa_mul<NP>(off ^ fa_ctab(ctab, g0), true, xv, acc);
+    else
+      fa_mul<NP>(off ^ fa_ctab(ctab, g), false, xv, acc);
+    if (inv) {
+#pragma unroll
+      for (int p = 0; p < NP; p++) pu[4 * p] ^= acc[p];
+    } else {
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        const uint32_t un = pu[4 * p] ^ acc[p];
+        pu[4 * p] = un;
+        pv[4 * p] = xv[p] ^ un;
+      }
+    }
+  }
+  __syncthreads();
+}
+
+// layer k = c: half 0 ^= delta * half 1, delta = C(bits above c), one constant
+// for the tile (its own inverse)
+__device__ __forceinline__ void fa_contract(const FaArgs& a, uint32_t* lds, const uint32_t* ctab, int64_t ebase) {
+  constexpr int ST = fa_stride<32>();
+  const uint32_t delta = __builtin_amdgcn_readfirstlane(fa_ctab(ctab, (uint32_t)(ebase >> a.c)));
+  const int TC = 1 << (a.R + a.lgC);
+  for (int tau = threadIdx.x; tau < TC * 4; tau += fa_threads<32>()) {
+    uint32_t* pe = lds + fa_slot(tau >> 2) * ST + (tau & 3);
+    uint32_t v[16], acc[16];
+#pragma unroll
+    for (int p = 0; p < 16; p++) v[p] = pe[4 * (16 + p)];
+    gf16_mulc(v, delta, acc);
+#pragma unroll
+    for (int p = 0; p < 16; p++) pe[4 * p] ^= acc[p];
+  }
+  __syncthreads();
+}
+
+// chunk maps on the staged tile: 8 coefficient planes -> 16 coordinates, and
+// 16 coordinates -> 16 coefficient planes, per half and element word
+template <int NP, int KC, bool UN>
+__device__ __forceinline__ void fa_chunks(const FaArgs& a, uint32_t* lds) {
+  constexpr int ST = fa_stride<NP>();
+  const int TC = 1 << (a.R + a.lgC);
+  for (int tau = threadIdx.x; tau < TC * 4 * (NP / 16); tau += fa_threads<NP>()) {
+    const int w = tau & 3, h = NP == 32 ? (tau >> 2) & 1 : 0, el = tau >> (NP == 32 ? 3 : 2);
+    uint32_t* pe = lds + fa_slot(el) * ST + 64 * h + w;
+    uint32_t in[16], out[16];
+#pragma unroll
+    for (int p = 0; p < (UN ? 16 : 8); p++) in[p] = pe[4 * p];
+    if constexpr (UN)
+      fa_unpack_planes<KC>(in, out);
+    else
+      fa_pack_planes<KC>(in, out);
+#pragma unroll
+    for (int p = 0; p < 16; p++) pe[4 * p] = out[p];
+  }
+  __syncthreads();
+}
+
+// pointwise product by A^
+__device__ __forceinline__ void fa_pointwise(const FaArgs& a, const uint32_t* __restrict__ ahat, uint32_t* lds,
+                                             int64_t ebase) {
+  constexpr int ST = fa_stride<32>();
+  const int TC = 1 << (a.R + a.lgC);  // the lowest pass: consecutive elements
+  for (int tau = threadIdx.x; tau < TC * 4; tau += fa_threads<32>()) {
+    const int el = tau >> 2;
+    uint32_t* pe = lds + fa_slot(el) * ST + (tau & 3);
+    uint32_t x[32], y[32];
+#pragma unroll
+    for (int p = 0; p < 32; p++) x[p] = pe[4 * p];
+    gf32_mulc<false>(x, ahat[ebase + el], y);
+#pragma unroll
+    for (int p = 0; p < 32; p++) pe[4 * p] = y[p];
+  }
+  __syncthreads();
+}
+
+// KC: chunk maps of the first / last pass (see qc_fa.h); -1: neither
+template <int NP, int KC>
+__global__ __launch_bounds__(fa_threads<NP>()) __attribute__((amdgpu_waves_per_eu(NP == 16 ? 4 : 2))) void fa_pass(
+    FaArgs a) {
+  extern __shared__ uint32_t lds[];
+  constexpr int ST = fa_stride<NP>();
+  constexpr int NT = fa_threads<NP>();
+  constexpr int LD = fa_ld<NP>();
+  const int64_t ioff = (int64_t)blockIdx.y * a.XS;
+  uint4* E = a.E + ioff;
+  const uint4* nin = a.nat_in + ioff;
+  uint4* nout = a.nat_out + ioff;
+  const uint32_t* ahat = a.ahats ? a.ahats[blockIdx.y] : a.ahat;
+  const int h = NP == 16 ? (int)blockIdx.z : 0;
+  const int C = 1 << a.lgC;
+  const int TC = 1 << (a.R + a.lgC);
+  const int64_t cblocks = ((int64_t)1 << a.lo) >> a.lgC;
+  const int64_t ntiles = ((int64_t)1 << (a.K - 5)) / TC;
+  uint32_t* ctab = lds + TC * ST;
+  fa_ctab_fill(ctab, threadIdx.x, NT);  // read after the first barrier
+  uint4 v[LD];
+  // staging addresses come from an opaque copy of the lane index, so that the
+  // compiler recomputes them per phase instead of holding them through the
+  // layers
+  auto opaque_tid = [] {
+    int t = (int)threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+  };
+  auto tile_base = [&](int64_t tile) {
+    return ((tile >> (a.lo - a.lgC)) << (a.lo + a.R)) | ((tile & (cblocks - 1)) << a.lgC);
+  };
+  // element-major staging word f: plane fastest; element t * C + c of the tile
+  auto e_addr = [&](int64_t eb, int f, int& el) {
+    el = f / NP;
+    const int t = el >> a.lgC, c = el & (C - 1);
+    return (eb + ((int64_t)t << a.lo) + c) * 32 + 16 * h + (f % NP);
+  };
+  // natural-order staging word f: element fastest, then (half, coefficient
+  // plane) of np planes per half
+  auto n_addr = [&](int64_t eb, int f, int lgnp, int& el, int& p) {
+    el = f & (TC - 1);
+    const int hp = f >> (a.R + a.lgC);
+    const int q = hp & ((1 << lgnp) - 1), hh = NP == 32 ? hp >> lgnp : h;
+    p = (NP == 32 ? 16 * hh : 0) + q;
+    const int64_t e = eb + ((int64_t)(el >> a.lgC) << a.lo) + (el & (C - 1));
+    return ((int64_t)q << (a.K - 4)) | ((e >> a.c) << (a.c + 1)) | ((int64_t)hh << a.c) |
+           (e & (((int64_t)1 << a.c) - 1));
+  };
+  const int n4 = TC * NP;
+  auto load_tile = [&](int64_t tile) {
+    const int tid = opaque_tid();
+    const int64_t eb = tile_base(tile);
+#pragma unroll
+    for (int u = 0; u < LD; u++) {
+      const int f = tid + u * NT;
+      int el, p;
+      v[u] = z4();
+      if (KC >= 0 && a.first) {
+        if (u < LD / 2 && f < n4 / 2) v[u] = nin[n_addr(eb, f, 3, el, p)];
+      } else if (f < n4) {
+        v[u] = E[e_addr(eb, f, el)];
+      }
+    }
+  };
+  // workgroups are dealt to the 8 XCDs in turn: one XCD's take neighbouring tiles
+  const int64_t G = gridDim.x, bx = blockIdx.x;
+  const int64_t slot = (G & 7) ? bx : (bx & 7) * (G >> 3) + (bx >> 3);
+  if (slot < ntiles) load_tile(slot);
+  for (int64_t tile = slot; tile < ntiles; tile += G) {
+    const int64_t eb = tile_base(tile);
+    {
+      const int tid = opaque_tid();
+#pragma unroll
+      for (int u = 0; u < LD; u++) {
+        const int f = tid + u * NT;
+        int el, p;
+        if (KC >= 0 && a.first) {
+          if (u < LD / 2 && f < n4 / 2) {
+            n_addr(eb, f, 3, el, p);
+            *(uint4*)&lds[fa_slot(el) * ST + p * 4] = v[u];
+          }
+        } else if (f < n4) {
+          el = f / NP;
+          *(uint4*)&lds[fa_slot(el) * ST + (f % NP) * 4] = v[u];
+        }
+      }
+    }
+    __syncthreads();
+    if constexpr (KC >= 0) {
+      if (a.first) fa_chunks<NP, KC, false>(a, lds);
+    }
+    if constexpr (NP == 32) {
+      if (a.contract && a.mode == FA_FWD) fa_contract(a, lds, ctab, eb);
+    }
+    // one step loop so that the layer body is instantiated once
+    const int s_fwd = a.mode != FA_INV ? a.R : 0;
+    const int s_pw = a.mode == FA_FUSED ? 1 : 0;
+    const int s_inv = a.mode != FA_FWD ? a.R : 0;
+    for (int step = 0; step < s_fwd + s_pw + s_inv; step++) {
+      if (step == s_fwd && s_pw) {
+        if constexpr (NP == 32) fa_pointwise(a, ahat, lds, eb);
+      } else {
+        const bool inv = step >= s_fwd;
+        fa_layer<NP>(a, lds, ctab, eb, inv ? step - s_fwd - s_pw : a.R - 1 - step, inv);
+      }
+    }
+    if constexpr (NP == 32) {
+      if (a.contract && a.mode == FA_INV) fa_contract(a, lds, ctab, eb);
+    }
+    if constexpr (KC >= 0) {
+      if (a.last) fa_chunks<NP, KC, true>(a, lds);
+    }
+    uint4 w[LD];
+    const int tid = opaque_tid();
+#pragma unroll
+    for (int u = 0; u < LD; u++) {
+      const int f = tid + u * NT;
+      w[u] = z4();
+      if (f < n4) {
+        int el, p = f % NP;
+        if (KC >= 0 && a.last)
+          n_addr(eb, f, 4, el, p);
+        else
+          el = f / NP;
+        w[u] = *(const uint4*)&lds[fa_slot(el) * ST + p * 4];
+      }
+    }
+    // the next tile's loads are issued before this tile's stores
+    if (tile + G < ntiles) load_tile(tile + G);
+#pragma unroll
+    for (int u = 0; u < LD; u++) {
+      const int f = tid + u * NT;
+      if (f < n4) {
+        int el, p;
+        if (KC >= 0 && a.last)
+          nout[n_addr(eb, f, 4, el, p)] = w[u];
+        else
+          E[e_addr(eb, f, el)] = w[u];
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// ---- input: blocks x_{n+i} to 128 bit-row strings of N = 2^(K-1) bits -----------
+__global__ __launch_bounds__(256) void fa_rows_in(const QcIo* __restrict__ io, QcIo io1, int64_t N,
+                                                  uint32_t* __restrict__ rows, int64_t inst_words) {
+  __shared__ uint32_t sm[128][33];
+  const QcIo q = io ? io[blockIdx.y] : io1;
+  const uint4* in = q.x + q.n;
+  rows += (int64_t)blockIdx.y * inst_words;
+  const int lane = threadIdx.x & 31;
+  const int grp = threadIdx.x >> 5;
+  const int64_t ntile = N / 32;  // a multiple of 32 (N >= 2^13)
+  for (int64_t t0 = (int64_t)blockIdx.x * 32; t0 < ntile; t0 += (int64_t)gridDim.x * 32) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int tl = grp * 4 + r;
+      const int64_t i = (t0 + tl) * 32 + lane;
+      uint4 v = z4();
+      if (i < q.n) v = in[i];
+      sm[0 * 32 + lane][tl] = cuot_transpose32(v.x, lane);
+      sm[1 * 32 + lane][tl] = cuot_transpose32(v.y, lane);
+      sm[2 * 32 + lane][tl] = cuot_transpose32(v.z, lane);
+      sm[3 * 32 + lane][tl] = cuot_transpose32(v.w, lane);
+    }
+    __syncthreads();
+    for (int f = threadIdx.x; f < 128 * 8; f += 256) {
+      const int k = f >> 3, tl = (f & 7) * 4;
+      *(uint4*)&rows[(int64_t)k * ntile + t0 + tl] = make_uint4(sm[k][tl], sm[k][tl + 1], sm[k][tl + 2], sm[k][tl + 3]);
+    }
+    __syncthreads();
+  }
+}
+
+// ---- conversion levels on blocks (levels >= 20) ------------------------------------
+// Division by s_k on chunks of 2^(k+1) coefficients (forward), or the product
+// back (conv_bits.h states both); one level, out of place, N coefficients.
+// SRC: the source is the instance's x_{n+i}, zero from n on.
+CUOT_DEV int fa_terms(int k, uint32_t* e) {
+  int c = 0;
+  for (int j = 0; j < k; j++)
+    if ((j & ~k) == 0) e[c++] = 1u << j;
+  return c;
+}
+
+template <bool INV, bool SRC>
+__global__ __launch_bounds__(256) void fa_conv_level(const QcIo* __restrict__ io, QcIo io1,
+                                                     const uint4* __restrict__ in, uint4* __restrict__ out, int64_t XS,
+                                                     int64_t N, int k) {
+  uint32_t e[16];
+  const int ne = fa_terms(k, e);
+  const int64_t emax = ne ? e[ne - 1] : 0;
+  const int64_t half = (int64_t)1 << k;
+  int64_t lim = N;
+  const uint4* src;
+  if (SRC) {
+    const QcIo q = io ? io[blockIdx.y] : io1;
+    src = q.x + q.n;
+    lim = q.n;
+  } else {
+    src = in + (int64_t)blockIdx.y * XS;
+  }
+  uint4* dst = out + (int64_t)blockIdx.y * XS;
+  auto at = [&](int64_t i) { return (!SRC || i < lim) ? src[i] : z4(); };
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < N; i += (int64_t)gridDim.x * 256) {
+    const int64_t pos = i & (2 * half - 1);
+    const int64_t lo = i - pos, hi = lo + half;
+    uint4 v = at(i);
+    if (pos < half) {
+      for (int q = 0; q < ne; q++) {
+        if ((int64_t)e[q] > pos) break;
+        const int64_t s = pos - e[q];
+        v = x4(v, at(hi + s));
+        if (!INV && s < emax) {
+          for (int r = 0; r < ne; r++)
+            if ((int64_t)e[r] > s) v = x4(v, at(hi + s + half - e[r]));
+        }
+      }
+    } else {
+      const int64_t s = pos - half;
+      if (s < emax) {
+        for (int r = 0; r < ne; r++)
+          if ((int64_t)e[r] > s) v = x4(v, at(hi + s + half - e[r]));
+      }
+    }
+    dst[i] = v;
+  }
+}
+
+// ---- output -------------------------------------------------------------------------
+// y_i = x_i ^ H_i ^ H_{i+n}, H the product's coefficients; with top >= 0 the
+// level k = top of the inverse conversion (the whole product's two halves) is
+// applied on the fly
+__global__ __launch_bounds__(256) void fa_output(const uint4* __restrict__ H, int64_t XS, int top,
+                                                 const QcIo* __restrict__ io, QcIo io1) {
+  const QcIo q = io ? io[blockIdx.y] : io1;
+  H += (int64_t)blockIdx.y * XS;
+  uint32_t e[16];
+  const int ne = top >= 0 ? fa_terms(top, e) : 0;
+  const int64_t half = top >= 0 ? (int64_t)1 << top : 0;
+  auto h_at = [&](int64_t i) {
+    uint4 v = H[i];
+    if (top < 0) return v;
+    if (i < half) {
+      for (int t = 0; t < ne; t++) {
+        if ((int64_t)e[t] > i) break;
+        v = x4(v, H[half + i - e[t]]);
+      }
+    } else {
+      const int64_t s = i - half;
+      for (int t = 0; t < ne; t++)
+        if ((int64_t)e[t] > s) v = x4(v, H[half + s + half - e[t]]);
+    }
+    return v;
+  };
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < q.n; i += (int64_t)gridDim.x * 256)
+    q.y[i] = x4(q.x[i], x4(h_at(i), h_at(i + q.n)));
+}
+
+// ---- A^: the scalar transform of the single polynomial a ------------------------------
+// One 32-bit word per point.  The words behind A^ (a word per point again) hold
+// a's bits while they are converted.
+CUOT_DEV uint32_t gf16_mul_dev(uint32_t a, uint32_t b) {
+  uint32_t r = 0;
+#pragma unroll
+  for (int i = 0; i < 16; i++) r ^= (a << i) & (0u - ((b >> i) & 1u));
+  // z^16 = z^5 + z^3 + z + 1, twice (the first fold leaves degree <= 19)
+#pragma unroll
+  for (int f = 0; f < 2; f++) {
+    const uint32_t t = r >> 16;
+    r = (r & 0xffffu) ^ t ^ (t << 1) ^ (t << 3) ^ (t << 5);
+  }
+  return r;
+}
+
+CUOT_DEV uint32_t gf32_mul_dev(uint32_t a, uint32_t b) {
+  const uint32_t a0 = a & 0xFFFFu, a1 = a >> 16, b0 = b & 0xFFFFu, b1 = b >> 16;
+  const uint32_t p0 = gf16_mul_dev(a0, b0), p1 = gf16_mul_dev(a1, b1), p2 = gf16_mul_dev(a0 ^ a1, b0 ^ b1);
+  return (p0 ^ gf16_times_nu(p1)) | ((p2 ^ p0) << 16);
+}
+
+__global__ __launch_bounds__(256) void fa_prep_bits(const QcPrep* __restrict__ pr, QcPrep pr1, int K) {
+  const QcPrep q = pr ? pr[blockIdx.y] : pr1;
+  uint32_t* T = q.ahat + ((int64_t)1 << (K - 5));
+  const int64_t nb = (q.n + 7) / 8;
+  for (int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x; w < ((int64_t)1 << (K - 6)); w += (int64_t)gridDim.x * 256) {
+    uint32_t v = 0;
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+      if (4 * w + b < nb) v |= (uint32_t)q.a_bits[4 * w + b] << (8 * b);
+    const int64_t left = q.n - 32 * w;
+    if (left <= 0)
+      v = 0;
+    else if (left < 32)
+      v &= (1u << left) - 1u;
+    T[w] = v;
+  }
+}
+
+// forward conversion level k >= 20 on a's bit string, out of place (from the
+// first or second half of the words behind A^ to the other)
+__global__ __launch_bounds__(256) void fa_prep_level(const QcPrep* __restrict__ pr, QcPrep pr1, int K, int k, int src) {
+  const QcPrep q = pr ? pr[blockIdx.y] : pr1;
+  const int64_t NW = (int64_t)1 << (K - 6);
+  const uint32_t* in = q.ahat + ((int64_t)1 << (K - 5)) + (src ? NW : 0);
+  uint32_t* out = q.ahat + ((int64_t)1 << (K - 5)) + (src ? 0 : NW);
+  uint32_t e[16];
+  const int ne = fa_terms(k, e);
+  const int64_t hw = (int64_t)1 << (k - 5);  // words per half
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < NW; i += (int64_t)gridDim.x * 256) {
+    const int64_t pos = i & (2 * hw - 1);
+    const uint32_t* hi = in + (i - pos) + hw;
+    // word s of the quotient's half: hi with its first e_max bits corrected
+    auto quot = [&](int64_t s) {
+      uint32_t v = hi[s];
+      for (int r = 0; r < ne; r++) {
+        const int64_t ew = e[r] >> 5;
+        if (e[r] >= 32) {
+          if (s < ew) v ^= hi[s + hw - ew];
+        } else if (s == 0) {
+          v ^= hi[hw - 1] >> (32 - e[r]);
+        }
+      }
+      return v;
+    };
+    uint32_t v;
+    if (pos >= hw) {
+      v = quot(pos - hw);
+    } else {
+      v = in[i];
+      for (int t = 0; t < ne; t++) {
+        const int64_t ew = e[t] >> 5;
+        const int sh = (int)(e[t] & 31);
+        if (pos < ew) continue;
+        const uint32_t x = quot(pos - ew);
+        if (sh == 0)
+          v ^= x;
+        else
+          v ^= (x << sh) | (pos - ew >= 1 ? quot(pos - ew - 1) >> (32 - sh) : 0u);
+      }
+    }
+    out[i] = v;
+  }
+}
+
+struct FaSync {
+  __device__ void operator()() const { __syncthreads(); }
+};
+
+// levels below 2^mp on each string of 2^mp bits, in place (one workgroup each)
+__global__ __launch_bounds__(1024) void fa_prep_rows(const QcPrep* __restrict__ pr, QcPrep pr1, int K, int mp, int src) {
+  extern __shared__ uint32_t sw[];
+  const QcPrep q = pr ? pr[blockIdx.y] : pr1;
+  const int64_t nw = (int64_t)1 << (mp - 5);
+  uint32_t* g = q.ahat + ((int64_t)1 << (K - 5)) + (src ? (int64_t)1 << (K - 6) : 0) + (int64_t)blockIdx.x * nw;
+  for (int64_t i = threadIdx.x; i < nw; i += 1024) sw[cbp_at<true>(i)] = g[i];
+  __syncthreads();
+  cbp_convert<true, false>(sw, 0, mp, threadIdx.x, 1024, FaSync());
+  for (int64_t i = threadIdx.x; i < nw; i += 1024) g[i] = sw[cbp_at<true>(i)];
+}
+
+constexpr int FA_PT = 10;  // log2 words of a preparation tile
+
+// Element bits lo .. lo + R - 1 on tiles of 2^R words 2^lo apart times 2^lgC
+// consecutive ones; the first tile pass takes the words from a's converted bits.
+__global__ __launch_bounds__(512) void fa_prep_fft(const QcPrep* __restrict__ pr, QcPrep pr1, int K, int c, int aidx,
+                                                   int lo, int R, int lgC, int first, int src) {
+  __shared__ uint32_t L[1 << FA_PT];
+  __shared__ uint32_t ctab[FA_CTAB];
+  const QcPrep q = pr ? pr[blockIdx.y] : pr1;
+  uint32_t* A = q.ahat;
+  const int nt = blockDim.x;
+  fa_ctab_fill(ctab, threadIdx.x, nt);
+  const int C = 1 << lgC, TW = 1 << (R + lgC);
+  const int64_t tile = blockIdx.x;
+  const int64_t cb = tile & ((((int64_t)1 << lo) >> lgC) - 1), hib = tile >> (lo - lgC);
+  auto eidx = [&](int i) { return (hib << (lo + R)) | ((int64_t)(i >> lgC) << lo) | (cb * C + (i & (C - 1))); };
+  if (first) {
+    const uint32_t* T = A + ((int64_t)1 << (K - 5)) + (src ? (int64_t)1 << (K - 6) : 0);
+    const uint32_t* pk = c_fa_pack[K <= 20 ? 0 : K - 20];
+    for (int i = threadIdx.x; i < TW; i += nt) {
+      const int64_t e = eidx(i);
+      uint32_t v = 0;
+      for (int h = 0; h < 2; h++) {
+        const int64_t idx = ((e >> c) << (c + 1)) | ((int64_t)h << c) | (e & (((int64_t)1 << c) - 1));
+        uint32_t x = 0;
+        for (int b = 0; b < 8; b++) {
+          const int64_t ci = ((int64_t)b << (K - 4)) | idx;
+          if ((T[ci >> 5] >> (ci & 31)) & 1u) x ^= pk[b];
+        }
+        v |= x << (16 * h);
+      }
+      L[i] = v;
+    }
+  } else {
+    for (int i = threadIdx.x; i < TW; i += nt) L[i] = A[eidx(i)];
+  }
+  __syncthreads();
+  for (int s = R - 1; s >= 0; s--) {
+    const int b = lo + s;  // element bit
+    if (b == c - 1 && K - 5 > c) {
+      // layer k = c between the two kinds: half 0 ^= C(bits above) * half 1
+      for (int i = threadIdx.x; i < TW; i += nt) {
+        const uint32_t x = L[i];
+        L[i] = x ^ gf16_mul_dev(fa_ctab(ctab, (uint32_t)(eidx(i) >> c)), x >> 16);
+      }
+      __syncthreads();
+    }
+    const int k = b >= c ? b + 1 : b;
+    const uint32_t off = c_fa_beta[aidx - k];
+    for (int t = threadIdx.x; t < (TW >> 1); t += nt) {
+      const int cc = t & (C - 1), bp = t >> lgC;
+      const int tu = ((bp >> s) << (s + 1)) | (bp & ((1 << s) - 1));
+      const int u = tu * C + cc, v = u + (C << s);
+      const uint32_t e = (uint32_t)eidx(u);
+      const uint32_t xv = L[v];
+      uint32_t xu = L[u];
+      if (b >= c) {
+        const uint32_t cst = off ^ fa_ctab(ctab, e >> (b + 1));
+        xu ^= gf16_mul_dev(cst, xv & 0xffffu) | (gf16_mul_dev(cst, xv >> 16) << 16);
+      } else {
+        const uint32_t g = ((e >> c) << (c - k)) | ((e & ((1u << c) - 1)) >> (k + 1));
+        xu ^= gf32_mul_dev(off ^ fa_ctab(ctab, g), xv);
+      }
+      L[u] = xu;
+      L[v] = xv ^ xu;
+    }
+    __syncthreads();
+  }
+  for (int i = threadIdx.x; i < TW; i += nt) A[eidx(i)] = L[i];
+}
+
+// ---- host -------------------------------------------------------------------------------
+int g_fa_ready = 0;
+
+template <int NP, int KC>
+hipError_t fa_allow_lds() {
+  return hipFuncSetAttribute((const void*)fa_pass<NP, KC>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (fa_tile<NP>() * fa_stride<NP>() + FA_CTAB) * 4);
+}
+
+hipError_t fa_configure() {
+  if (g_fa_ready) return hipSuccess;
+  uint32_t beta[32], pack[FA_KC_MAX + 1][8];
+  fa_basis(beta);
+  const FaChunk ch[FA_KC_MAX + 1] = {kFaChunk<0>, kFaChunk<1>, kFaChunk<2>, kFaChunk<3>, kFaChunk<4>, kFaChunk<5>};
+  // pack[b]: bits 0..2 of b are index bits K-4 .. K-2
+  for (int i = 0; i <= FA_KC_MAX; i++)
+    for (int q = 0; q < 8; q++) pack[i][q] = ch[i].pack[q];
+  hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(c_fa_beta), beta, sizeof(beta));
+  if (!e) e = hipMemcpyToSymbol(HIP_SYMBOL(c_fa_pack), pack, sizeof(pack));
+  if (!e) e = fa_allow_lds<32, -1>();
+  if (!e) e = fa_allow_lds<32, 0>();
+  if (!e) e = fa_allow_lds<16, 1>();
+  if (!e) e = fa_allow_lds<16, 2>();
+  if (!e) e = fa_allow_lds<16, 3>();
+  if (!e) e = fa_allow_lds<16, 4>();
+  if (!e) e = fa_allow_lds<16, 5>();
+  if (!e)
+    e = hipFuncSetAttribute((const void*)fa_prep_rows, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)cbp_words(32 * 1024, true) * 4);
+  if (!e) g_fa_ready = 1;
+  return e;
+}
+
+int fa_log(int64_t n) {  // K: 2^(K-1) >= n
+  int K = 1;
+  while (((int64_t)1 << (K - 1)) < n) K++;
+  return K;
+}
+
+unsigned capg(int64_t v, int64_t cap) { return (unsigned)(v < 1 ? 1 : (v > cap ? cap : v)); }
+
+template <int NP, int KC>
+void fa_launch(const FaArgs& a, int B, hipStream_t st) {
+  constexpr int Z = 32 / NP;
+  const int64_t ntiles = ((int64_t)1 << (a.K - 5)) >> (a.R + a.lgC);
+  // two resident workgroups on each of the 256 CUs; every one walks many tiles
+  const int64_t cap = 512 / (B * Z) < 1 ? 1 : 512 / (B * Z);
+  const double per = 512.0 * (double)((int64_t)1 << (a.K - 5)) * B;
+  cuot_rec_begin(st, NP == 16 ? "fa_pass<16>" : "fa_pass<32>", a.first ? per * 1.5 : per * 2.0);
+  hipLaunchKernelGGL((fa_pass<NP, KC>), dim3(capg(ntiles, cap), (unsigned)B, (unsigned)Z), dim3(fa_threads<NP>()),
+                     ((size_t)fa_stride<NP>() * ((size_t)1 << (a.R + a.lgC)) + FA_CTAB) * 4, st, a);
+  cuot_rec_end(st);
+}
+
+template <int NP>
+void fa_launch_kc(const FaArgs& a, int kc, int B, hipStream_t st) {
+  switch (kc) {
+    case 1: fa_launch<16, 1>(a, B, st); break;
+    case 2: fa_launch<16, 2>(a, B, st); break;
+    case 3: fa_launch<16, 3>(a, B, st); break;
+    case 4: fa_launch<16, 4>(a, B, st); break;
+    default: fa_launch<16, 5>(a, B, st); break;
+  }
+}
+
+// Layers of the upper GF(2^32) passes, from bit c-1 down to the fused pass's 7:
+// tiles of 2^4 elements times 8 columns (up to 5 layers in one pass where that
+// saves a launch): the columns and the four words share a twiddle, so most
+// wavefronts take scalar branches.  The knobs set layers and columns.
+int fa_pass_layers(int left) {
+  const int knob = cuot_knobs().qc_radix;
+  int R = knob > 0 ? (knob < 7 ? knob : 7) : (left <= 5 ? left : 4);
+  return R < left ? R : left;
+}
+
+int fa_columns(int R, int lo) {
+  const int knob = cuot_knobs().qc_cols;
+  int lgC = 7 - R;
+  if (knob > 0 && __builtin_ctz(knob) < lgC) lgC = __builtin_ctz(knob);
+  return lgC < lo ? lgC : lo;
+}
+
+hipError_t fa_transform(const FaArgs& base, int B, hipStream_t st) {
+  const int K = base.K, c = base.c, r = K - 5 - c;
+  const int R0 = c < 7 ? c : 7;
+  // upper passes: [lo, lo + R) from the top
+  int los[16], Rs[16], np = 0;
+  for (int top = c; top > R0;) {
+    Rs[np] = fa_pass_layers(top - R0);
+    los[np] = top - Rs[np];
+    top = los[np++];
+  }
+  FaArgs a = base;
+  if (r > 0) {
+    a.lo = c;
+    a.R = r;
+    a.lgC = 8 - r;
+    a.mode = FA_FWD;
+    a.first = 1;
+    fa_launch_kc<16>(a, K - 20, B, st);
+  }
+  for (int i = 0; i < np; i++) {
+    a = base;
+    a.lo = los[i];
+    a.R = Rs[i];
+    a.lgC = fa_columns(a.R, a.lo);
+    a.mode = FA_FWD;
+    a.first = r == 0 && i == 0;
+    a.contract = r > 0 && i == 0;
+    if (a.first)
+      fa_launch<32, 0>(a, B, st);
+    else
+      fa_launch<32, -1>(a, B, st);
+  }
+  a = base;
+  a.R = R0;
+  a.mode = FA_FUSED;
+  fa_launch<32, -1>(a, B, st);
+  for (int i = np - 1; i >= 0; i--) {
+    a = base;
+    a.lo = los[i];
+    a.R = Rs[i];
+    a.lgC = fa_columns(a.R, a.lo);
+    a.mode = FA_INV;
+    a.last = r == 0 && i == 0;
+    a.contract = r > 0 && i == 0;
+    if (a.last)
+      fa_launch<32, 0>(a, B, st);
+    else
+      fa_launch<32, -1>(a, B, st);
+  }
+  if (r > 0) {
+    a = base;
+    a.lo = c;
+    a.R = r;
+    a.lgC = 8 - r;
+    a.mode = FA_INV;
+    a.last = 1;
+    fa_launch_kc<16>(a, K - 20, B, st);
+  }
+  return hipGetLastError();
+}
+
+}  // namespace
+
+bool cuot_qc_fa_selected(int64_t n) {
+  const int K = fa_log(n);
+  return K >= FA_KMIN && K <= FA_KMAX;
+}
+
+hipError_t cuot_qc_fa_configure() { return fa_configure(); }
+
+// two buffers of 2^K blocks per instance (the matrix-core encoder of small
+// codes asks for four)
+size_t cuot_qc_fa_scratch_bytes(int64_t n, int B) {
+  return (size_t)B * (cuot_qc_mfma_eligible(n) ? 4 : 2) * ((size_t)16 << fa_log(n));
+}
+
+hipError_t cuot_launch_qc_fa_prepare(const QcPrep* pr, QcPrep pr1, int B, int K, hipStream_t st) {
+  hipError_t e = fa_configure();
+  if (e != hipSuccess) return e;
+  const int c = K - 5 < 15 ? K - 5 : 15, aidx = 16 + c;
+  const int64_t nw = (int64_t)1 << (K - 6);
+  hipLaunchKernelGGL(fa_prep_bits, dim3(capg(nw / 256, 1024), (unsigned)B), dim3(256), 0, st, pr, pr1, K);
+  int src = 0;
+  for (int k = K - 2; k >= FA_STR; k--, src ^= 1)
+    hipLaunchKernelGGL(fa_prep_level, dim3(capg(nw / 256, 1024), (unsigned)B), dim3(256), 0, st, pr, pr1, K, k, src);
+  const int mp = K - 1 < FA_STR ? K - 1 : FA_STR;
+  hipLaunchKernelGGL(fa_prep_rows, dim3(1u << (K - 1 - mp), (unsigned)B), dim3(1024),
+                     (size_t)cbp_words((int64_t)1 << (mp - 5), true) * 4, st, pr, pr1, K, mp, src);
+  const int bits = K - 5;
+  const int Rl = bits < FA_PT ? bits : FA_PT, Ru = bits - Rl;
+  if (Ru > 0)
+    hipLaunchKernelGGL(fa_prep_fft, dim3(1u << (bits - FA_PT), (unsigned)B), dim3(512), 0, st, pr, pr1, K, c, aidx, Rl,
+                       Ru, FA_PT - Ru, 1, src);
+  hipLaunchKernelGGL(fa_prep_fft, dim3(1u << (bits - Rl), (unsigned)B), dim3(512), 0, st, pr, pr1, K, c, aidx, 0, Rl, 0,
+                     Ru > 0 ? 0 : 1, src);
+  return hipGetLastError();
+}
+
+hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ahat1, const uint32_t* const* ahats, int B,
+                                    int K, int64_t nmax, void* scratch, hipStream_t st) {
+  hipError_t e = fa_configure();
+  if (e != hipSuccess) return e;
+  const int64_t XS = (int64_t)1 << K;  // blocks per instance and buffer
+  uint4* X = (uint4*)scratch;
+  uint4* Y = X + (int64_t)B * XS;
+  const int64_t Nin = XS >> 1;
+  // forward conversion; the natural-order coefficients end up in X
+  if (K - 1 <= FA_STR) {
+    const int64_t words = Nin / 32;
+    cuot_rec_begin(st, "fa_rows_in", 32.0 * (double)Nin * B);
+    hipLaunchKernelGGL(fa_rows_in, dim3(capg(words / 32, 4096), (unsigned)B), dim3(256), 0, st, io, io1, Nin,
+                       (uint32_t*)Y, XS * 4);
+    cuot_rec_end(st);
+    if ((e = cuot_launch_conv_rows(4096, st, (uint32_t*)Y, words, 128ll * B, 128, XS * 4, K - 1, 0))) return e;
+    if ((e = cuot_launch_transpose_planes2(Y, Nin, X, true, B, 1, XS * 4, 128 * words, XS, Nin, st))) return e;
+  } else {
+    // levels K-2 .. 20 on blocks; their last output lies in X
+    const int nlev = K - 1 - FA_STR;
+    uint4* cur = nullptr;
+    for (int j = 0; j < nlev; j++) {
+      uint4* dst = ((nlev - 1 - j) & 1) ? Y : X;
+      const dim3 grid(capg(Nin / 256, 16384), (unsigned)B);
+      cuot_rec_begin(st, "fa_conv_level", 32.0 * (double)Nin * B);
+      if (j == 0)
+        hipLaunchKernelGGL((fa_conv_level<false, true>), grid, dim3(256), 0, st, io, io1, cur, dst, XS, Nin, K - 2 - j);
+      else
+        hipLaunchKernelGGL((fa_conv_level<false, false>), grid, dim3(256), 0, st, io, io1, cur, dst, XS, Nin, K - 2 - j);
+      cuot_rec_end(st);
+      cur = dst;
+    }
+    const int64_t S = (int64_t)1 << FA_STR, words = S / 32;
+    const int P = (int)(Nin >> FA_STR);
+    if ((e = cuot_launch_transpose_planes2(X, S, Y, false, B * P, P, XS, S, XS * 4, 128 * words, st))) return e;
+    if ((e = cuot_launch_conv_rows(4096, st, (uint32_t*)Y, words, 128ll * P * B, 128ll * P, XS * 4, FA_STR, 0)))
+      return e;
+    if ((e = cuot_launch_transpose_planes2(Y, S, X, true, B * P, P, XS * 4, 128 * words, XS, S, st))) return e;
+  }
+  FaArgs a;
+  memset(&a, 0, sizeof(a));
+  a.nat_in = X;
+  a.nat_out = X;
+  a.E = Y;
+  a.ahat = ahat1;
+  a.ahats = ahats;
+  a.XS = XS;
+  a.K = K;
+  a.c = K - 5 < 15 ? K - 5 : 15;
+  a.a = 16 + a.c;
+  if ((e = fa_transform(a, B, st))) return e;
+  // inverse conversion of the 2^K coefficients in X
+  const int mp = K < FA_STR ? K : FA_STR;
+  const int64_t S = (int64_t)1 << mp, words = S / 32;
+  const int P = 1 << (K - mp);
+  if ((e = cuot_launch_transpose_planes2(X, S, Y, false, B * P, P, XS, S, XS * 4, 128 * words, st))) return e;
+  if ((e = cuot_launch_conv_rows(8192, st, (uint32_t*)Y, words, 128ll * P * B, 128ll * P, XS * 4, mp, 1))) return e;
+  if ((e = cuot_launch_transpose_planes2(Y, S, X, true, B * P, P, XS * 4, 128 * words, XS, S, st))) return e;
+  uint4* cur = X;
+  for (int k = FA_STR; k < K - 1; k++) {
+    uint4* dst = cur == X ? Y : X;
+    cuot_rec_begin(st, "fa_conv_level", 32.0 * (double)XS * B);
+    hipLaunchKernelGGL((fa_conv_level<true, false>), dim3(capg(XS / 256, 16384), (unsigned)B), dim3(256), 0, st, io, io1,
+                       cur, dst, XS, XS, k);
+    cuot_rec_end(st);
+    cur = dst;
+  }
+  cuot_rec_begin(st, "fa_output", 48.0 * (double)nmax * B);
+  hipLaunchKernelGGL(fa_output, dim3(capg((nmax + 255) / 256, 16384), (unsigned)B), dim3(256), 0, st, cur, XS,
+                     K > FA_STR ? K - 1 : -1, io, io1);
+  cuot_rec_end(st);
+  return hipGetLastError();
+}

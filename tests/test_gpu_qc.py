@@ -175,3 +175,40 @@ def test_transpose(ctx, N):
     back = dev_blocks(N)
     ctx.bit_untranspose(rows, N, back)
     assert np.array_equal(to_np(back), x)
+
+
+# the product on Frobenius orbits (2^12 < n <= 2^24): both ends of every padded
+# length and the neighbours outside its range.  A circulant with a few ones is a
+# XOR of rotations at any length; random ones against Karatsuba at small ends.
+@pytest.mark.parametrize("n", [4096, 4097, 8192, 8193, 65536, 131073, (1 << 18) + 1, 1 << 19, (1 << 19) + 1,
+                               (1 << 20) + 1, (1 << 21) + 1, (1 << 22) + 1, (1 << 23) + 1, 1 << 24])
+def test_qc_orbit_product_rotations(ctx, knob_mfma, n):
+    import torch
+
+    print(f"qc orbits rotations n={n}", flush=True)
+    knob_mfma(-1)
+    r = rng(n + 21)
+    pos = sorted({0, 1, n - 1, n // 2, int(r.integers(0, n)), int(r.integers(0, n))})
+    a = np.zeros((n + 7) // 8, dtype=np.uint8)
+    for s in pos:
+        a[s >> 3] |= 1 << (s & 7)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randint(-(1 << 63), (1 << 63) - 1, (2 * n, 2), dtype=torch.int64, device="cuda", generator=g)
+    ahat = torch.zeros(ctx.qc_ahat_len(n), dtype=torch.int32, device="cuda")
+    scratch = torch.full((ctx.qc_scratch_bytes(n),), 0xA5, dtype=torch.uint8, device="cuda")
+    ctx.qc_prepare(n, dev_bits(a, n), ahat, scratch)
+    y = dev_blocks(n)
+    ctx.qc_encode(n, ahat, x, y, scratch)
+    want = x[:n].clone()
+    for s in pos:
+        want ^= torch.roll(x[n:], s, 0)
+    assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("n", [4097, 8193, 20000, 131073, (1 << 19) + 1])
+def test_qc_orbit_product_vs_karatsuba(ctx, knob_mfma, n):
+    print(f"qc orbits karatsuba n={n}", flush=True)
+    knob_mfma(-1)
+    r = rng(n + 23)
+    a, x = rand_bits(r, n), rand_blocks(r, 2 * n)
+    assert np.array_equal(qc_gpu(ctx, x, a, n), po.qc_encode_fast(x, a, n, nthreads=8))
