@@ -30,9 +30,10 @@
 //
 // Encode (per party), blocks x_{n+i} being coefficient i of all 128 rows:
 //   128-row bit transpose, novel-basis conversion of every row string in LDS
-//   (conv_fast.h), transpose back (levels of 2^20 coefficients and more act on
-//   the blocks before that); a first pass (GF(2^16) layers, halves of the
-//   elements apart), passes of GF(2^32) layers, the lowest of them with the
+//   (conv_fast.h), transpose back (for K > 21 the strings are the 2^16
+//   coefficients of an expansion in powers of s_16, made on the blocks before
+//   that, and the first pass converts across the strings); a first pass
+//   (GF(2^16) layers, halves of the elements apart), passes of GF(2^32) layers, the lowest of them with the
 //   product by A^ and the inverse layers; the mirror image back; y.
 // Between passes the data is element major: element e is 32 planes x 16 bytes
 // in one run, so that every tile reads and writes whole lines.
@@ -218,6 +219,71 @@ __device__ __forceinline__ void fa_chunks(const FaArgs& a, uint32_t* lds) {
   __syncthreads();
 }
 
+// Conversion of the coefficient rows of a half-mode tile between the s_16-adic
+// and the novel basis: row rho (index bits 16 up) is a coefficient of X = s_16,
+// whose subspace polynomials are s_k(X) = X^(2^k) + sum of X^e, e = 2^j for the
+// proper submasks j of k (levels as in conv_bits.h, one row instead of one
+// bit).  Row rho lies in plane rho >> r of element (rho mod 2^r) * C + column,
+// r = KC.  The terms are compile-time constants: with runtime term lists the two
+// passes took 1000 us more at n = 2^24, where this adds 170 and 250 us to
+// passes of 315 and 365.
+constexpr bool fa_is_term(int k, int j) { return j < k && (j & ~k) == 0; }
+constexpr int fa_jmax(int k) {
+  int m = 0;
+  for (int j = 0; j < k; j++)
+    if (fa_is_term(k, j)) m = j;
+  return m;
+}
+
+template <int KC>
+__device__ __forceinline__ uint4& fa_row(uint32_t* lds, int rho, int c) {
+  return *(uint4*)&lds[fa_slot(((rho & ((1 << KC) - 1)) << (8 - KC)) + c) * fa_stride<16>() + 4 * (rho >> KC)];
+}
+
+// v ^= rows hb + s + half - e for the terms e = 2^J > s (FIX) or lb-side rows
+// hb + s - e for e <= s
+template <int KC, int K, bool FIX, int J = 0>
+__device__ __forceinline__ void fa_row_terms(uint32_t* lds, uint4& v, int hb, int s, int c) {
+  if constexpr (J < K) {
+    if constexpr (fa_is_term(K, J)) {
+      constexpr int e = 1 << J;
+      if (FIX ? e > s : e <= s) v = x4(v, fa_row<KC>(lds, FIX ? hb + s + (1 << K) - e : hb + s - e, c));
+    }
+    fa_row_terms<KC, K, FIX, J + 1>(lds, v, hb, s, c);
+  }
+}
+
+template <int KC, bool INV, int STEP = 1>
+__device__ __forceinline__ void fa_outer(uint32_t* lds) {
+  constexpr int NB = KC + (INV ? 4 : 3);  // row bits; level 0 has no lower terms
+  if constexpr (STEP < NB) {
+    constexpr int K = INV ? STEP : NB - STEP, half = 1 << K, LGC = 8 - KC, C = 1 << LGC, LGE = fa_jmax(K);
+#pragma unroll
+    for (int phase = 0; phase < 2; phase++) {
+      if ((phase == 0) != INV) {
+        constexpr int cnt = (1 << (NB - 1 - K)) << (LGE + LGC);  // hi rows i < e_max
+        for (int x = threadIdx.x; x < cnt; x += fa_threads<16>()) {
+          const int c = x & (C - 1), i = (x >> LGC) & ((1 << LGE) - 1), hb = ((x >> (LGC + LGE)) * 2 + 1) * half;
+          uint4 v = fa_row<KC>(lds, hb + i, c);
+          fa_row_terms<KC, K, true>(lds, v, hb, i, c);
+          fa_row<KC>(lds, hb + i, c) = v;
+        }
+      } else {
+        constexpr int cnt = 1 << (NB - 1 + LGC);
+#pragma unroll 1
+        for (int x = threadIdx.x; x < cnt; x += fa_threads<16>()) {
+          const int c = x & (C - 1), lo = x >> LGC, j = lo & (half - 1), lb = (lo >> K) * 2 * half;
+          uint4 v = fa_row<KC>(lds, lb + j, c);
+          fa_row_terms<KC, K, false>(lds, v, lb + half, j, c);
+          fa_row<KC>(lds, lb + j, c) = v;
+        }
+      }
+      __syncthreads();
+    }
+    fa_outer<KC, INV, STEP + 1>(lds);
+  }
+}
+
 // pointwise product by A^
 __device__ __forceinline__ void fa_pointwise(const FaArgs& a, const uint32_t* __restrict__ ahat, uint32_t* lds,
                                              int64_t ebase) {
@@ -326,6 +392,9 @@ __global__ __launch_bounds__(fa_threads<NP>()) __attribute__((amdgpu_waves_per_e
     }
     __syncthreads();
     if constexpr (KC >= 0) {
+      if constexpr (NP == 16 && KC > 1) {
+        if (a.first) fa_outer<KC, false>(lds);
+      }
       if (a.first) fa_chunks<NP, KC, false>(a, lds);
     }
     if constexpr (NP == 32) {
@@ -348,6 +417,9 @@ __global__ __launch_bounds__(fa_threads<NP>()) __attribute__((amdgpu_waves_per_e
     }
     if constexpr (KC >= 0) {
       if (a.last) fa_chunks<NP, KC, true>(a, lds);
+      if constexpr (NP == 16 && KC > 1) {
+        if (a.last) fa_outer<KC, true>(lds);
+      }
     }
     uint4 w[LD];
     const int tid = opaque_tid();
@@ -381,120 +453,235 @@ __global__ __launch_bounds__(fa_threads<NP>()) __attribute__((amdgpu_waves_per_e
   }
 }
 
-// ---- input: blocks x_{n+i} to 128 bit-row strings of N = 2^(K-1) bits -----------
-__global__ __launch_bounds__(256) void fa_rows_in(const QcIo* __restrict__ io, QcIo io1, int64_t N,
-                                                  uint32_t* __restrict__ rows, int64_t inst_words) {
+// ---- s_16-adic levels on blocks (K > 21) ------------------------------------------
+// Expansion of a polynomial in powers of s_16 = x^65536 + x: s_16^(2^i) has one
+// lower term, so the level of index bit b = 16 + i takes, with half = 2^b and
+// e = 2^i, q = hi with its first e coefficients corrected by its last ones, and
+// lo_j ^= q_{j-e} (backwards the same with the two steps exchanged).  Away from
+// the first coefficients of a half all levels are their own inverses, commute
+// and move coefficient j of a row 2^b further to j + e of this one, so R of them
+// are one pass over skewed columns (below), bound by memory: 2^24 coefficients
+// 16 bytes wide in 102 us (5.26 TB/s).  At n = 2^24 the forward levels take 207
+// us and the backward ones with the output 490.  The novel basis' own levels
+// (s_23 has 15 lower terms) one pass each took 934 and 1510 with the same
+// output, the s_16-adic ones as a gather of (3/2)^R reads per output 310 and 1000.
+// At K = 21 a single level of three terms is left, done in the output: 388 us an
+// encode of n = 2^20 against 413 this way.
+// The source: an instance's natural-order buffer, or x_{n+i}, zero from n on.
+struct FaSrc {
+  const uint4* p;
+  int64_t n;
+  __device__ __forceinline__ uint4 operator[](int64_t i) const { return i < n ? p[i] : make_uint4(0, 0, 0, 0); }
+};
+
+// exact value of index I after the levels of bits b0 .. b (backwards) or
+// b .. b0 + R - 1 (forwards); only near the start of a half
+template <bool INV, int L>
+__device__ __attribute__((noinline)) uint4 fa_s16_slow(const FaSrc& in, int64_t I, int b0, int R) {
+  if constexpr (L == 0) {
+    return in[I];
+  } else {
+    const int b = INV ? b0 + L - 1 : b0 + R - L;
+    const int64_t half = (int64_t)1 << b, e = half >> 16;
+    const int64_t pos = I & (2 * half - 1), hi = I - pos + half;
+    uint4 v = fa_s16_slow<INV, L - 1>(in, I, b0, R);
+    if (pos < half) {
+      if (pos >= e) {
+        const int64_t s = pos - e;
+        v = x4(v, fa_s16_slow<INV, L - 1>(in, hi + s, b0, R));
+        if (!INV && s < e) v = x4(v, fa_s16_slow<INV, L - 1>(in, hi + s + half - e, b0, R));
+      }
+    } else if (pos - half < e) {
+      v = x4(v, fa_s16_slow<INV, L - 1>(in, I + half - e, b0, R));
+    }
+    return v;
+  }
+}
+
+// the first 2 * (sum of the shifts) coefficients above bit b0 take the exact form
+constexpr int64_t fa_s16_edge(int R, int b0) { return (int64_t)2 << (R + b0 - 16); }
+
+// Skewed column c of the 2^R rows of 2^b0 coefficients at base: coefficient
+// c - T 2^(b0-16) of row T.  The levels stay inside a column, where they are a
+// butterfly of R stages, so every coefficient is read and written once.  Rows
+// whose coefficient lies below the exact ones or past the row are not valid
+// (and no valid one takes them in).  Rows below FROM are left out.
+template <int R, int FROM = 0>
+__device__ __forceinline__ void fa_s16_column(const FaSrc& in, int64_t base, int64_t c, int b0, uint4 (&v)[1 << R]) {
+#pragma unroll
+  for (int T = FROM; T < (1 << R); T++) {
+    const int64_t j = c - ((int64_t)T << (b0 - 16));
+    v[T] = j >= 0 && j < ((int64_t)1 << b0) ? in[base + ((int64_t)T << b0) + j] : make_uint4(0, 0, 0, 0);
+  }
+#pragma unroll
+  for (int b = 0; b < R; b++)
+#pragma unroll
+    for (int T = FROM; T < (1 << R); T++)
+      if (!(T >> b & 1)) v[T] = x4(v[T], v[T | 1 << b]);
+}
+
+// columns from the first valid coefficient of row 0 to the last one of row 2^R - 1
+constexpr int64_t fa_s16_columns(int R, int b0) {
+  return ((int64_t)1 << b0) - fa_s16_edge(R, b0) + ((((int64_t)1 << R) - 1) << (b0 - 16));
+}
+
+// Bits B0 .. B0 + R - 1 of N coefficients, a column per lane.  The rows' first
+// coefficients, whose exact form is a long chain of dependent reads, go to
+// workgroups of their own, one per lane.
+template <bool INV, bool SRC, int R, int B0>
+__global__ __launch_bounds__(256) void fa_s16_level(const QcIo* __restrict__ io, QcIo io1, const uint4* __restrict__ in,
+                                                    uint4* __restrict__ out, int64_t XS, int64_t N) {
+  FaSrc src;
+  if (SRC) {
+    const QcIo q = io ? io[blockIdx.y] : io1;
+    src.p = q.x + q.n;
+    src.n = q.n;
+  } else {
+    src.p = in + (int64_t)blockIdx.y * XS;
+    src.n = N;
+  }
+  uint4* dst = out + (int64_t)blockIdx.y * XS;
+  const int tid = threadIdx.x;
+  constexpr int64_t EDGE = fa_s16_edge(R, B0);
+  const int64_t edges = (N >> B0) * EDGE, nedge = (edges + 255) / 256;
+  if ((int64_t)blockIdx.x < nedge) {
+    const int64_t x = (int64_t)blockIdx.x * 256 + tid;
+    if (x >= edges) return;
+    const int64_t i = ((x / EDGE) << B0) | (x & (EDGE - 1));
+    dst[i] = fa_s16_slow<INV, R>(src, i, B0, R);
+    return;
+  }
+  constexpr int64_t per = (fa_s16_columns(R, B0) + 255) / 256;  // workgroups per 2^R rows
+  const int64_t tile = (int64_t)blockIdx.x - nedge;
+  const int64_t c = EDGE + (tile % per) * 256 + tid, base = (tile / per) << (B0 + R);
+  uint4 v[1 << R];
+  fa_s16_column<R>(src, base, c, B0, v);
+#pragma unroll
+  for (int T = 0; T < (1 << R); T++) {
+    const int64_t j = c - ((int64_t)T << (B0 - 16));
+    if (j >= EDGE && j < ((int64_t)1 << B0)) dst[base + ((int64_t)T << B0) + j] = v[T];
+  }
+}
+
+// ---- input: blocks to 128 bit-row strings of S = 2^mp bits ---------------------------
+// SRC: from x_{n+i}
+template <bool SRC>
+__global__ __launch_bounds__(256) void fa_rows_in(const QcIo* __restrict__ io, QcIo io1, const uint4* __restrict__ in,
+                                                  int64_t XS, int64_t N, int mp, uint32_t* __restrict__ rows) {
   __shared__ uint32_t sm[128][33];
-  const QcIo q = io ? io[blockIdx.y] : io1;
-  const uint4* in = q.x + q.n;
-  rows += (int64_t)blockIdx.y * inst_words;
+  FaSrc src;
+  if (SRC) {
+    const QcIo q = io ? io[blockIdx.y] : io1;
+    src.p = q.x + q.n;
+    src.n = q.n;
+  } else {
+    src.p = in + (int64_t)blockIdx.y * XS;
+    src.n = N;
+  }
+  rows += (int64_t)blockIdx.y * XS * 4;
   const int lane = threadIdx.x & 31;
   const int grp = threadIdx.x >> 5;
-  const int64_t ntile = N / 32;  // a multiple of 32 (N >= 2^13)
-  for (int64_t t0 = (int64_t)blockIdx.x * 32; t0 < ntile; t0 += (int64_t)gridDim.x * 32) {
+  const int64_t rw = (int64_t)1 << (mp - 5);  // words per row string
+  // tiles of 1024 blocks (32 words of every row)
+  for (int64_t tile = blockIdx.x; tile < (N >> 10); tile += gridDim.x) {
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int tl = grp * 4 + r;
-      const int64_t i = (t0 + tl) * 32 + lane;
-      uint4 v = z4();
-      if (i < q.n) v = in[i];
+      const int64_t i = (tile << 10) + tl * 32 + lane;
+      const uint4 v = src[i];
       sm[0 * 32 + lane][tl] = cuot_transpose32(v.x, lane);
       sm[1 * 32 + lane][tl] = cuot_transpose32(v.y, lane);
       sm[2 * 32 + lane][tl] = cuot_transpose32(v.z, lane);
       sm[3 * 32 + lane][tl] = cuot_transpose32(v.w, lane);
     }
     __syncthreads();
+    const int64_t str = (tile << 10) >> mp, w0 = ((tile << 10) & (((int64_t)1 << mp) - 1)) >> 5;
+    uint32_t* dst = rows + str * 128 * rw + w0;
     for (int f = threadIdx.x; f < 128 * 8; f += 256) {
       const int k = f >> 3, tl = (f & 7) * 4;
-      *(uint4*)&rows[(int64_t)k * ntile + t0 + tl] = make_uint4(sm[k][tl], sm[k][tl + 1], sm[k][tl + 2], sm[k][tl + 3]);
+      *(uint4*)&dst[(int64_t)k * rw + tl] = make_uint4(sm[k][tl], sm[k][tl + 1], sm[k][tl + 2], sm[k][tl + 3]);
     }
     __syncthreads();
   }
 }
 
-// ---- conversion levels on blocks (levels >= 20) ------------------------------------
-// Division by s_k on chunks of 2^(k+1) coefficients (forward), or the product
-// back (conv_bits.h states both); one level, out of place, N coefficients.
-// SRC: the source is the instance's x_{n+i}, zero from n on.
-CUOT_DEV int fa_terms(int k, uint32_t* e) {
-  int c = 0;
-  for (int j = 0; j < k; j++)
-    if ((j & ~k) == 0) e[c++] = 1u << j;
-  return c;
-}
-
-template <bool INV, bool SRC>
-__global__ __launch_bounds__(256) void fa_conv_level(const QcIo* __restrict__ io, QcIo io1,
-                                                     const uint4* __restrict__ in, uint4* __restrict__ out, int64_t XS,
-                                                     int64_t N, int k) {
-  uint32_t e[16];
-  const int ne = fa_terms(k, e);
-  const int64_t emax = ne ? e[ne - 1] : 0;
-  const int64_t half = (int64_t)1 << k;
-  int64_t lim = N;
-  const uint4* src;
-  if (SRC) {
-    const QcIo q = io ? io[blockIdx.y] : io1;
-    src = q.x + q.n;
-    lim = q.n;
-  } else {
-    src = in + (int64_t)blockIdx.y * XS;
-  }
-  uint4* dst = out + (int64_t)blockIdx.y * XS;
-  auto at = [&](int64_t i) { return (!SRC || i < lim) ? src[i] : z4(); };
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < N; i += (int64_t)gridDim.x * 256) {
-    const int64_t pos = i & (2 * half - 1);
-    const int64_t lo = i - pos, hi = lo + half;
-    uint4 v = at(i);
-    if (pos < half) {
-      for (int q = 0; q < ne; q++) {
-        if ((int64_t)e[q] > pos) break;
-        const int64_t s = pos - e[q];
-        v = x4(v, at(hi + s));
-        if (!INV && s < emax) {
-          for (int r = 0; r < ne; r++)
-            if ((int64_t)e[r] > s) v = x4(v, at(hi + s + half - e[r]));
-        }
-      }
-    } else {
-      const int64_t s = pos - half;
-      if (s < emax) {
-        for (int r = 0; r < ne; r++)
-          if ((int64_t)e[r] > s) v = x4(v, at(hi + s + half - e[r]));
-      }
-    }
-    dst[i] = v;
-  }
-}
-
 // ---- output -------------------------------------------------------------------------
-// y_i = x_i ^ H_i ^ H_{i+n}, H the product's coefficients; with top >= 0 the
-// level k = top of the inverse conversion (the whole product's two halves) is
-// applied on the fly
-__global__ __launch_bounds__(256) void fa_output(const uint4* __restrict__ H, int64_t XS, int top,
-                                                 const QcIo* __restrict__ io, QcIo io1) {
+// y_i = x_i ^ H_i ^ H_{i+n}, H the product's coefficients.  TOP (K = 21): its two
+// halves go through the last level on the way, s_20 = x^(2^20) + x^65536 + x^16 + x.
+template <bool TOP>
+__global__ __launch_bounds__(256) void fa_output(const uint4* __restrict__ H, int64_t XS, const QcIo* __restrict__ io,
+                                                 QcIo io1) {
   const QcIo q = io ? io[blockIdx.y] : io1;
   H += (int64_t)blockIdx.y * XS;
-  uint32_t e[16];
-  const int ne = top >= 0 ? fa_terms(top, e) : 0;
-  const int64_t half = top >= 0 ? (int64_t)1 << top : 0;
   auto h_at = [&](int64_t i) {
     uint4 v = H[i];
-    if (top < 0) return v;
-    if (i < half) {
-      for (int t = 0; t < ne; t++) {
-        if ((int64_t)e[t] > i) break;
-        v = x4(v, H[half + i - e[t]]);
+    if constexpr (TOP) {
+      constexpr int64_t half = (int64_t)1 << 20;
+#pragma unroll
+      for (int e = 1; e <= 65536; e = e == 1 ? 16 : e * 4096) {
+        if (i < half ? i >= e : i - half < e) v = x4(v, H[i < half ? half + i - e : i + half - e]);
       }
-    } else {
-      const int64_t s = i - half;
-      for (int t = 0; t < ne; t++)
-        if ((int64_t)e[t] > s) v = x4(v, H[half + s + half - e[t]]);
     }
     return v;
   };
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < q.n; i += (int64_t)gridDim.x * 256)
     q.y[i] = x4(q.x[i], x4(h_at(i), h_at(i + q.n)));
+}
+
+// The same through the last levels, bits 20 .. K-1 (R of them).  With n = m 2^20
+// + r, the coefficients i + n of one skewed column's i are again one column, r +
+// 16 m further, m rows up, or one row more and 2^20 back where j + r passes the
+// row's end.  That column goes through LDS, as m is no constant.  i or i + n at
+// a row's start: lanes of their own, 2 EDGE per row of y.
+constexpr int FA_OT = 128;
+
+template <int R>
+__global__ __launch_bounds__(FA_OT) void fa_output_s16(const uint4* __restrict__ H, int64_t XS,
+                                                       const QcIo* __restrict__ io, QcIo io1) {
+  constexpr int B0 = 20, LOW = 1 << (R - 2);  // n > 2^(K-2)
+  constexpr int64_t EDGE = fa_s16_edge(R, B0), ROW = (int64_t)1 << B0;
+  __shared__ uint4 second[((1 << R) - LOW) * FA_OT];
+  const QcIo q = io ? io[blockIdx.y] : io1;
+  FaSrc src;
+  src.p = H + (int64_t)blockIdx.y * XS;
+  src.n = XS;
+  const int64_t m = q.n >> B0, r = q.n & (ROW - 1), rows = (q.n + ROW - 1) >> B0;
+  const int64_t nedge = rows * 2 * EDGE / FA_OT;
+  if ((int64_t)blockIdx.x < nedge) {
+    const int64_t x = (int64_t)blockIdx.x * FA_OT + threadIdx.x, k = x & (EDGE - 1);
+    const int64_t j = x & EDGE ? (k - r) & (ROW - 1) : k, i = (x / (2 * EDGE)) << B0 | j;
+    if (i >= q.n || ((x & EDGE) && j < EDGE)) return;
+    uint4 v = q.x[i];
+#pragma unroll 1
+    for (int s = 0; s < 2; s++) v = x4(v, fa_s16_slow<true, R>(src, s ? i + q.n : i, B0, R));
+    q.y[i] = v;
+    return;
+  }
+  const int64_t c = EDGE + ((int64_t)blockIdx.x - nedge) * FA_OT + threadIdx.x;
+  if (c - 16 * (rows - 1) >= ROW) return;
+  const bool carry = c - 16 * (rows - 1) + r >= ROW;
+  const int up = (int)m + (carry ? 1 : 0);
+  {
+    uint4 v[1 << R];
+    fa_s16_column<R, LOW>(src, 0, c + r + 16 * m + (carry ? 16 - ROW : 0), B0, v);
+#pragma unroll
+    for (int T = LOW; T < (1 << R); T++) second[(T - LOW) * FA_OT + threadIdx.x] = v[T];
+  }
+  uint4 v[1 << R];
+  fa_s16_column<R>(src, 0, c, B0, v);
+#pragma unroll
+  for (int T = 0; T <= (1 << (R - 1)); T++) {
+    const int64_t j = c - 16 * T, i = (int64_t)T << B0 | j;
+    if (T < rows && j >= EDGE && j < ROW && ((j + r) & (ROW - 1)) >= EDGE && i < q.n)
+      q.y[i] = x4(q.x[i], x4(v[T], second[(T + up - LOW) * FA_OT + threadIdx.x]));
+  }
+}
+
+CUOT_DEV int fa_terms(int k, uint32_t* e) {
+  int c = 0;
+  for (int j = 0; j < k; j++)
+    if ((j & ~k) == 0) e[c++] = 1u << j;
+  return c;
 }
 
 // ---- A^: the scalar transform of the single polynomial a ------------------------------
@@ -711,6 +898,17 @@ int fa_log(int64_t n) {  // K: 2^(K-1) >= n
 
 unsigned capg(int64_t v, int64_t cap) { return (unsigned)(v < 1 ? 1 : (v > cap ? cap : v)); }
 
+template <bool INV, bool SRC, int R, int B0>
+void fa_launch_level(const QcIo* io, QcIo io1, const uint4* in, uint4* out, int64_t XS, int64_t N, int B,
+                     hipStream_t st) {
+  const int64_t wgs =
+      ((N >> B0) * fa_s16_edge(R, B0) + 255) / 256 + (N >> (B0 + R)) * ((fa_s16_columns(R, B0) + 255) / 256);
+  cuot_rec_begin(st, "fa_s16_level", 32.0 * (double)N * B);
+  hipLaunchKernelGGL((fa_s16_level<INV, SRC, R, B0>), dim3((unsigned)wgs, (unsigned)B), dim3(256), 0, st, io, io1, in,
+                     out, XS, N);
+  cuot_rec_end(st);
+}
+
 template <int NP, int KC>
 void fa_launch(const FaArgs& a, int B, hipStream_t st) {
   constexpr int Z = 32 / NP;
@@ -858,35 +1056,31 @@ hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ah
   uint4* X = (uint4*)scratch;
   uint4* Y = X + (int64_t)B * XS;
   const int64_t Nin = XS >> 1;
-  // forward conversion; the natural-order coefficients end up in X
-  if (K - 1 <= FA_STR) {
-    const int64_t words = Nin / 32;
-    cuot_rec_begin(st, "fa_rows_in", 32.0 * (double)Nin * B);
-    hipLaunchKernelGGL(fa_rows_in, dim3(capg(words / 32, 4096), (unsigned)B), dim3(256), 0, st, io, io1, Nin,
-                       (uint32_t*)Y, XS * 4);
-    cuot_rec_end(st);
-    if ((e = cuot_launch_conv_rows(4096, st, (uint32_t*)Y, words, 128ll * B, 128, XS * 4, K - 1, 0))) return e;
-    if ((e = cuot_launch_transpose_planes2(Y, Nin, X, true, B, 1, XS * 4, 128 * words, XS, Nin, st))) return e;
-  } else {
-    // levels K-2 .. 20 on blocks; their last output lies in X
-    const int nlev = K - 1 - FA_STR;
-    uint4* cur = nullptr;
-    for (int j = 0; j < nlev; j++) {
-      uint4* dst = ((nlev - 1 - j) & 1) ? Y : X;
-      const dim3 grid(capg(Nin / 256, 16384), (unsigned)B);
-      cuot_rec_begin(st, "fa_conv_level", 32.0 * (double)Nin * B);
-      if (j == 0)
-        hipLaunchKernelGGL((fa_conv_level<false, true>), grid, dim3(256), 0, st, io, io1, cur, dst, XS, Nin, K - 2 - j);
-      else
-        hipLaunchKernelGGL((fa_conv_level<false, false>), grid, dim3(256), 0, st, io, io1, cur, dst, XS, Nin, K - 2 - j);
-      cuot_rec_end(st);
-      cur = dst;
+  // forward conversion; the natural-order coefficients end up in X: row strings
+  // of the whole length, or for K > 21 of 2^16 coefficients under s_16-adic
+  // levels (the first pass converts the rows of those)
+  const bool adic = K > 21;
+  {
+    const int mp = adic ? 16 : K - 1;
+    if (adic) {
+      switch (K - 21) {
+        case 1: fa_launch_level<false, true, 1, 20>(io, io1, X, Y, XS, Nin, B, st); break;
+        case 2: fa_launch_level<false, true, 2, 20>(io, io1, X, Y, XS, Nin, B, st); break;
+        case 3: fa_launch_level<false, true, 3, 20>(io, io1, X, Y, XS, Nin, B, st); break;
+        default: fa_launch_level<false, true, 4, 20>(io, io1, X, Y, XS, Nin, B, st); break;
+      }
+      fa_launch_level<false, false, 4, 16>(io, io1, Y, X, XS, Nin, B, st);
     }
-    const int64_t S = (int64_t)1 << FA_STR, words = S / 32;
-    const int P = (int)(Nin >> FA_STR);
-    if ((e = cuot_launch_transpose_planes2(X, S, Y, false, B * P, P, XS, S, XS * 4, 128 * words, st))) return e;
-    if ((e = cuot_launch_conv_rows(4096, st, (uint32_t*)Y, words, 128ll * P * B, 128ll * P, XS * 4, FA_STR, 0)))
-      return e;
+    cuot_rec_begin(st, "fa_rows_in", 32.0 * (double)Nin * B);
+    const dim3 rgrid(capg(Nin >> 10, 8192), (unsigned)B);
+    if (!adic)
+      hipLaunchKernelGGL(fa_rows_in<true>, rgrid, dim3(256), 0, st, io, io1, X, XS, Nin, mp, (uint32_t*)Y);
+    else
+      hipLaunchKernelGGL(fa_rows_in<false>, rgrid, dim3(256), 0, st, io, io1, X, XS, Nin, mp, (uint32_t*)Y);
+    cuot_rec_end(st);
+    const int64_t S = (int64_t)1 << mp, words = S / 32;
+    const int P = (int)(Nin >> mp);
+    if ((e = cuot_launch_conv_rows(4096, st, (uint32_t*)Y, words, 128ll * P * B, 128ll * P, XS * 4, mp, 0))) return e;
     if ((e = cuot_launch_transpose_planes2(Y, S, X, true, B * P, P, XS * 4, 128 * words, XS, S, st))) return e;
   }
   FaArgs a;
@@ -902,24 +1096,37 @@ hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ah
   a.a = 16 + a.c;
   if ((e = fa_transform(a, B, st))) return e;
   // inverse conversion of the 2^K coefficients in X
-  const int mp = K < FA_STR ? K : FA_STR;
+  const int mp = adic ? 16 : (K < 20 ? K : 20);
   const int64_t S = (int64_t)1 << mp, words = S / 32;
   const int P = 1 << (K - mp);
   if ((e = cuot_launch_transpose_planes2(X, S, Y, false, B * P, P, XS, S, XS * 4, 128 * words, st))) return e;
   if ((e = cuot_launch_conv_rows(8192, st, (uint32_t*)Y, words, 128ll * P * B, 128ll * P, XS * 4, mp, 1))) return e;
   if ((e = cuot_launch_transpose_planes2(Y, S, X, true, B * P, P, XS * 4, 128 * words, XS, S, st))) return e;
-  uint4* cur = X;
-  for (int k = FA_STR; k < K - 1; k++) {
-    uint4* dst = cur == X ? Y : X;
-    cuot_rec_begin(st, "fa_conv_level", 32.0 * (double)XS * B);
-    hipLaunchKernelGGL((fa_conv_level<true, false>), dim3(capg(XS / 256, 16384), (unsigned)B), dim3(256), 0, st, io, io1,
-                       cur, dst, XS, XS, k);
-    cuot_rec_end(st);
-    cur = dst;
-  }
+  if (adic) fa_launch_level<true, false, 4, 16>(io, io1, X, Y, XS, XS, B, st);
   cuot_rec_begin(st, "fa_output", 48.0 * (double)nmax * B);
-  hipLaunchKernelGGL(fa_output, dim3(capg((nmax + 255) / 256, 16384), (unsigned)B), dim3(256), 0, st, cur, XS,
-                     K > FA_STR ? K - 1 : -1, io, io1);
+  switch (K <= 20 ? 0 : K - 20) {
+    case 0:
+      hipLaunchKernelGGL(fa_output<false>, dim3(capg((nmax + 255) / 256, 16384), (unsigned)B), dim3(256), 0, st, X, XS,
+                         io, io1);
+      break;
+    case 1:
+      hipLaunchKernelGGL(fa_output<true>, dim3(capg((nmax + 255) / 256, 16384), (unsigned)B), dim3(256), 0, st, X, XS,
+                         io, io1);
+      break;
+#define FA_CASE(R)                                                                                               \
+  case R:                                                                                                        \
+    hipLaunchKernelGGL(fa_output_s16<R>,                                                                         \
+                       dim3((unsigned)(((nmax + ((int64_t)1 << 20) - 1) >> 20) * 2 * fa_s16_edge(R, 20) / FA_OT + \
+                                       (fa_s16_columns(R, 20) + FA_OT - 1) / FA_OT),                             \
+                            (unsigned)B),                                                                        \
+                       dim3(FA_OT), 0, st, Y, XS, io, io1);                                                      \
+    break;
+    FA_CASE(2)
+    FA_CASE(3)
+    FA_CASE(4)
+    FA_CASE(5)
+#undef FA_CASE
+  }
   cuot_rec_end(st);
   return hipGetLastError();
 }

@@ -205,6 +205,14 @@ def test_qc_orbit_product_rotations(ctx, knob_mfma, n):
     assert torch.equal(y, want)
 
 
+# n > 2^20: rows of 2^20 coefficients in skewed columns; i + n near a row's ends,
+# whole and ragged last rows, with and without a carry into the next row
+@pytest.mark.parametrize("n", [(1 << 21) - 1, (1 << 22) - 100, 3 * (1 << 20) + 513, (1 << 22) + (1 << 20),
+                               (1 << 23) - (1 << 18) + 3, (1 << 24) - 1040])
+def test_qc_columns_rotations(ctx, knob_mfma, n):
+    test_qc_orbit_product_rotations(ctx, knob_mfma, n)
+
+
 @pytest.mark.parametrize("n", [4097, 8193, 20000, 131073, (1 << 19) + 1])
 def test_qc_orbit_product_vs_karatsuba(ctx, knob_mfma, n):
     print(f"qc orbits karatsuba n={n}", flush=True)
