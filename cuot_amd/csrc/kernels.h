@@ -163,7 +163,7 @@ void cuot_rec_end(hipStream_t st);
 // the built-in rule.  Knobs never change outputs.
 struct CuotKnobs {
   int qc_radix;  // FFT layers per upper pass (2..8)
-  int qc_cols;   // FFT columns per tile (1, 2, 4, 8)
+  int qc_cols;   // FFT columns per tile (1, 2, 4, 8; n > 2^24)
   int ggm_dfs;   // per-lane depth-first levels L (h - 10 <= L <= min(h - 8, 6))
   int lpn_wgs;   // LPN grid cap
   int qc_mfma_max;  // matrix-core QC encoder for n at or below (-1: never)

@@ -32,9 +32,10 @@
 //   128-row bit transpose, novel-basis conversion of every row string in LDS
 //   (conv_fast.h), transpose back (for K > 21 the strings are the 2^16
 //   coefficients of an expansion in powers of s_16, made on the blocks before
-//   that, and the first pass converts across the strings); a first pass
-//   (GF(2^16) layers, halves of the elements apart), passes of GF(2^32) layers, the lowest of them with the
-//   product by A^ and the inverse layers; the mirror image back; y.
+//   that, and the first pass converts across the strings); for K > 20 a pass of
+//   the GF(2^16) layers, halves of the elements apart; a pass of up to seven
+//   GF(2^32) layers; one of the lowest eight, the product by A^ and the inverse
+//   of the eight; the mirror image back; y.
 // Between passes the data is element major: element e is 32 planes x 16 bytes
 // in one run, so that every tile reads and writes whole lines.
 #include <string.h>
@@ -46,7 +47,7 @@
 
 namespace {
 
-__constant__ uint32_t c_fa_beta[32];
+__constant__ uint2 c_fa_beta[32];  // beta_i and nu times its theta part
 __constant__ uint32_t c_fa_pack[FA_KC_MAX + 1][8];
 
 constexpr int FA_KMIN = 14, FA_KMAX = 25;
@@ -56,28 +57,26 @@ CUOT_DEV uint4 x4(uint4 a, uint4 b) { return make_uint4(a.x ^ b.x, a.y ^ b.y, a.
 CUOT_DEV uint4 z4() { return make_uint4(0, 0, 0, 0); }
 
 // ---- twiddles -----------------------------------------------------------------
-// C(g) from three 256-entry tables of the low 24 bits of g
+// C(g) and nu times its theta part from three 256-entry tables of the low 24 bits of g
 constexpr int FA_CTAB = 3 * 256;
 
-CUOT_DEV void fa_ctab_fill(uint32_t* tab, int tid, int nth) {
+CUOT_DEV uint2 x2(uint2 a, uint2 b) { return make_uint2(a.x ^ b.x, a.y ^ b.y); }
+
+CUOT_DEV void fa_ctab_fill(uint2* tab, int tid, int nth) {
   for (int i = tid; i < FA_CTAB; i += nth) {
     const int q = i >> 8, v = i & 255;
-    uint32_t c = 0;
+    uint2 c = make_uint2(0, 0);
     for (int b = 0; b < 8; b++)
-      if ((v >> b) & 1) c ^= c_fa_beta[8 * q + b + 1];
+      if ((v >> b) & 1) c = x2(c, c_fa_beta[8 * q + b + 1]);
     tab[i] = c;
   }
 }
 
-CUOT_DEV uint32_t fa_ctab(const uint32_t* tab, uint32_t g) {
-  return tab[g & 255] ^ tab[256 + ((g >> 8) & 255)] ^ tab[512 + ((g >> 16) & 255)];
+CUOT_DEV uint2 fa_ctab(const uint2* tab, uint32_t g) {
+  return x2(x2(tab[g & 255], tab[256 + ((g >> 8) & 255)]), tab[512 + ((g >> 16) & 255)]);
 }
 
-// ---- passes ---------------------------------------------------------------------
-// LDS tile: TC = 2^R * C elements (2^R of them 2^lo apart times C consecutive
-// ones) of NP planes x 4 words, 4 pad words per element.  NP = 32: whole
-// elements, layers k < c.  NP = 16: one half (blockIdx.z) of the elements, the
-// layers above c, where the halves transform apart under GF(2^16) constants.
+// ---- GF(2^16) layers (K > 20) -------------------------------------------------------
 enum { FA_FWD = 0, FA_INV = 1, FA_FUSED = 2 };
 
 struct FaArgs {
@@ -88,124 +87,58 @@ struct FaArgs {
   const uint32_t* const* ahats;  // per-instance A^ (batch) or NULL
   int64_t XS;                    // instance stride of all three buffers in blocks
   int K, c, a;
-  int lo, R, lgC;
-  int mode;
-  int first, last;  // reads nat_in / writes nat_out
-  int contract;     // the layer k = c before the forward or after the inverse layers
+  int lo, R;     // layers of element bits lo .. lo + R - 1
+  int contract;  // the layer k = c before the forward or after the inverse layers
 };
 
-template <int NP>
-constexpr int fa_stride() {
-  return NP * 4 + 4;
-}
-template <int NP>
-constexpr int fa_tile() {
-  return 4096 / NP;  // elements per tile: 64 KB of data, two workgroups per CU
-}
-template <int NP>
-constexpr int fa_threads() {
-  return NP == 16 ? 512 : 256;  // one (butterfly, word) task per lane and layer
-}
-template <int NP>
-constexpr int fa_ld() {
-  return 4096 / fa_threads<NP>();  // staged 16-byte words per lane
-}
+constexpr int FA_TL = 8;    // log2 elements of a tile
+constexpr int FA_NT = 512;  // lanes
+
+// First and last pass: the layers above c, KC of them, where the halves of the
+// elements transform apart under GF(2^16) constants (blockIdx.z: the half).  LDS
+// tile: 2^KC elements 2^c apart times 2^(8-KC) consecutive ones, 16 planes x 4
+// words each and 4 words of padding; one (butterfly, word) per lane and layer.
+constexpr int FA_ST16 = 68;
 
 // LDS slot of tile element e: the butterflies of the lowest tile layers touch
 // elements whose slots share their residue mod 8 (the element stride is 4 mod
 // 64 banks); reflecting every odd group of eight spreads them
 CUOT_DEV int fa_slot(int e) { return e ^ (((e >> 3) & 1) * 7); }
 
-template <int NP>
-__device__ __forceinline__ void fa_mul(uint32_t cst_lane, bool uniform, const uint32_t* xv, uint32_t* acc) {
-  const uint32_t cst = uniform ? __builtin_amdgcn_readfirstlane(cst_lane) : cst_lane;
-  if constexpr (NP == 16)
-    gf16_mulc(xv, cst, acc);
-  else
-    gf32_mulc<false>(xv, cst, acc);
-}
-
-template <int NP>
-__device__ __forceinline__ void fa_layer(const FaArgs& a, uint32_t* lds, const uint32_t* ctab, int64_t ebase, int s,
-                                         bool inv) {
-  constexpr int ST = fa_stride<NP>();
-  const int C = 1 << a.lgC;
-  const int k = NP == 16 ? a.c + 1 + s : a.lo + s;  // coefficient index bit
-  const uint32_t off = c_fa_beta[a.a - k];
-  const int ntask = (1 << (a.R - 1)) * C * 4;
-  for (int tau = threadIdx.x; tau < ntask; tau += fa_threads<NP>()) {
-    const int w = tau & 3;
-    const int cc = (tau >> 2) & (C - 1);
-    const int bp = (tau >> 2) >> a.lgC;
-    const int tu = ((bp >> s) << (s + 1)) | (bp & ((1 << s) - 1));
-    const int tv = tu | (1 << s);
-    uint32_t g;
-    if constexpr (NP == 16) {
-      g = (uint32_t)(tu >> (s + 1));
-    } else {
-      const uint32_t e = (uint32_t)ebase | (uint32_t)(tu << a.lo);  // columns lie below bit k
-      g = ((e >> a.c) << (a.c - k)) | ((e & ((1u << a.c) - 1)) >> (k + 1));
-    }
-    uint32_t* pu = lds + fa_slot(tu * C + cc) * ST + w;
-    uint32_t* pv = lds + fa_slot(tv * C + cc) * ST + w;
-    uint32_t xv[NP], acc[NP];
-    if (inv) {
+template <int KC, bool INV>
+__device__ __forceinline__ void fa_layer16(const FaArgs& a, uint32_t* lds, const uint2* ctab, int s) {
+  constexpr int LGC = FA_TL - KC, C = 1 << LGC;
+  const int w = threadIdx.x & 3, cc = (threadIdx.x >> 2) & (C - 1), bp = (threadIdx.x >> 2) >> LGC;
+  const int tu = ((bp >> s) << (s + 1)) | (bp & ((1 << s) - 1)), tv = tu | (1 << s);
+  uint32_t* pu = lds + fa_slot(tu * C + cc) * FA_ST16 + w;
+  uint32_t* pv = lds + fa_slot(tv * C + cc) * FA_ST16 + w;
+  uint32_t xv[16], acc[16];
 #pragma unroll
-      for (int p = 0; p < NP; p++) {
-        xv[p] = pv[4 * p] ^ pu[4 * p];
-        pv[4 * p] = xv[p];
-      }
-    } else {
-#pragma unroll
-      for (int p = 0; p < NP; p++) xv[p] = pv[4 * p];
-    }
-    const uint32_t g0 = __builtin_amdgcn_readfirstlane(g);
-    if (__all(g == g0))
-      fa_mul<NP>(off ^ fa_ctab(ctab, g0), true, xv, acc);
-    else
-      fa_mul<NP>(off ^ fa_ctab(ctab, g), false, xv, acc);
-    if (inv) {
-#pragma unroll
-      for (int p = 0; p < NP; p++) pu[4 * p] ^= acc[p];
-    } else {
-#pragma unroll
-      for (int p = 0; p < NP; p++) {
-        const uint32_t un = pu[4 * p] ^ acc[p];
-        pu[4 * p] = un;
-        pv[4 * p] = xv[p] ^ un;
-      }
-    }
+  for (int p = 0; p < 16; p++) {
+    xv[p] = pv[4 * p];
+    if (INV) pv[4 * p] = xv[p] ^= pu[4 * p];
   }
-  __syncthreads();
-}
-
-// layer k = c: half 0 ^= delta * half 1, delta = C(bits above c), one constant
-// for the tile (its own inverse)
-__device__ __forceinline__ void fa_contract(const FaArgs& a, uint32_t* lds, const uint32_t* ctab, int64_t ebase) {
-  constexpr int ST = fa_stride<32>();
-  const uint32_t delta = __builtin_amdgcn_readfirstlane(fa_ctab(ctab, (uint32_t)(ebase >> a.c)));
-  const int TC = 1 << (a.R + a.lgC);
-  for (int tau = threadIdx.x; tau < TC * 4; tau += fa_threads<32>()) {
-    uint32_t* pe = lds + fa_slot(tau >> 2) * ST + (tau & 3);
-    uint32_t v[16], acc[16];
+  // the first lane's constant for all, and what the others' g add to it: a
+  // wavefront covers 16 neighbouring (butterfly, column) pairs, so at most the
+  // low four bits of g differ
+  const uint32_t g = (uint32_t)(tu >> (s + 1)), g0 = __builtin_amdgcn_readfirstlane(g), d = g ^ g0;
+  fa_mulc16(xv, __builtin_amdgcn_readfirstlane(c_fa_beta[a.a - a.c - 1 - s].x ^ fa_ctab(ctab, g0).x), acc);
+  if (__any(d != 0)) fa_add_low(xv, d, acc);
 #pragma unroll
-    for (int p = 0; p < 16; p++) v[p] = pe[4 * (16 + p)];
-    gf16_mulc(v, delta, acc);
-#pragma unroll
-    for (int p = 0; p < 16; p++) pe[4 * p] ^= acc[p];
+  for (int p = 0; p < 16; p++) {
+    const uint32_t un = pu[4 * p] ^ acc[p];
+    pu[4 * p] = un;
+    if (!INV) pv[4 * p] = xv[p] ^ un;
   }
   __syncthreads();
 }
 
 // chunk maps on the staged tile: 8 coefficient planes -> 16 coordinates, and
-// 16 coordinates -> 16 coefficient planes, per half and element word
-template <int NP, int KC, bool UN>
-__device__ __forceinline__ void fa_chunks(const FaArgs& a, uint32_t* lds) {
-  constexpr int ST = fa_stride<NP>();
-  const int TC = 1 << (a.R + a.lgC);
-  for (int tau = threadIdx.x; tau < TC * 4 * (NP / 16); tau += fa_threads<NP>()) {
-    const int w = tau & 3, h = NP == 32 ? (tau >> 2) & 1 : 0, el = tau >> (NP == 32 ? 3 : 2);
-    uint32_t* pe = lds + fa_slot(el) * ST + 64 * h + w;
+// 16 coordinates -> 16 coefficient planes
+template <int KC, bool UN>
+__device__ __forceinline__ void fa_chunks(uint32_t* lds) {
+  for (int tau = threadIdx.x; tau < 4 << FA_TL; tau += FA_NT) {
+    uint32_t* pe = lds + fa_slot(tau >> 2) * FA_ST16 + (tau & 3);
     uint32_t in[16], out[16];
 #pragma unroll
     for (int p = 0; p < (UN ? 16 : 8); p++) in[p] = pe[4 * p];
@@ -225,8 +158,7 @@ __device__ __forceinline__ void fa_chunks(const FaArgs& a, uint32_t* lds) {
 // proper submasks j of k (levels as in conv_bits.h, one row instead of one
 // bit).  Row rho lies in plane rho >> r of element (rho mod 2^r) * C + column,
 // r = KC.  The terms are compile-time constants: with runtime term lists the two
-// passes took 1000 us more at n = 2^24, where this adds 170 and 250 us to
-// passes of 315 and 365.
+// passes took 1000 us more at n = 2^24, where this adds 170 and 250 us to theirs.
 constexpr bool fa_is_term(int k, int j) { return j < k && (j & ~k) == 0; }
 constexpr int fa_jmax(int k) {
   int m = 0;
@@ -237,7 +169,7 @@ constexpr int fa_jmax(int k) {
 
 template <int KC>
 __device__ __forceinline__ uint4& fa_row(uint32_t* lds, int rho, int c) {
-  return *(uint4*)&lds[fa_slot(((rho & ((1 << KC) - 1)) << (8 - KC)) + c) * fa_stride<16>() + 4 * (rho >> KC)];
+  return *(uint4*)&lds[fa_slot(((rho & ((1 << KC) - 1)) << (8 - KC)) + c) * FA_ST16 + 4 * (rho >> KC)];
 }
 
 // v ^= rows hb + s + half - e for the terms e = 2^J > s (FIX) or lb-side rows
@@ -262,7 +194,7 @@ __device__ __forceinline__ void fa_outer(uint32_t* lds) {
     for (int phase = 0; phase < 2; phase++) {
       if ((phase == 0) != INV) {
         constexpr int cnt = (1 << (NB - 1 - K)) << (LGE + LGC);  // hi rows i < e_max
-        for (int x = threadIdx.x; x < cnt; x += fa_threads<16>()) {
+        for (int x = threadIdx.x; x < cnt; x += FA_NT) {
           const int c = x & (C - 1), i = (x >> LGC) & ((1 << LGE) - 1), hb = ((x >> (LGC + LGE)) * 2 + 1) * half;
           uint4 v = fa_row<KC>(lds, hb + i, c);
           fa_row_terms<KC, K, true>(lds, v, hb, i, c);
@@ -271,7 +203,7 @@ __device__ __forceinline__ void fa_outer(uint32_t* lds) {
       } else {
         constexpr int cnt = 1 << (NB - 1 + LGC);
 #pragma unroll 1
-        for (int x = threadIdx.x; x < cnt; x += fa_threads<16>()) {
+        for (int x = threadIdx.x; x < cnt; x += FA_NT) {
           const int c = x & (C - 1), lo = x >> LGC, j = lo & (half - 1), lb = (lo >> K) * 2 * half;
           uint4 v = fa_row<KC>(lds, lb + j, c);
           fa_row_terms<KC, K, false>(lds, v, lb + half, j, c);
@@ -284,87 +216,45 @@ __device__ __forceinline__ void fa_outer(uint32_t* lds) {
   }
 }
 
-// pointwise product by A^
-__device__ __forceinline__ void fa_pointwise(const FaArgs& a, const uint32_t* __restrict__ ahat, uint32_t* lds,
-                                             int64_t ebase) {
-  constexpr int ST = fa_stride<32>();
-  const int TC = 1 << (a.R + a.lgC);  // the lowest pass: consecutive elements
-  for (int tau = threadIdx.x; tau < TC * 4; tau += fa_threads<32>()) {
-    const int el = tau >> 2;
-    uint32_t* pe = lds + fa_slot(el) * ST + (tau & 3);
-    uint32_t x[32], y[32];
-#pragma unroll
-    for (int p = 0; p < 32; p++) x[p] = pe[4 * p];
-    gf32_mulc<false>(x, ahat[ebase + el], y);
-#pragma unroll
-    for (int p = 0; p < 32; p++) pe[4 * p] = y[p];
-  }
-  __syncthreads();
+// address of element e's coefficient q of half h in natural order
+CUOT_DEV int64_t fa_nat(const FaArgs& a, int64_t e, int h, int q) {
+  return ((int64_t)q << (a.K - 4)) | ((e >> a.c) << (a.c + 1)) | ((int64_t)h << a.c) | (e & (((int64_t)1 << a.c) - 1));
 }
 
-// KC: chunk maps of the first / last pass (see qc_fa.h); -1: neither
-template <int NP, int KC>
-__global__ __launch_bounds__(fa_threads<NP>()) __attribute__((amdgpu_waves_per_eu(NP == 16 ? 4 : 2))) void fa_pass(
-    FaArgs a) {
+// staging addresses come from an opaque copy of the lane index, so that the
+// compiler recomputes them per phase instead of holding them through the layers
+__device__ __forceinline__ int opaque_tid() {
+  int t = (int)threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+template <int KC, bool INV>
+__global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void fa_pass16(FaArgs a) {
   extern __shared__ uint32_t lds[];
-  constexpr int ST = fa_stride<NP>();
-  constexpr int NT = fa_threads<NP>();
-  constexpr int LD = fa_ld<NP>();
+  constexpr int LGC = FA_TL - KC, C = 1 << LGC, TC = 1 << FA_TL;
   const int64_t ioff = (int64_t)blockIdx.y * a.XS;
   uint4* E = a.E + ioff;
   const uint4* nin = a.nat_in + ioff;
   uint4* nout = a.nat_out + ioff;
-  const uint32_t* ahat = a.ahats ? a.ahats[blockIdx.y] : a.ahat;
-  const int h = NP == 16 ? (int)blockIdx.z : 0;
-  const int C = 1 << a.lgC;
-  const int TC = 1 << (a.R + a.lgC);
-  const int64_t cblocks = ((int64_t)1 << a.lo) >> a.lgC;
-  const int64_t ntiles = ((int64_t)1 << (a.K - 5)) / TC;
-  uint32_t* ctab = lds + TC * ST;
-  fa_ctab_fill(ctab, threadIdx.x, NT);  // read after the first barrier
-  uint4 v[LD];
-  // staging addresses come from an opaque copy of the lane index, so that the
-  // compiler recomputes them per phase instead of holding them through the
-  // layers
-  auto opaque_tid = [] {
-    int t = (int)threadIdx.x;
-    asm volatile("" : "+v"(t));
-    return t;
-  };
-  auto tile_base = [&](int64_t tile) {
-    return ((tile >> (a.lo - a.lgC)) << (a.lo + a.R)) | ((tile & (cblocks - 1)) << a.lgC);
-  };
-  // element-major staging word f: plane fastest; element t * C + c of the tile
-  auto e_addr = [&](int64_t eb, int f, int& el) {
-    el = f / NP;
-    const int t = el >> a.lgC, c = el & (C - 1);
-    return (eb + ((int64_t)t << a.lo) + c) * 32 + 16 * h + (f % NP);
-  };
-  // natural-order staging word f: element fastest, then (half, coefficient
-  // plane) of np planes per half
-  auto n_addr = [&](int64_t eb, int f, int lgnp, int& el, int& p) {
-    el = f & (TC - 1);
-    const int hp = f >> (a.R + a.lgC);
-    const int q = hp & ((1 << lgnp) - 1), hh = NP == 32 ? hp >> lgnp : h;
-    p = (NP == 32 ? 16 * hh : 0) + q;
-    const int64_t e = eb + ((int64_t)(el >> a.lgC) << a.lo) + (el & (C - 1));
-    return ((int64_t)q << (a.K - 4)) | ((e >> a.c) << (a.c + 1)) | ((int64_t)hh << a.c) |
-           (e & (((int64_t)1 << a.c) - 1));
-  };
-  const int n4 = TC * NP;
+  const int h = (int)blockIdx.z;
+  const int64_t ntiles = ((int64_t)1 << (a.K - 5)) >> FA_TL;
+  uint2* ctab = (uint2*)(lds + TC * FA_ST16);
+  fa_ctab_fill(ctab, threadIdx.x, FA_NT);  // read after the first barrier
+  // a tile's base is its first column: the 2^KC elements are all those 2^c apart
+  auto elem = [&](int64_t tile, int el) { return (tile << LGC) + ((int64_t)(el >> LGC) << a.c) + (el & (C - 1)); };
+  // staged word f: plane fastest in element-major data, element fastest in natural order
+  uint4 v[8];
   auto load_tile = [&](int64_t tile) {
     const int tid = opaque_tid();
-    const int64_t eb = tile_base(tile);
 #pragma unroll
-    for (int u = 0; u < LD; u++) {
-      const int f = tid + u * NT;
-      int el, p;
+    for (int u = 0; u < (INV ? 8 : 4); u++) {
+      const int f = tid + u * FA_NT;
       v[u] = z4();
-      if (KC >= 0 && a.first) {
-        if (u < LD / 2 && f < n4 / 2) v[u] = nin[n_addr(eb, f, 3, el, p)];
-      } else if (f < n4) {
-        v[u] = E[e_addr(eb, f, el)];
-      }
+      if constexpr (INV)
+        v[u] = E[elem(tile, f >> 4) * 32 + 16 * h + (f & 15)];
+      else
+        v[u] = nin[fa_nat(a, elem(tile, f & (TC - 1)), h, f >> FA_TL)];
     }
   };
   // workgroups are dealt to the 8 XCDs in turn: one XCD's take neighbouring tiles
@@ -372,83 +262,306 @@ __global__ __launch_bounds__(fa_threads<NP>()) __attribute__((amdgpu_waves_per_e
   const int64_t slot = (G & 7) ? bx : (bx & 7) * (G >> 3) + (bx >> 3);
   if (slot < ntiles) load_tile(slot);
   for (int64_t tile = slot; tile < ntiles; tile += G) {
-    const int64_t eb = tile_base(tile);
-    {
-      const int tid = opaque_tid();
+    int tid = opaque_tid();
 #pragma unroll
-      for (int u = 0; u < LD; u++) {
-        const int f = tid + u * NT;
-        int el, p;
-        if (KC >= 0 && a.first) {
-          if (u < LD / 2 && f < n4 / 2) {
-            n_addr(eb, f, 3, el, p);
-            *(uint4*)&lds[fa_slot(el) * ST + p * 4] = v[u];
-          }
-        } else if (f < n4) {
-          el = f / NP;
-          *(uint4*)&lds[fa_slot(el) * ST + (f % NP) * 4] = v[u];
-        }
-      }
+    for (int u = 0; u < (INV ? 8 : 4); u++) {
+      const int f = tid + u * FA_NT;
+      *(uint4*)&lds[fa_slot(INV ? f >> 4 : f & (TC - 1)) * FA_ST16 + (INV ? f & 15 : f >> FA_TL) * 4] = v[u];
     }
     __syncthreads();
-    if constexpr (KC >= 0) {
-      if constexpr (NP == 16 && KC > 1) {
-        if (a.first) fa_outer<KC, false>(lds);
-      }
-      if (a.first) fa_chunks<NP, KC, false>(a, lds);
+    if constexpr (!INV) {
+      if constexpr (KC > 1) fa_outer<KC, false>(lds);
+      fa_chunks<KC, false>(lds);
     }
-    if constexpr (NP == 32) {
-      if (a.contract && a.mode == FA_FWD) fa_contract(a, lds, ctab, eb);
+    // one loop, so that the layer's code is there once
+#pragma unroll 1
+    for (int step = 0; step < KC; step++) fa_layer16<KC, INV>(a, lds, ctab, INV ? step : KC - 1 - step);
+    if constexpr (INV) {
+      fa_chunks<KC, true>(lds);
+      if constexpr (KC > 1) fa_outer<KC, true>(lds);
     }
-    // one step loop so that the layer body is instantiated once
-    const int s_fwd = a.mode != FA_INV ? a.R : 0;
-    const int s_pw = a.mode == FA_FUSED ? 1 : 0;
-    const int s_inv = a.mode != FA_FWD ? a.R : 0;
-    for (int step = 0; step < s_fwd + s_pw + s_inv; step++) {
-      if (step == s_fwd && s_pw) {
-        if constexpr (NP == 32) fa_pointwise(a, ahat, lds, eb);
-      } else {
-        const bool inv = step >= s_fwd;
-        fa_layer<NP>(a, lds, ctab, eb, inv ? step - s_fwd - s_pw : a.R - 1 - step, inv);
-      }
-    }
-    if constexpr (NP == 32) {
-      if (a.contract && a.mode == FA_INV) fa_contract(a, lds, ctab, eb);
-    }
-    if constexpr (KC >= 0) {
-      if (a.last) fa_chunks<NP, KC, true>(a, lds);
-      if constexpr (NP == 16 && KC > 1) {
-        if (a.last) fa_outer<KC, true>(lds);
-      }
-    }
-    uint4 w[LD];
-    const int tid = opaque_tid();
+    uint4 w[8];
+    tid = opaque_tid();
 #pragma unroll
-    for (int u = 0; u < LD; u++) {
-      const int f = tid + u * NT;
+    for (int u = 0; u < 8; u++) {
+      const int f = tid + u * FA_NT;
       w[u] = z4();
-      if (f < n4) {
-        int el, p = f % NP;
-        if (KC >= 0 && a.last)
-          n_addr(eb, f, 4, el, p);
-        else
-          el = f / NP;
-        w[u] = *(const uint4*)&lds[fa_slot(el) * ST + p * 4];
-      }
+      w[u] = *(const uint4*)&lds[fa_slot(INV ? f & (TC - 1) : f >> 4) * FA_ST16 + (INV ? f >> FA_TL : f & 15) * 4];
     }
     // the next tile's loads are issued before this tile's stores
     if (tile + G < ntiles) load_tile(tile + G);
 #pragma unroll
-    for (int u = 0; u < LD; u++) {
-      const int f = tid + u * NT;
-      if (f < n4) {
-        int el, p;
-        if (KC >= 0 && a.last)
-          nout[n_addr(eb, f, 4, el, p)] = w[u];
-        else
-          E[e_addr(eb, f, el)] = w[u];
-      }
+    for (int u = 0; u < 8; u++) {
+      const int f = tid + u * FA_NT;
+      if constexpr (INV)
+        nout[fa_nat(a, elem(tile, f & (TC - 1)), h, f >> FA_TL)] = w[u];
+      else
+        E[elem(tile, f >> 4) * 32 + 16 * h + (f & 15)] = w[u];
     }
+    __syncthreads();
+  }
+}
+
+// ---- GF(2^32) passes: layers k < c ------------------------------------------------
+// A workgroup of 512 lanes holds a tile of 256 elements (2^R of them 2^lo apart
+// times 2^lgC consecutive ones) in registers: lane P * 4 + w has word w of the
+// two elements of butterfly P, all 32 planes of both.  Between layers a lane
+// gives one of the two to the lane whose P differs in the next layer's bit and
+// takes one: through LDS where that is another wavefront, by lane swaps inside
+// one.  Held in LDS (128 elements a tile, 256 lanes at 250 registers, every layer
+// reading and writing all of it), two wavefronts per SIMD waited half of the
+// time; registers hold twice the tile at four wavefronts, and three passes do
+// where five did.  At n = 2^24 the passes took 355 + 312 + 924 + 314 + 342 us, now
+// 298 + 645 + 305; the middle one issues vector operations all the time, the
+// others run at 3.6 TB/s.  Tiles of 128 elements (twice the workgroups where
+// there are few) gain 3 to 4 % of an encode at n = 2^16 .. 2^17, 1 % at 2^18 and
+// lose from there on: not worth the second set of kernels.
+constexpr int FA_ST = 132;  // LDS words of a staged element: 32 planes x 4, 4 of padding
+
+// give u (where this lane's P has bit b set) or v to the lane whose P differs in
+// that bit and take the same from it
+// (N lanes further; the quads of a row whose bit is set are the BANKS)
+template <int N, int BANKS>
+__device__ __forceinline__ void fa_swap_dpp(uint32_t* u, uint32_t* v) {
+#pragma unroll
+  for (int p = 0; p < 32; p++) {
+    const int a = (int)u[p], b = (int)v[p];
+    u[p] = (uint32_t)__builtin_amdgcn_update_dpp(a, b, 0x110 | N, 0xF, BANKS, false);       // row_shr
+    v[p] = (uint32_t)__builtin_amdgcn_update_dpp(b, a, 0x100 | N, 0xF, 0xF ^ BANKS, false);  // row_shl
+  }
+}
+
+__device__ __forceinline__ void fa_swap_lds(uint32_t* lds, uint32_t* g, int other) {
+#pragma unroll
+  for (int p = 0; p < 32; p++) lds[p * FA_NT + threadIdx.x] = g[p];
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < 32; p++) g[p] = lds[p * FA_NT + other];
+  __syncthreads();
+}
+
+__device__ __forceinline__ void fa_swap(uint32_t* lds, uint32_t* u, uint32_t* v, int P, int b) {
+  // (b opaque in between: as one chain of choices the compiler merges all ways
+  // behind 64 moves)
+#define FA_OPAQUE(x) \
+  x = __builtin_amdgcn_readfirstlane(x); \
+  asm volatile("" : "+s"(x))
+  if (b >= 4) {  // another wavefront; the bit is this one's
+    const int other = (int)threadIdx.x ^ (4 << b);
+    int bit = __builtin_amdgcn_readfirstlane(P >> b) & 1;
+    if (bit) fa_swap_lds(lds, u, other);
+    FA_OPAQUE(bit);
+    if (!bit) fa_swap_lds(lds, v, other);
+  }
+  FA_OPAQUE(b);
+  if (b == 3) {
+#pragma unroll
+    for (int p = 0; p < 32; p++) {
+      const auto r = __builtin_amdgcn_permlane32_swap(u[p], v[p], false, false);
+      u[p] = r[0];
+      v[p] = r[1];
+    }
+  }
+  FA_OPAQUE(b);
+  if (b == 2) {
+#pragma unroll
+    for (int p = 0; p < 32; p++) {
+      const auto r = __builtin_amdgcn_permlane16_swap(u[p], v[p], false, false);
+      u[p] = r[0];
+      v[p] = r[1];
+    }
+  }
+  FA_OPAQUE(b);
+  if (b == 1) fa_swap_dpp<8, 0xC>(u, v);
+  FA_OPAQUE(b);
+  if (b == 0) fa_swap_dpp<4, 0xA>(u, v);
+}
+
+CUOT_DEV int fa_insert(int P, int b, int r) { return ((P >> b) << (b + 1)) | (r << b) | (P & ((1 << b) - 1)); }
+
+template <int MODE, bool NAT>
+__global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void fa_pass32(FaArgs a) {
+  extern __shared__ uint32_t lds[];
+  constexpr int TL = FA_TL, NT = FA_NT, NH = 1 << (TL - 1);  // NH: elements of half a tile
+  const int64_t ioff = (int64_t)blockIdx.y * a.XS;
+  uint4* E = a.E + ioff;
+  const uint4* nin = a.nat_in + ioff;
+  uint4* nout = a.nat_out + ioff;
+  const uint32_t* ahat = a.ahats ? a.ahats[blockIdx.y] : a.ahat;
+  const int tid = threadIdx.x, w = tid & 3, P = tid >> 2;
+  const int lgC = TL - a.R, C = 1 << lgC;
+  const int64_t cblocks = ((int64_t)1 << a.lo) >> lgC;
+  const int64_t ntiles = ((int64_t)1 << (a.K - 5)) >> TL;
+  uint2* ctab = (uint2*)(lds + NH * FA_ST);
+  fa_ctab_fill(ctab, tid, NT);  // read after the first barrier
+  // the register bit of the tile index when the tile is read and written
+  const int rin = MODE == FA_INV ? lgC : TL - 1, rout = MODE == FA_FWD ? lgC : TL - 1;
+  const int64_t G = gridDim.x, bx = blockIdx.x;
+  // workgroups are dealt to the 8 XCDs in turn: one XCD's take neighbouring tiles
+  const int64_t slot = (G & 7) ? bx : (bx & 7) * (G >> 3) + (bx >> 3);
+  for (int64_t tile = slot; tile < ntiles; tile += G) {
+    const int64_t eb = ((tile >> (a.lo - lgC)) << (a.lo + a.R)) | ((tile & (cblocks - 1)) << lgC);
+    // Addresses are sums over the bits of the index: a part of the lane's bits (32
+    // bits of it) and a scalar one, both per half of the tile (register bit r).
+    auto off = [&](int i) { return ((uint32_t)(i >> lgC) << a.lo) | (uint32_t)(i & (C - 1)); };
+    uint32_t u[32], v[32];
+    // the tile's two halves, NH elements each, through LDS
+    uint4 st[8];
+    constexpr bool NIN = NAT && MODE == FA_FWD, NOUT = NAT && MODE == FA_INV;
+    // natural order, word f = tid + NT k: element fastest, then coefficient (QB
+    // bits) and half; else plane fastest, then element
+    auto addr = [&](uint4* p, bool nat, int QB, int reg, int r, int tid, int k) {
+      const int fh = nat ? 4 * k : (NT >> 5) * k, fl = nat ? tid >> (TL - 1) : tid >> 5;  // the index above the fastest part
+      int64_t sc;
+      uint32_t ln;
+      if (nat) {
+        auto hq = [&](int x) { return (uint32_t)(x & ((1 << QB) - 1)) << (a.K - 4) | (uint32_t)(x >> QB) << a.c; };
+        sc = eb + off(r << reg) + hq(fh);
+        ln = off(fa_insert(tid & (NH - 1), reg, 0)) + hq(fl);
+      } else {
+        sc = (eb + off(fa_insert(fh, reg, r))) * 32;
+        ln = off(fa_insert(fl, reg, 0)) * 32 + (tid & 31);
+      }
+      return (uint4*)((char*)(p + sc) + (size_t)(ln * 16));
+    };
+    auto fetch = [&](int r) {
+      const int tid = opaque_tid();
+#pragma unroll
+      for (int k = 0; k < (NIN ? 4 : 8); k++) {
+        st[k] = z4();
+        st[k] = *addr(NIN ? (uint4*)nin : E, NIN, 3, rin, r, tid, k);
+      }
+    };
+    auto take = [&]() {
+      const int tid = opaque_tid();
+#pragma unroll
+      for (int k = 0; k < (NIN ? 4 : 8); k++) {
+        const int f = tid + k * NT;
+        if constexpr (NIN)
+          *(uint4*)&lds[(f & (NH - 1)) * FA_ST + (f >> (TL + 2)) * 64 + ((f >> (TL - 1)) & 7) * 4] = st[k];
+        else
+          *(uint4*)&lds[(f >> 5) * FA_ST + (f & 31) * 4] = st[k];
+      }
+    };
+    auto read = [&](uint32_t* x) {
+      if constexpr (NIN) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          uint32_t t[8];
+#pragma unroll
+          for (int q = 0; q < 8; q++) t[q] = lds[P * FA_ST + h * 64 + q * 4 + w];
+          fa_pack_planes<0>(t, x + 16 * h);
+        }
+      } else {
+#pragma unroll
+        for (int p = 0; p < 32; p++) x[p] = lds[P * FA_ST + p * 4 + w];
+      }
+    };
+    fetch(0);
+    take();
+    __syncthreads();
+    fetch(1);
+    read(u);
+    __syncthreads();
+    take();
+    __syncthreads();
+    read(v);
+    __syncthreads();
+    uint2 ac = make_uint2(0, 0), an = make_uint2(0, 0);
+    if constexpr (MODE == FA_FUSED) {
+      ac = *(const uint2*)&ahat[eb + 2 * P];
+      an = *(const uint2*)&ahat[((int64_t)1 << (a.K - 5)) + eb + 2 * P];
+    }
+    // layer k = c: half 0 ^= delta * half 1, delta = C(bits above c), one constant
+    // for the tile (its own inverse)
+    auto contract = [&]() {
+      const uint32_t delta = __builtin_amdgcn_readfirstlane(fa_ctab(ctab, (uint32_t)(eb >> a.c)).x);
+      uint32_t t[16];
+      fa_mulc16(u + 16, delta, t);
+#pragma unroll
+      for (int p = 0; p < 16; p++) u[p] ^= t[p];
+      fa_mulc16(v + 16, delta, t);
+#pragma unroll
+      for (int p = 0; p < 16; p++) v[p] ^= t[p];
+    };
+    if (MODE == FA_FWD && a.contract) contract();
+    const int layers = TL - lgC;
+    // forward from tile bit 7 down to lgC, then back up; one loop, so that the
+    // layer's code is there once
+    for (int step = 0; step < (MODE == FA_FUSED ? 2 * layers : layers); step++) {
+      const bool inv = MODE == FA_INV || (MODE == FA_FUSED && step >= layers);
+      const int up = MODE == FA_FUSED ? step - layers : step;
+      const int b = inv ? lgC + up : TL - 1 - step;
+      int sw = step == 0 ? -1 : inv ? b - 1 : b;  // the bit of P to swap with
+      if constexpr (MODE == FA_FUSED) {
+        if (step == layers) {
+          sw = -1;
+          asm volatile("" : "+v"(ac.x), "+v"(ac.y), "+v"(an.x), "+v"(an.y));  // their 96 masks stay in here
+          fa_mulv32(u, ac.x, an.x);
+          __builtin_amdgcn_sched_barrier(0);
+          fa_mulv32(v, ac.y, an.y);
+        }
+      }
+      FA_OPAQUE(sw);
+      fa_swap(lds, u, v, P, sw);
+      const int k = a.lo + b - lgC;
+      const uint32_t e = (uint32_t)eb + off(fa_insert(P, b, 0));
+      const uint32_t g = ((e >> a.c) << (a.c - k)) | ((e & ((1u << a.c) - 1)) >> (k + 1));
+      // the first lane's constant for all, and what the others' g add to it: a
+      // wavefront covers 16 neighbouring P, so at most the low four bits differ
+      const uint32_t g0 = __builtin_amdgcn_readfirstlane(g), d = g ^ g0;
+      const uint2 c = x2(c_fa_beta[a.a - k], fa_ctab(ctab, g0));
+      // (fused: by a mask, as a branch costs moves of both)
+      auto add_u = [&](bool now) {
+        if constexpr (MODE == FA_FUSED) {
+#pragma unroll
+          for (int p = 0; p < 32; p++) asm("v_bitop3_b32 %0, %0, %1, %2 bitop3:0x78" : "+v"(v[p]) : "v"(u[p]), "s"(0 - (int)now));
+        } else if (now) {
+#pragma unroll
+          for (int p = 0; p < 32; p++) v[p] ^= u[p];
+        }
+      };
+      add_u(inv);
+      fa_add_mul32(u, v, __builtin_amdgcn_readfirstlane(c.x), __builtin_amdgcn_readfirstlane(c.y));
+      if (__any(d != 0)) {
+        fa_add_low(v, d, u);
+        fa_add_low(v + 16, d, u + 16);
+      }
+      add_u(!inv);
+    }
+    if (MODE == FA_INV && a.contract) contract();
+    auto put = [&](const uint32_t* x) {
+      if constexpr (NOUT) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          uint32_t t[16];
+          fa_unpack_planes<0>(x + 16 * h, t);
+#pragma unroll
+          for (int q = 0; q < 16; q++) lds[P * FA_ST + h * 64 + q * 4 + w] = t[q];
+        }
+      } else {
+#pragma unroll
+        for (int p = 0; p < 32; p++) lds[P * FA_ST + p * 4 + w] = x[p];
+      }
+    };
+    auto store = [&](int r) {
+      const int tid = opaque_tid();
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const int f = tid + k * NT;
+        *addr(NOUT ? nout : E, NOUT, 4, rout, r, tid, k) =
+            *(const uint4*)&lds[NOUT ? (f & (NH - 1)) * FA_ST + (f >> (TL + 3)) * 64 + ((f >> (TL - 1)) & 15) * 4
+                                     : (f >> 5) * FA_ST + (f & 31) * 4];
+      }
+    };
+    __syncthreads();
+    put(u);
+    __syncthreads();
+    store(0);
+    __syncthreads();
+    put(v);
+    __syncthreads();
+    store(1);
     __syncthreads();
   }
 }
@@ -686,26 +799,7 @@ CUOT_DEV int fa_terms(int k, uint32_t* e) {
 
 // ---- A^: the scalar transform of the single polynomial a ------------------------------
 // One 32-bit word per point.  The words behind A^ (a word per point again) hold
-// a's bits while they are converted.
-CUOT_DEV uint32_t gf16_mul_dev(uint32_t a, uint32_t b) {
-  uint32_t r = 0;
-#pragma unroll
-  for (int i = 0; i < 16; i++) r ^= (a << i) & (0u - ((b >> i) & 1u));
-  // z^16 = z^5 + z^3 + z + 1, twice (the first fold leaves degree <= 19)
-#pragma unroll
-  for (int f = 0; f < 2; f++) {
-    const uint32_t t = r >> 16;
-    r = (r & 0xffffu) ^ t ^ (t << 1) ^ (t << 3) ^ (t << 5);
-  }
-  return r;
-}
-
-CUOT_DEV uint32_t gf32_mul_dev(uint32_t a, uint32_t b) {
-  const uint32_t a0 = a & 0xFFFFu, a1 = a >> 16, b0 = b & 0xFFFFu, b1 = b >> 16;
-  const uint32_t p0 = gf16_mul_dev(a0, b0), p1 = gf16_mul_dev(a1, b1), p2 = gf16_mul_dev(a0 ^ a1, b0 ^ b1);
-  return (p0 ^ gf16_times_nu(p1)) | ((p2 ^ p0) << 16);
-}
-
+// a's bits while they are converted and nu times the values' theta parts in the end.
 __global__ __launch_bounds__(256) void fa_prep_bits(const QcPrep* __restrict__ pr, QcPrep pr1, int K) {
   const QcPrep q = pr ? pr[blockIdx.y] : pr1;
   uint32_t* T = q.ahat + ((int64_t)1 << (K - 5));
@@ -793,7 +887,7 @@ constexpr int FA_PT = 10;  // log2 words of a preparation tile
 __global__ __launch_bounds__(512) void fa_prep_fft(const QcPrep* __restrict__ pr, QcPrep pr1, int K, int c, int aidx,
                                                    int lo, int R, int lgC, int first, int src) {
   __shared__ uint32_t L[1 << FA_PT];
-  __shared__ uint32_t ctab[FA_CTAB];
+  __shared__ uint2 ctab[FA_CTAB];
   const QcPrep q = pr ? pr[blockIdx.y] : pr1;
   uint32_t* A = q.ahat;
   const int nt = blockDim.x;
@@ -829,12 +923,12 @@ __global__ __launch_bounds__(512) void fa_prep_fft(const QcPrep* __restrict__ pr
       // layer k = c between the two kinds: half 0 ^= C(bits above) * half 1
       for (int i = threadIdx.x; i < TW; i += nt) {
         const uint32_t x = L[i];
-        L[i] = x ^ gf16_mul_dev(fa_ctab(ctab, (uint32_t)(eidx(i) >> c)), x >> 16);
+        L[i] = x ^ fa_mul16_dev(x >> 16, fa_ctab(ctab, (uint32_t)(eidx(i) >> c)).x);
       }
       __syncthreads();
     }
     const int k = b >= c ? b + 1 : b;
-    const uint32_t off = c_fa_beta[aidx - k];
+    const uint2 off = c_fa_beta[aidx - k];
     for (int t = threadIdx.x; t < (TW >> 1); t += nt) {
       const int cc = t & (C - 1), bp = t >> lgC;
       const int tu = ((bp >> s) << (s + 1)) | (bp & ((1 << s) - 1));
@@ -843,46 +937,70 @@ __global__ __launch_bounds__(512) void fa_prep_fft(const QcPrep* __restrict__ pr
       const uint32_t xv = L[v];
       uint32_t xu = L[u];
       if (b >= c) {
-        const uint32_t cst = off ^ fa_ctab(ctab, e >> (b + 1));
-        xu ^= gf16_mul_dev(cst, xv & 0xffffu) | (gf16_mul_dev(cst, xv >> 16) << 16);
+        const uint32_t cst = off.x ^ fa_ctab(ctab, e >> (b + 1)).x;
+        xu ^= fa_mul16_dev(xv & 0xffffu, cst) | (fa_mul16_dev(xv >> 16, cst) << 16);
       } else {
         const uint32_t g = ((e >> c) << (c - k)) | ((e & ((1u << c) - 1)) >> (k + 1));
-        xu ^= gf32_mul_dev(off ^ fa_ctab(ctab, g), xv);
+        const uint2 cst = x2(off, fa_ctab(ctab, g));
+        xu ^= fa_mul32_dev(xv, cst.x, cst.y);
       }
       L[u] = xu;
       L[v] = xv ^ xu;
     }
     __syncthreads();
   }
-  for (int i = threadIdx.x; i < TW; i += nt) A[eidx(i)] = L[i];
+  for (int i = threadIdx.x; i < TW; i += nt) {
+    const int64_t e = eidx(i);
+    A[e] = L[i];
+    if (lo == 0) A[((int64_t)1 << (K - 5)) + e] = fa_mul16_dev(L[i] >> 16, FA_NU);
+  }
 }
 
 // ---- host -------------------------------------------------------------------------------
 int g_fa_ready = 0;
 
-template <int NP, int KC>
-hipError_t fa_allow_lds() {
-  return hipFuncSetAttribute((const void*)fa_pass<NP, KC>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (fa_tile<NP>() * fa_stride<NP>() + FA_CTAB) * 4);
+constexpr size_t FA_LDS16 = 256 * FA_ST16 * 4 + FA_CTAB * sizeof(uint2);
+
+template <int KC>
+hipError_t fa_allow_lds16() {
+  hipError_t e = hipFuncSetAttribute((const void*)fa_pass16<KC, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)FA_LDS16);
+  if (!e)
+    e = hipFuncSetAttribute((const void*)fa_pass16<KC, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)FA_LDS16);
+  return e;
+}
+
+constexpr size_t FA_LDS32 = (FA_ST * 4 << (FA_TL - 1)) + FA_CTAB * sizeof(uint2);
+
+template <int MODE, bool NAT>
+hipError_t fa_allow_lds32() {
+  return hipFuncSetAttribute((const void*)fa_pass32<MODE, NAT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)FA_LDS32);
 }
 
 hipError_t fa_configure() {
   if (g_fa_ready) return hipSuccess;
-  uint32_t beta[32], pack[FA_KC_MAX + 1][8];
-  fa_basis(beta);
+  uint32_t basis[32], pack[FA_KC_MAX + 1][8];
+  fa_basis(basis);
+  uint2 beta[32];
+  for (int i = 0; i < 32; i++) beta[i] = make_uint2(basis[i], fa_mul16(FA_NU, basis[i] >> 16));
   const FaChunk ch[FA_KC_MAX + 1] = {kFaChunk<0>, kFaChunk<1>, kFaChunk<2>, kFaChunk<3>, kFaChunk<4>, kFaChunk<5>};
   // pack[b]: bits 0..2 of b are index bits K-4 .. K-2
   for (int i = 0; i <= FA_KC_MAX; i++)
     for (int q = 0; q < 8; q++) pack[i][q] = ch[i].pack[q];
   hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(c_fa_beta), beta, sizeof(beta));
   if (!e) e = hipMemcpyToSymbol(HIP_SYMBOL(c_fa_pack), pack, sizeof(pack));
-  if (!e) e = fa_allow_lds<32, -1>();
-  if (!e) e = fa_allow_lds<32, 0>();
-  if (!e) e = fa_allow_lds<16, 1>();
-  if (!e) e = fa_allow_lds<16, 2>();
-  if (!e) e = fa_allow_lds<16, 3>();
-  if (!e) e = fa_allow_lds<16, 4>();
-  if (!e) e = fa_allow_lds<16, 5>();
+  if (!e) e = fa_allow_lds32<FA_FWD, false>();
+  if (!e) e = fa_allow_lds32<FA_FWD, true>();
+  if (!e) e = fa_allow_lds32<FA_FUSED, false>();
+  if (!e) e = fa_allow_lds32<FA_INV, false>();
+  if (!e) e = fa_allow_lds32<FA_INV, true>();
+  if (!e) e = fa_allow_lds16<1>();
+  if (!e) e = fa_allow_lds16<2>();
+  if (!e) e = fa_allow_lds16<3>();
+  if (!e) e = fa_allow_lds16<4>();
+  if (!e) e = fa_allow_lds16<5>();
   if (!e)
     e = hipFuncSetAttribute((const void*)fa_prep_rows, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)cbp_words(32 * 1024, true) * 4);
@@ -909,105 +1027,75 @@ void fa_launch_level(const QcIo* io, QcIo io1, const uint4* in, uint4* out, int6
   cuot_rec_end(st);
 }
 
-template <int NP, int KC>
-void fa_launch(const FaArgs& a, int B, hipStream_t st) {
-  constexpr int Z = 32 / NP;
-  const int64_t ntiles = ((int64_t)1 << (a.K - 5)) >> (a.R + a.lgC);
+template <bool INV>
+void fa_launch16(const FaArgs& a, int B, hipStream_t st) {
+  const int64_t ntiles = ((int64_t)1 << (a.K - 5)) >> FA_TL;
   // two resident workgroups on each of the 256 CUs; every one walks many tiles
-  const int64_t cap = 512 / (B * Z) < 1 ? 1 : 512 / (B * Z);
+  const dim3 grid(capg(ntiles, 256 / B < 1 ? 1 : 256 / B), (unsigned)B, 2);
   const double per = 512.0 * (double)((int64_t)1 << (a.K - 5)) * B;
-  cuot_rec_begin(st, NP == 16 ? "fa_pass<16>" : "fa_pass<32>", a.first ? per * 1.5 : per * 2.0);
-  hipLaunchKernelGGL((fa_pass<NP, KC>), dim3(capg(ntiles, cap), (unsigned)B, (unsigned)Z), dim3(fa_threads<NP>()),
-                     ((size_t)fa_stride<NP>() * ((size_t)1 << (a.R + a.lgC)) + FA_CTAB) * 4, st, a);
+  cuot_rec_begin(st, "fa_pass16", INV ? per * 2.0 : per * 1.5);
+  switch (a.K - 20) {
+#define FA_CASE(KC) \
+  case KC: hipLaunchKernelGGL((fa_pass16<KC, INV>), grid, dim3(FA_NT), FA_LDS16, st, a); break;
+    FA_CASE(1)
+    FA_CASE(2)
+    FA_CASE(3)
+    FA_CASE(4)
+    FA_CASE(5)
+#undef FA_CASE
+  }
   cuot_rec_end(st);
 }
 
-template <int NP>
-void fa_launch_kc(const FaArgs& a, int kc, int B, hipStream_t st) {
-  switch (kc) {
-    case 1: fa_launch<16, 1>(a, B, st); break;
-    case 2: fa_launch<16, 2>(a, B, st); break;
-    case 3: fa_launch<16, 3>(a, B, st); break;
-    case 4: fa_launch<16, 4>(a, B, st); break;
-    default: fa_launch<16, 5>(a, B, st); break;
-  }
-}
-
-// Layers of the upper GF(2^32) passes, from bit c-1 down to the fused pass's 7:
-// tiles of 2^4 elements times 8 columns (up to 5 layers in one pass where that
-// saves a launch): the columns and the four words share a twiddle, so most
-// wavefronts take scalar branches.  The knobs set layers and columns.
-int fa_pass_layers(int left) {
-  const int knob = cuot_knobs().qc_radix;
-  int R = knob > 0 ? (knob < 7 ? knob : 7) : (left <= 5 ? left : 4);
-  return R < left ? R : left;
-}
-
-int fa_columns(int R, int lo) {
-  const int knob = cuot_knobs().qc_cols;
-  int lgC = 7 - R;
-  if (knob > 0 && __builtin_ctz(knob) < lgC) lgC = __builtin_ctz(knob);
-  return lgC < lo ? lgC : lo;
+template <int MODE, bool NAT>
+void fa_launch32(const FaArgs& a, int B, hipStream_t st) {
+  const int64_t ntiles = ((int64_t)1 << (a.K - 5)) >> FA_TL;
+  // two resident workgroups on each of the 256 CUs; every one walks many tiles
+  const int64_t cap = 512 / B < 1 ? 1 : 512 / B;
+  const double per = 512.0 * (double)((int64_t)1 << (a.K - 5)) * B;
+  cuot_rec_begin(st, MODE == FA_FUSED ? "fa_pass32 fused" : "fa_pass32", NAT && MODE == FA_FWD ? per * 1.5 : per * 2.0);
+  hipLaunchKernelGGL((fa_pass32<MODE, NAT>), dim3(capg(ntiles, cap), (unsigned)B), dim3(FA_NT), FA_LDS32, st, a);
+  cuot_rec_end(st);
 }
 
 hipError_t fa_transform(const FaArgs& base, int B, hipStream_t st) {
   const int K = base.K, c = base.c, r = K - 5 - c;
-  const int R0 = c < 7 ? c : 7;
-  // upper passes: [lo, lo + R) from the top
+  // upper passes, [lo, lo + R) from the top down to the fused pass's eight layers:
+  // one, of at most seven (fewer layers each with the knob)
+  const int knob = cuot_knobs().qc_radix;
   int los[16], Rs[16], np = 0;
-  for (int top = c; top > R0;) {
-    Rs[np] = fa_pass_layers(top - R0);
+  for (int top = c; top > FA_TL;) {
+    Rs[np] = top - FA_TL < 7 ? top - FA_TL : 7;
+    if (knob > 0 && knob < Rs[np]) Rs[np] = knob;
     los[np] = top - Rs[np];
     top = los[np++];
   }
-  FaArgs a = base;
-  if (r > 0) {
-    a.lo = c;
-    a.R = r;
-    a.lgC = 8 - r;
-    a.mode = FA_FWD;
-    a.first = 1;
-    fa_launch_kc<16>(a, K - 20, B, st);
-  }
+  if (r > 0) fa_launch16<false>(base, B, st);
+  FaArgs a;
   for (int i = 0; i < np; i++) {
     a = base;
     a.lo = los[i];
     a.R = Rs[i];
-    a.lgC = fa_columns(a.R, a.lo);
-    a.mode = FA_FWD;
-    a.first = r == 0 && i == 0;
     a.contract = r > 0 && i == 0;
-    if (a.first)
-      fa_launch<32, 0>(a, B, st);
+    if (r == 0 && i == 0)
+      fa_launch32<FA_FWD, true>(a, B, st);
     else
-      fa_launch<32, -1>(a, B, st);
+      fa_launch32<FA_FWD, false>(a, B, st);
   }
   a = base;
-  a.R = R0;
-  a.mode = FA_FUSED;
-  fa_launch<32, -1>(a, B, st);
+  a.R = FA_TL;
+  fa_launch32<FA_FUSED, false>(a, B, st);
   for (int i = np - 1; i >= 0; i--) {
     a = base;
     a.lo = los[i];
     a.R = Rs[i];
-    a.lgC = fa_columns(a.R, a.lo);
-    a.mode = FA_INV;
-    a.last = r == 0 && i == 0;
     a.contract = r > 0 && i == 0;
-    if (a.last)
-      fa_launch<32, 0>(a, B, st);
+    if (r == 0 && i == 0)
+      fa_launch32<FA_INV, true>(a, B, st);
     else
-      fa_launch<32, -1>(a, B, st);
+      fa_launch32<FA_INV, false>(a, B, st);
   }
-  if (r > 0) {
-    a = base;
-    a.lo = c;
-    a.R = r;
-    a.lgC = 8 - r;
-    a.mode = FA_INV;
-    a.last = 1;
-    fa_launch_kc<16>(a, K - 20, B, st);
-  }
+  if (r > 0) fa_launch16<true>(base, B, st);
   return hipGetLastError();
 }
 

@@ -11,7 +11,8 @@ speed.
 
 Stages and knobs:
   * "qc"  -- quasi-cyclic encode of one party at n COTs: FFT layers per upper
-             pass (qc_radix 4..7) and columns per tile (qc_cols 1, 2, 4, 8);
+             pass (qc_radix 4..7) and, for n > 2^24, columns per tile (qc_cols
+             1, 2, 4, 8);
              features (log2 n, m, radix, log2 cols);
   * "ggm" -- GGM expansion of t trees of depth h: per-lane depth-first levels
              L (ggm_dfs, h-10 <= L <= min(h-8, 6)); features (h, log2 t, L).

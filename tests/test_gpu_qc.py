@@ -213,6 +213,19 @@ def test_qc_columns_rotations(ctx, knob_mfma, n):
     test_qc_orbit_product_rotations(ctx, knob_mfma, n)
 
 
+# fewer layers per upper pass: several passes, tiles of 2^2 .. 2^5 rows
+@pytest.mark.parametrize("radix", [2, 3, 5])
+@pytest.mark.parametrize("n", [70001, (1 << 20) + 1])
+def test_qc_orbit_layers_per_pass(ctx, knob_mfma, n, radix):
+    from cuot_amd import tune
+
+    tune.set_knobs(qc_radix=radix, qc_mfma_max=-1)
+    try:
+        test_qc_orbit_product_rotations(ctx, lambda v: None, n)
+    finally:
+        tune.set_knobs()
+
+
 @pytest.mark.parametrize("n", [4097, 8193, 20000, 131073, (1 << 19) + 1])
 def test_qc_orbit_product_vs_karatsuba(ctx, knob_mfma, n):
     print(f"qc orbits karatsuba n={n}", flush=True)
