@@ -309,9 +309,13 @@ extern "C" int cuot_sot_run_stages(cuot_ctx* ctx, const cuot_sot_config* cfg, vo
 
 // Whole instance with the independent stages overlapped on two streams (the
 // caller's and the context's second stream, joined before returning):
-//   caller: setup -> sender GGM + masked rows -> [A^] -> sender QC -> [join]
-//   second: [setup] -> A^ prepare -> sparse -> [rows] -> receiver GGM -> receiver QC
-// The two encodes use separate scratch.  Same bytes as the staged run.
+//   caller: setup -> sender GGM + masked rows -> A^ prepare -> sender QC -> sparse -> [join]
+//   second: [rows] -> receiver GGM -> receiver QC (from its pointwise product on behind [A^])
+// The two encodes use separate scratch.  Same bytes as the staged run.  A^ and
+// the sparse product beside the sender's trees instead, ahead of the receiver's,
+// and both encodes behind A^ took 829 us at n = 2^20 and 448 at 190731, this
+// way 746 and 415 (the receiver's trees start with the rows, and the caller's
+// stream has the sparse product while the receiver's encode ends).
 extern "C" int cuot_sot_run(cuot_ctx* ctx, const cuot_sot_config* cfg, void* ws_d, size_t ws_bytes, cuot_block* v_d,
                             cuot_block* w_d, uint8_t* b_d, cuot_block* delta_d, void* stream) {
   CUOT_CHECK_ARG(ctx && cfg, "ctx/cfg NULL");
@@ -327,23 +331,20 @@ extern "C" int cuot_sot_run(cuot_ctx* ctx, const cuot_sot_config* cfg, void* ws_
   CUOT_HIP_TRY(ctx->ensure_aux());
   CUOT_HIP_TRY(cuot_qc_configure());
   hipStream_t st = ctx->st(stream), ax = ctx->aux;
-  hipEvent_t e_setup = ctx->ev[0], e_prep = ctx->ev[1], e_rows = ctx->ev[2], e_done = ctx->ev[3];
+  hipEvent_t e_prep = ctx->ev[1], e_rows = ctx->ev[2], e_done = ctx->ev[3];
   CUOT_HIP_TRY(p.run_setup((blk*)delta_d, st));
-  CUOT_HIP_TRY(hipEventRecord(e_setup, st));
-  CUOT_HIP_TRY(hipStreamWaitEvent(ax, e_setup, 0));
-  // both encodes follow in this call: when they take the matrix cores, A^ is
-  // not needed (its 33 small launches took 95 us beside n = 2^14's 45 us encodes)
-  CUOT_HIP_TRY(p.run_prepare(!cuot_qc_mfma_selected(p.cfg.n), ax));
-  CUOT_HIP_TRY(hipEventRecord(e_prep, ax));
-  CUOT_HIP_TRY(cuot_launch_sparse(p.a_words, p.cfg.n, p.pos, (int)p.cfg.t, (uint32_t*)b_d, ax));
   CUOT_HIP_TRY(p.run_expand_sender(st));
   CUOT_HIP_TRY(hipEventRecord(e_rows, st));
   CUOT_HIP_TRY(hipStreamWaitEvent(ax, e_rows, 0));
   CUOT_HIP_TRY(p.run_expand_recver(ax));
-  CUOT_HIP_TRY(cuot_launch_qc_encode(p.ahat, p.cfg.n, p.leaves_r, (blk*)w_d, p.qc_scratch2, ax));
-  CUOT_HIP_TRY(hipEventRecord(e_done, ax));
-  CUOT_HIP_TRY(hipStreamWaitEvent(st, e_prep, 0));
+  // both encodes follow in this call: when they take the matrix cores, A^ is
+  // not needed (its 33 small launches took 95 us beside n = 2^14's 45 us encodes)
+  CUOT_HIP_TRY(p.run_prepare(!cuot_qc_mfma_selected(p.cfg.n), st));
+  CUOT_HIP_TRY(hipEventRecord(e_prep, st));
   CUOT_HIP_TRY(cuot_launch_qc_encode(p.ahat, p.cfg.n, p.leaves_s, (blk*)v_d, p.qc_scratch, st));
+  CUOT_HIP_TRY(cuot_launch_qc_encode(p.ahat, p.cfg.n, p.leaves_r, (blk*)w_d, p.qc_scratch2, ax, e_prep));
+  CUOT_HIP_TRY(hipEventRecord(e_done, ax));
+  CUOT_HIP_TRY(cuot_launch_sparse(p.a_words, p.cfg.n, p.pos, (int)p.cfg.t, (uint32_t*)b_d, st));
   CUOT_HIP_TRY(hipStreamWaitEvent(st, e_done, 0));
   return CUOT_OK;
 }

@@ -87,8 +87,9 @@ size_t cuot_qc_scratch_bytes_for(int64_t n);
 // whose encodes run in the same call and take it (cuot_qc_mfma_selected)
 hipError_t cuot_launch_qc_prepare(const uint8_t* a_bits, int64_t n, uint32_t* ahat, void* scratch, bool transform,
                                   hipStream_t st);
+// ready: A^ is complete at this event (of another stream; NULL: already in st's order)
 hipError_t cuot_launch_qc_encode(const uint32_t* ahat, int64_t n, const void* x, void* y, void* scratch,
-                                 hipStream_t st);
+                                 hipStream_t st, hipEvent_t ready = nullptr);
 // Batches of instances with the same transform length 2^m (one launch per
 // step, blockIdx.y = instance).  Tables live in device memory.
 struct QcIo {
@@ -115,7 +116,7 @@ hipError_t cuot_qc_fa_configure();
 size_t cuot_qc_fa_scratch_bytes(int64_t n, int B);
 hipError_t cuot_launch_qc_fa_prepare(const QcPrep* pr, QcPrep pr1, int B, int K, hipStream_t st);
 hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ahat1, const uint32_t* const* ahats, int B,
-                                    int K, int64_t nmax, void* scratch, hipStream_t st);
+                                    int K, int64_t nmax, void* scratch, hipStream_t st, hipEvent_t ready);
 // novel-basis conversion of ntiles row strings of 2^mp bits in place (qc.hip);
 // tpi strings per instance, instances inst_words apart
 hipError_t cuot_launch_conv_rows(unsigned cap, hipStream_t st, uint32_t* Bw, int64_t tile_words, int64_t ntiles,

@@ -1357,12 +1357,14 @@ hipError_t fft_inverse_upper(const Bufs& b, int m, int from, bool grouped, bool*
 }
 
 hipError_t encode_batch(const QcIo* io, QcIo io1, const uint32_t* ahat1, const uint32_t* const* ahats, int B, int m,
-                        void* scratch, hipStream_t st) {
+                        void* scratch, hipStream_t st, hipEvent_t ready = nullptr) {
   hipError_t e = configure_lds();
   if (e != hipSuccess) return e;
   if (B > 1 && !row_path(m - 1)) return hipErrorInvalidValue;
   if (cuot_qc_fa_selected(((int64_t)1 << (m + 2)) + 1))
-    return cuot_launch_qc_fa_encode(io, io1, ahat1, ahats, B, m + 4, io ? (int64_t)1 << (m + 3) : io1.n, scratch, st);
+    return cuot_launch_qc_fa_encode(io, io1, ahat1, ahats, B, m + 4, io ? (int64_t)1 << (m + 3) : io1.n, scratch, st,
+                                    ready);
+  if (ready && (e = hipStreamWaitEvent(st, ready, 0)) != hipSuccess) return e;
   const int64_t M = (int64_t)1 << m;
   Bufs b = bufs(scratch, M, B);
   cuot_rec_begin(st, "qc_pack_x", 2.0 * 16.0 * (double)(M >> 1) * 16 * B);
@@ -1495,15 +1497,17 @@ hipError_t cuot_launch_qc_prepare_batch(const QcPrep* prep_d, int B, int m, bool
 }
 
 hipError_t cuot_launch_qc_encode(const uint32_t* ahat, int64_t n, const void* x, void* y, void* scratch,
-                                 hipStream_t st) {
+                                 hipStream_t st, hipEvent_t ready) {
   QcIo io1;
   io1.x = (const uint4*)x;
   io1.y = (uint4*)y;
   io1.n = n;
   const int m = cuot_qc_log_len(n);
-  if (cuot_qc_mfma_selected(n))
-    return cuot_launch_qc_mfma(nullptr, io1, ahat + ((int64_t)1 << m), nullptr, 1, m, n, scratch, st);
-  return encode_batch(nullptr, io1, ahat, nullptr, 1, m, scratch, st);
+  if (cuot_qc_mfma_selected(n)) {
+    hipError_t e = ready ? hipStreamWaitEvent(st, ready, 0) : hipSuccess;
+    return e ? e : cuot_launch_qc_mfma(nullptr, io1, ahat + ((int64_t)1 << m), nullptr, 1, m, n, scratch, st);
+  }
+  return encode_batch(nullptr, io1, ahat, nullptr, 1, m, scratch, st, ready);
 }
 
 hipError_t cuot_launch_qc_encode_batch(const QcIo* io_d, const uint32_t* const* ahats_d, int B, int m, int64_t nmax,

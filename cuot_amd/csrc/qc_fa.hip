@@ -1058,7 +1058,7 @@ void fa_launch32(const FaArgs& a, int B, hipStream_t st) {
   cuot_rec_end(st);
 }
 
-hipError_t fa_transform(const FaArgs& base, int B, hipStream_t st) {
+hipError_t fa_transform(const FaArgs& base, int B, hipStream_t st, hipEvent_t ready) {
   const int K = base.K, c = base.c, r = K - 5 - c;
   // upper passes, [lo, lo + R) from the top down to the fused pass's eight layers:
   // one, of at most seven (fewer layers each with the knob)
@@ -1081,6 +1081,11 @@ hipError_t fa_transform(const FaArgs& base, int B, hipStream_t st) {
       fa_launch32<FA_FWD, true>(a, B, st);
     else
       fa_launch32<FA_FWD, false>(a, B, st);
+  }
+  // the first launch that reads A^
+  if (ready) {
+    hipError_t e = hipStreamWaitEvent(st, ready, 0);
+    if (e != hipSuccess) return e;
   }
   a = base;
   a.R = FA_TL;
@@ -1137,7 +1142,7 @@ hipError_t cuot_launch_qc_fa_prepare(const QcPrep* pr, QcPrep pr1, int B, int K,
 }
 
 hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ahat1, const uint32_t* const* ahats, int B,
-                                    int K, int64_t nmax, void* scratch, hipStream_t st) {
+                                    int K, int64_t nmax, void* scratch, hipStream_t st, hipEvent_t ready) {
   hipError_t e = fa_configure();
   if (e != hipSuccess) return e;
   const int64_t XS = (int64_t)1 << K;  // blocks per instance and buffer
@@ -1182,7 +1187,7 @@ hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ah
   a.K = K;
   a.c = K - 5 < 15 ? K - 5 : 15;
   a.a = 16 + a.c;
-  if ((e = fa_transform(a, B, st))) return e;
+  if ((e = fa_transform(a, B, st, ready))) return e;
   // inverse conversion of the 2^K coefficients in X
   const int mp = adic ? 16 : (K < 20 ? K : 20);
   const int64_t S = (int64_t)1 << mp, words = S / 32;
