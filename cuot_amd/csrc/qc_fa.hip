@@ -29,16 +29,18 @@
 //     k = c-1 .. 0     butterflies over GF(2^32)
 //
 // Encode (per party), blocks x_{n+i} being coefficient i of all 128 rows:
-//   128-row bit transpose, novel-basis conversion of every row string in LDS
-//   (conv_fast.h), transpose back (for K > 21 the strings are the 2^16
-//   coefficients of an expansion in powers of s_16, made on the blocks before
-//   that, and the first pass converts across the strings); for K > 20 a pass of
-//   the GF(2^16) layers, halves of the elements apart; a pass of up to seven
-//   GF(2^32) layers; one of the lowest eight, the product by A^ and the inverse
-//   of the eight; the mirror image back; y.
+//   conversion to the novel basis on the blocks: passes over columns for the
+//   powers of s_16 and s_8, two over tiles for the 16 bits below (bits 16 up: in
+//   the first pass of the transform); for K > 20 a pass of the GF(2^16) layers,
+//   halves of the elements apart; a pass of up to seven GF(2^32) layers; one of
+//   the lowest eight, the product by A^ and the inverse of the eight; the mirror
+//   image back; y.  For K <= 16 the conversion runs on 128 strings of bits, one a
+//   row, transposed there and back (conv_fast.h).
 // Between passes the data is element major: element e is 32 planes x 16 bytes
 // in one run, so that every tile reads and writes whole lines.
 #include <string.h>
+
+#include <type_traits>
 
 #include "conv_fast.h"
 #include "kernels.h"
@@ -152,67 +154,185 @@ __device__ __forceinline__ void fa_chunks(uint32_t* lds) {
   __syncthreads();
 }
 
-// Conversion of the coefficient rows of a half-mode tile between the s_16-adic
-// and the novel basis: row rho (index bits 16 up) is a coefficient of X = s_16,
-// whose subspace polynomials are s_k(X) = X^(2^k) + sum of X^e, e = 2^j for the
-// proper submasks j of k (levels as in conv_bits.h, one row instead of one
-// bit).  Row rho lies in plane rho >> r of element (rho mod 2^r) * C + column,
-// r = KC.  The terms are compile-time constants: with runtime term lists the two
-// passes took 1000 us more at n = 2^24, where this adds 170 and 250 us to theirs.
-constexpr bool fa_is_term(int k, int j) { return j < k && (j & ~k) == 0; }
-constexpr int fa_jmax(int k) {
-  int m = 0;
-  for (int j = 0; j < k; j++)
-    if (fa_is_term(k, j)) m = j;
-  return m;
+// ---- basis conversion in registers ----------------------------------------------------
+// Between the monomial basis and the novel one, every split of the index bits at
+// r = 16, 8, 4, 2, 1 is an expansion in powers of s_r = x^(2^r) + x, followed by
+// the same for the bits above the split (X = s_r) and below it.  s_r^(2^i) has
+// one lower term, so the level of bit b = r + i takes, with half = 2^b and e =
+// 2^i, q = hi with its first e coefficients corrected by its last ones, and
+// lo_j ^= q_{j-e} (backwards the same with the two steps exchanged): 32 such
+// levels for 16 bits, where the novel basis' own levels, bit by bit, have 65
+// lower terms (s_15 alone 15).
+CUOT_DEV void fa_add(uint32_t& a, uint32_t b, uint32_t k) { a ^= b & k; }
+CUOT_DEV void fa_add(uint4& a, uint4 b, uint32_t k) {
+  a.x ^= b.x & k;
+  a.y ^= b.y & k;
+  a.z ^= b.z & k;
+  a.w ^= b.w & k;
 }
-
-template <int KC>
-__device__ __forceinline__ uint4& fa_row(uint32_t* lds, int rho, int c) {
-  return *(uint4*)&lds[fa_slot(((rho & ((1 << KC) - 1)) << (8 - KC)) + c) * FA_ST16 + 4 * (rho >> KC)];
+CUOT_DEV void fa_add(uint2& a, uint2 b, uint32_t k) {
+  a.x ^= b.x & k;
+  a.y ^= b.y & k;
 }
+CUOT_DEV void fa_add(uint32_t& a, uint32_t b) { a ^= b; }
+CUOT_DEV void fa_add(uint2& a, uint2 b) { a = x2(a, b); }
+CUOT_DEV void fa_add(uint4& a, uint4 b) { a = x4(a, b); }
 
-// v ^= rows hb + s + half - e for the terms e = 2^J > s (FIX) or lb-side rows
-// hb + s - e for e <= s
-template <int KC, int K, bool FIX, int J = 0>
-__device__ __forceinline__ void fa_row_terms(uint32_t* lds, uint4& v, int hb, int s, int c) {
-  if constexpr (J < K) {
-    if constexpr (fa_is_term(K, J)) {
-      constexpr int e = 1 << J;
-      if (FIX ? e > s : e <= s) v = x4(v, fa_row<KC>(lds, FIX ? hb + s + (1 << K) - e : hb + s - e, c));
+// The levels of R bits from b0 on stay inside the columns
+//     c + T (2^b0 - u),   T = 0 .. 2^R,   u = 2^(b0-r),   c < 2^b0 - u
+// of a group of 2^(b0+R) coefficients (the last one exists for c < 2^R u): at bit
+// b0 + i element T meets element T + 2^i, whether as q_{j-e} of its lower
+// coefficient, as correction or not at all.  Element T lies in row T of 2^b0
+// coefficients for T <= m = c / u, at the end of row T - 1 above; where m >= 2^R
+// (no EDGE) all levels are plain butterflies and commute.  Where a group has 2^b0
+// rows (b0 = R = 4, u = 1) column 0 has one element more, the group's last.
+template <bool INV, int R, bool EDGE, int FROM = 0, int N, typename V>
+__device__ __forceinline__ void fa_column_levels(V (&v)[N], int m) {
+  if constexpr (!EDGE) {
+#pragma unroll
+    for (int i = 0; i < R; i++)
+#pragma unroll
+      for (int T = FROM; T < (1 << R); T++)
+        if (!(T >> i & 1)) fa_add(v[T], v[T | 1 << i]);
+  } else {
+#pragma unroll
+    for (int s = 0; s < R; s++) {
+      const int i = INV ? s : R - 1 - s, d = 1 << i;
+#pragma unroll
+      for (int ph = 0; ph < 2; ph++) {
+#pragma unroll
+        for (int T = FROM; T + d <= (1 << R); T++) {
+          if ((ph == 0) != INV) {  // a half's first e coefficients
+            if ((T & (2 * d - 1)) == d) fa_add(v[T], v[T + d], T <= m && T + d > m ? ~0u : 0u);
+          } else {
+            const bool lo = !(T & d), lo1 = T > 0 && !((T - 1) & d);  // row T's bit, row T - 1's
+            if (lo || lo1) fa_add(v[T], v[T + d], (T > m ? lo1 : lo && ((T & (d - 1)) || T + d <= m)) ? ~0u : 0u);
+          }
+        }
+        if (N == (1 << R) + 2 && (ph == 0) != INV) fa_add(v[(1 << R) + 1 - d], v[(1 << R) + 1], m == 0 ? ~0u : 0u);
+      }
     }
-    fa_row_terms<KC, K, FIX, J + 1>(lds, v, hb, s, c);
   }
 }
 
-template <int KC, bool INV, int STEP = 1>
-__device__ __forceinline__ void fa_outer(uint32_t* lds) {
-  constexpr int NB = KC + (INV ? 4 : 3);  // row bits; level 0 has no lower terms
-  if constexpr (STEP < NB) {
-    constexpr int K = INV ? STEP : NB - STEP, half = 1 << K, LGC = 8 - KC, C = 1 << LGC, LGE = fa_jmax(K);
+// one level on 2^N coefficients in registers
+template <int N, int B, int E, bool INV, typename V>
+__device__ __forceinline__ void fa_reg_level(V (&v)[1 << N]) {
 #pragma unroll
-    for (int phase = 0; phase < 2; phase++) {
-      if ((phase == 0) != INV) {
-        constexpr int cnt = (1 << (NB - 1 - K)) << (LGE + LGC);  // hi rows i < e_max
-        for (int x = threadIdx.x; x < cnt; x += FA_NT) {
-          const int c = x & (C - 1), i = (x >> LGC) & ((1 << LGE) - 1), hb = ((x >> (LGC + LGE)) * 2 + 1) * half;
-          uint4 v = fa_row<KC>(lds, hb + i, c);
-          fa_row_terms<KC, K, true>(lds, v, hb, i, c);
-          fa_row<KC>(lds, hb + i, c) = v;
-        }
-      } else {
-        constexpr int cnt = 1 << (NB - 1 + LGC);
-#pragma unroll 1
-        for (int x = threadIdx.x; x < cnt; x += FA_NT) {
-          const int c = x & (C - 1), lo = x >> LGC, j = lo & (half - 1), lb = (lo >> K) * 2 * half;
-          uint4 v = fa_row<KC>(lds, lb + j, c);
-          fa_row_terms<KC, K, false>(lds, v, lb + half, j, c);
-          fa_row<KC>(lds, lb + j, c) = v;
+  for (int ph = 0; ph < 2; ph++)
+#pragma unroll
+    for (int g = 0; g < (1 << N); g += 2 << B)
+#pragma unroll
+      for (int j = 0; j < (1 << B); j++) {
+        const int hi = g + (1 << B);
+        if ((ph == 0) != INV) {
+          if (j < E) fa_add(v[hi + j], v[hi + j + (1 << B) - E]);
+        } else {
+          if (j >= E) fa_add(v[g + j], v[hi + j - E]);
         }
       }
-      __syncthreads();
+}
+
+// whole conversion of N <= 4 bits in registers
+template <int N, bool INV, typename V>
+__device__ __forceinline__ void fa_reg_conv(V (&v)[1 << N]) {
+  if constexpr (!INV) {
+    if constexpr (N == 4) fa_reg_level<N, 3, 2, INV>(v);  // powers of s_2
+    if constexpr (N >= 3) fa_reg_level<N, 2, 1, INV>(v);
+    if constexpr (N == 4) fa_reg_level<N, 3, 4, INV>(v);  // bits 2, 3
+    if constexpr (N >= 2) fa_reg_level<N, 1, 1, INV>(v);  // bits 0, 1
+  } else {
+    if constexpr (N >= 2) fa_reg_level<N, 1, 1, INV>(v);
+    if constexpr (N == 4) fa_reg_level<N, 3, 4, INV>(v);
+    if constexpr (N >= 3) fa_reg_level<N, 2, 1, INV>(v);
+    if constexpr (N == 4) fa_reg_level<N, 3, 2, INV>(v);
+  }
+}
+
+// Conversion of 2^(4+H) rows, H <= 4, as three steps on registers between which
+// the rows go through LDS: the powers of s_4 in columns (c < 15), the bits below
+// (16 neighbouring rows) and the bits above (2^H rows 16 apart).
+template <int H, bool INV, typename V, typename L, typename S>
+__device__ __forceinline__ void fa_step_s4(int c, const L& ld, const S& st) {
+  V v[(1 << H) + (H == 4 ? 2 : 1)];
+#pragma unroll
+  for (int T = 0; T < (1 << H); T++) v[T] = ld(c + 15 * T);
+  v[1 << H] = V();
+  if (c < (1 << H)) v[1 << H] = ld(c + (15 << H));
+  if constexpr (H == 4) {
+    v[17] = V();
+    if (c == 0) v[17] = ld(255);
+  }
+  fa_column_levels<INV, H, true>(v, c);
+#pragma unroll
+  for (int T = 0; T < (1 << H); T++) st(c + 15 * T, v[T]);
+  if (c < (1 << H)) st(c + (15 << H), v[1 << H]);
+  if constexpr (H == 4) {
+    if (c == 0) st(255, v[17]);
+  }
+}
+
+template <int N, int STRIDE, bool INV, typename V, typename L, typename S>
+__device__ __forceinline__ void fa_step_conv(int row, const L& ld, const S& st) {
+  V v[1 << N];
+#pragma unroll
+  for (int k = 0; k < (1 << N); k++) v[k] = ld(row + k * STRIDE);
+  fa_reg_conv<N, INV>(v);
+#pragma unroll
+  for (int k = 0; k < (1 << N); k++) st(row + k * STRIDE, v[k]);
+}
+
+// The coefficient rows of a half-mode tile, from powers of s_16 to the novel basis
+// (INV: back): row rho (index bits 16 up, X = s_16) lies in plane rho >> KC of
+// element (rho mod 2^KC) * C + column.  A lane takes one word of a row.  At n = 2^24
+// the two passes take 300 and 445 us; level by level over the whole tile in LDS,
+// with the novel basis' own terms, 365 and 515.
+template <int KC>
+__device__ __forceinline__ uint32_t& fa_row(uint32_t* lds, int rho, int col, int w) {
+  return lds[fa_slot(((rho & ((1 << KC) - 1)) << (FA_TL - KC)) + col) * FA_ST16 + 4 * (rho >> KC) + w];
+}
+
+template <int KC, bool INV>
+__device__ __forceinline__ void fa_outer(uint32_t* lds) {
+  constexpr int NB = KC + (INV ? 4 : 3), H = NB > 8 ? 4 : NB - 4, LGW = FA_TL - KC + 2;  // words of a row: columns x 4
+  const int w = threadIdx.x & 3, col = (threadIdx.x >> 2) & ((1 << (LGW - 2)) - 1);
+  auto halves = [&](auto step, int tasks) {  // tasks per 2^(4+H) rows
+    for (int x = threadIdx.x >> LGW; x < tasks << (NB - 4 - H); x += FA_NT >> LGW) {
+      const int base = NB > 8 ? (x / tasks) << 8 : 0;
+      step(
+          NB > 8 ? x % tasks : x, [&](int r) { return fa_row<KC>(lds, base + r, col, w); },
+          [&](int r, uint32_t v) { fa_row<KC>(lds, base + r, col, w) = v; });
     }
-    fa_outer<KC, INV, STEP + 1>(lds);
+    __syncthreads();
+  };
+  [[maybe_unused]] auto s4 = [&] {
+    halves([](int c, const auto& ld, const auto& st) { if (c < 15) fa_step_s4<H, INV, uint32_t>(c, ld, st); }, 16);
+  };
+  auto s8 = [&] {  // bit 8 of nine: lo_j ^= q_{j-1}
+    if constexpr (NB > 8) {
+      if (!INV) {
+        if ((int)threadIdx.x >> LGW == 0) fa_row<KC>(lds, 256, col, w) ^= fa_row<KC>(lds, 511, col, w);
+        __syncthreads();
+      }
+      for (int x = (threadIdx.x >> LGW) + 1; x < 256; x += FA_NT >> LGW)
+        fa_row<KC>(lds, x, col, w) ^= fa_row<KC>(lds, 255 + x, col, w);
+      __syncthreads();
+      if (INV) {
+        if ((int)threadIdx.x >> LGW == 0) fa_row<KC>(lds, 256, col, w) ^= fa_row<KC>(lds, 511, col, w);
+        __syncthreads();
+      }
+    }
+  };
+  if constexpr (!INV) {
+    s8();
+    if constexpr (H > 0) s4();
+  }
+  halves([](int r, const auto& ld, const auto& st) { fa_step_conv<4, 1, INV, uint32_t>(16 * r, ld, st); }, 1 << H);
+  if constexpr (H > 1)
+    halves([](int r, const auto& ld, const auto& st) { fa_step_conv<H, 16, INV, uint32_t>(r, ld, st); }, 16);
+  if constexpr (INV) {
+    if constexpr (H > 0) s4();
+    s8();
   }
 }
 
@@ -270,7 +390,7 @@ __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void
     }
     __syncthreads();
     if constexpr (!INV) {
-      if constexpr (KC > 1) fa_outer<KC, false>(lds);
+      fa_outer<KC, false>(lds);
       fa_chunks<KC, false>(lds);
     }
     // one loop, so that the layer's code is there once
@@ -278,7 +398,7 @@ __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void
     for (int step = 0; step < KC; step++) fa_layer16<KC, INV>(a, lds, ctab, INV ? step : KC - 1 - step);
     if constexpr (INV) {
       fa_chunks<KC, true>(lds);
-      if constexpr (KC > 1) fa_outer<KC, true>(lds);
+      fa_outer<KC, true>(lds);
     }
     uint4 w[8];
     tid = opaque_tid();
@@ -450,6 +570,9 @@ __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void
           uint32_t t[8];
 #pragma unroll
           for (int q = 0; q < 8; q++) t[q] = lds[P * FA_ST + h * 64 + q * 4 + w];
+          // planes of index bits 16 up: from powers of s_16 to the novel basis
+          if (a.K == 20) fa_reg_conv<3, false>(t);
+          if (a.K == 19) fa_reg_level<3, 2, 2, false>(t);
           fa_pack_planes<0>(t, x + 16 * h);
         }
       } else {
@@ -536,6 +659,12 @@ __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void
         for (int h = 0; h < 2; h++) {
           uint32_t t[16];
           fa_unpack_planes<0>(x + 16 * h, t);
+          if (a.K == 20) fa_reg_conv<4, true>(t);
+          if (a.K == 19) {
+            fa_reg_level<4, 2, 2, true>(t);
+            fa_reg_level<4, 3, 2, true>(t);
+          }
+          if (a.K == 18) fa_reg_level<4, 3, 4, true>(t);
 #pragma unroll
           for (int q = 0; q < 16; q++) lds[P * FA_ST + h * 64 + q * 4 + w] = t[q];
         }
@@ -566,20 +695,14 @@ __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void
   }
 }
 
-// ---- s_16-adic levels on blocks (K > 21) ------------------------------------------
-// Expansion of a polynomial in powers of s_16 = x^65536 + x: s_16^(2^i) has one
-// lower term, so the level of index bit b = 16 + i takes, with half = 2^b and
-// e = 2^i, q = hi with its first e coefficients corrected by its last ones, and
-// lo_j ^= q_{j-e} (backwards the same with the two steps exchanged).  Away from
-// the first coefficients of a half all levels are their own inverses, commute
-// and move coefficient j of a row 2^b further to j + e of this one, so R of them
-// are one pass over skewed columns (below), bound by memory: 2^24 coefficients
-// 16 bytes wide in 102 us (5.26 TB/s).  At n = 2^24 the forward levels take 207
-// us and the backward ones with the output 490.  The novel basis' own levels
-// (s_23 has 15 lower terms) one pass each took 934 and 1510 with the same
-// output, the s_16-adic ones as a gather of (3/2)^R reads per output 310 and 1000.
-// At K = 21 a single level of three terms is left, done in the output: 388 us an
-// encode of n = 2^20 against 413 this way.
+// ---- s_16- and s_8-adic levels on blocks (K > 16) ------------------------------------
+// All R levels of a call are one pass, each coefficient read and written once and
+// memory the bound: 2^24 blocks in 100 us (5.4 TB/s).  The novel basis' own levels
+// from bit 20 up, one pass each, took 934 us forward and 1510 back with the output
+// at n = 2^24; the powers of s_16 take 200 and 490, and in bit strings, as the
+// bits below then were, the conversion cost 50 us each way at n = 2^20 beside the
+// transposes (76 us of an encode before the transform, now 44, and 107 behind it,
+// now 64).
 // The source: an instance's natural-order buffer, or x_{n+i}, zero from n on.
 struct FaSrc {
   const uint4* p;
@@ -587,63 +710,23 @@ struct FaSrc {
   __device__ __forceinline__ uint4 operator[](int64_t i) const { return i < n ? p[i] : make_uint4(0, 0, 0, 0); }
 };
 
-// exact value of index I after the levels of bits b0 .. b (backwards) or
-// b .. b0 + R - 1 (forwards); only near the start of a half
-template <bool INV, int L>
-__device__ __attribute__((noinline)) uint4 fa_s16_slow(const FaSrc& in, int64_t I, int b0, int R) {
-  if constexpr (L == 0) {
-    return in[I];
-  } else {
-    const int b = INV ? b0 + L - 1 : b0 + R - L;
-    const int64_t half = (int64_t)1 << b, e = half >> 16;
-    const int64_t pos = I & (2 * half - 1), hi = I - pos + half;
-    uint4 v = fa_s16_slow<INV, L - 1>(in, I, b0, R);
-    if (pos < half) {
-      if (pos >= e) {
-        const int64_t s = pos - e;
-        v = x4(v, fa_s16_slow<INV, L - 1>(in, hi + s, b0, R));
-        if (!INV && s < e) v = x4(v, fa_s16_slow<INV, L - 1>(in, hi + s + half - e, b0, R));
-      }
-    } else if (pos - half < e) {
-      v = x4(v, fa_s16_slow<INV, L - 1>(in, I + half - e, b0, R));
-    }
-    return v;
-  }
+// elements FROM .. 2^R of column c of the group at base (the last one, beyond
+// the group for most columns, only with EDGE)
+template <int R, bool EDGE, int FROM = 0, typename SRC, typename V>
+__device__ __forceinline__ void fa_column_load(const SRC& in, int64_t base, int64_t c, int64_t ncol, int64_t group,
+                                               V (&v)[(1 << R) + 1]) {
+#pragma unroll
+  for (int T = FROM; T < (1 << R); T++) v[T] = in[base + c + T * ncol];
+  v[1 << R] = V();
+  if (EDGE && c + (ncol << R) < group) v[1 << R] = in[base + c + (ncol << R)];
 }
 
-// the first 2 * (sum of the shifts) coefficients above bit b0 take the exact form
-constexpr int64_t fa_s16_edge(int R, int b0) { return (int64_t)2 << (R + b0 - 16); }
-
-// Skewed column c of the 2^R rows of 2^b0 coefficients at base: coefficient
-// c - T 2^(b0-16) of row T.  The levels stay inside a column, where they are a
-// butterfly of R stages, so every coefficient is read and written once.  Rows
-// whose coefficient lies below the exact ones or past the row are not valid
-// (and no valid one takes them in).  Rows below FROM are left out.
-template <int R, int FROM = 0>
-__device__ __forceinline__ void fa_s16_column(const FaSrc& in, int64_t base, int64_t c, int b0, uint4 (&v)[1 << R]) {
-#pragma unroll
-  for (int T = FROM; T < (1 << R); T++) {
-    const int64_t j = c - ((int64_t)T << (b0 - 16));
-    v[T] = j >= 0 && j < ((int64_t)1 << b0) ? in[base + ((int64_t)T << b0) + j] : make_uint4(0, 0, 0, 0);
-  }
-#pragma unroll
-  for (int b = 0; b < R; b++)
-#pragma unroll
-    for (int T = FROM; T < (1 << R); T++)
-      if (!(T >> b & 1)) v[T] = x4(v[T], v[T | 1 << b]);
-}
-
-// columns from the first valid coefficient of row 0 to the last one of row 2^R - 1
-constexpr int64_t fa_s16_columns(int R, int b0) {
-  return ((int64_t)1 << b0) - fa_s16_edge(R, b0) + ((((int64_t)1 << R) - 1) << (b0 - 16));
-}
-
-// Bits B0 .. B0 + R - 1 of N coefficients, a column per lane.  The rows' first
-// coefficients, whose exact form is a long chain of dependent reads, go to
-// workgroups of their own, one per lane.
-template <bool INV, bool SRC, int R, int B0>
-__global__ __launch_bounds__(256) void fa_s16_level(const QcIo* __restrict__ io, QcIo io1, const uint4* __restrict__ in,
-                                                    uint4* __restrict__ out, int64_t XS, int64_t N) {
+// Bits B0 .. B0 + R - 1 of N coefficients, a column per lane.
+template <bool INV, bool SRC, int S, int R, int B0>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void fa_adic_level(const QcIo* __restrict__ io, QcIo io1, const uint4* __restrict__ in,
+                                                     uint4* __restrict__ out, int64_t XS, int64_t N) {
+  constexpr int64_t U = (int64_t)1 << (B0 - S), NCOL = ((int64_t)1 << B0) - U, GROUP = (int64_t)1 << (B0 + R);
+  constexpr int64_t per = (NCOL + 255) / 256;  // workgroups per group
   FaSrc src;
   if (SRC) {
     const QcIo q = io ? io[blockIdx.y] : io1;
@@ -654,43 +737,31 @@ __global__ __launch_bounds__(256) void fa_s16_level(const QcIo* __restrict__ io,
     src.n = N;
   }
   uint4* dst = out + (int64_t)blockIdx.y * XS;
-  const int tid = threadIdx.x;
-  constexpr int64_t EDGE = fa_s16_edge(R, B0);
-  const int64_t edges = (N >> B0) * EDGE, nedge = (edges + 255) / 256;
-  if ((int64_t)blockIdx.x < nedge) {
-    const int64_t x = (int64_t)blockIdx.x * 256 + tid;
-    if (x >= edges) return;
-    const int64_t i = ((x / EDGE) << B0) | (x & (EDGE - 1));
-    dst[i] = fa_s16_slow<INV, R>(src, i, B0, R);
-    return;
+  const int64_t c0 = (int64_t)(blockIdx.x % per) * 256, c = c0 + threadIdx.x;
+  const int64_t base = (int64_t)(blockIdx.x / per) << (B0 + R);
+  if (c >= NCOL) return;
+  uint4 v[(1 << R) + 1];
+  if (c0 < U << R) {
+    fa_column_load<R, true>(src, base, c, NCOL, GROUP, v);
+    fa_column_levels<INV, R, true>(v, (int)(c / U));
+    if (c < U << R) dst[base + c + (NCOL << R)] = v[1 << R];
+  } else {
+    fa_column_load<R, false>(src, base, c, NCOL, GROUP, v);
+    fa_column_levels<INV, R, false>(v, 0);
   }
-  constexpr int64_t per = (fa_s16_columns(R, B0) + 255) / 256;  // workgroups per 2^R rows
-  const int64_t tile = (int64_t)blockIdx.x - nedge;
-  const int64_t c = EDGE + (tile % per) * 256 + tid, base = (tile / per) << (B0 + R);
-  uint4 v[1 << R];
-  fa_s16_column<R>(src, base, c, B0, v);
 #pragma unroll
-  for (int T = 0; T < (1 << R); T++) {
-    const int64_t j = c - ((int64_t)T << (B0 - 16));
-    if (j >= EDGE && j < ((int64_t)1 << B0)) dst[base + ((int64_t)T << B0) + j] = v[T];
-  }
+  for (int T = 0; T < (1 << R); T++) dst[base + c + T * NCOL] = v[T];
 }
 
-// ---- input: blocks to 128 bit-row strings of S = 2^mp bits ---------------------------
-// SRC: from x_{n+i}
-template <bool SRC>
-__global__ __launch_bounds__(256) void fa_rows_in(const QcIo* __restrict__ io, QcIo io1, const uint4* __restrict__ in,
-                                                  int64_t XS, int64_t N, int mp, uint32_t* __restrict__ rows) {
+// ---- input: blocks x_{n+i} to 128 bit-row strings of N = 2^mp bits ---------------------
+__global__ __launch_bounds__(256) void fa_rows_in(const QcIo* __restrict__ io, QcIo io1, int64_t XS, int mp,
+                                                  uint32_t* __restrict__ rows) {
   __shared__ uint32_t sm[128][33];
+  const QcIo q = io ? io[blockIdx.y] : io1;
   FaSrc src;
-  if (SRC) {
-    const QcIo q = io ? io[blockIdx.y] : io1;
-    src.p = q.x + q.n;
-    src.n = q.n;
-  } else {
-    src.p = in + (int64_t)blockIdx.y * XS;
-    src.n = N;
-  }
+  src.p = q.x + q.n;
+  src.n = q.n;
+  const int64_t N = (int64_t)1 << mp;
   rows += (int64_t)blockIdx.y * XS * 4;
   const int lane = threadIdx.x & 31;
   const int grp = threadIdx.x >> 5;
@@ -708,8 +779,7 @@ __global__ __launch_bounds__(256) void fa_rows_in(const QcIo* __restrict__ io, Q
       sm[3 * 32 + lane][tl] = cuot_transpose32(v.w, lane);
     }
     __syncthreads();
-    const int64_t str = (tile << 10) >> mp, w0 = ((tile << 10) & (((int64_t)1 << mp) - 1)) >> 5;
-    uint32_t* dst = rows + str * 128 * rw + w0;
+    uint32_t* dst = rows + (tile << 5);
     for (int f = threadIdx.x; f < 128 * 8; f += 256) {
       const int k = f >> 3, tl = (f & 7) * 4;
       *(uint4*)&dst[(int64_t)k * rw + tl] = make_uint4(sm[k][tl], sm[k][tl + 1], sm[k][tl + 2], sm[k][tl + 3]);
@@ -719,74 +789,158 @@ __global__ __launch_bounds__(256) void fa_rows_in(const QcIo* __restrict__ io, Q
 }
 
 // ---- output -------------------------------------------------------------------------
-// y_i = x_i ^ H_i ^ H_{i+n}, H the product's coefficients.  TOP (K = 21): its two
-// halves go through the last level on the way, s_20 = x^(2^20) + x^65536 + x^16 + x.
-template <bool TOP>
+// y_i = x_i ^ H_i ^ H_{i+n}, H the product's coefficients
 __global__ __launch_bounds__(256) void fa_output(const uint4* __restrict__ H, int64_t XS, const QcIo* __restrict__ io,
                                                  QcIo io1) {
   const QcIo q = io ? io[blockIdx.y] : io1;
   H += (int64_t)blockIdx.y * XS;
-  auto h_at = [&](int64_t i) {
-    uint4 v = H[i];
-    if constexpr (TOP) {
-      constexpr int64_t half = (int64_t)1 << 20;
-#pragma unroll
-      for (int e = 1; e <= 65536; e = e == 1 ? 16 : e * 4096) {
-        if (i < half ? i >= e : i - half < e) v = x4(v, H[i < half ? half + i - e : i + half - e]);
-      }
-    }
-    return v;
-  };
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < q.n; i += (int64_t)gridDim.x * 256)
-    q.y[i] = x4(q.x[i], x4(h_at(i), h_at(i + q.n)));
+    q.y[i] = x4(q.x[i], x4(H[i], H[i + q.n]));
 }
 
-// The same through the last levels, bits 20 .. K-1 (R of them).  With n = m 2^20
-// + r, the coefficients i + n of one skewed column's i are again one column, r +
-// 16 m further, m rows up, or one row more and 2^20 back where j + r passes the
-// row's end.  That column goes through LDS, as m is no constant.  i or i + n at
-// a row's start: lanes of their own, 2 EDGE per row of y.
+// The same through the last levels, bits B0 .. K-1 (R of them, B0 = 16 or 20).  The
+// coefficients i + n of a column's i are a column again: with n = Q (2^B0 - u) + r,
+// the one r further, Q elements up (or past the last column around to the first, one more
+// up).  It goes through LDS, as Q is no constant.
+// A lane takes a block or, with 33 of them to a column, half of one (at n =
+// 2^20 19 us, with whole ones, at 190 registers, 40).
 constexpr int FA_OT = 128;
 
 template <int R>
-__global__ __launch_bounds__(FA_OT) void fa_output_s16(const uint4* __restrict__ H, int64_t XS,
-                                                       const QcIo* __restrict__ io, QcIo io1) {
-  constexpr int B0 = 20, LOW = 1 << (R - 2);  // n > 2^(K-2)
-  constexpr int64_t EDGE = fa_s16_edge(R, B0), ROW = (int64_t)1 << B0;
-  __shared__ uint4 second[((1 << R) - LOW) * FA_OT];
-  const QcIo q = io ? io[blockIdx.y] : io1;
-  FaSrc src;
-  src.p = H + (int64_t)blockIdx.y * XS;
-  src.n = XS;
-  const int64_t m = q.n >> B0, r = q.n & (ROW - 1), rows = (q.n + ROW - 1) >> B0;
-  const int64_t nedge = rows * 2 * EDGE / FA_OT;
-  if ((int64_t)blockIdx.x < nedge) {
-    const int64_t x = (int64_t)blockIdx.x * FA_OT + threadIdx.x, k = x & (EDGE - 1);
-    const int64_t j = x & EDGE ? (k - r) & (ROW - 1) : k, i = (x / (2 * EDGE)) << B0 | j;
-    if (i >= q.n || ((x & EDGE) && j < EDGE)) return;
-    uint4 v = q.x[i];
-#pragma unroll 1
-    for (int s = 0; s < 2; s++) v = x4(v, fa_s16_slow<true, R>(src, s ? i + q.n : i, B0, R));
-    q.y[i] = v;
-    return;
-  }
-  const int64_t c = EDGE + ((int64_t)blockIdx.x - nedge) * FA_OT + threadIdx.x;
-  if (c - 16 * (rows - 1) >= ROW) return;
-  const bool carry = c - 16 * (rows - 1) + r >= ROW;
-  const int up = (int)m + (carry ? 1 : 0);
-  {
-    uint4 v[1 << R];
-    fa_s16_column<R, LOW>(src, 0, c + r + 16 * m + (carry ? 16 - ROW : 0), B0, v);
+struct FaOut {
+  static constexpr int PARTS = R > 4 ? 2 : 1;
+  using V = std::conditional_t<PARTS == 2, uint2, uint4>;
+  const V* p;
+  __device__ __forceinline__ V operator[](int64_t i) const { return p[i * PARTS]; }
+};
+
+template <int R, int B0, bool EDGE, typename V = typename FaOut<R>::V>
+__device__ __forceinline__ void fa_output_column(const FaOut<R>& H, const FaOut<R>& x, V* y, int64_t n, int64_t c,
+                                                 int64_t c2, int up, V* second) {
+  constexpr int LOW = R > 1 ? 1 << (R - 2) : 0, LU = B0 - 16;  // Q >= LOW: n > 2^(K-2)
+  constexpr int64_t NCOL = ((int64_t)1 << B0) - (1 << LU), GROUP = (int64_t)1 << (B0 + R);
+  V v[(1 << R) + 1];
+  fa_column_load<R, EDGE, LOW>(H, 0, c2, NCOL, GROUP, v);
+  fa_column_levels<true, R, EDGE, LOW>(v, (int)(c2 >> LU));
 #pragma unroll
-    for (int T = LOW; T < (1 << R); T++) second[(T - LOW) * FA_OT + threadIdx.x] = v[T];
-  }
-  uint4 v[1 << R];
-  fa_s16_column<R>(src, 0, c, B0, v);
+  for (int T = LOW; T <= (1 << R); T++)
+    if (T >= up && T - up <= (1 << (R - 1))) second[(T - up) * FA_OT + threadIdx.x] = v[T];
+  fa_column_load<R, EDGE>(H, 0, c, NCOL, GROUP, v);
+  fa_column_levels<true, R, EDGE>(v, (int)(c >> LU));
 #pragma unroll
   for (int T = 0; T <= (1 << (R - 1)); T++) {
-    const int64_t j = c - 16 * T, i = (int64_t)T << B0 | j;
-    if (T < rows && j >= EDGE && j < ROW && ((j + r) & (ROW - 1)) >= EDGE && i < q.n)
-      q.y[i] = x4(q.x[i], x4(v[T], second[(T + up - LOW) * FA_OT + threadIdx.x]));
+    const int64_t i = c + T * NCOL;
+    if (i < n) {
+      V o = x[i];
+      fa_add(o, v[T]);
+      fa_add(o, second[T * FA_OT + threadIdx.x]);
+      y[i * FaOut<R>::PARTS] = o;
+    }
+  }
+}
+
+template <int R, int B0>
+__global__ __launch_bounds__(FA_OT) __attribute__((amdgpu_waves_per_eu(2))) void fa_output_adic(
+    const uint4* __restrict__ H, int64_t XS, const QcIo* __restrict__ io, QcIo io1) {
+  using V = typename FaOut<R>::V;
+  constexpr int64_t U = (int64_t)1 << (B0 - 16), NCOL = ((int64_t)1 << B0) - U, ECOL = U << R;
+  constexpr int PARTS = FaOut<R>::PARTS, COLS = FA_OT / PARTS;
+  __shared__ V second[((1 << (R - 1)) + 1) * FA_OT];
+  const QcIo q = io ? io[blockIdx.y] : io1;
+  const int part = threadIdx.x % PARTS;
+  FaOut<R> h, x;
+  h.p = (const V*)(H + (int64_t)blockIdx.y * XS) + part;
+  x.p = (const V*)q.x + part;
+  V* y = (V*)q.y + part;
+  const int64_t c0 = (int64_t)blockIdx.x * COLS, c = c0 + threadIdx.x / PARTS, r = q.n % NCOL;
+  if (c >= NCOL) return;
+  const bool wrap = c + r >= NCOL;
+  const int up = (int)(q.n / NCOL) + (wrap ? 1 : 0);
+  const int64_t d0 = c0 + r >= NCOL ? c0 + r - NCOL : c0 + r;  // first lane's second column
+  const int64_t c2 = c + r - (wrap ? NCOL : 0);
+  if (c0 < ECOL || d0 < ECOL || d0 + COLS > NCOL)
+    fa_output_column<R, B0, true>(h, x, y, q.n, c, c2, up, second);
+  else
+    fa_output_column<R, B0, false>(h, x, y, q.n, c, c2, up, second);
+}
+
+// ---- conversion of 2^16 coefficients on blocks (K > 16) --------------------------------
+// A workgroup of 256 lanes converts 2^12 blocks, 16 or 17 per lane and step, the
+// steps exchanging through LDS.  ROWS: the outer bits 8 .. 15, 256 rows 256 apart
+// times 16 consecutive columns; else 4096 consecutive blocks, the s_8-adic levels
+// of bits 8 .. 11 (those of 12 .. 15: fa_adic_level) and the bits below 8.
+// Memory is the bound: 2^24 blocks in 108 us and, ROWS, 88.  As strings of bits, transposed there and back, the
+// 16 bits took 531 us for 2^24 coefficients and 971 back for 2^25, level by level
+// on blocks in LDS (tiles of 512 lanes, two barriers a level) 387 and 677 with bits
+// 12 .. 15.
+constexpr int FA_CT = 256;
+
+template <bool INV, bool ROWS>
+__global__ __launch_bounds__(FA_CT) __attribute__((amdgpu_waves_per_eu(2))) void fa_conv_tile(const uint4* in, uint4* out,
+                                                                                              int64_t XS) {
+  extern __shared__ uint4 sm[];
+  const int tid = threadIdx.x, x = tid & 15, y = tid >> 4;
+  const int64_t tile = blockIdx.x;
+  const int64_t g0 = (int64_t)blockIdx.y * XS + (ROWS ? ((tile >> 4) << 16) + ((tile & 15) << 4) : tile << 12);
+  // row r of column (or block of 256) cl, in memory and in LDS (padded: 16 lanes
+  // 256 bytes apart otherwise meet in the same banks)
+  auto mem = [&](int cl, int r) { return g0 + (ROWS ? (r << 8) + cl : (cl << 8) + r); };
+  auto slot = [&](int cl, int r) -> uint4& {
+    const int i = ROWS ? (r << 4) + cl : (cl << 8) + r;
+    return sm[i + (i >> 4)];
+  };
+  // lanes of a step: the faster index where neighbours are contiguous
+  const int xc = ROWS ? x : y, xr = ROWS ? y : x;
+  auto lds_ld = [&](int r) { return slot(xc, r); };
+  auto lds_st = [&](int r, uint4 v) { slot(xc, r) = v; };
+  auto mem_ld = [&](int r) { return in[mem(xc, r)]; };
+  auto mem_st = [&](int r, uint4 v) { out[mem(xc, r)] = v; };
+  // 16 neighbouring rows per lane
+  auto low = [&] {
+    fa_step_conv<4, 1, INV, uint4>(16 * xr, lds_ld, lds_st);
+    __syncthreads();
+  };
+  // the s_8-adic levels of 16 blocks of 256
+  auto s8 = [&](const auto& ld, const auto& st) {
+    if (tid < 255) {
+      uint4 v[17];
+#pragma unroll
+      for (int T = 0; T < 16; T++) v[T] = ld(tid + 255 * T);
+      v[16] = z4();
+      if (tid < 16) v[16] = ld(tid + 255 * 16);
+      if (tid < 64)
+        fa_column_levels<INV, 4, true>(v, tid);
+      else
+        fa_column_levels<INV, 4, false>(v, 0);
+#pragma unroll
+      for (int T = 0; T < 16; T++) st(tid + 255 * T, v[T]);
+      if (tid < 16) st(tid + 255 * 16, v[16]);
+    }
+  };
+  auto lin_ld = [&](int i) { return sm[i + (i >> 4)]; };
+  auto lin_st = [&](int i, uint4 v) { sm[i + (i >> 4)] = v; };
+  if constexpr (!INV) {
+    if constexpr (ROWS) {
+      if (xr < 15) fa_step_s4<4, INV, uint4>(xr, mem_ld, lds_st);
+    } else {
+      s8([&](int i) { return in[g0 + i]; }, lin_st);
+      __syncthreads();
+      if (xr < 15) fa_step_s4<4, INV, uint4>(xr, lds_ld, lds_st);
+    }
+    __syncthreads();
+    low();
+    fa_step_conv<4, 16, INV, uint4>(xr, lds_ld, mem_st);
+  } else {
+    fa_step_conv<4, 16, INV, uint4>(xr, mem_ld, lds_st);
+    __syncthreads();
+    low();
+    if constexpr (ROWS) {
+      if (xr < 15) fa_step_s4<4, INV, uint4>(xr, lds_ld, mem_st);
+    } else {
+      if (xr < 15) fa_step_s4<4, INV, uint4>(xr, lds_ld, lds_st);
+      __syncthreads();
+      s8(lin_ld, [&](int i, uint4 v) { out[g0 + i] = v; });
+    }
   }
 }
 
@@ -961,6 +1115,14 @@ int g_fa_ready = 0;
 
 constexpr size_t FA_LDS16 = 256 * FA_ST16 * 4 + FA_CTAB * sizeof(uint2);
 
+constexpr size_t FA_LDSC = (4096 + 256) * 16;
+
+template <bool INV, bool ROWS>
+hipError_t fa_allow_ldsc() {
+  return hipFuncSetAttribute((const void*)fa_conv_tile<INV, ROWS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)FA_LDSC);
+}
+
 template <int KC>
 hipError_t fa_allow_lds16() {
   hipError_t e = hipFuncSetAttribute((const void*)fa_pass16<KC, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -996,6 +1158,10 @@ hipError_t fa_configure() {
   if (!e) e = fa_allow_lds32<FA_FUSED, false>();
   if (!e) e = fa_allow_lds32<FA_INV, false>();
   if (!e) e = fa_allow_lds32<FA_INV, true>();
+  if (!e) e = fa_allow_ldsc<false, false>();
+  if (!e) e = fa_allow_ldsc<false, true>();
+  if (!e) e = fa_allow_ldsc<true, false>();
+  if (!e) e = fa_allow_ldsc<true, true>();
   if (!e) e = fa_allow_lds16<1>();
   if (!e) e = fa_allow_lds16<2>();
   if (!e) e = fa_allow_lds16<3>();
@@ -1016,14 +1182,21 @@ int fa_log(int64_t n) {  // K: 2^(K-1) >= n
 
 unsigned capg(int64_t v, int64_t cap) { return (unsigned)(v < 1 ? 1 : (v > cap ? cap : v)); }
 
-template <bool INV, bool SRC, int R, int B0>
+template <bool INV, bool SRC, int S, int R, int B0>
 void fa_launch_level(const QcIo* io, QcIo io1, const uint4* in, uint4* out, int64_t XS, int64_t N, int B,
                      hipStream_t st) {
-  const int64_t wgs =
-      ((N >> B0) * fa_s16_edge(R, B0) + 255) / 256 + (N >> (B0 + R)) * ((fa_s16_columns(R, B0) + 255) / 256);
-  cuot_rec_begin(st, "fa_s16_level", 32.0 * (double)N * B);
-  hipLaunchKernelGGL((fa_s16_level<INV, SRC, R, B0>), dim3((unsigned)wgs, (unsigned)B), dim3(256), 0, st, io, io1, in,
+  const int64_t wgs = (N >> (B0 + R)) * ((((int64_t)1 << B0) - ((int64_t)1 << (B0 - S)) + 255) / 256);
+  cuot_rec_begin(st, "fa_adic_level", 32.0 * (double)N * B);
+  hipLaunchKernelGGL((fa_adic_level<INV, SRC, S, R, B0>), dim3((unsigned)wgs, (unsigned)B), dim3(256), 0, st, io, io1, in,
                      out, XS, N);
+  cuot_rec_end(st);
+}
+
+template <bool INV, bool ROWS>
+void fa_launch_conv(const uint4* in, uint4* out, int64_t XS, int64_t N, int B, hipStream_t st) {
+  cuot_rec_begin(st, "fa_conv_tile", 32.0 * (double)N * B);
+  hipLaunchKernelGGL((fa_conv_tile<INV, ROWS>), dim3((unsigned)(N >> 12), (unsigned)B), dim3(FA_CT), FA_LDSC, st, in, out,
+                     XS);
   cuot_rec_end(st);
 }
 
@@ -1149,32 +1322,46 @@ hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ah
   uint4* X = (uint4*)scratch;
   uint4* Y = X + (int64_t)B * XS;
   const int64_t Nin = XS >> 1;
-  // forward conversion; the natural-order coefficients end up in X: row strings
-  // of the whole length, or for K > 21 of 2^16 coefficients under s_16-adic
-  // levels (the first pass converts the rows of those)
-  const bool adic = K > 21;
-  {
-    const int mp = adic ? 16 : K - 1;
-    if (adic) {
-      switch (K - 21) {
-        case 1: fa_launch_level<false, true, 1, 20>(io, io1, X, Y, XS, Nin, B, st); break;
-        case 2: fa_launch_level<false, true, 2, 20>(io, io1, X, Y, XS, Nin, B, st); break;
-        case 3: fa_launch_level<false, true, 3, 20>(io, io1, X, Y, XS, Nin, B, st); break;
-        default: fa_launch_level<false, true, 4, 20>(io, io1, X, Y, XS, Nin, B, st); break;
-      }
-      fa_launch_level<false, false, 4, 16>(io, io1, Y, X, XS, Nin, B, st);
+  // forward conversion; the natural-order coefficients end up in X: for K <= 16
+  // row strings, above levels of powers of s_16 and, for the 2^16 coefficients
+  // of those, the rest on blocks (the first pass converts index bits 16 up)
+  const bool adic = K > 16;
+  if (adic) {
+    switch (K - 17) {
+#define FA_CASE(R)                                                                        \
+  case R:                                                                                 \
+    fa_launch_level<false, true, 16, R, 16>(io, io1, nullptr, X, XS, Nin, B, st);        \
+    break;
+#define FA_CASE2(R)                                                                       \
+  case 4 + R:                                                                             \
+    fa_launch_level<false, true, 16, R, 20>(io, io1, nullptr, Y, XS, Nin, B, st);        \
+    fa_launch_level<false, false, 16, 4, 16>(io, io1, Y, X, XS, Nin, B, st);             \
+    break;
+      FA_CASE(1)
+      FA_CASE(2)
+      FA_CASE(3)
+      FA_CASE(4)
+      FA_CASE(5)
+      FA_CASE2(2)
+      FA_CASE2(3)
+      FA_CASE2(4)
+#undef FA_CASE
+#undef FA_CASE2
     }
-    cuot_rec_begin(st, "fa_rows_in", 32.0 * (double)Nin * B);
-    const dim3 rgrid(capg(Nin >> 10, 8192), (unsigned)B);
-    if (!adic)
-      hipLaunchKernelGGL(fa_rows_in<true>, rgrid, dim3(256), 0, st, io, io1, X, XS, Nin, mp, (uint32_t*)Y);
+    if (K == 17)
+      fa_launch_level<false, true, 8, 4, 12>(io, io1, nullptr, Y, XS, Nin, B, st);
     else
-      hipLaunchKernelGGL(fa_rows_in<false>, rgrid, dim3(256), 0, st, io, io1, X, XS, Nin, mp, (uint32_t*)Y);
+      fa_launch_level<false, false, 8, 4, 12>(io, io1, X, Y, XS, Nin, B, st);
+    fa_launch_conv<false, false>(Y, X, XS, Nin, B, st);
+    fa_launch_conv<false, true>(X, X, XS, Nin, B, st);
+  } else {
+    const int64_t S = Nin, words = S / 32;
+    cuot_rec_begin(st, "fa_rows_in", 32.0 * (double)Nin * B);
+    hipLaunchKernelGGL(fa_rows_in, dim3(capg(Nin >> 10, 8192), (unsigned)B), dim3(256), 0, st, io, io1, XS, K - 1,
+                       (uint32_t*)Y);
     cuot_rec_end(st);
-    const int64_t S = (int64_t)1 << mp, words = S / 32;
-    const int P = (int)(Nin >> mp);
-    if ((e = cuot_launch_conv_rows(4096, st, (uint32_t*)Y, words, 128ll * P * B, 128ll * P, XS * 4, mp, 0))) return e;
-    if ((e = cuot_launch_transpose_planes2(Y, S, X, true, B * P, P, XS * 4, 128 * words, XS, S, st))) return e;
+    if ((e = cuot_launch_conv_rows(4096, st, (uint32_t*)Y, words, 128ll * B, 128, XS * 4, K - 1, 0))) return e;
+    if ((e = cuot_launch_transpose_planes2(Y, S, X, true, B, 1, XS * 4, 128 * words, XS, S, st))) return e;
   }
   FaArgs a;
   memset(&a, 0, sizeof(a));
@@ -1189,35 +1376,36 @@ hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ah
   a.a = 16 + a.c;
   if ((e = fa_transform(a, B, st, ready))) return e;
   // inverse conversion of the 2^K coefficients in X
-  const int mp = adic ? 16 : (K < 20 ? K : 20);
-  const int64_t S = (int64_t)1 << mp, words = S / 32;
-  const int P = 1 << (K - mp);
-  if ((e = cuot_launch_transpose_planes2(X, S, Y, false, B * P, P, XS, S, XS * 4, 128 * words, st))) return e;
-  if ((e = cuot_launch_conv_rows(8192, st, (uint32_t*)Y, words, 128ll * P * B, 128ll * P, XS * 4, mp, 1))) return e;
-  if ((e = cuot_launch_transpose_planes2(Y, S, X, true, B * P, P, XS * 4, 128 * words, XS, S, st))) return e;
-  if (adic) fa_launch_level<true, false, 4, 16>(io, io1, X, Y, XS, XS, B, st);
+  if (adic) {
+    fa_launch_conv<true, true>(X, X, XS, XS, B, st);
+    fa_launch_conv<true, false>(X, Y, XS, XS, B, st);
+    fa_launch_level<true, false, 8, 4, 12>(io, io1, Y, X, XS, XS, B, st);
+    if (K > 21) fa_launch_level<true, false, 16, 4, 16>(io, io1, X, Y, XS, XS, B, st);
+  } else {
+    const int64_t words = XS / 32;
+    if ((e = cuot_launch_transpose_planes2(X, XS, Y, false, B, 1, XS, XS, XS * 4, 128 * words, st))) return e;
+    if ((e = cuot_launch_conv_rows(8192, st, (uint32_t*)Y, words, 128ll * B, 128, XS * 4, K, 1))) return e;
+    if ((e = cuot_launch_transpose_planes2(Y, XS, X, true, B, 1, XS * 4, 128 * words, XS, XS, st))) return e;
+  }
   cuot_rec_begin(st, "fa_output", 48.0 * (double)nmax * B);
-  switch (K <= 20 ? 0 : K - 20) {
-    case 0:
-      hipLaunchKernelGGL(fa_output<false>, dim3(capg((nmax + 255) / 256, 16384), (unsigned)B), dim3(256), 0, st, X, XS,
-                         io, io1);
+  switch (K - 16) {
+    default:
+      hipLaunchKernelGGL(fa_output, dim3(capg((nmax + 255) / 256, 16384), (unsigned)B), dim3(256), 0, st, X, XS, io, io1);
       break;
-    case 1:
-      hipLaunchKernelGGL(fa_output<true>, dim3(capg((nmax + 255) / 256, 16384), (unsigned)B), dim3(256), 0, st, X, XS,
-                         io, io1);
-      break;
-#define FA_CASE(R)                                                                                               \
-  case R:                                                                                                        \
-    hipLaunchKernelGGL(fa_output_s16<R>,                                                                         \
-                       dim3((unsigned)(((nmax + ((int64_t)1 << 20) - 1) >> 20) * 2 * fa_s16_edge(R, 20) / FA_OT + \
-                                       (fa_s16_columns(R, 20) + FA_OT - 1) / FA_OT),                             \
-                            (unsigned)B),                                                                        \
-                       dim3(FA_OT), 0, st, Y, XS, io, io1);                                                      \
+#define FA_CASE(N, R, B0, SRC)                                                                                      \
+  case N:                                                                                                           \
+    hipLaunchKernelGGL((fa_output_adic<R, B0>), dim3((FaOut<R>::PARTS << B0) / FA_OT, (unsigned)B), dim3(FA_OT), 0, st, SRC, XS, \
+                       io, io1);                                                                                    \
     break;
-    FA_CASE(2)
-    FA_CASE(3)
-    FA_CASE(4)
-    FA_CASE(5)
+    FA_CASE(1, 1, 16, X)
+    FA_CASE(2, 2, 16, X)
+    FA_CASE(3, 3, 16, X)
+    FA_CASE(4, 4, 16, X)
+    FA_CASE(5, 5, 16, X)
+    FA_CASE(6, 2, 20, Y)
+    FA_CASE(7, 3, 20, Y)
+    FA_CASE(8, 4, 20, Y)
+    FA_CASE(9, 5, 20, Y)
 #undef FA_CASE
   }
   cuot_rec_end(st);

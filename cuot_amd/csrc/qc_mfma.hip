@@ -43,7 +43,11 @@ constexpr int64_t MF_NMAX = 1 << 16;          // bits of a are kept after the tr
 constexpr int64_t MF_TARGET_WGS = 1024;       // rows x slices aimed for (four per CU)
 constexpr int64_t MF_KLEN_MIN = 256, MF_KLEN_MAX = 16384;
 constexpr int MF_WIN_BYTES = MF_KLEN_MAX + MF_RW + 16;
-constexpr int64_t MF_DEFAULT_MAX = 49152;  // built-in crossover (n at or below: matrix cores), measured
+// Built-in crossover (n at or below: matrix cores), measured as one encode / two on
+// two streams, us: n = 32768 105 / 176 here and 182 / 190 by the transform (whose
+// padded length doubles at 32769, but whose conversion is on blocks from there on),
+// 36000 123 / 206 and 134 / 142, 40000 149 / 248 and 134 / 142.
+constexpr int64_t MF_DEFAULT_MAX = 36864;
 
 struct MfPlan {
   int64_t gx;    // row workgroups

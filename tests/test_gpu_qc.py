@@ -205,9 +205,10 @@ def test_qc_orbit_product_rotations(ctx, knob_mfma, n):
     assert torch.equal(y, want)
 
 
-# n > 2^20: rows of 2^20 coefficients in skewed columns; i + n near a row's ends,
-# whole and ragged last rows, with and without a carry into the next row
-@pytest.mark.parametrize("n", [(1 << 21) - 1, (1 << 22) - 100, 3 * (1 << 20) + 513, (1 << 22) + (1 << 20),
+# conversion and output in columns of 2^16 - 1 (n <= 2^20) or 2^20 - 16 rows: i + n
+# near a column's ends, whole and ragged last rows, with and without a wrap
+@pytest.mark.parametrize("n", [32769, 65535, 99991, 131072, (1 << 18) - 5, (1 << 20) - 17, 1 << 20,
+                               (1 << 21) - 1, (1 << 22) - 100, 3 * (1 << 20) + 513, (1 << 22) + (1 << 20),
                                (1 << 23) - (1 << 18) + 3, (1 << 24) - 1040])
 def test_qc_columns_rotations(ctx, knob_mfma, n):
     test_qc_orbit_product_rotations(ctx, knob_mfma, n)
