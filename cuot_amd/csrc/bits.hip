@@ -34,69 +34,77 @@ CUOT_DEV uint32_t cyc_window(const uint32_t* __restrict__ a, int64_t n, int64_t 
   return out;
 }
 
-__global__ void sparse_encode_kernel(const uint32_t* __restrict__ a, int64_t n, const int64_t* __restrict__ pos,
-                                     int w, uint32_t* __restrict__ out) {
-  const int64_t nw = (n + 31) / 32;
-  for (int64_t W = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; W < nw; W += (int64_t)gridDim.x * blockDim.x) {
-    uint32_t acc = 0;
-    const int64_t lo = W * 32;
-    for (int q = 0; q < w; q++) {
-      const int64_t p = pos[q];
-      if (p < 0 || p >= 2 * n) continue;
-      if (p < n) {
-        if ((p >> 5) == W) acc ^= 1u << (p & 31);
-      } else {
-        const int64_t s = p - n;  // out_i ^= a_{(i - s) mod n}
-        int64_t start = lo - s;  // in (-n, n): lo < n and 0 <= s < n
-        if (start < 0) start += n;
-        acc ^= cyc_window(a, n, start);
-      }
-    }
-    if (lo + 32 > n) acc &= (1u << (n - lo)) - 1u;
-    out[W] = acc;
-  }
-}
+// out = e_0 ^ a * e_1 for the w set positions of e.  A wavefront takes 128 output
+// words (two a lane, which share their middle word) and every fourth position,
+// four of them in flight; the four wavefronts' sums meet in LDS.  Bound by L2
+// reads at large n (2^24 bits, 1024 positions: 249 us) and by the chain of
+// positions at small ones: with all positions in turn in one lane 2^20 bits and
+// 128 positions took 27 us, now 9, 190731 and 94 20, now 8, 4000037 and 512 105,
+// now 40.
+constexpr int SP_WORDS = 128, SP_CHUNK = 512;
 
-// n a multiple of 32 (and at least 64 words): the window of position s starts
-// at the same bit offset sb = s mod 32 in every word, so output word W takes
-// (a[W - so] << sb) | (a[W - so - 1] >> (32 - sb)) with so = s / 32 (indices mod
-// n / 32); SPR consecutive output words per lane share their loads.
-constexpr int SPR = 2;  // measured at n = 2^24: 1 -> 0.31 ms, 2 -> 0.27 ms, 4 -> 0.37 ms
-__global__ void sparse_encode_w32(const uint32_t* __restrict__ a, int64_t n, const int64_t* __restrict__ pos, int w,
-                                  uint32_t* __restrict__ out) {
-  const int64_t nw = n >> 5;
-  for (int64_t W0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * SPR; W0 < nw;
-       W0 += (int64_t)gridDim.x * blockDim.x * SPR) {
-    uint32_t acc[SPR];
+__global__ __launch_bounds__(256) void sparse_encode(const uint32_t* __restrict__ a, int64_t n,
+                                                     const int64_t* __restrict__ pos, int w,
+                                                     uint32_t* __restrict__ out) {
+  __shared__ int64_t shift[SP_CHUNK];
+  __shared__ uint32_t res[SP_WORDS];
+  const int64_t nw = (n + 31) >> 5, last = (n - 1) >> 5;
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const int64_t B0 = (int64_t)blockIdx.x * SP_WORDS, W0 = B0 + 2 * (tid & 63), lo = W0 * 32;
+  if (tid < SP_WORDS) res[tid] = 0u;
+  uint32_t acc[2] = {0u, 0u};
+  for (int q0 = 0; q0 < w; q0 += SP_CHUNK) {
+    const int cnt = w - q0 < SP_CHUNK ? w - q0 : SP_CHUNK;
+    __syncthreads();
+    for (int q = tid; q < SP_CHUNK; q += 256) {
+      const int64_t p = q < cnt ? pos[q0 + q] : -1;
+      shift[q] = p >= n && p < 2 * n ? p - n : -1;
+      const int64_t rel = (p >> 5) - B0;
+      if (p >= 0 && p < n && rel >= 0 && rel < SP_WORDS) atomicXor(&res[rel], 1u << (p & 31));
+    }
+    __syncthreads();
+    if (W0 >= nw) continue;
+    for (int q = wave; q < cnt; q += 16) {
+      uint32_t x[4][3];
+      int sh[4];
+      bool whole[4];
+      int64_t start[4];
 #pragma unroll
-    for (int r = 0; r < SPR; r++) acc[r] = 0u;
-    for (int q = 0; q < w; q++) {
-      const int64_t p = pos[q];
-      if (p < 0 || p >= 2 * n) continue;
-      if (p < n) {
-        const int64_t pw = (p >> 5) - W0;
-#pragma unroll
-        for (int r = 0; r < SPR; r++)
-          if (pw == r) acc[r] ^= 1u << (p & 31);
-        continue;
+      for (int k = 0; k < 4; k++) {
+        const int64_t s = q + 4 * k < SP_CHUNK ? shift[q + 4 * k] : -1;  // out_i ^= a_{(i - s) mod n}
+        start[k] = lo - s;                                               // in (-n, n)
+        if (start[k] < 0) start[k] += n;
+        whole[k] = s >= 0 && start[k] + 64 <= n;
+        if (s < 0) start[k] = -1;
+        const int64_t wi = whole[k] ? start[k] >> 5 : 0;
+        sh[k] = (int)(start[k] & 31);
+        x[k][0] = a[wi];
+        x[k][1] = a[wi + 1 < last ? wi + 1 : last];
+        x[k][2] = a[wi + 2 < last ? wi + 2 : last];
       }
-      const int64_t sft = p - n;  // out_i ^= a_{(i - sft) mod n}
-      const int64_t so = sft >> 5;
-      const int sb = (int)(sft & 31);
-      int64_t i = W0 - so - 1;  // in [-nw, nw)
-      if (i < 0) i += nw;
-      uint32_t prev = a[i];
 #pragma unroll
-      for (int r = 0; r < SPR; r++) {
-        if (++i == nw) i = 0;
-        const uint32_t cur = a[i];
-        acc[r] ^= sb ? (cur << sb) | (prev >> (32 - sb)) : cur;
-        prev = cur;
+      for (int k = 0; k < 4; k++) {
+        if (whole[k]) {
+          acc[0] ^= (uint32_t)(((uint64_t)x[k][1] << 32 | x[k][0]) >> sh[k]);
+          acc[1] ^= (uint32_t)(((uint64_t)x[k][2] << 32 | x[k][1]) >> sh[k]);
+        } else if (start[k] >= 0) {  // past the row's end
+#pragma unroll
+          for (int r = 0; r < 2; r++)
+            if (lo + 32 * r < n) acc[r] ^= cyc_window(a, n, (start[k] + 32 * r) % n);
+        }
       }
     }
+  }
+  __syncthreads();
 #pragma unroll
-    for (int r = 0; r < SPR; r++)
-      if (W0 + r < nw) out[W0 + r] = acc[r];
+  for (int r = 0; r < 2; r++)
+    if (acc[r]) atomicXor(&res[2 * (tid & 63) + r], acc[r]);
+  __syncthreads();
+  if (tid < SP_WORDS && B0 + tid < nw) {
+    uint32_t v = res[tid];
+    const int64_t left = n - (B0 + tid) * 32;
+    if (left < 32) v &= (1u << left) - 1u;
+    out[B0 + tid] = v;
   }
 }
 
@@ -204,13 +212,9 @@ unsigned grid_for(int64_t total, int64_t cap = 1 << 16) {
 
 hipError_t cuot_launch_sparse(const uint32_t* a_words, int64_t n, const int64_t* pos, int w, uint32_t* out,
                               hipStream_t st) {
-  if ((n & 31) == 0 && (n >> 5) >= 64) {
-    hipLaunchKernelGGL(sparse_encode_w32, dim3(grid_for(((n >> 5) + SPR - 1) / SPR)), dim3(256), 0, st, a_words, n,
-                       pos, w, out);
-    return hipGetLastError();
-  }
-  hipLaunchKernelGGL(sparse_encode_kernel, dim3(grid_for((n + 31) / 32)), dim3(256), 0, st, a_words, n, pos, w,
-                     out);
+  const int64_t nw = (n + 31) >> 5;
+  hipLaunchKernelGGL(sparse_encode, dim3((unsigned)((nw + SP_WORDS - 1) / SP_WORDS)), dim3(256), 0, st, a_words, n, pos,
+                     w, out);
   return hipGetLastError();
 }
 

@@ -53,7 +53,9 @@ __constant__ uint2 c_fa_beta[32];  // beta_i and nu times its theta part
 __constant__ uint32_t c_fa_pack[FA_KC_MAX + 1][8];
 
 constexpr int FA_KMIN = 14, FA_KMAX = 25;
-constexpr int FA_STR = 20;  // longest row string converted in LDS (128 KB, 144 KB padded)
+// longest string of a's bits converted in LDS: 36 KB padded, so that a workgroup
+// fits beside the trees' (2^20 bits at a time waited for a whole CU's LDS)
+constexpr int FA_STR = 18;
 
 CUOT_DEV uint4 x4(uint4 a, uint4 b) { return make_uint4(a.x ^ b.x, a.y ^ b.y, a.z ^ b.z, a.w ^ b.w); }
 CUOT_DEV uint4 z4() { return make_uint4(0, 0, 0, 0); }
@@ -944,13 +946,6 @@ __global__ __launch_bounds__(FA_CT) __attribute__((amdgpu_waves_per_eu(2))) void
   }
 }
 
-CUOT_DEV int fa_terms(int k, uint32_t* e) {
-  int c = 0;
-  for (int j = 0; j < k; j++)
-    if ((j & ~k) == 0) e[c++] = 1u << j;
-  return c;
-}
-
 // ---- A^: the scalar transform of the single polynomial a ------------------------------
 // One 32-bit word per point.  The words behind A^ (a word per point again) hold
 // a's bits while they are converted and nu times the values' theta parts in the end.
@@ -972,50 +967,20 @@ __global__ __launch_bounds__(256) void fa_prep_bits(const QcPrep* __restrict__ p
   }
 }
 
-// forward conversion level k >= 20 on a's bit string, out of place (from the
-// first or second half of the words behind A^ to the other)
-__global__ __launch_bounds__(256) void fa_prep_level(const QcPrep* __restrict__ pr, QcPrep pr1, int K, int k, int src) {
+// one step of the forward conversion level KL on a's bit string, in place: the
+// correction of the upper halves or (LO) the lower halves' update.  Two launches
+// of a few us a level; as one, out of place, the update worked every correction
+// out again, and with its runs of terms in memory it took 180 us at n = 2^24 for
+// levels 20 .. 23, 690 beside the receiver's trees.
+template <int KL, bool LO>
+__global__ __launch_bounds__(256) void fa_prep_level(const QcPrep* __restrict__ pr, QcPrep pr1, int K) {
   const QcPrep q = pr ? pr[blockIdx.y] : pr1;
-  const int64_t NW = (int64_t)1 << (K - 6);
-  const uint32_t* in = q.ahat + ((int64_t)1 << (K - 5)) + (src ? NW : 0);
-  uint32_t* out = q.ahat + ((int64_t)1 << (K - 5)) + (src ? 0 : NW);
-  uint32_t e[16];
-  const int ne = fa_terms(k, e);
-  const int64_t hw = (int64_t)1 << (k - 5);  // words per half
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < NW; i += (int64_t)gridDim.x * 256) {
-    const int64_t pos = i & (2 * hw - 1);
-    const uint32_t* hi = in + (i - pos) + hw;
-    // word s of the quotient's half: hi with its first e_max bits corrected
-    auto quot = [&](int64_t s) {
-      uint32_t v = hi[s];
-      for (int r = 0; r < ne; r++) {
-        const int64_t ew = e[r] >> 5;
-        if (e[r] >= 32) {
-          if (s < ew) v ^= hi[s + hw - ew];
-        } else if (s == 0) {
-          v ^= hi[hw - 1] >> (32 - e[r]);
-        }
-      }
-      return v;
-    };
-    uint32_t v;
-    if (pos >= hw) {
-      v = quot(pos - hw);
-    } else {
-      v = in[i];
-      for (int t = 0; t < ne; t++) {
-        const int64_t ew = e[t] >> 5;
-        const int sh = (int)(e[t] & 31);
-        if (pos < ew) continue;
-        const uint32_t x = quot(pos - ew);
-        if (sh == 0)
-          v ^= x;
-        else
-          v ^= (x << sh) | (pos - ew >= 1 ? quot(pos - ew - 1) >> (32 - sh) : 0u);
-      }
-    }
-    out[i] = v;
-  }
+  uint32_t* T = q.ahat + ((int64_t)1 << (K - 5));
+  const int64_t tid = (int64_t)blockIdx.x * 256 + threadIdx.x, nth = (int64_t)gridDim.x * 256;
+  if (LO)
+    cbt_lo_update<KL>(T, (int64_t)1 << (K - 6), tid, nth);
+  else
+    cbt_hi_fix<KL>(T, (int64_t)1 << (K - 6), tid, nth);
 }
 
 struct FaSync {
@@ -1023,11 +988,11 @@ struct FaSync {
 };
 
 // levels below 2^mp on each string of 2^mp bits, in place (one workgroup each)
-__global__ __launch_bounds__(1024) void fa_prep_rows(const QcPrep* __restrict__ pr, QcPrep pr1, int K, int mp, int src) {
+__global__ __launch_bounds__(1024) void fa_prep_rows(const QcPrep* __restrict__ pr, QcPrep pr1, int K, int mp) {
   extern __shared__ uint32_t sw[];
   const QcPrep q = pr ? pr[blockIdx.y] : pr1;
   const int64_t nw = (int64_t)1 << (mp - 5);
-  uint32_t* g = q.ahat + ((int64_t)1 << (K - 5)) + (src ? (int64_t)1 << (K - 6) : 0) + (int64_t)blockIdx.x * nw;
+  uint32_t* g = q.ahat + ((int64_t)1 << (K - 5)) + (int64_t)blockIdx.x * nw;
   for (int64_t i = threadIdx.x; i < nw; i += 1024) sw[cbp_at<true>(i)] = g[i];
   __syncthreads();
   cbp_convert<true, false>(sw, 0, mp, threadIdx.x, 1024, FaSync());
@@ -1039,7 +1004,7 @@ constexpr int FA_PT = 10;  // log2 words of a preparation tile
 // Element bits lo .. lo + R - 1 on tiles of 2^R words 2^lo apart times 2^lgC
 // consecutive ones; the first tile pass takes the words from a's converted bits.
 __global__ __launch_bounds__(512) void fa_prep_fft(const QcPrep* __restrict__ pr, QcPrep pr1, int K, int c, int aidx,
-                                                   int lo, int R, int lgC, int first, int src) {
+                                                   int lo, int R, int lgC, int first) {
   __shared__ uint32_t L[1 << FA_PT];
   __shared__ uint2 ctab[FA_CTAB];
   const QcPrep q = pr ? pr[blockIdx.y] : pr1;
@@ -1051,7 +1016,7 @@ __global__ __launch_bounds__(512) void fa_prep_fft(const QcPrep* __restrict__ pr
   const int64_t cb = tile & ((((int64_t)1 << lo) >> lgC) - 1), hib = tile >> (lo - lgC);
   auto eidx = [&](int i) { return (hib << (lo + R)) | ((int64_t)(i >> lgC) << lo) | (cb * C + (i & (C - 1))); };
   if (first) {
-    const uint32_t* T = A + ((int64_t)1 << (K - 5)) + (src ? (int64_t)1 << (K - 6) : 0);
+    const uint32_t* T = A + ((int64_t)1 << (K - 5));
     const uint32_t* pk = c_fa_pack[K <= 20 ? 0 : K - 20];
     for (int i = threadIdx.x; i < TW; i += nt) {
       const int64_t e = eidx(i);
@@ -1298,19 +1263,33 @@ hipError_t cuot_launch_qc_fa_prepare(const QcPrep* pr, QcPrep pr1, int B, int K,
   const int c = K - 5 < 15 ? K - 5 : 15, aidx = 16 + c;
   const int64_t nw = (int64_t)1 << (K - 6);
   hipLaunchKernelGGL(fa_prep_bits, dim3(capg(nw / 256, 1024), (unsigned)B), dim3(256), 0, st, pr, pr1, K);
-  int src = 0;
-  for (int k = K - 2; k >= FA_STR; k--, src ^= 1)
-    hipLaunchKernelGGL(fa_prep_level, dim3(capg(nw / 256, 1024), (unsigned)B), dim3(256), 0, st, pr, pr1, K, k, src);
+  for (int k = K - 2; k >= FA_STR; k--) {
+    const dim3 grid(capg(nw / 512, 1024), (unsigned)B);
+    switch (k) {
+#define FA_CASE(KL)                                                                     \
+  case KL:                                                                              \
+    hipLaunchKernelGGL((fa_prep_level<KL, false>), grid, dim3(256), 0, st, pr, pr1, K); \
+    hipLaunchKernelGGL((fa_prep_level<KL, true>), grid, dim3(256), 0, st, pr, pr1, K);  \
+    break;
+      FA_CASE(18)
+      FA_CASE(19)
+      FA_CASE(20)
+      FA_CASE(21)
+      FA_CASE(22)
+      FA_CASE(23)
+#undef FA_CASE
+    }
+  }
   const int mp = K - 1 < FA_STR ? K - 1 : FA_STR;
   hipLaunchKernelGGL(fa_prep_rows, dim3(1u << (K - 1 - mp), (unsigned)B), dim3(1024),
-                     (size_t)cbp_words((int64_t)1 << (mp - 5), true) * 4, st, pr, pr1, K, mp, src);
+                     (size_t)cbp_words((int64_t)1 << (mp - 5), true) * 4, st, pr, pr1, K, mp);
   const int bits = K - 5;
   const int Rl = bits < FA_PT ? bits : FA_PT, Ru = bits - Rl;
   if (Ru > 0)
     hipLaunchKernelGGL(fa_prep_fft, dim3(1u << (bits - FA_PT), (unsigned)B), dim3(512), 0, st, pr, pr1, K, c, aidx, Rl,
-                       Ru, FA_PT - Ru, 1, src);
+                       Ru, FA_PT - Ru, 1);
   hipLaunchKernelGGL(fa_prep_fft, dim3(1u << (bits - Rl), (unsigned)B), dim3(512), 0, st, pr, pr1, K, c, aidx, 0, Rl, 0,
-                     Ru > 0 ? 0 : 1, src);
+                     Ru > 0 ? 0 : 1);
   return hipGetLastError();
 }
 

@@ -163,6 +163,19 @@ def test_sparse_vs_oracle(ctx, n):
     assert np.array_equal(got, po.qc_sparse(pos, a, n))
 
 
+# tiles of 128 words, chunks of 512 positions, four in flight per wavefront
+@pytest.mark.parametrize("n, w", [(63, 5), (64, 1), (4095, 600), (4097, 512), (8192, 513), (100003, 1027), (1 << 17, 17)])
+def test_sparse_tiles_and_chunks(ctx, n, w):
+    import torch
+
+    r = rng(n + 5)
+    a = rand_bits(r, n)
+    pos = np.sort(r.choice(2 * n, size=w, replace=False)).astype(np.int64)
+    out = torch.full((((n + 31) // 32) * 4,), 0xA5, dtype=torch.uint8, device="cuda")
+    ctx.qc_sparse(n, dev_bits(a, n), torch.from_numpy(pos).cuda(), out)
+    assert np.array_equal(out.cpu().numpy()[: (n + 7) // 8], po.qc_sparse(pos, a, n))
+
+
 @pytest.mark.parametrize("N", [32, 1024, 32 * 1000, 1 << 16])
 def test_transpose(ctx, N):
     import torch
