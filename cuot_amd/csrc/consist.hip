@@ -87,17 +87,6 @@ CUOT_DEV blk mk(uint64_t lo, uint64_t hi) {
 }
 CUOT_DEV blk bx(blk a, blk b) { return make_uint4(a.x ^ b.x, a.y ^ b.y, a.z ^ b.z, a.w ^ b.w); }
 
-CUOT_DEV void clmul64(uint64_t a, uint64_t b, uint64_t& lo, uint64_t& hi) {
-  uint64_t l = 0, h = 0;
-  for (int i = 0; i < 64; i++) {
-    const uint64_t m = 0 - ((b >> i) & 1);
-    l ^= (a << i) & m;
-    h ^= (i ? (a >> (64 - i)) : 0) & m;
-  }
-  lo = l;
-  hi = h;
-}
-
 // p[0..3] (256 bits, p[0] lowest) mod x^128 + x^7 + x^2 + x + 1
 CUOT_DEV blk reduce256(uint64_t p0, uint64_t p1, uint64_t p2, uint64_t p3) {
 #pragma unroll
@@ -111,17 +100,37 @@ CUOT_DEV blk reduce256(uint64_t p0, uint64_t p1, uint64_t p2, uint64_t p3) {
   return mk(p0, p1);
 }
 
+// N products by one e, bit by bit from its top: a shift with the reduction folded
+// in and one masked XOR a word (the masks serve all N; through 64-bit carry-less
+// products one took 3600 operations, here 1300)
+template <int N>
+CUOT_DEV void gf_mul_n(blk e, const blk (&x)[N], blk (&r)[N]) {
+  const uint32_t ew[4] = {e.x, e.y, e.z, e.w};
+#pragma unroll
+  for (int k = 0; k < N; k++) r[k] = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+  for (int w = 3; w >= 0; w--) {
+    uint32_t v = ew[w];
+#pragma unroll 4
+    for (int b = 0; b < 32; b++, v <<= 1) {
+      const uint32_t m = (uint32_t)((int32_t)v >> 31);
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        const uint32_t top = (uint32_t)((int32_t)r[k].w >> 31) & 0x87u;
+        r[k].w = (r[k].w << 1 | r[k].z >> 31) ^ (x[k].w & m);
+        r[k].z = (r[k].z << 1 | r[k].y >> 31) ^ (x[k].z & m);
+        r[k].y = (r[k].y << 1 | r[k].x >> 31) ^ (x[k].y & m);
+        r[k].x = (r[k].x << 1) ^ top ^ (x[k].x & m);
+      }
+    }
+  }
+}
+
 CUOT_DEV blk gf_mul(blk a, blk b) {
-  uint64_t l, h, p0, p1, p2, p3;
-  clmul64(lo64(a), lo64(b), p0, p1);
-  clmul64(hi64(a), hi64(b), p2, p3);
-  clmul64(lo64(a), hi64(b), l, h);
-  p1 ^= l;
-  p2 ^= h;
-  clmul64(hi64(a), lo64(b), l, h);
-  p1 ^= l;
-  p2 ^= h;
-  return reduce256(p0, p1, p2, p3);
+  const blk x[1] = {b};
+  blk r[1];
+  gf_mul_n<1>(a, x, r);
+  return r[0];
 }
 
 // bits of x at the even positions of a 64-bit word
@@ -138,12 +147,6 @@ CUOT_DEV uint64_t spread32(uint32_t v) {
 // a^2: in characteristic 2 the square of sum a_i x^i is sum a_i x^(2i)
 CUOT_DEV blk gf_sqr(blk a) {
   return reduce256(spread32(a.x), spread32(a.y), spread32(a.z), spread32(a.w));
-}
-
-// a * x
-CUOT_DEV blk gf_mul_x(blk a) {
-  const uint64_t l = lo64(a), h = hi64(a);
-  return reduce256(l << 1, (h << 1) | (l >> 63), h >> 63, 0);
 }
 
 // a * x^j, 0 <= j < 128
@@ -180,12 +183,17 @@ struct ConsistArgs {
   blk* chia;
 };
 
-__global__ __launch_bounds__(256) void consist_tree_kernel(ConsistArgs a) {
-  __shared__ uint4 B[3][128];     // K x^i for the three table constants
+// Bound by the table lookups (10.6 GB of LDS reads for 1270 trees of 8192 leaves)
+// and the instructions around them.  30 KB of LDS, so that five workgroups fit a
+// CU and those trees run in one wave of workgroups: 236 us, 345 with 39 KB, the powers of x
+// one after the other and 64-bit carry-less products for the last three.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void consist_tree_kernel(ConsistArgs a) {
   __shared__ uint4 T[3][32][16];  // window tables of S = seed^P, seed, seed^16
-  __shared__ uint4 red[2][256];
+  __shared__ uint4 B[3][128];     // K x^i for the three table constants
   __shared__ uint4 cs[4];
   __shared__ uint4 PW[2][17];     // seed^b and seed^(16a), a, b = 0..16
+  // the lanes' terms: over the tables of seed and seed^16, whose last use is PW
+  uint4(*red)[256] = (uint4(*)[256])&T[1][0][0];
   const int64_t tr = blockIdx.x;
   const int L = 1 << a.h;
   const int P = L < 256 ? L : 256;
@@ -205,13 +213,7 @@ __global__ __launch_bounds__(256) void consist_tree_kernel(ConsistArgs a) {
     }
   }
   __syncthreads();
-  if (tid < 3) {
-    blk c = cs[tid];
-    for (int i = 0; i < 128; i++) {
-      B[tid][i] = c;
-      c = gf_mul_x(c);
-    }
-  }
+  for (int f = tid; f < 3 * 128; f += 256) B[f >> 7][f & 127] = gf_mul_xj(cs[f >> 7], f & 127);
   __syncthreads();
   for (int f = tid; f < 3 * 512; f += 256) {
     const int q = f >> 9, k = (f >> 4) & 31, v = f & 15;
@@ -257,8 +259,11 @@ __global__ __launch_bounds__(256) void consist_tree_kernel(ConsistArgs a) {
       }
     }
     const blk e = gf_mul(PW[1][(tid + 1) >> 4], PW[0][(tid + 1) & 15]);  // seed^(tid+1)
-    hs = gf_mul(e, hs);
-    hr = gf_mul(e, hr);
+    const blk x[2] = {hs, hr};
+    blk r[2];
+    gf_mul_n<2>(e, x, r);
+    hs = r[0];
+    hr = r[1];
   }
   red[0][tid] = hs;
   red[1][tid] = hr;

@@ -309,13 +309,15 @@ extern "C" int cuot_sot_run_stages(cuot_ctx* ctx, const cuot_sot_config* cfg, vo
 
 // Whole instance with the independent stages overlapped on two streams (the
 // caller's and the context's second stream, joined before returning):
-//   caller: setup -> sender GGM + masked rows -> A^ prepare -> sender QC -> sparse -> [join]
-//   second: [rows] -> receiver GGM -> receiver QC (from its pointwise product on behind [A^])
+//   caller: setup -> sender GGM + masked rows -> A^ prepare -> sender QC -> [join]
+//   second: [rows] -> receiver GGM -> receiver QC (from its pointwise product on behind [A^]) -> sparse
 // The two encodes use separate scratch.  Same bytes as the staged run.  A^ and
 // the sparse product beside the sender's trees instead, ahead of the receiver's,
 // and both encodes behind A^ took 829 us at n = 2^20 and 448 at 190731, this
-// way 746 and 415 (the receiver's trees start with the rows, and the caller's
-// stream has the sparse product while the receiver's encode ends).
+// way 746 and 415: the receiver's trees start with the rows, and its stream is the
+// first to end (the sparse product behind the sender's encode costs 10 us at
+// 190731, 15 at 2^20 and 100 at 2^24; with the matrix cores' encodes, which wait
+// for no A^, it belongs there: 134 us at 2^14, 140 behind the receiver's).
 extern "C" int cuot_sot_run(cuot_ctx* ctx, const cuot_sot_config* cfg, void* ws_d, size_t ws_bytes, cuot_block* v_d,
                             cuot_block* w_d, uint8_t* b_d, cuot_block* delta_d, void* stream) {
   CUOT_CHECK_ARG(ctx && cfg, "ctx/cfg NULL");
@@ -343,8 +345,11 @@ extern "C" int cuot_sot_run(cuot_ctx* ctx, const cuot_sot_config* cfg, void* ws_
   CUOT_HIP_TRY(hipEventRecord(e_prep, st));
   CUOT_HIP_TRY(cuot_launch_qc_encode(p.ahat, p.cfg.n, p.leaves_s, (blk*)v_d, p.qc_scratch, st));
   CUOT_HIP_TRY(cuot_launch_qc_encode(p.ahat, p.cfg.n, p.leaves_r, (blk*)w_d, p.qc_scratch2, ax, e_prep));
+  // behind the encode that ends first: the receiver's where the sender's waited for A^
+  const bool mfma = cuot_qc_mfma_selected(p.cfg.n);
+  if (!mfma) CUOT_HIP_TRY(cuot_launch_sparse(p.a_words, p.cfg.n, p.pos, (int)p.cfg.t, (uint32_t*)b_d, ax));
   CUOT_HIP_TRY(hipEventRecord(e_done, ax));
-  CUOT_HIP_TRY(cuot_launch_sparse(p.a_words, p.cfg.n, p.pos, (int)p.cfg.t, (uint32_t*)b_d, st));
+  if (mfma) CUOT_HIP_TRY(cuot_launch_sparse(p.a_words, p.cfg.n, p.pos, (int)p.cfg.t, (uint32_t*)b_d, st));
   CUOT_HIP_TRY(hipStreamWaitEvent(st, e_done, 0));
   return CUOT_OK;
 }
