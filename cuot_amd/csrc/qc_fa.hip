@@ -98,63 +98,73 @@ struct FaArgs {
 constexpr int FA_TL = 8;    // log2 elements of a tile
 constexpr int FA_NT = 512;  // lanes
 
-// First and last pass: the layers above c, KC of them, where the halves of the
-// elements transform apart under GF(2^16) constants (blockIdx.z: the half).  LDS
-// tile: 2^KC elements 2^c apart times 2^(8-KC) consecutive ones, 16 planes x 4
-// words each and 4 words of padding; one (butterfly, word) per lane and layer.
-constexpr int FA_ST16 = 68;
-
-// LDS slot of tile element e: the butterflies of the lowest tile layers touch
-// elements whose slots share their residue mod 8 (the element stride is 4 mod
-// 64 banks); reflecting every odd group of eight spreads them
-CUOT_DEV int fa_slot(int e) { return e ^ (((e >> 3) & 1) * 7); }
-
-template <int KC, bool INV>
-__device__ __forceinline__ void fa_layer16(const FaArgs& a, uint32_t* lds, const uint2* ctab, int s) {
-  constexpr int LGC = FA_TL - KC, C = 1 << LGC;
-  const int w = threadIdx.x & 3, cc = (threadIdx.x >> 2) & (C - 1), bp = (threadIdx.x >> 2) >> LGC;
-  const int tu = ((bp >> s) << (s + 1)) | (bp & ((1 << s) - 1)), tv = tu | (1 << s);
-  uint32_t* pu = lds + fa_slot(tu * C + cc) * FA_ST16 + w;
-  uint32_t* pv = lds + fa_slot(tv * C + cc) * FA_ST16 + w;
-  uint32_t xv[16], acc[16];
+// A pass holds a tile of 256 elements (rows 2^lo apart times consecutive columns)
+// in registers: lane P * 4 + w has word w of the two elements of butterfly P.
+// Between layers a lane gives one of the two to the lane whose P differs in the
+// next layer's bit and takes one: through LDS where that is another wavefront, by
+// lane swaps inside one.
+// give u (where this lane's P has bit b set) or v to the lane whose P differs in
+// that bit and take the same from it
+// (N lanes further; the quads of a row whose bit is set are the BANKS)
+template <int NP, int N, int BANKS>
+__device__ __forceinline__ void fa_swap_dpp(uint32_t* u, uint32_t* v) {
 #pragma unroll
-  for (int p = 0; p < 16; p++) {
-    xv[p] = pv[4 * p];
-    if (INV) pv[4 * p] = xv[p] ^= pu[4 * p];
+  for (int p = 0; p < NP; p++) {
+    const int a = (int)u[p], b = (int)v[p];
+    u[p] = (uint32_t)__builtin_amdgcn_update_dpp(a, b, 0x110 | N, 0xF, BANKS, false);       // row_shr
+    v[p] = (uint32_t)__builtin_amdgcn_update_dpp(b, a, 0x100 | N, 0xF, 0xF ^ BANKS, false);  // row_shl
   }
-  // the first lane's constant for all, and what the others' g add to it: a
-  // wavefront covers 16 neighbouring (butterfly, column) pairs, so at most the
-  // low four bits of g differ
-  const uint32_t g = (uint32_t)(tu >> (s + 1)), g0 = __builtin_amdgcn_readfirstlane(g), d = g ^ g0;
-  fa_mulc16(xv, __builtin_amdgcn_readfirstlane(c_fa_beta[a.a - a.c - 1 - s].x ^ fa_ctab(ctab, g0).x), acc);
-  if (__any(d != 0)) fa_add_low(xv, d, acc);
+}
+
+template <int NP>
+__device__ __forceinline__ void fa_swap_lds(uint32_t* lds, uint32_t* g, int other) {
 #pragma unroll
-  for (int p = 0; p < 16; p++) {
-    const uint32_t un = pu[4 * p] ^ acc[p];
-    pu[4 * p] = un;
-    if (!INV) pv[4 * p] = xv[p] ^ un;
-  }
+  for (int p = 0; p < NP; p++) lds[p * FA_NT + threadIdx.x] = g[p];
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < NP; p++) g[p] = lds[p * FA_NT + other];
   __syncthreads();
 }
 
-// chunk maps on the staged tile: 8 coefficient planes -> 16 coordinates, and
-// 16 coordinates -> 16 coefficient planes
-template <int KC, bool UN>
-__device__ __forceinline__ void fa_chunks(uint32_t* lds) {
-  for (int tau = threadIdx.x; tau < 4 << FA_TL; tau += FA_NT) {
-    uint32_t* pe = lds + fa_slot(tau >> 2) * FA_ST16 + (tau & 3);
-    uint32_t in[16], out[16];
-#pragma unroll
-    for (int p = 0; p < (UN ? 16 : 8); p++) in[p] = pe[4 * p];
-    if constexpr (UN)
-      fa_unpack_planes<KC>(in, out);
-    else
-      fa_pack_planes<KC>(in, out);
-#pragma unroll
-    for (int p = 0; p < 16; p++) pe[4 * p] = out[p];
+template <int NP>
+__device__ __forceinline__ void fa_swap(uint32_t* lds, uint32_t* u, uint32_t* v, int P, int b) {
+  // (b opaque in between: as one chain of choices the compiler merges all ways
+  // behind 64 moves)
+#define FA_OPAQUE(x) \
+  x = __builtin_amdgcn_readfirstlane(x); \
+  asm volatile("" : "+s"(x))
+  if (b >= 4) {  // another wavefront; the bit is this one's
+    const int other = (int)threadIdx.x ^ (4 << b);
+    int bit = __builtin_amdgcn_readfirstlane(P >> b) & 1;
+    if (bit) fa_swap_lds<NP>(lds, u, other);
+    FA_OPAQUE(bit);
+    if (!bit) fa_swap_lds<NP>(lds, v, other);
   }
-  __syncthreads();
+  FA_OPAQUE(b);
+  if (b == 3) {
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const auto r = __builtin_amdgcn_permlane32_swap(u[p], v[p], false, false);
+      u[p] = r[0];
+      v[p] = r[1];
+    }
+  }
+  FA_OPAQUE(b);
+  if (b == 2) {
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const auto r = __builtin_amdgcn_permlane16_swap(u[p], v[p], false, false);
+      u[p] = r[0];
+      v[p] = r[1];
+    }
+  }
+  FA_OPAQUE(b);
+  if (b == 1) fa_swap_dpp<NP, 8, 0xC>(u, v);
+  FA_OPAQUE(b);
+  if (b == 0) fa_swap_dpp<NP, 4, 0xA>(u, v);
 }
+
+CUOT_DEV int fa_insert(int P, int b, int r) { return ((P >> b) << (b + 1)) | (r << b) | (P & ((1 << b) - 1)); }
 
 // ---- basis conversion in registers ----------------------------------------------------
 // Between the monomial basis and the novel one, every split of the index bits at
@@ -284,22 +294,38 @@ __device__ __forceinline__ void fa_step_conv(int row, const L& ld, const S& st) 
   for (int k = 0; k < (1 << N); k++) st(row + k * STRIDE, v[k]);
 }
 
+constexpr int FA_ST16 = 68;
+
+// LDS slot of tile element e where a step's lanes touch elements eight apart (the
+// element stride is 4 mod 64 banks): reflecting every odd group of eight spreads them
+CUOT_DEV int fa_slot(int e) { return e ^ (((e >> 3) & 1) * 7); }
+
 // The coefficient rows of a half-mode tile, from powers of s_16 to the novel basis
 // (INV: back): row rho (index bits 16 up, X = s_16) lies in plane rho >> KC of
-// element (rho mod 2^KC) * C + column.  A lane takes one word of a row.  At n = 2^24
-// the two passes take 300 and 445 us; level by level over the whole tile in LDS,
-// with the novel basis' own terms, 365 and 515.
+// element (rho mod 2^KC) * C + column.  A lane takes one word of a row.  Level by
+// level over the whole tile in LDS, with the novel basis' own terms, the two
+// passes took 65 and 70 us more at n = 2^24.
 template <int KC>
 __device__ __forceinline__ uint32_t& fa_row(uint32_t* lds, int rho, int col, int w) {
   return lds[fa_slot(((rho & ((1 << KC) - 1)) << (FA_TL - KC)) + col) * FA_ST16 + 4 * (rho >> KC) + w];
 }
 
+// staging (and the rows' conversion) addresses come from an opaque copy of the lane index, so that the
+// compiler recomputes them per phase instead of holding them through the layers
+__device__ __forceinline__ int opaque_tid() {
+  int t = (int)threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 template <int KC, bool INV>
 __device__ __forceinline__ void fa_outer(uint32_t* lds) {
   constexpr int NB = KC + (INV ? 4 : 3), H = NB > 8 ? 4 : NB - 4, LGW = FA_TL - KC + 2;  // words of a row: columns x 4
-  const int w = threadIdx.x & 3, col = (threadIdx.x >> 2) & ((1 << (LGW - 2)) - 1);
+  // (the longest conversions' addresses would spill the next tile's loads)
+  const int tid = INV && KC > 3 ? opaque_tid() : (int)threadIdx.x;
+  const int w = tid & 3, col = (tid >> 2) & ((1 << (LGW - 2)) - 1);
   auto halves = [&](auto step, int tasks) {  // tasks per 2^(4+H) rows
-    for (int x = threadIdx.x >> LGW; x < tasks << (NB - 4 - H); x += FA_NT >> LGW) {
+    for (int x = tid >> LGW; x < tasks << (NB - 4 - H); x += FA_NT >> LGW) {
       const int base = NB > 8 ? (x / tasks) << 8 : 0;
       step(
           NB > 8 ? x % tasks : x, [&](int r) { return fa_row<KC>(lds, base + r, col, w); },
@@ -313,14 +339,14 @@ __device__ __forceinline__ void fa_outer(uint32_t* lds) {
   auto s8 = [&] {  // bit 8 of nine: lo_j ^= q_{j-1}
     if constexpr (NB > 8) {
       if (!INV) {
-        if ((int)threadIdx.x >> LGW == 0) fa_row<KC>(lds, 256, col, w) ^= fa_row<KC>(lds, 511, col, w);
+        if (tid >> LGW == 0) fa_row<KC>(lds, 256, col, w) ^= fa_row<KC>(lds, 511, col, w);
         __syncthreads();
       }
-      for (int x = (threadIdx.x >> LGW) + 1; x < 256; x += FA_NT >> LGW)
+      for (int x = (tid >> LGW) + 1; x < 256; x += FA_NT >> LGW)
         fa_row<KC>(lds, x, col, w) ^= fa_row<KC>(lds, 255 + x, col, w);
       __syncthreads();
       if (INV) {
-        if ((int)threadIdx.x >> LGW == 0) fa_row<KC>(lds, 256, col, w) ^= fa_row<KC>(lds, 511, col, w);
+        if (tid >> LGW == 0) fa_row<KC>(lds, 256, col, w) ^= fa_row<KC>(lds, 511, col, w);
         __syncthreads();
       }
     }
@@ -343,40 +369,51 @@ CUOT_DEV int64_t fa_nat(const FaArgs& a, int64_t e, int h, int q) {
   return ((int64_t)q << (a.K - 4)) | ((e >> a.c) << (a.c + 1)) | ((int64_t)h << a.c) | (e & (((int64_t)1 << a.c) - 1));
 }
 
-// staging addresses come from an opaque copy of the lane index, so that the
-// compiler recomputes them per phase instead of holding them through the layers
-__device__ __forceinline__ int opaque_tid() {
-  int t = (int)threadIdx.x;
-  asm volatile("" : "+v"(t));
-  return t;
-}
-
+// First and last pass (K > 20): the layers above c, KC of them, where the halves of
+// the elements transform apart under GF(2^16) constants (blockIdx.z: the half).
+// Tiles of 2^KC elements 2^c apart times 2^(8-KC) consecutive ones.  On the natural
+// side the tile's coefficients lie in LDS for the rows' conversion, 16 planes x 4
+// words an element and 4 words of padding.  At n = 2^24 the two passes take 240 and
+// 440 us (3.4 and 2.4 TB/s); with the whole tile in LDS through the layers 300 and
+// 445, of which 190 and 310 were vector operations.
 template <int KC, bool INV>
 __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void fa_pass16(FaArgs a) {
   extern __shared__ uint32_t lds[];
-  constexpr int LGC = FA_TL - KC, C = 1 << LGC, TC = 1 << FA_TL;
+  constexpr int LGC = FA_TL - KC, C = 1 << LGC, TC = 1 << FA_TL, NH = TC / 2;
   const int64_t ioff = (int64_t)blockIdx.y * a.XS;
   uint4* E = a.E + ioff;
   const uint4* nin = a.nat_in + ioff;
   uint4* nout = a.nat_out + ioff;
-  const int h = (int)blockIdx.z;
+  const int h = (int)blockIdx.z, w = threadIdx.x & 3, P = threadIdx.x >> 2;
   const int64_t ntiles = ((int64_t)1 << (a.K - 5)) >> FA_TL;
   uint2* ctab = (uint2*)(lds + TC * FA_ST16);
   fa_ctab_fill(ctab, threadIdx.x, FA_NT);  // read after the first barrier
-  // a tile's base is its first column: the 2^KC elements are all those 2^c apart
-  auto elem = [&](int64_t tile, int el) { return (tile << LGC) + ((int64_t)(el >> LGC) << a.c) + (el & (C - 1)); };
-  // staged word f: plane fastest in element-major data, element fastest in natural order
-  uint4 v[8];
+  // Staged word f = tid + 512 k: plane fastest in element-major data, element fastest
+  // in natural order.  A tile's base is its first column (the 2^KC elements are all
+  // those 2^c apart); an address is a scalar part of the base and k's bits plus one
+  // of the lane's.
+  auto off = [&](int el) { return ((int64_t)(el >> LGC) << a.c) + (el & (C - 1)); };
+  auto eptr = [&](int64_t tile, int tid, int k) {
+    const uint32_t ln = (uint32_t)off(tid >> 4) * 32 + (tid & 15);
+    return (uint4*)((char*)(E + ((tile << LGC) + off(32 * k)) * 32 + 16 * h) + (size_t)(ln * 16));
+  };
+  auto nptr = [&](uint4* p, int64_t tile, int tid, int k) {
+    const uint32_t ln = (uint32_t)fa_nat(a, off(tid & (TC - 1)), 0, tid >> FA_TL);
+    return (uint4*)((char*)(p + fa_nat(a, tile << LGC, h, 2 * k)) + (size_t)(ln * 16));
+  };
+  // LDS slot of an element on the element-major side: by register bit (tile bit
+  // LGC), then P
+  auto eslot = [&](int el) { return ((el >> LGC) & 1) * NH + ((el >> (LGC + 1)) << LGC | (el & (C - 1))); };
+  uint4 st[8];
   auto load_tile = [&](int64_t tile) {
     const int tid = opaque_tid();
 #pragma unroll
-    for (int u = 0; u < (INV ? 8 : 4); u++) {
-      const int f = tid + u * FA_NT;
-      v[u] = z4();
+    for (int k = 0; k < (INV ? 8 : 4); k++) {
+      st[k] = z4();
       if constexpr (INV)
-        v[u] = E[elem(tile, f >> 4) * 32 + 16 * h + (f & 15)];
+        st[k] = *eptr(tile, tid, k);
       else
-        v[u] = nin[fa_nat(a, elem(tile, f & (TC - 1)), h, f >> FA_TL)];
+        st[k] = *nptr((uint4*)nin, tile, tid, k);
     }
   };
   // workgroups are dealt to the 8 XCDs in turn: one XCD's take neighbouring tiles
@@ -386,51 +423,90 @@ __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void
   for (int64_t tile = slot; tile < ntiles; tile += G) {
     int tid = opaque_tid();
 #pragma unroll
-    for (int u = 0; u < (INV ? 8 : 4); u++) {
-      const int f = tid + u * FA_NT;
-      *(uint4*)&lds[fa_slot(INV ? f >> 4 : f & (TC - 1)) * FA_ST16 + (INV ? f & 15 : f >> FA_TL) * 4] = v[u];
+    for (int k = 0; k < (INV ? 8 : 4); k++) {
+      const int f = tid + k * FA_NT;
+      *(uint4*)&lds[(INV ? eslot(f >> 4) : fa_slot(f & (TC - 1))) * FA_ST16 + (INV ? f & 15 : f >> FA_TL) * 4] = st[k];
+    }
+    __syncthreads();
+    uint32_t u[16], v[16];
+    if constexpr (!INV) {
+      fa_outer<KC, false>(lds);
+      uint32_t t[8];
+#pragma unroll
+      for (int p = 0; p < 8; p++) t[p] = lds[fa_slot(P) * FA_ST16 + 4 * p + w];
+      fa_pack_planes<KC>(t, u);
+#pragma unroll
+      for (int p = 0; p < 8; p++) t[p] = lds[fa_slot(NH + P) * FA_ST16 + 4 * p + w];
+      fa_pack_planes<KC>(t, v);
+    } else {
+#pragma unroll
+      for (int p = 0; p < 16; p++) u[p] = lds[P * FA_ST16 + 4 * p + w];
+#pragma unroll
+      for (int p = 0; p < 16; p++) v[p] = lds[(NH + P) * FA_ST16 + 4 * p + w];
+    }
+    __syncthreads();
+    // tile bits 7 .. LGC, or back up; one loop, so that the layer's code is there once
+#pragma unroll 1
+    for (int step = 0; step < KC; step++) {
+      const int b = INV ? LGC + step : FA_TL - 1 - step;
+      int sw = step == 0 ? -1 : INV ? b - 1 : b;  // the bit of P to swap with
+      FA_OPAQUE(sw);
+      fa_swap<16>(lds, u, v, P, sw);
+      // the first lane's constant for all, and what the others' g add to it
+      const uint32_t g = (uint32_t)(P >> b), g0 = __builtin_amdgcn_readfirstlane(g), d = g ^ g0;
+      const uint2 c = x2(c_fa_beta[a.a - a.c - 1 - (b - LGC)], fa_ctab(ctab, g0));
+      uint32_t acc[16];
+      if constexpr (INV) {
+#pragma unroll
+        for (int p = 0; p < 16; p++) v[p] ^= u[p];
+      }
+      fa_mulc16(v, __builtin_amdgcn_readfirstlane(c.x), acc);
+#pragma unroll
+      for (int p = 0; p < 16; p++) u[p] ^= acc[p];
+      if (__any(d != 0)) fa_add_low(v, d, u);
+      if constexpr (!INV) {
+#pragma unroll
+        for (int p = 0; p < 16; p++) v[p] ^= u[p];
+      }
     }
     __syncthreads();
     if constexpr (!INV) {
-      fa_outer<KC, false>(lds);
-      fa_chunks<KC, false>(lds);
-    }
-    // one loop, so that the layer's code is there once
-#pragma unroll 1
-    for (int step = 0; step < KC; step++) fa_layer16<KC, INV>(a, lds, ctab, INV ? step : KC - 1 - step);
-    if constexpr (INV) {
-      fa_chunks<KC, true>(lds);
-      fa_outer<KC, true>(lds);
-    }
-    uint4 w[8];
-    tid = opaque_tid();
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const int f = tid + u * FA_NT;
-      w[u] = z4();
-      w[u] = *(const uint4*)&lds[fa_slot(INV ? f & (TC - 1) : f >> 4) * FA_ST16 + (INV ? f >> FA_TL : f & 15) * 4];
+      for (int p = 0; p < 16; p++) lds[P * FA_ST16 + 4 * p + w] = u[p];
+#pragma unroll
+      for (int p = 0; p < 16; p++) lds[(NH + P) * FA_ST16 + 4 * p + w] = v[p];
+      __syncthreads();
+    } else {
+      uint32_t t[16];
+      fa_unpack_planes<KC>(u, t);
+#pragma unroll
+      for (int p = 0; p < 16; p++) lds[fa_slot(P) * FA_ST16 + 4 * p + w] = t[p];
+      fa_unpack_planes<KC>(v, t);
+#pragma unroll
+      for (int p = 0; p < 16; p++) lds[fa_slot(NH + P) * FA_ST16 + 4 * p + w] = t[p];
+      __syncthreads();
+      fa_outer<KC, true>(lds);
     }
     // the next tile's loads are issued before this tile's stores
     if (tile + G < ntiles) load_tile(tile + G);
+    tid = opaque_tid();
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const int f = tid + u * FA_NT;
+    for (int k = 0; k < 8; k++) {
+      const int f = tid + k * FA_NT;
+      const uint4 o = *(const uint4*)&lds[(INV ? fa_slot(f & (TC - 1)) : eslot(f >> 4)) * FA_ST16 +
+                                          (INV ? f >> FA_TL : f & 15) * 4];
       if constexpr (INV)
-        nout[fa_nat(a, elem(tile, f & (TC - 1)), h, f >> FA_TL)] = w[u];
+        *nptr(nout, tile, tid, k) = o;
       else
-        E[elem(tile, f >> 4) * 32 + 16 * h + (f & 15)] = w[u];
+        *eptr(tile, tid, k) = o;
     }
     __syncthreads();
   }
 }
 
 // ---- GF(2^32) passes: layers k < c ------------------------------------------------
-// A workgroup of 512 lanes holds a tile of 256 elements (2^R of them 2^lo apart
-// times 2^lgC consecutive ones) in registers: lane P * 4 + w has word w of the
-// two elements of butterfly P, all 32 planes of both.  Between layers a lane
-// gives one of the two to the lane whose P differs in the next layer's bit and
-// takes one: through LDS where that is another wavefront, by lane swaps inside
-// one.  Held in LDS (128 elements a tile, 256 lanes at 250 registers, every layer
+// Tiles of 2^R elements 2^lo apart times 2^(8-R) consecutive ones, all 32 planes.
+// Held in LDS (128 elements a tile, 256 lanes at 250 registers, every layer
 // reading and writing all of it), two wavefronts per SIMD waited half of the
 // time; registers hold twice the tile at four wavefronts, and three passes do
 // where five did.  At n = 2^24 the passes took 355 + 312 + 924 + 314 + 342 us, now
@@ -439,67 +515,6 @@ __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void
 // there are few) gain 3 to 4 % of an encode at n = 2^16 .. 2^17, 1 % at 2^18 and
 // lose from there on: not worth the second set of kernels.
 constexpr int FA_ST = 132;  // LDS words of a staged element: 32 planes x 4, 4 of padding
-
-// give u (where this lane's P has bit b set) or v to the lane whose P differs in
-// that bit and take the same from it
-// (N lanes further; the quads of a row whose bit is set are the BANKS)
-template <int N, int BANKS>
-__device__ __forceinline__ void fa_swap_dpp(uint32_t* u, uint32_t* v) {
-#pragma unroll
-  for (int p = 0; p < 32; p++) {
-    const int a = (int)u[p], b = (int)v[p];
-    u[p] = (uint32_t)__builtin_amdgcn_update_dpp(a, b, 0x110 | N, 0xF, BANKS, false);       // row_shr
-    v[p] = (uint32_t)__builtin_amdgcn_update_dpp(b, a, 0x100 | N, 0xF, 0xF ^ BANKS, false);  // row_shl
-  }
-}
-
-__device__ __forceinline__ void fa_swap_lds(uint32_t* lds, uint32_t* g, int other) {
-#pragma unroll
-  for (int p = 0; p < 32; p++) lds[p * FA_NT + threadIdx.x] = g[p];
-  __syncthreads();
-#pragma unroll
-  for (int p = 0; p < 32; p++) g[p] = lds[p * FA_NT + other];
-  __syncthreads();
-}
-
-__device__ __forceinline__ void fa_swap(uint32_t* lds, uint32_t* u, uint32_t* v, int P, int b) {
-  // (b opaque in between: as one chain of choices the compiler merges all ways
-  // behind 64 moves)
-#define FA_OPAQUE(x) \
-  x = __builtin_amdgcn_readfirstlane(x); \
-  asm volatile("" : "+s"(x))
-  if (b >= 4) {  // another wavefront; the bit is this one's
-    const int other = (int)threadIdx.x ^ (4 << b);
-    int bit = __builtin_amdgcn_readfirstlane(P >> b) & 1;
-    if (bit) fa_swap_lds(lds, u, other);
-    FA_OPAQUE(bit);
-    if (!bit) fa_swap_lds(lds, v, other);
-  }
-  FA_OPAQUE(b);
-  if (b == 3) {
-#pragma unroll
-    for (int p = 0; p < 32; p++) {
-      const auto r = __builtin_amdgcn_permlane32_swap(u[p], v[p], false, false);
-      u[p] = r[0];
-      v[p] = r[1];
-    }
-  }
-  FA_OPAQUE(b);
-  if (b == 2) {
-#pragma unroll
-    for (int p = 0; p < 32; p++) {
-      const auto r = __builtin_amdgcn_permlane16_swap(u[p], v[p], false, false);
-      u[p] = r[0];
-      v[p] = r[1];
-    }
-  }
-  FA_OPAQUE(b);
-  if (b == 1) fa_swap_dpp<8, 0xC>(u, v);
-  FA_OPAQUE(b);
-  if (b == 0) fa_swap_dpp<4, 0xA>(u, v);
-}
-
-CUOT_DEV int fa_insert(int P, int b, int r) { return ((P >> b) << (b + 1)) | (r << b) | (P & ((1 << b) - 1)); }
 
 template <int MODE, bool NAT>
 __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void fa_pass32(FaArgs a) {
@@ -533,7 +548,8 @@ __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void
     // natural order, word f = tid + NT k: element fastest, then coefficient (QB
     // bits) and half; else plane fastest, then element
     auto addr = [&](uint4* p, bool nat, int QB, int reg, int r, int tid, int k) {
-      const int fh = nat ? 4 * k : (NT >> 5) * k, fl = nat ? tid >> (TL - 1) : tid >> 5;  // the index above the fastest part
+      // the index above the fastest part
+      const int fh = nat ? 4 * k : (NT >> 5) * k, fl = nat ? tid >> (TL - 1) : tid >> 5;
       int64_t sc;
       uint32_t ln;
       if (nat) {
@@ -628,7 +644,7 @@ __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void
         }
       }
       FA_OPAQUE(sw);
-      fa_swap(lds, u, v, P, sw);
+      fa_swap<32>(lds, u, v, P, sw);
       const int k = a.lo + b - lgC;
       const uint32_t e = (uint32_t)eb + off(fa_insert(P, b, 0));
       const uint32_t g = ((e >> a.c) << (a.c - k)) | ((e & ((1u << a.c) - 1)) >> (k + 1));
@@ -640,7 +656,8 @@ __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void
       auto add_u = [&](bool now) {
         if constexpr (MODE == FA_FUSED) {
 #pragma unroll
-          for (int p = 0; p < 32; p++) asm("v_bitop3_b32 %0, %0, %1, %2 bitop3:0x78" : "+v"(v[p]) : "v"(u[p]), "s"(0 - (int)now));
+          for (int p = 0; p < 32; p++)
+            asm("v_bitop3_b32 %0, %0, %1, %2 bitop3:0x78" : "+v"(v[p]) : "v"(u[p]), "s"(0 - (int)now));
         } else if (now) {
 #pragma unroll
           for (int p = 0; p < 32; p++) v[p] ^= u[p];
@@ -725,8 +742,8 @@ __device__ __forceinline__ void fa_column_load(const SRC& in, int64_t base, int6
 
 // Bits B0 .. B0 + R - 1 of N coefficients, a column per lane.
 template <bool INV, bool SRC, int S, int R, int B0>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void fa_adic_level(const QcIo* __restrict__ io, QcIo io1, const uint4* __restrict__ in,
-                                                     uint4* __restrict__ out, int64_t XS, int64_t N) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void fa_adic_level(
+    const QcIo* __restrict__ io, QcIo io1, const uint4* __restrict__ in, uint4* __restrict__ out, int64_t XS, int64_t N) {
   constexpr int64_t U = (int64_t)1 << (B0 - S), NCOL = ((int64_t)1 << B0) - U, GROUP = (int64_t)1 << (B0 + R);
   constexpr int64_t per = (NCOL + 255) / 256;  // workgroups per group
   FaSrc src;
@@ -878,8 +895,8 @@ __global__ __launch_bounds__(FA_OT) __attribute__((amdgpu_waves_per_eu(2))) void
 constexpr int FA_CT = 256;
 
 template <bool INV, bool ROWS>
-__global__ __launch_bounds__(FA_CT) __attribute__((amdgpu_waves_per_eu(2))) void fa_conv_tile(const uint4* in, uint4* out,
-                                                                                              int64_t XS) {
+__global__ __launch_bounds__(FA_CT) __attribute__((amdgpu_waves_per_eu(2))) void fa_conv_tile(
+    const uint4* in, uint4* out, int64_t XS) {
   extern __shared__ uint4 sm[];
   const int tid = threadIdx.x, x = tid & 15, y = tid >> 4;
   const int64_t tile = blockIdx.x;
