@@ -250,8 +250,10 @@ def collect_counters():
             row["hbm_bytes_per_launch"] = round(tb)
             a = (algo or {}).get(k["base"])
             if a and a["launches"] and a["bytes"] > 0:
-                row["algorithmic_bytes_per_launch"] = round(a["bytes"] / a["launches"])
-                row["traffic_over_algorithmic"] = round(tb / (a["bytes"] / a["launches"]), 3)
+                # one recorded launch can be several kernels (the LPN's slices)
+                alg = a["bytes"] / max(a["launches"], sum(o["n0"] for o in table.values() if o["base"] == k["base"]))
+                row["algorithmic_bytes_per_launch"] = round(alg)
+                row["traffic_over_algorithmic"] = round(tb / alg, 3)
         out[full] = row
     note = (f"rocprofv3 --pmc, two passes over bench.py --counter-run; FETCH_SIZE x {fscale:.3f}, "
             f"WRITE_SIZE x {wscale:.3f} (KiB -> bytes, from the 256 MiB copy); VALU util = VALU instructions x 64 "
@@ -358,8 +360,7 @@ def cpu_baseline(threads: int):
     }
 
 
-QC_ENCODE_KERNELS = ("qc_pack_x", "transpose_fwd", "qc_conv_rows", "transpose_inv", "qc_fft_pass", "qc_unpack_x",
-                     "qc_rows_fold", "qc_output_planes", "qc_output")
+QC_ENCODE_KERNELS = ("fa_adic_level", "fa_conv_tile", "fa_pass16", "fa_pass32", "fa_output", "fa_output_adic")
 
 
 def qc_encode_bound(counters, qc_ms):
@@ -942,7 +943,8 @@ def main():
                 "hbm_frac_algorithmic": round(lk["algorithmic_GBps"] / HBM_PEAK_GBS, 4),
                 "algorithmic_bytes_per_launch": lk["algorithmic_bytes_per_launch"],
                 "bytes_per_row_per_role": 16 * 12,
-                "hbm_bytes_per_launch": lpn_row.get("hbm_bytes_per_launch") if lpn_row else None,
+                "hbm_bytes_per_launch": (lpn_row["hbm_bytes_per_launch"] * lpn_row["launches"]  # one per slice
+                                         if lpn_row and "hbm_bytes_per_launch" in lpn_row else None),
                 "traffic_over_algorithmic": lpn_row.get("traffic_over_algorithmic") if lpn_row else None,
                 "valu_util": lpn_row.get("valu_util") if lpn_row else None,
             }

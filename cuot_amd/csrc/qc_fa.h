@@ -96,7 +96,7 @@ static inline void fa_basis(uint32_t beta[32]) {
 // beta_{a-k}: four bits (three in a half-length input) are one GF(2^16) value.
 // kc = 0 for K <= 20, K - 20 above.
 struct FaChunk {
-  uint32_t pack[16];    // value of chunk bit pattern 1 << q ... pack[q] = product over the bits b of q of beta_{a-(K-4+b)}
+  uint32_t pack[16];    // pack[q] = product over the bits b of q of beta_{a-(K-4+b)}
   uint32_t unpack[16];  // bit j of unpack[q]: coordinate j contributes to coefficient q
 };
 
@@ -215,11 +215,16 @@ struct FaOp {
 #define FA_ADD3(a, x, y) "v_bitop3_b32 " a ", " a ", " x ", " y " bitop3:0x96\n"
 #define FA_SET2(a, x) "v_mov_b32 " a ", " x "\n"
 #define FA_SET3(a, x, y) "v_xor_b32 " a ", " x ", " y "\n"
-#define FA_CASE(D, X2, X3)                                                                                           \
-  "FA" #D "_%=:\n" FA_D##D(X2, X3, "%[a0]", "%[a1]", "%[a2]", "%[a3]", "%[p0]", "%[p1]", "%[p2]", "%[p3]", "%[l0]", "%[h0]") \
-      FA_D##D(X2, X3, "%[a4]", "%[a5]", "%[a6]", "%[a7]", "%[p4]", "%[p5]", "%[p6]", "%[p7]", "%[l1]", "%[h1]") \
-      FA_D##D(X2, X3, "%[a8]", "%[a9]", "%[a10]", "%[a11]", "%[p8]", "%[p9]", "%[p10]", "%[p11]", "%[l2]", "%[h2]") \
-      FA_D##D(X2, X3, "%[a12]", "%[a13]", "%[a14]", "%[a15]", "%[p12]", "%[p13]", "%[p14]", "%[p15]", "%[l3]", "%[h3]") \
+#define FA_CASE(D, X2, X3) \
+  "FA" #D "_%=:\n" \
+  FA_D##D(X2, X3, "%[a0]", "%[a1]", "%[a2]", "%[a3]", "%[p0]", "%[p1]", "%[p2]", "%[p3]", \
+          "%[l0]", "%[h0]") \
+  FA_D##D(X2, X3, "%[a4]", "%[a5]", "%[a6]", "%[a7]", "%[p4]", "%[p5]", "%[p6]", "%[p7]", \
+          "%[l1]", "%[h1]") \
+  FA_D##D(X2, X3, "%[a8]", "%[a9]", "%[a10]", "%[a11]", "%[p8]", "%[p9]", "%[p10]", "%[p11]", \
+          "%[l2]", "%[h2]") \
+  FA_D##D(X2, X3, "%[a12]", "%[a13]", "%[a14]", "%[a15]", "%[p12]", "%[p13]", "%[p14]", "%[p15]", \
+          "%[l3]", "%[h3]") \
   "s_branch FAend_%=\n"
 #define FA_BIT(B, ONE) "s_bitcmp1_b32 %[d], " #B "\ns_cbranch_scc1 FA" #ONE "_%=\n"
 #define FA_CASES(X2, X3)                                                                                            \
@@ -234,10 +239,22 @@ struct FaOp {
   "FAt14_%=:\n" FA_BIT(0, 15) FA_CASE(14, X2, X3) FA_CASE(15, X2, X3) "FAend_%=:\n"
 #define FA_ADD2_ZERO
 #define FA_SET2_ZERO \
-  "v_mov_b32 %[a0], 0\n" "v_mov_b32 %[a1], 0\n" "v_mov_b32 %[a2], 0\n" "v_mov_b32 %[a3], 0\n" "v_mov_b32 %[a4], 0\n" "v_mov_b32 %[a5], 0\n" "v_mov_b32 %[a6], 0\n" "v_mov_b32 %[a7], 0\n" "v_mov_b32 %[a8], 0\n" "v_mov_b32 %[a9], 0\n" "v_mov_b32 %[a10], 0\n" "v_mov_b32 %[a11], 0\n" "v_mov_b32 %[a12], 0\n" "v_mov_b32 %[a13], 0\n" "v_mov_b32 %[a14], 0\n" "v_mov_b32 %[a15], 0\n"
-#define FA_OPERANDS(C)                                                                                              \
-  [a0] C(a[0]), [a1] C(a[1]), [a2] C(a[2]), [a3] C(a[3]), [a4] C(a[4]), [a5] C(a[5]), [a6] C(a[6]), [a7] C(a[7]), [a8] C(a[8]), [a9] C(a[9]), [a10] C(a[10]), [a11] C(a[11]), [a12] C(a[12]), [a13] C(a[13]), [a14] C(a[14]), [a15] C(a[15]) \
-      : [p0] "v"(v.p[0]), [p1] "v"(v.p[1]), [p2] "v"(v.p[2]), [p3] "v"(v.p[3]), [p4] "v"(v.p[4]), [p5] "v"(v.p[5]), [p6] "v"(v.p[6]), [p7] "v"(v.p[7]), [p8] "v"(v.p[8]), [p9] "v"(v.p[9]), [p10] "v"(v.p[10]), [p11] "v"(v.p[11]), [p12] "v"(v.p[12]), [p13] "v"(v.p[13]), [p14] "v"(v.p[14]), [p15] "v"(v.p[15]), [l0] "v"(v.lo[0]), [h0] "v"(v.hi[0]), [l1] "v"(v.lo[1]), [h1] "v"(v.hi[1]), [l2] "v"(v.lo[2]), [h2] "v"(v.hi[2]), [l3] "v"(v.lo[3]), [h3] "v"(v.hi[3]), [d] "s"(d) \
+  "v_mov_b32 %[a0], 0\n" "v_mov_b32 %[a1], 0\n" "v_mov_b32 %[a2], 0\n" "v_mov_b32 %[a3], 0\n" \
+  "v_mov_b32 %[a4], 0\n" "v_mov_b32 %[a5], 0\n" "v_mov_b32 %[a6], 0\n" "v_mov_b32 %[a7], 0\n" \
+  "v_mov_b32 %[a8], 0\n" "v_mov_b32 %[a9], 0\n" "v_mov_b32 %[a10], 0\n" "v_mov_b32 %[a11], 0\n" \
+  "v_mov_b32 %[a12], 0\n" "v_mov_b32 %[a13], 0\n" "v_mov_b32 %[a14], 0\n" "v_mov_b32 %[a15], 0\n"
+#define FA_OPERANDS(C) \
+  [a0] C(a[0]), [a1] C(a[1]), [a2] C(a[2]), [a3] C(a[3]), \
+  [a4] C(a[4]), [a5] C(a[5]), [a6] C(a[6]), [a7] C(a[7]), \
+  [a8] C(a[8]), [a9] C(a[9]), [a10] C(a[10]), [a11] C(a[11]), \
+  [a12] C(a[12]), [a13] C(a[13]), [a14] C(a[14]), [a15] C(a[15]) \
+      : [p0] "v"(v.p[0]), [p1] "v"(v.p[1]), [p2] "v"(v.p[2]), [p3] "v"(v.p[3]), \
+        [p4] "v"(v.p[4]), [p5] "v"(v.p[5]), [p6] "v"(v.p[6]), [p7] "v"(v.p[7]), \
+        [p8] "v"(v.p[8]), [p9] "v"(v.p[9]), [p10] "v"(v.p[10]), [p11] "v"(v.p[11]), \
+        [p12] "v"(v.p[12]), [p13] "v"(v.p[13]), [p14] "v"(v.p[14]), [p15] "v"(v.p[15]), \
+        [l0] "v"(v.lo[0]), [h0] "v"(v.hi[0]), [l1] "v"(v.lo[1]), [h1] "v"(v.hi[1]), \
+        [l2] "v"(v.lo[2]), [h2] "v"(v.hi[2]), [l3] "v"(v.lo[3]), [h3] "v"(v.hi[3]), \
+        [d] "s"(d) \
       : "scc"
 #define FA_OUT(x) "=&v"(x)
 #define FA_INOUT(x) "+&v"(x)

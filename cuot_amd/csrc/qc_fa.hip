@@ -1208,7 +1208,7 @@ void fa_launch32(const FaArgs& a, int B, hipStream_t st) {
   // two resident workgroups on each of the 256 CUs; every one walks many tiles
   const int64_t cap = 512 / B < 1 ? 1 : 512 / B;
   const double per = 512.0 * (double)((int64_t)1 << (a.K - 5)) * B;
-  cuot_rec_begin(st, MODE == FA_FUSED ? "fa_pass32 fused" : "fa_pass32", NAT && MODE == FA_FWD ? per * 1.5 : per * 2.0);
+  cuot_rec_begin(st, "fa_pass32", NAT && MODE == FA_FWD ? per * 1.5 : per * 2.0);
   hipLaunchKernelGGL((fa_pass32<MODE, NAT>), dim3(capg(ntiles, cap), (unsigned)B), dim3(FA_NT), FA_LDS32, st, a);
   cuot_rec_end(st);
 }
@@ -1383,7 +1383,7 @@ hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ah
     if ((e = cuot_launch_conv_rows(8192, st, (uint32_t*)Y, words, 128ll * B, 128, XS * 4, K, 1))) return e;
     if ((e = cuot_launch_transpose_planes2(Y, XS, X, true, B, 1, XS * 4, 128 * words, XS, XS, st))) return e;
   }
-  cuot_rec_begin(st, "fa_output", 48.0 * (double)nmax * B);
+  cuot_rec_begin(st, K > 16 ? "fa_output_adic" : "fa_output", 48.0 * (double)nmax * B);
   switch (K - 16) {
     default:
       hipLaunchKernelGGL(fa_output, dim3(capg((nmax + 255) / 256, 16384), (unsigned)B), dim3(256), 0, st, X, XS, io, io1);
