@@ -53,9 +53,15 @@ __constant__ uint2 c_fa_beta[32];  // beta_i and nu times its theta part
 __constant__ uint32_t c_fa_pack[FA_KC_MAX + 1][8];
 
 constexpr int FA_KMIN = 14, FA_KMAX = 25;
-// longest string of a's bits converted in LDS: 36 KB padded, so that a workgroup
-// fits beside the trees' (2^20 bits at a time waited for a whole CU's LDS)
-constexpr int FA_STR = 18;
+// Log2 of the strings of a's bits that are converted in LDS.  A run prepares A^
+// beside the receiver's trees, which from n = 2^19 on have a workgroup on every
+// CU; 1024 lanes need the registers of a whole CU and wait for its trees to end:
+// at n = 2^20 strings of 2^18 bits took 83 us there, 23 alone.  K > 20: strings of
+// 2^16 bits on 512 lanes, which fit beside a tree (31 us there; the added level
+// launches cost 3 of 73 us where A^ is prepared alone): run of n = 2^20 607 ->
+// 580 us, 2^21 1091 -> 1015, 2^24 8660 -> 8480.  K <= 20: the trees mostly leave CUs
+// free, and the launches or half the lanes cost what they save (n = 300000 367 -> 375).
+constexpr int fa_str(int K) { return K > 20 ? 16 : K > 19 ? 18 : K - 1; }
 
 CUOT_DEV uint4 x4(uint4 a, uint4 b) { return make_uint4(a.x ^ b.x, a.y ^ b.y, a.z ^ b.z, a.w ^ b.w); }
 CUOT_DEV uint4 z4() { return make_uint4(0, 0, 0, 0); }
@@ -1006,14 +1012,15 @@ struct FaSync {
 
 // levels below 2^mp on each string of 2^mp bits, in place (one workgroup each)
 __global__ __launch_bounds__(1024) void fa_prep_rows(const QcPrep* __restrict__ pr, QcPrep pr1, int K, int mp) {
+  const int nl = (int)blockDim.x;
   extern __shared__ uint32_t sw[];
   const QcPrep q = pr ? pr[blockIdx.y] : pr1;
   const int64_t nw = (int64_t)1 << (mp - 5);
   uint32_t* g = q.ahat + ((int64_t)1 << (K - 5)) + (int64_t)blockIdx.x * nw;
-  for (int64_t i = threadIdx.x; i < nw; i += 1024) sw[cbp_at<true>(i)] = g[i];
+  for (int64_t i = threadIdx.x; i < nw; i += nl) sw[cbp_at<true>(i)] = g[i];
   __syncthreads();
-  cbp_convert<true, false>(sw, 0, mp, threadIdx.x, 1024, FaSync());
-  for (int64_t i = threadIdx.x; i < nw; i += 1024) g[i] = sw[cbp_at<true>(i)];
+  cbp_convert<true, false>(sw, 0, mp, threadIdx.x, nl, FaSync());
+  for (int64_t i = threadIdx.x; i < nw; i += nl) g[i] = sw[cbp_at<true>(i)];
 }
 
 constexpr int FA_PT = 10;  // log2 words of a preparation tile
@@ -1149,9 +1156,6 @@ hipError_t fa_configure() {
   if (!e) e = fa_allow_lds16<3>();
   if (!e) e = fa_allow_lds16<4>();
   if (!e) e = fa_allow_lds16<5>();
-  if (!e)
-    e = hipFuncSetAttribute((const void*)fa_prep_rows, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)cbp_words(32 * 1024, true) * 4);
   if (!e) g_fa_ready = 1;
   return e;
 }
@@ -1280,7 +1284,8 @@ hipError_t cuot_launch_qc_fa_prepare(const QcPrep* pr, QcPrep pr1, int B, int K,
   const int c = K - 5 < 15 ? K - 5 : 15, aidx = 16 + c;
   const int64_t nw = (int64_t)1 << (K - 6);
   hipLaunchKernelGGL(fa_prep_bits, dim3(capg(nw / 256, 1024), (unsigned)B), dim3(256), 0, st, pr, pr1, K);
-  for (int k = K - 2; k >= FA_STR; k--) {
+  const int mp = fa_str(K);
+  for (int k = K - 2; k >= mp; k--) {
     const dim3 grid(capg(nw / 512, 1024), (unsigned)B);
     switch (k) {
 #define FA_CASE(KL)                                                                     \
@@ -1288,6 +1293,8 @@ hipError_t cuot_launch_qc_fa_prepare(const QcPrep* pr, QcPrep pr1, int B, int K,
     hipLaunchKernelGGL((fa_prep_level<KL, false>), grid, dim3(256), 0, st, pr, pr1, K); \
     hipLaunchKernelGGL((fa_prep_level<KL, true>), grid, dim3(256), 0, st, pr, pr1, K);  \
     break;
+      FA_CASE(16)
+      FA_CASE(17)
       FA_CASE(18)
       FA_CASE(19)
       FA_CASE(20)
@@ -1297,9 +1304,9 @@ hipError_t cuot_launch_qc_fa_prepare(const QcPrep* pr, QcPrep pr1, int B, int K,
 #undef FA_CASE
     }
   }
-  const int mp = K - 1 < FA_STR ? K - 1 : FA_STR;
-  hipLaunchKernelGGL(fa_prep_rows, dim3(1u << (K - 1 - mp), (unsigned)B), dim3(1024),
-                     (size_t)cbp_words((int64_t)1 << (mp - 5), true) * 4, st, pr, pr1, K, mp);
+  const dim3 strings(1u << (K - 1 - mp), (unsigned)B);
+  const size_t lds = (size_t)cbp_words((int64_t)1 << (mp - 5), true) * 4;
+  hipLaunchKernelGGL(fa_prep_rows, strings, dim3(K > 20 ? 512 : 1024), lds, st, pr, pr1, K, mp);
   const int bits = K - 5;
   const int Rl = bits < FA_PT ? bits : FA_PT, Ru = bits - Rl;
   if (Ru > 0)
