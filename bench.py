@@ -360,7 +360,8 @@ def cpu_baseline(threads: int):
     }
 
 
-QC_ENCODE_KERNELS = ("fa_adic_level", "fa_conv_tile", "fa_pass16", "fa_pass32", "fa_output", "fa_output_adic")
+QC_ENCODE_KERNELS = ("fa_adic_level", "fa_conv_tile", "fa_pass16", "fa_pass32", "fa_output", "fa_output_adic",
+                     "fa_output_cyclic")
 
 
 def qc_encode_bound(counters, qc_ms):

@@ -735,6 +735,34 @@ struct FaSrc {
   __device__ __forceinline__ uint4 operator[](int64_t i) const { return i < n ? p[i] : make_uint4(0, 0, 0, 0); }
 };
 
+// The product's 2n coefficients (in p, digits of powers of s_16 of 2^16 coefficients
+// each, before the levels of bits 16 up) folded to n = 2^(K-1): with e = n / 2^16,
+// s_16^e = x^n + x^e, so modulo x^n + 1 the upper half h counts 1 + x^e times.  In
+// the digits, x^e h is h rotated by e and, for a digit's last e coefficients,
+// which x^(2^16) = s_16 + x carries into the next digit, once more one further in
+// their own; the last digit's carry is 1 + x^e again.  EDGE: with what falls on a
+// digit's first coefficients; the others' is the rotation alone.
+template <typename V, int PARTS, bool EDGE>
+struct FaFold {
+  const V* p;
+  int64_t n, e;
+  __device__ __forceinline__ V operator[](int64_t i) const {
+    V v = p[i * PARTS];
+    fa_add(v, p[(n + i) * PARTS]);
+    fa_add(v, p[(n + ((i - e) & (n - 1))) * PARTS]);
+    if (EDGE) {
+      const int64_t j = i & 65535;
+      if (j >= 1 && j <= e) fa_add(v, p[(n + i + 65535 - e) * PARTS]);
+      if (i >= e && i < 2 * e) fa_add(v, p[(2 * n - 2 * e + i) * PARTS]);
+    }
+    return v;
+  }
+};
+
+// columns of 2^16 - 1 from here on hold no coefficient below 2e of a digit (element
+// T of column c is coefficient c - T or, for c < T, one of the digit before)
+__device__ __forceinline__ int64_t fa_fold_edge(int64_t n) { return (n >> 15) + 32; }
+
 // elements FROM .. 2^R of column c of the group at base (the last one, beyond
 // the group for most columns, only with EDGE)
 template <int R, bool EDGE, int FROM = 0, typename SRC, typename V>
@@ -746,14 +774,16 @@ __device__ __forceinline__ void fa_column_load(const SRC& in, int64_t base, int6
   if (EDGE && c + (ncol << R) < group) v[1 << R] = in[base + c + (ncol << R)];
 }
 
-// Bits B0 .. B0 + R - 1 of N coefficients, a column per lane.
-template <bool INV, bool SRC, int S, int R, int B0>
+// Bits B0 .. B0 + R - 1 of N coefficients, a column per lane; from a buffer, x or a
+// buffer of 2N folded.
+enum { FA_BUF, FA_X, FA_FOLD };
+template <bool INV, int SRC, int S, int R, int B0>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void fa_adic_level(
     const QcIo* __restrict__ io, QcIo io1, const uint4* __restrict__ in, uint4* __restrict__ out, int64_t XS, int64_t N) {
   constexpr int64_t U = (int64_t)1 << (B0 - S), NCOL = ((int64_t)1 << B0) - U, GROUP = (int64_t)1 << (B0 + R);
   constexpr int64_t per = (NCOL + 255) / 256;  // workgroups per group
   FaSrc src;
-  if (SRC) {
+  if (SRC == FA_X) {
     const QcIo q = io ? io[blockIdx.y] : io1;
     src.p = q.x + q.n;
     src.n = q.n;
@@ -766,12 +796,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   const int64_t base = (int64_t)(blockIdx.x / per) << (B0 + R);
   if (c >= NCOL) return;
   uint4 v[(1 << R) + 1];
-  if (c0 < U << R) {
-    fa_column_load<R, true>(src, base, c, NCOL, GROUP, v);
+  if (c0 < U << R || (SRC == FA_FOLD && c0 < fa_fold_edge(N))) {
+    if constexpr (SRC == FA_FOLD)
+      fa_column_load<R, true>(FaFold<uint4, 1, true>{src.p, N, N >> 16}, base, c, NCOL, GROUP, v);
+    else
+      fa_column_load<R, true>(src, base, c, NCOL, GROUP, v);
     fa_column_levels<INV, R, true>(v, (int)(c / U));
     if (c < U << R) dst[base + c + (NCOL << R)] = v[1 << R];
   } else {
-    fa_column_load<R, false>(src, base, c, NCOL, GROUP, v);
+    if constexpr (SRC == FA_FOLD)
+      fa_column_load<R, false>(FaFold<uint4, 1, false>{src.p, N, N >> 16}, base, c, NCOL, GROUP, v);
+    else
+      fa_column_load<R, false>(src, base, c, NCOL, GROUP, v);
     fa_column_levels<INV, R, false>(v, 0);
   }
 #pragma unroll
@@ -887,6 +923,48 @@ __global__ __launch_bounds__(FA_OT) __attribute__((amdgpu_waves_per_eu(2))) void
     fa_output_column<R, B0, true>(h, x, y, q.n, c, c2, up, second);
   else
     fa_output_column<R, B0, false>(h, x, y, q.n, c, c2, up, second);
+}
+
+// The same for n = 2^(K-1), H folded to n coefficients (or FOLD: still to be): one
+// column a lane gives its outputs, no column is worked out twice.  At n = 2^24 the
+// folding level and this take 175 + 172 us, the level and the output above 204 + 291
+// (of which x and y are 107 at the copy rate).
+template <int R, int B0, bool FOLD>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void fa_output_cyclic(
+    const uint4* __restrict__ H, QcIo q) {
+  using V = typename FaOut<R>::V;
+  constexpr int PARTS = FaOut<R>::PARTS;
+  constexpr int64_t U = (int64_t)1 << (B0 - 16), NCOL = ((int64_t)1 << B0) - U, GROUP = (int64_t)1 << (B0 + R);
+  const int part = threadIdx.x % PARTS;
+  const int64_t c0 = (int64_t)blockIdx.x * (256 / PARTS), c = c0 + threadIdx.x / PARTS;
+  if (c >= NCOL) return;
+  FaOut<R> h, x;
+  h.p = (const V*)H + part;
+  x.p = (const V*)q.x + part;
+  V* y = (V*)q.y + part;
+  V v[(1 << R) + 1];
+  if (c0 < U << R || (FOLD && c0 < fa_fold_edge(GROUP))) {
+    if constexpr (FOLD)
+      fa_column_load<R, true>(FaFold<V, PARTS, true>{h.p, GROUP, GROUP >> 16}, 0, c, NCOL, GROUP, v);
+    else
+      fa_column_load<R, true>(h, 0, c, NCOL, GROUP, v);
+    fa_column_levels<true, R, true>(v, (int)(c / U));
+  } else {
+    if constexpr (FOLD)
+      fa_column_load<R, false>(FaFold<V, PARTS, false>{h.p, GROUP, GROUP >> 16}, 0, c, NCOL, GROUP, v);
+    else
+      fa_column_load<R, false>(h, 0, c, NCOL, GROUP, v);
+    fa_column_levels<true, R, false>(v, 0);
+  }
+#pragma unroll
+  for (int T = 0; T <= (1 << R); T++) {
+    const int64_t i = c + T * NCOL;
+    if (i < GROUP) {
+      V o = x[i];
+      fa_add(o, v[T]);
+      y[i * PARTS] = o;
+    }
+  }
 }
 
 // ---- conversion of 2^16 coefficients on blocks (K > 16) --------------------------------
@@ -1168,7 +1246,7 @@ int fa_log(int64_t n) {  // K: 2^(K-1) >= n
 
 unsigned capg(int64_t v, int64_t cap) { return (unsigned)(v < 1 ? 1 : (v > cap ? cap : v)); }
 
-template <bool INV, bool SRC, int S, int R, int B0>
+template <bool INV, int SRC, int S, int R, int B0>
 void fa_launch_level(const QcIo* io, QcIo io1, const uint4* in, uint4* out, int64_t XS, int64_t N, int B,
                      hipStream_t st) {
   const int64_t wgs = (N >> (B0 + R)) * ((((int64_t)1 << B0) - ((int64_t)1 << (B0 - S)) + 255) / 256);
@@ -1333,12 +1411,12 @@ hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ah
     switch (K - 17) {
 #define FA_CASE(R)                                                                        \
   case R:                                                                                 \
-    fa_launch_level<false, true, 16, R, 16>(io, io1, nullptr, X, XS, Nin, B, st);        \
+    fa_launch_level<false, FA_X, 16, R, 16>(io, io1, nullptr, X, XS, Nin, B, st);        \
     break;
 #define FA_CASE2(R)                                                                       \
   case 4 + R:                                                                             \
-    fa_launch_level<false, true, 16, R, 20>(io, io1, nullptr, Y, XS, Nin, B, st);        \
-    fa_launch_level<false, false, 16, 4, 16>(io, io1, Y, X, XS, Nin, B, st);             \
+    fa_launch_level<false, FA_X, 16, R, 20>(io, io1, nullptr, Y, XS, Nin, B, st);        \
+    fa_launch_level<false, FA_BUF, 16, 4, 16>(io, io1, Y, X, XS, Nin, B, st);             \
     break;
       FA_CASE(1)
       FA_CASE(2)
@@ -1352,9 +1430,9 @@ hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ah
 #undef FA_CASE2
     }
     if (K == 17)
-      fa_launch_level<false, true, 8, 4, 12>(io, io1, nullptr, Y, XS, Nin, B, st);
+      fa_launch_level<false, FA_X, 8, 4, 12>(io, io1, nullptr, Y, XS, Nin, B, st);
     else
-      fa_launch_level<false, false, 8, 4, 12>(io, io1, X, Y, XS, Nin, B, st);
+      fa_launch_level<false, FA_BUF, 8, 4, 12>(io, io1, X, Y, XS, Nin, B, st);
     fa_launch_conv<false, false>(Y, X, XS, Nin, B, st);
     fa_launch_conv<false, true>(X, X, XS, Nin, B, st);
   } else {
@@ -1378,20 +1456,29 @@ hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ah
   a.c = K - 5 < 15 ? K - 5 : 15;
   a.a = 16 + a.c;
   if ((e = fa_transform(a, B, st, ready))) return e;
-  // inverse conversion of the 2^K coefficients in X
+  // inverse conversion of the 2^K coefficients in X, for one n = 2^(K-1) folded
+  // to n of them before the levels of bits 16 up.  Encode, general form -> folded:
+  // n = 2^24 3505 -> 3357 us, 2^23 1647 -> 1581, 2^22 806 -> 783, 2^21 406 -> 403; 2^20 266
+  // -> 269 and 2^19, 2^18 the same, where the output is short either way.  A batch's
+  // members differ in n and take the general form.
+  const bool cyclic = K > 21 && !io && io1.n == Nin;
   if (adic) {
     fa_launch_conv<true, true>(X, X, XS, XS, B, st);
     fa_launch_conv<true, false>(X, Y, XS, XS, B, st);
-    fa_launch_level<true, false, 8, 4, 12>(io, io1, Y, X, XS, XS, B, st);
-    if (K > 21) fa_launch_level<true, false, 16, 4, 16>(io, io1, X, Y, XS, XS, B, st);
+    fa_launch_level<true, FA_BUF, 8, 4, 12>(io, io1, Y, X, XS, XS, B, st);
+    if (cyclic) {
+      if (K > 22) fa_launch_level<true, FA_FOLD, 16, 4, 16>(io, io1, X, Y, XS, XS / 2, B, st);
+    } else if (K > 21) {
+      fa_launch_level<true, FA_BUF, 16, 4, 16>(io, io1, X, Y, XS, XS, B, st);
+    }
   } else {
     const int64_t words = XS / 32;
     if ((e = cuot_launch_transpose_planes2(X, XS, Y, false, B, 1, XS, XS, XS * 4, 128 * words, st))) return e;
     if ((e = cuot_launch_conv_rows(8192, st, (uint32_t*)Y, words, 128ll * B, 128, XS * 4, K, 1))) return e;
     if ((e = cuot_launch_transpose_planes2(Y, XS, X, true, B, 1, XS * 4, 128 * words, XS, XS, st))) return e;
   }
-  cuot_rec_begin(st, K > 16 ? "fa_output_adic" : "fa_output", 48.0 * (double)nmax * B);
-  switch (K - 16) {
+  cuot_rec_begin(st, cyclic ? "fa_output_cyclic" : adic ? "fa_output_adic" : "fa_output", 48.0 * (double)nmax * B);
+  switch (cyclic ? K : K - 16) {
     default:
       hipLaunchKernelGGL(fa_output, dim3(capg((nmax + 255) / 256, 16384), (unsigned)B), dim3(256), 0, st, X, XS, io, io1);
       break;
@@ -1409,6 +1496,15 @@ hipError_t cuot_launch_qc_fa_encode(const QcIo* io, QcIo io1, const uint32_t* ah
     FA_CASE(7, 3, 20, Y)
     FA_CASE(8, 4, 20, Y)
     FA_CASE(9, 5, 20, Y)
+#undef FA_CASE
+#define FA_CASE(N, R, B0, FOLD, SRC)                                                                                 \
+  case N:                                                                                                            \
+    hipLaunchKernelGGL((fa_output_cyclic<R, B0, FOLD>), dim3((FaOut<R>::PARTS << B0) / 256), dim3(256), 0, st, SRC, io1); \
+    break;
+    FA_CASE(22, 5, 16, true, X)
+    FA_CASE(23, 2, 20, false, Y)
+    FA_CASE(24, 3, 20, false, Y)
+    FA_CASE(25, 4, 20, false, Y)
 #undef FA_CASE
   }
   cuot_rec_end(st);

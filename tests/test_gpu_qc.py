@@ -227,6 +227,13 @@ def test_qc_columns_rotations(ctx, knob_mfma, n):
     test_qc_orbit_product_rotations(ctx, knob_mfma, n)
 
 
+# n a power of two from 2^21 on: folded before the upper levels, one form of the
+# output each (2^20: the general one)
+@pytest.mark.parametrize("lg", [20, 21, 22, 23, 24])
+def test_qc_cyclic_fold_rotations(ctx, knob_mfma, lg):
+    test_qc_orbit_product_rotations(ctx, knob_mfma, 1 << lg)
+
+
 # fewer layers per upper pass: several passes, tiles of 2^2 .. 2^5 rows
 @pytest.mark.parametrize("radix", [2, 3, 5])
 @pytest.mark.parametrize("n", [70001, (1 << 20) + 1])
