@@ -972,10 +972,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 // steps exchanging through LDS.  ROWS: the outer bits 8 .. 15, 256 rows 256 apart
 // times 16 consecutive columns; else 4096 consecutive blocks, the s_8-adic levels
 // of bits 8 .. 11 (those of 12 .. 15: fa_adic_level) and the bits below 8.
-// Memory is the bound: 2^24 blocks in 108 us and, ROWS, 88.  As strings of bits, transposed there and back, the
-// 16 bits took 531 us for 2^24 coefficients and 971 back for 2^25, level by level
-// on blocks in LDS (tiles of 512 lanes, two barriers a level) 387 and 677 with bits
-// 12 .. 15.
+// Memory is the bound: 2^24 blocks in 108 us and, ROWS, 88; back 2^25 in 226 and
+// 171 (with the next tile's blocks fetched ahead 225, and ROWS spills).  As strings
+// of bits, transposed there and back, the 16 bits took 531 us for 2^24 coefficients
+// and 971 back for 2^25, level by level on blocks in LDS (tiles of 512 lanes, two
+// barriers a level) 387 and 677 with bits 12 .. 15.
 constexpr int FA_CT = 256;
 
 template <bool INV, bool ROWS>
