@@ -350,13 +350,15 @@ hipError_t launch_all(cuot_batch* b, uint32_t stages, hipStream_t st, hipStream_
     if ((e = hipStreamWaitEvent(ax, ev[0], 0))) return e;
     sp = ax;
   }
-  if (stages & CUOT_BATCH_STAGE_QC_PREPARE)
+  if (stages & (CUOT_BATCH_STAGE_QC_PREPARE | CUOT_BATCH_STAGE_QC))
     for (const PrepGroup& pg : b->prep) {
       // a whole run whose encodes of this length all take the matrix cores
-      // needs only the bits of a
+      // needs only the bits of a; an encode stage by itself may then have to
+      // prepare A^ first
       int64_t nmax = 0;
       for (int i : pg.members) nmax = std::max(nmax, b->inst[i].n);
-      const bool transform = stages != CUOT_BATCH_STAGE_ALL || !cuot_qc_mfma_selected(nmax);
+      if (!(stages & CUOT_BATCH_STAGE_QC_PREPARE) && !cuot_qc_ahat_late(nmax)) continue;
+      const bool transform = stages != CUOT_BATCH_STAGE_ALL || !cuot_qc_ahat_left_out(nmax);
       if ((e = cuot_launch_qc_prepare_batch((const QcPrep*)(ws + pg.off), (int)pg.members.size(), pg.m, transform,
                                             sp)))
         return e;

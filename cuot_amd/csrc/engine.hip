@@ -295,7 +295,10 @@ extern "C" int cuot_sot_run_stages(cuot_ctx* ctx, const cuot_sot_config* cfg, vo
   CUOT_HIP_TRY(hipSetDevice(ctx->device));
   hipStream_t st = ctx->st(stream);
   if (stages & CUOT_SOT_STAGE_SETUP) CUOT_HIP_TRY(p.run_setup((blk*)delta_d, st));
-  if (stages & CUOT_SOT_STAGE_QC_PREPARE) CUOT_HIP_TRY(p.run_prepare(true, st));
+  // (a whole run may have left A^ out)
+  if ((stages & CUOT_SOT_STAGE_QC_PREPARE) ||
+      ((stages & (CUOT_SOT_STAGE_QC_SENDER | CUOT_SOT_STAGE_QC_RECVER)) && cuot_qc_ahat_late(p.cfg.n)))
+    CUOT_HIP_TRY(p.run_prepare(true, st));
   if (stages & CUOT_SOT_STAGE_GGM_SENDER) CUOT_HIP_TRY(p.run_expand_sender(st));
   if (stages & CUOT_SOT_STAGE_GGM_RECVER) CUOT_HIP_TRY(p.run_expand_recver(st));
   if (stages & CUOT_SOT_STAGE_QC_SENDER)
@@ -339,9 +342,10 @@ extern "C" int cuot_sot_run(cuot_ctx* ctx, const cuot_sot_config* cfg, void* ws_
   CUOT_HIP_TRY(hipEventRecord(e_rows, st));
   CUOT_HIP_TRY(hipStreamWaitEvent(ax, e_rows, 0));
   CUOT_HIP_TRY(p.run_expand_recver(ax));
-  // both encodes follow in this call: when they take the matrix cores, A^ is
-  // not needed (its 33 small launches took 95 us beside n = 2^14's 45 us encodes)
-  CUOT_HIP_TRY(p.run_prepare(!cuot_qc_mfma_selected(p.cfg.n), st));
+  // both encodes follow in this call: when they take the matrix cores, A^ is not
+  // needed.  Preparing it beside the sender's trees all the same took (run without
+  // -> with it, us) n = 1000 86 -> 146, 24000 177 -> 212, 36000 289 -> 319, 2^14 137 -> 137.
+  CUOT_HIP_TRY(p.run_prepare(!cuot_qc_ahat_left_out(p.cfg.n), st));
   CUOT_HIP_TRY(hipEventRecord(e_prep, st));
   CUOT_HIP_TRY(cuot_launch_qc_encode(p.ahat, p.cfg.n, p.leaves_s, (blk*)v_d, p.qc_scratch, st));
   CUOT_HIP_TRY(cuot_launch_qc_encode(p.ahat, p.cfg.n, p.leaves_r, (blk*)w_d, p.qc_scratch2, ax, e_prep));

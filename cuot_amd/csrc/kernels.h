@@ -84,7 +84,7 @@ hipError_t cuot_launch_lpn_batch(const void* tabs_d, const int64_t* wg_start_d, 
 int cuot_qc_log_len(int64_t n);
 size_t cuot_qc_scratch_bytes_for(int64_t n);
 // transform = false: only a's bits for the matrix-core encoder, for callers
-// whose encodes run in the same call and take it (cuot_qc_mfma_selected)
+// whose encodes run in the same call (cuot_qc_ahat_left_out)
 hipError_t cuot_launch_qc_prepare(const uint8_t* a_bits, int64_t n, uint32_t* ahat, void* scratch, bool transform,
                                   hipStream_t st);
 // ready: A^ is complete at this event (of another stream; NULL: already in st's order)
@@ -127,6 +127,13 @@ hipError_t cuot_launch_conv_rows(unsigned cap, hipStream_t st, uint32_t* Bw, int
 bool cuot_qc_mfma_eligible(int64_t n);
 bool cuot_qc_mfma_selected(int64_t n);  // eligible and at or below the crossover knob
 int64_t cuot_qc_mfma_limit();           // the crossover in force (knob or built-in)
+// A whole run leaves A^ unprepared where the built-in crossover sends n to the
+// matrix cores.  A later call may run the encode alone under a knob that sends it
+// to the transform: cuot_qc_ahat_late says that A^ may be missing there, and the
+// encode stage prepares it from the bits of a in the workspace.  Under a knob, whole
+// runs leave nothing out, so that above the built-in crossover A^ is always there.
+bool cuot_qc_ahat_left_out(int64_t n);
+bool cuot_qc_ahat_late(int64_t n);
 int64_t cuot_qc_ahat_words(int64_t n);
 hipError_t cuot_launch_qc_keep_bits(const QcPrep* pr, QcPrep pr1, int B, int m, int64_t nmax, hipStream_t st);
 hipError_t cuot_launch_qc_mfma(const QcIo* io, QcIo io1, const uint32_t* bits1, const uint32_t* const* ahats, int B,

@@ -270,6 +270,14 @@ int64_t cuot_qc_mfma_limit() {
 
 bool cuot_qc_mfma_selected(int64_t n) { return cuot_qc_mfma_eligible(n) && n <= cuot_qc_mfma_limit(); }
 
+bool cuot_qc_ahat_left_out(int64_t n) {
+  return cuot_knobs().qc_mfma_max == 0 && cuot_qc_mfma_eligible(n) && n <= MF_DEFAULT_MAX;
+}
+
+bool cuot_qc_ahat_late(int64_t n) {
+  return cuot_qc_mfma_eligible(n) && n <= MF_DEFAULT_MAX && !cuot_qc_mfma_selected(n);
+}
+
 hipError_t cuot_launch_qc_keep_bits(const QcPrep* pr, QcPrep pr1, int B, int m, int64_t nmax, hipStream_t st) {
   const int64_t bytes = 4 * ((nmax + 31) / 32);
   hipLaunchKernelGGL(qc_mf_keep_bits, dim3((unsigned)((bytes + 255) / 256), (unsigned)B), dim3(256), 0, st, pr, pr1,
