@@ -8,6 +8,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+#include <mutex>
+
 #include "../../include/cuot_amd.h"
 
 #define CUOT_DEV __device__ __forceinline__
@@ -58,5 +61,26 @@ CUOT_DEV void stb(blk* p, blk v) { *(blk_gptr)p = blk_vec{v.x, v.y, v.z, v.w}; }
       return CUOT_ERR_HIP;                                  \
     }                                                       \
   } while (0)
+
+// One-time set-up of each device (function attributes hold for the device that is
+// current when they are set); safe with several threads.
+struct CuotDeviceOnce {
+  std::mutex mu;
+  std::atomic<bool> done[64] = {};
+
+  template <typename F>
+  hipError_t run(const F& setup) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
+    if (done[dev].load(std::memory_order_acquire)) return hipSuccess;
+    std::lock_guard<std::mutex> lk(mu);
+    if (done[dev].load(std::memory_order_relaxed)) return hipSuccess;
+    e = setup();
+    if (e == hipSuccess) done[dev].store(true, std::memory_order_release);
+    return e;
+  }
+};
 
 void cuot_set_last_error(const char* msg, const char* file, int line);

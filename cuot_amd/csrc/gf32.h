@@ -101,8 +101,8 @@ constexpr uint32_t gf32_pack_chunk(uint32_t u) {
 // ---- Cantor basis: beta_0 = 1, beta_i^2 + beta_i = beta_{i-1} ----------------
 // Solves the GF(2)-linear system x^2 + x = c by elimination; the root with
 // coordinate 0 clear is taken (the other root is x + 1).  Returns 0 on success.
-static inline int gf32_cantor_basis(uint32_t beta[32]) {
-  uint32_t col[32];
+constexpr int gf32_cantor_basis(uint32_t* beta) {
+  uint32_t col[32] = {0};
   for (int j = 0; j < 32; j++) {
     uint32_t tj = 1u << j;
     col[j] = gf32_mul(tj, tj) ^ tj;

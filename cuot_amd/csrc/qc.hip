@@ -65,8 +65,14 @@ struct Beta {
   uint32_t v[32];
 };
 
-// Cantor basis beta_0..beta_31 (uploaded once per process by configure_lds)
-__constant__ uint32_t c_beta[32];
+constexpr Beta cantor_basis() {
+  Beta b{};
+  gf32_cantor_basis(b.v);
+  return b;
+}
+
+// Cantor basis beta_0..beta_31 (part of the code object, so that every device has it)
+__constant__ Beta c_beta = cantor_basis();
 
 // lower terms of s_k: e = 2^j for j a proper submask of k (at most 15 for k < 31)
 CUOT_DEV int lower_terms(int k, uint32_t* e) {
@@ -93,7 +99,7 @@ CUOT_DEV void ctab_fill(uint32_t* tab, int tid, int nth) {
     const int q = i >> 8, v = i & 255;
     uint32_t c = 0;
     for (int b = 0; b < 8; b++)
-      if ((v >> b) & 1) c ^= c_beta[8 * q + b + 1];
+      if ((v >> b) & 1) c ^= c_beta.v[8 * q + b + 1];
     tab[i] = c;
   }
 }
@@ -810,7 +816,7 @@ __global__ void qcs_fft_layer(const QcPrep* __restrict__ pr, QcPrep pr1, int64_t
   for (int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; b < (M >> 1); b += (int64_t)gridDim.x * blockDim.x) {
     const int64_t g = b >> k, j = b & (half - 1);
     const int64_t u = g * 2 * half + j, v = u + half;
-    const uint32_t c = chunk_const(c_beta, (uint64_t)g);
+    const uint32_t c = chunk_const(c_beta.v, (uint64_t)g);
     const uint32_t xu = A[u] ^ gf32_mul_dev(c, A[v]);
     A[u] = xu;
     A[v] = A[v] ^ xu;
@@ -873,7 +879,7 @@ __global__ __launch_bounds__(1024) void qcs_prepare_lds(const QcPrep* __restrict
     for (int64_t b = tid; b < Mh; b += nth) {
       const int64_t g = b >> k, j = b & (half - 1);
       const int64_t u = g * 2 * half + j, v = u + half;
-      const uint32_t c = chunk_const(c_beta, (uint64_t)g);
+      const uint32_t c = chunk_const(c_beta.v, (uint64_t)g);
       const uint32_t xu = L[u] ^ gf32_mul_dev(c, L[v]);
       L[u] = xu;
       L[v] = L[v] ^ xu;
@@ -944,7 +950,7 @@ __global__ __launch_bounds__(1024) void qcs_fft_tile(const QcPrep* __restrict__ 
     for (int b = threadIdx.x; b < (TW >> 1); b += blockDim.x) {
       const int c = b & (C - 1), bp = b >> lgC;
       const int tu = ((bp >> s) << (s + 1)) | (bp & ((1 << s) - 1)), tv = tu | (1 << s);
-      const uint32_t cst = chunk_const(c_beta, (uint64_t)gidx(tu, c) >> (k + 1));
+      const uint32_t cst = chunk_const(c_beta.v, (uint64_t)gidx(tu, c) >> (k + 1));
       const int u = tu * C + c, v = tv * C + c;
       const uint32_t xu = L[u] ^ gf32_mul_dev(cst, L[v]);
       L[u] = xu;
@@ -1015,25 +1021,7 @@ unsigned grid_for(int64_t total, int64_t cap = 1 << 16) {
   return (unsigned)g;
 }
 
-Beta g_beta;
-bool g_beta_ready = false;
-
-const Beta& beta() {
-  if (!g_beta_ready) {
-    gf32_cantor_basis(g_beta.v);
-    g_beta_ready = true;
-  }
-  return g_beta;
-}
-
-int g_sm_configured = 0;
-
-hipError_t configure_lds() {
-  if (g_sm_configured) return hipSuccess;
-  {
-    hipError_t e0 = hipMemcpyToSymbol(HIP_SYMBOL(c_beta), beta().v, sizeof(uint32_t) * 32);
-    if (e0 != hipSuccess) return e0;
-  }
+hipError_t allow_lds() {
   hipError_t e = hipFuncSetAttribute((const void*)qc_fft_pass<32>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (ftc_max<32>() * fstride<32>() + CTAB_WORDS) * 4);
   if (e != hipSuccess) return e;
@@ -1061,9 +1049,12 @@ hipError_t configure_lds() {
   if (e != hipSuccess) return e;
   e = hipFuncSetAttribute((const void*)qc_conv_lds<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (1 << CONV_B) * 16);
-  if (e != hipSuccess) return e;
-  g_sm_configured = 1;
-  return hipSuccess;
+  return e;
+}
+
+hipError_t configure_lds() {
+  static CuotDeviceOnce once;
+  return once.run(allow_lds);
 }
 
 struct Bufs {

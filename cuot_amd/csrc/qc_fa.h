@@ -60,15 +60,23 @@ static_assert(kFaBeta.v[0] == 1, "nu has trace 1");
 static_assert(kFaBeta.v[1] == 7 && kFaBeta.v[2] == 4 && kFaBeta.v[3] == 8 && kFaBeta.v[4] == 0x140,
               "what the products by lane-dependent constants assume");
 
-// all 32 (host)
-static inline void fa_basis(uint32_t beta[32]) {
+// all 32
+struct FaBasis {
+  uint32_t v[32];
+};
+
+constexpr FaBasis fa_basis() {
+  FaBasis b{};
+  uint32_t* beta = b.v;
   for (int i = 0; i < 16; i++) beta[i] = kFaBeta.v[i];
   beta[16] = 0x10000u;
+  uint32_t img[32] = {0};
+  for (int j = 1; j < 32; j++) img[j] = fa_mul32(1u << j, 1u << j) ^ (1u << j);
   for (int i = 17; i < 32; i++) {
     // x^2 + x = beta[i-1]: elimination on the images of the 31 unit vectors
     uint32_t bv[32] = {0}, bm[32] = {0};
     for (int j = 1; j < 32; j++) {
-      uint32_t v = fa_mul32(1u << j, 1u << j) ^ (1u << j), m = 1u << j;
+      uint32_t v = img[j], m = 1u << j;
       while (v) {
         const int h = 31 - __builtin_clz(v);
         if (!bm[h]) {
@@ -88,6 +96,7 @@ static inline void fa_basis(uint32_t beta[32]) {
     }
     beta[i] = m;
   }
+  return b;
 }
 
 // Transform of products of 2^K coefficients: the points are beta_a + the span

@@ -49,8 +49,28 @@
 
 namespace {
 
-__constant__ uint2 c_fa_beta[32];  // beta_i and nu times its theta part
-__constant__ uint32_t c_fa_pack[FA_KC_MAX + 1][8];
+struct alignas(8) FaConsts {
+  uint32_t beta[32][2];              // beta_i and nu times its theta part
+  uint32_t pack[FA_KC_MAX + 1][8];  // [kc][q]: bits 0..2 of q are index bits K-4 .. K-2
+};
+
+constexpr FaConsts fa_consts() {
+  FaConsts c{};
+  const FaBasis b = fa_basis();
+  for (int i = 0; i < 32; i++) {
+    c.beta[i][0] = b.v[i];
+    c.beta[i][1] = fa_mul16(FA_NU, b.v[i] >> 16);
+  }
+  const FaChunk ch[FA_KC_MAX + 1] = {kFaChunk<0>, kFaChunk<1>, kFaChunk<2>, kFaChunk<3>, kFaChunk<4>, kFaChunk<5>};
+  for (int i = 0; i <= FA_KC_MAX; i++)
+    for (int q = 0; q < 8; q++) c.pack[i][q] = ch[i].pack[q];
+  return c;
+}
+
+// part of the code object, so that every device has them
+__constant__ FaConsts c_fa = fa_consts();
+
+CUOT_DEV uint2 fa_beta(int i) { return make_uint2(c_fa.beta[i][0], c_fa.beta[i][1]); }
 
 constexpr int FA_KMIN = 14, FA_KMAX = 25;
 // Log2 of the strings of a's bits that are converted in LDS.  A run prepares A^
@@ -77,7 +97,7 @@ CUOT_DEV void fa_ctab_fill(uint2* tab, int tid, int nth) {
     const int q = i >> 8, v = i & 255;
     uint2 c = make_uint2(0, 0);
     for (int b = 0; b < 8; b++)
-      if ((v >> b) & 1) c = x2(c, c_fa_beta[8 * q + b + 1]);
+      if ((v >> b) & 1) c = x2(c, fa_beta(8 * q + b + 1));
     tab[i] = c;
   }
 }
@@ -460,7 +480,7 @@ __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void
       fa_swap<16>(lds, u, v, P, sw);
       // the first lane's constant for all, and what the others' g add to it
       const uint32_t g = (uint32_t)(P >> b), g0 = __builtin_amdgcn_readfirstlane(g), d = g ^ g0;
-      const uint2 c = x2(c_fa_beta[a.a - a.c - 1 - (b - LGC)], fa_ctab(ctab, g0));
+      const uint2 c = x2(fa_beta(a.a - a.c - 1 - (b - LGC)), fa_ctab(ctab, g0));
       uint32_t acc[16];
       if constexpr (INV) {
 #pragma unroll
@@ -657,7 +677,7 @@ __global__ __launch_bounds__(FA_NT) __attribute__((amdgpu_waves_per_eu(4))) void
       // the first lane's constant for all, and what the others' g add to it: a
       // wavefront covers 16 neighbouring P, so at most the low four bits differ
       const uint32_t g0 = __builtin_amdgcn_readfirstlane(g), d = g ^ g0;
-      const uint2 c = x2(c_fa_beta[a.a - k], fa_ctab(ctab, g0));
+      const uint2 c = x2(fa_beta(a.a - k), fa_ctab(ctab, g0));
       // (fused: by a mask, as a branch costs moves of both)
       auto add_u = [&](bool now) {
         if constexpr (MODE == FA_FUSED) {
@@ -1120,7 +1140,7 @@ __global__ __launch_bounds__(512) void fa_prep_fft(const QcPrep* __restrict__ pr
   auto eidx = [&](int i) { return (hib << (lo + R)) | ((int64_t)(i >> lgC) << lo) | (cb * C + (i & (C - 1))); };
   if (first) {
     const uint32_t* T = A + ((int64_t)1 << (K - 5));
-    const uint32_t* pk = c_fa_pack[K <= 20 ? 0 : K - 20];
+    const uint32_t* pk = c_fa.pack[K <= 20 ? 0 : K - 20];
     for (int i = threadIdx.x; i < TW; i += nt) {
       const int64_t e = eidx(i);
       uint32_t v = 0;
@@ -1150,7 +1170,7 @@ __global__ __launch_bounds__(512) void fa_prep_fft(const QcPrep* __restrict__ pr
       __syncthreads();
     }
     const int k = b >= c ? b + 1 : b;
-    const uint2 off = c_fa_beta[aidx - k];
+    const uint2 off = fa_beta(aidx - k);
     for (int t = threadIdx.x; t < (TW >> 1); t += nt) {
       const int cc = t & (C - 1), bp = t >> lgC;
       const int tu = ((bp >> s) << (s + 1)) | (bp & ((1 << s) - 1));
@@ -1179,8 +1199,6 @@ __global__ __launch_bounds__(512) void fa_prep_fft(const QcPrep* __restrict__ pr
 }
 
 // ---- host -------------------------------------------------------------------------------
-int g_fa_ready = 0;
-
 constexpr size_t FA_LDS16 = 256 * FA_ST16 * 4 + FA_CTAB * sizeof(uint2);
 
 constexpr size_t FA_LDSC = (4096 + 256) * 16;
@@ -1209,19 +1227,8 @@ hipError_t fa_allow_lds32() {
                              (int)FA_LDS32);
 }
 
-hipError_t fa_configure() {
-  if (g_fa_ready) return hipSuccess;
-  uint32_t basis[32], pack[FA_KC_MAX + 1][8];
-  fa_basis(basis);
-  uint2 beta[32];
-  for (int i = 0; i < 32; i++) beta[i] = make_uint2(basis[i], fa_mul16(FA_NU, basis[i] >> 16));
-  const FaChunk ch[FA_KC_MAX + 1] = {kFaChunk<0>, kFaChunk<1>, kFaChunk<2>, kFaChunk<3>, kFaChunk<4>, kFaChunk<5>};
-  // pack[b]: bits 0..2 of b are index bits K-4 .. K-2
-  for (int i = 0; i <= FA_KC_MAX; i++)
-    for (int q = 0; q < 8; q++) pack[i][q] = ch[i].pack[q];
-  hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(c_fa_beta), beta, sizeof(beta));
-  if (!e) e = hipMemcpyToSymbol(HIP_SYMBOL(c_fa_pack), pack, sizeof(pack));
-  if (!e) e = fa_allow_lds32<FA_FWD, false>();
+hipError_t fa_allow_lds() {
+  hipError_t e = fa_allow_lds32<FA_FWD, false>();
   if (!e) e = fa_allow_lds32<FA_FWD, true>();
   if (!e) e = fa_allow_lds32<FA_FUSED, false>();
   if (!e) e = fa_allow_lds32<FA_INV, false>();
@@ -1235,8 +1242,12 @@ hipError_t fa_configure() {
   if (!e) e = fa_allow_lds16<3>();
   if (!e) e = fa_allow_lds16<4>();
   if (!e) e = fa_allow_lds16<5>();
-  if (!e) g_fa_ready = 1;
   return e;
+}
+
+hipError_t fa_configure() {
+  static CuotDeviceOnce once;
+  return once.run(fa_allow_lds);
 }
 
 int fa_log(int64_t n) {  // K: 2^(K-1) >= n

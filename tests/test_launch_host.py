@@ -1,0 +1,31 @@
+"""What the library asks the HIP runtime for (launch shapes, per-device set-up),
+checked on the CPU: a program whose own stand-ins for the runtime's entry points
+take the place of the real ones links the built library."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    from cuot_amd import _lib
+
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built")
+    exe = str(tmp_path_factory.mktemp("launch") / "check")
+    libdir = os.path.dirname(_lib.LIB_PATH)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-rdynamic", "-o", exe, os.path.join(HERE, "launch_host_check.cpp"),
+                    f"-L{libdir}", "-lcuot_amd", f"-Wl,-rpath,{libdir}", "-Wl,--allow-shlib-undefined"], check=True)
+
+    def run(what):
+        r = subprocess.run([exe, what], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0 and f"{what} ok" in r.stdout, r.stdout + r.stderr
+
+    return run
+
+
+def test_every_device_is_set_up(check):
+    check("devices")
