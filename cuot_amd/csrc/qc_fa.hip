@@ -143,28 +143,33 @@ __device__ __forceinline__ void fa_swap_dpp(uint32_t* u, uint32_t* v) {
 }
 
 template <int NP>
-__device__ __forceinline__ void fa_swap_lds(uint32_t* lds, uint32_t* g, int other) {
-#pragma unroll
-  for (int p = 0; p < NP; p++) lds[p * FA_NT + threadIdx.x] = g[p];
-  __syncthreads();
-#pragma unroll
-  for (int p = 0; p < NP; p++) g[p] = lds[p * FA_NT + other];
-  __syncthreads();
-}
-
-template <int NP>
 __device__ __forceinline__ void fa_swap(uint32_t* lds, uint32_t* u, uint32_t* v, int P, int b) {
   // (b opaque in between: as one chain of choices the compiler merges all ways
   // behind 64 moves)
 #define FA_OPAQUE(x) \
   x = __builtin_amdgcn_readfirstlane(x); \
   asm volatile("" : "+s"(x))
-  if (b >= 4) {  // another wavefront; the bit is this one's
-    const int other = (int)threadIdx.x ^ (4 << b);
+  if (b >= 4) {  // another wavefront; the bit is this one's, b the workgroup's
+    auto put = [&](const uint32_t* g) {
+#pragma unroll
+      for (int p = 0; p < NP; p++) lds[p * FA_NT + threadIdx.x] = g[p];
+    };
+    auto get = [&](uint32_t* g) {
+      const int other = (int)threadIdx.x ^ (4 << b);
+#pragma unroll
+      for (int p = 0; p < NP; p++) g[p] = lds[p * FA_NT + other];
+    };
+    // only the copies depend on the bit: all wavefronts meet at the same barriers
     int bit = __builtin_amdgcn_readfirstlane(P >> b) & 1;
-    if (bit) fa_swap_lds<NP>(lds, u, other);
+    if (bit) put(u);
     FA_OPAQUE(bit);
-    if (!bit) fa_swap_lds<NP>(lds, v, other);
+    if (!bit) put(v);
+    __syncthreads();
+    FA_OPAQUE(bit);
+    if (bit) get(u);
+    FA_OPAQUE(bit);
+    if (!bit) get(v);
+    __syncthreads();
   }
   FA_OPAQUE(b);
   if (b == 3) {
