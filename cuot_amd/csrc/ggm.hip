@@ -411,14 +411,23 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void gg
 }
 
 // Depth-first levels L per lane.  Every lane of the workgroup has a subtree from
-// depth 9 on, so L = h - 9 (the knob may ask for the neighbouring splits);
-// depth 16 keeps L = 6 for the registers and puts two subtrees on a lane.
-int ggm_split(int h) {
-  const int k = cuot_knobs().ggm_dfs;
-  const int hi = h - 8 < LMAX ? h - 8 : LMAX;
-  if (k >= 1 && k <= hi && h - k <= MAXTOP) return k;
+// depth 9 on, so L = h - 9; depth 16 keeps L = 6 for the registers and puts two
+// subtrees on a lane.
+int ggm_rule(int h) {
   if (h <= 9) return 0;
   return h - 9 < LMAX ? h - 9 : LMAX;
+}
+
+// the split of whole trees that the knob asks for, 0 where it has none for this depth
+int ggm_knob(int h) {
+  const int k = cuot_knobs().ggm_dfs;
+  const int hi = h - 8 < LMAX ? h - 8 : LMAX;
+  return k >= 1 && k <= hi && h - k <= MAXTOP ? k : 0;
+}
+
+int ggm_split(int h) {
+  const int k = ggm_knob(h);
+  return k ? k : ggm_rule(h);
 }
 
 // L, plus 16 when the breadth-first top is deeper than 2^9 nodes
@@ -472,9 +481,9 @@ hipError_t launch_form(const GgmKArgs& a, int L, int64_t wgs, hipStream_t st) {
 
 hipError_t launch_ggm(GgmKArgs a, bool recv, hipStream_t st) {
   const int64_t nl = (a.t << a.h) < a.n_out ? (a.t << a.h) : a.n_out;
-  a.s = ggm_wg_split(a.t, a.h, recv);
-  if ((recv && a.part == nullptr) || cuot_knobs().ggm_dfs) a.s = 0;  // the knob picks a split of whole trees
-  const int L = ggm_split(a.h - a.s);
+  const int k = ggm_knob(a.h);
+  a.s = k || (recv && a.part == nullptr) ? 0 : ggm_wg_split(a.t, a.h, recv);
+  const int L = k ? k : ggm_rule(a.h - a.s);
   hipError_t e = hipSuccess;
   cuot_rec_begin(st, recv ? "ggm_kernel<recv>" : "ggm_kernel<send>", 16.0 * (double)nl);
   if (!recv) {

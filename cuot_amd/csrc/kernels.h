@@ -172,7 +172,7 @@ void cuot_rec_end(hipStream_t st);
 struct CuotKnobs {
   int qc_radix;  // FFT layers per upper pass (2..8)
   int qc_cols;   // FFT columns per tile (1, 2, 4, 8; n > 2^24)
-  int ggm_dfs;   // per-lane depth-first levels L (h - 10 <= L <= min(h - 8, 6))
+  int ggm_dfs;   // per-lane depth-first levels L of whole trees (h - 10 <= L <= min(h - 8, 6))
   int lpn_wgs;   // LPN grid cap
   int qc_mfma_max;  // matrix-core QC encoder for n at or below (-1: never)
   int aes_impl;     // AES streams: 0 rule / 1 LDS T-table / 2 bitsliced

@@ -14,8 +14,10 @@ Stages and knobs:
              pass (qc_radix 4..7) and, for n > 2^24, columns per tile (qc_cols
              1, 2, 4, 8);
              features (log2 n, m, radix, log2 cols);
-  * "ggm" -- GGM expansion of t trees of depth h: per-lane depth-first levels
-             L (ggm_dfs, h-10 <= L <= min(h-8, 6)); features (h, log2 t, L).
+  * "ggm" -- GGM expansion of t trees of depth h: the built-in rule (ggm_dfs 0,
+             which gives a few deep trees several workgroups each) or per-lane
+             depth-first levels L of whole trees (ggm_dfs, h-10 <= L <=
+             min(h-8, 6)); features (h, log2 t, L).
 """
 from __future__ import annotations
 
@@ -149,9 +151,8 @@ QC_DEFAULT = dict(qc_radix=7, qc_cols=2)
 
 
 def ggm_space(h: int):
-    if h <= 8:
-        return [dict(ggm_dfs=0)]
-    return [dict(ggm_dfs=L) for L in range(max(1, h - 10), min(h - 8, 6) + 1)]
+    """The built-in rule, then the splits of whole trees that are valid at depth h."""
+    return [dict(ggm_dfs=L) for L in (0, *range(max(1, h - 10), min(h - 8, 6) + 1))]
 
 
 def qc_log_len(n: int) -> int:

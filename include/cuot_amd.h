@@ -439,7 +439,8 @@ int cuot_mlp_adam(cuot_ctx *ctx, float *params_d, const float *grad_d, float *m_
 typedef struct {
   int32_t qc_radix; /* most FFT layers per upper pass, 2..8 (at most 7 for n <= 2^24) */
   int32_t qc_cols;  /* FFT columns per tile, 1, 2, 4 or 8 (n > 2^24 only; below, tiles are fixed) */
-  int32_t ggm_dfs;  /* GGM per-lane depth-first levels (valid: h-10 <= L <= min(h-8, 6); else the rule) */
+  int32_t ggm_dfs;  /* GGM per-lane depth-first levels (valid: h-10 <= L <= min(h-8, 6); else the rule).
+                       A valid one means one workgroup per tree; the rule gives a few deep trees several */
   int32_t lpn_wgs;  /* LPN grid cap */
   int32_t qc_mfma_max; /* QC encodes with 17 <= n <= this run as a 0/1 int8 matrix-core product
                           (at most 2^16; -1: never, 0: the built-in crossover) */

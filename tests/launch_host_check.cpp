@@ -49,10 +49,51 @@ static int check_devices() {
   return 0;
 }
 
+static std::string shapes() {
+  std::string s;
+  for (const Launch& l : g_launches) s += l.kernel + " " + std::to_string(l.grid.x) + "; ";
+  return s;
+}
+
+// A split that the knob has none of for a depth is the built-in rule, which gives a
+// few deep trees several workgroups each; a valid one means one workgroup per tree.
+static int check_ggm_dfs() {
+  cuot_ctx* ctx = nullptr;
+  REQUIRE(cuot_init(0, &ctx) == CUOT_OK);
+  for (int h = 9; h <= 16; h++) {
+    std::string rule;
+    for (int dfs = 0; dfs <= 6; dfs++) {
+      const cuot_knob_values k = {0, 0, dfs, 0, 0, 0};
+      REQUIRE(cuot_set_knobs(&k) == CUOT_OK);
+      cuot_ggm_params p;
+      memset(&p, 0, sizeof(p));
+      p.t = 3;
+      p.h = h;
+      p.mode = CUOT_MODE_SOT;
+      p.n_out = p.t << h;
+      g_launches.clear();
+      REQUIRE(cuot_ggm_sender(ctx, &p, (cuot_block*)buf, (cuot_block*)buf, (cuot_block*)buf, nullptr) == CUOT_OK);
+      const bool valid = dfs >= 1 && dfs >= h - 10 && dfs <= h - 8;
+      if (dfs == 0) {
+        rule = shapes();
+        REQUIRE(h < 12 || g_launches.back().grid.x > 3);
+      } else if (valid) {
+        REQUIRE(g_launches.size() == 1 && g_launches[0].grid.x == 3);
+      } else {
+        if (shapes() != rule) printf("h = %d, ggm_dfs = %d: %s not %s\n", h, dfs, shapes().c_str(), rule.c_str());
+        REQUIRE(shapes() == rule);
+      }
+    }
+  }
+  REQUIRE(cuot_destroy(ctx) == CUOT_OK);
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   int rc = 2;
   if (what == "devices") rc = check_devices();
+  if (what == "ggm_dfs") rc = check_ggm_dfs();
   if (!rc) printf("%s ok\n", what.c_str());
   return rc;
 }

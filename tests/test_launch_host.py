@@ -29,3 +29,16 @@ def check(tmp_path_factory):
 
 def test_every_device_is_set_up(check):
     check("devices")
+
+
+def test_ggm_knob_without_a_split_is_the_rule(check):
+    check("ggm_dfs")
+
+
+def test_tuner_can_choose_the_ggm_rule():
+    from cuot_amd import tune
+
+    for h in range(1, 17):
+        space = [k["ggm_dfs"] for k in tune.ggm_space(h)]
+        assert space[0] == 0
+        assert space[1:] == [L for L in range(1, 7) if h - 10 <= L <= h - 8], h
