@@ -254,3 +254,18 @@ def test_qc_orbit_product_vs_karatsuba(ctx, knob_mfma, n):
     r = rng(n + 23)
     a, x = rand_bits(r, n), rand_blocks(r, 2 * n)
     assert np.array_equal(qc_gpu(ctx, x, a, n), po.qc_encode_fast(x, a, n, nthreads=8))
+
+
+# n > 2^24 stays with the transform on packed chunks: one more upper pass than
+# 2^24 took (2^22 elements), an upper pass in full mode (2^24 elements), the
+# conversion level by level, A^ in tiles, and other pass shapes by the knobs
+@pytest.mark.parametrize("n, radix, cols", [((1 << 24) + 1, 0, 0), ((1 << 24) + 1, 3, 4), ((1 << 25) - 17, 8, 8),
+                                            ((1 << 25) + 1, 5, 1), ((1 << 26) + 1, 0, 0)])
+def test_qc_long_product_rotations(ctx, n, radix, cols):
+    from cuot_amd import tune
+
+    tune.set_knobs(qc_radix=radix, qc_cols=cols, qc_mfma_max=-1)
+    try:
+        test_qc_orbit_product_rotations(ctx, lambda v: None, n)
+    finally:
+        tune.set_knobs()
