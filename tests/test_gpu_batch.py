@@ -138,3 +138,24 @@ def test_batch_overlap_matches(ctx):
         for i, (wi, _) in enumerate(mix):
             assert _same(_batch_out(bt, i, wi), ref[i]), f"run {rep} (graph={graph}) instance {i} differs"
     bt.close()
+
+
+def test_batch_powers_of_two_match_plain(ctx):
+    """A single n = 2^21 or more is folded before its last levels; in a batch it
+    takes the general output, also where n is a whole number of columns."""
+    import torch
+
+    import cuot_amd
+    from cuot_amd.workloads import SOT, make_instance
+
+    rows = [make_instance(SOT, 1 << lg, (lg, 77)) for lg in (20, 21, 22, 23, 24)]
+    print("batch of powers of two", flush=True)
+    ins = [cuot_amd.make_instance_struct(SOT, w.n, w.t, w.h, 0, w.seed, k0=SOT_K0, k1=SOT_K1) for w in rows]
+    bt = cuot_amd.Batch(ctx, ins)
+    bt.run()
+    torch.cuda.synchronize()
+    for i, w in enumerate(rows):
+        v, u, b, d = run_sot_gpu(ctx, w.n, w.t, w.h, np.array(w.seed, dtype=np.uint64))
+        assert torch.equal(bt.out0[i], v[: w.n]) and torch.equal(bt.out1[i], u[: w.n]), w.n
+        assert torch.equal(bt.bits[i].view(torch.uint8)[: w.n // 8], b[: w.n // 8]), w.n
+    bt.close()

@@ -269,3 +269,25 @@ def test_qc_long_product_rotations(ctx, n, radix, cols):
         test_qc_orbit_product_rotations(ctx, lambda v: None, n)
     finally:
         tune.set_knobs()
+
+
+# y over x, on every form of the output: matrix cores, rows (by the knob), whole
+# and half blocks a lane, folded
+@pytest.mark.parametrize("n, mfma", [(1000, -1), (1000, 0), (9001, -1), (36000, 0), (50001, 0), (70000, 0), (400001, 0),
+                                     ((1 << 20) - 3, 0), (1 << 21, 0), (2500001, 0), (1 << 22, 0), (1 << 23, 0)])
+def test_qc_encode_in_place(ctx, knob_mfma, n, mfma):
+    import torch
+
+    print(f"qc in place n={n}", flush=True)
+    knob_mfma(mfma)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    a = torch.randint(0, 256, ((n + 7) // 8,), dtype=torch.uint8, device="cuda", generator=g)
+    x = torch.randint(-(1 << 63), (1 << 63) - 1, (2 * n, 2), dtype=torch.int64, device="cuda", generator=g)
+    ahat = torch.zeros(ctx.qc_ahat_len(n), dtype=torch.int32, device="cuda")
+    scratch = torch.full((ctx.qc_scratch_bytes(n),), 0xA5, dtype=torch.uint8, device="cuda")
+    ctx.qc_prepare(n, a, ahat, scratch)
+    y = dev_blocks(n)
+    ctx.qc_encode(n, ahat, x, y, scratch)
+    upper = x[n:].clone()
+    ctx.qc_encode(n, ahat, x, x, scratch)
+    assert torch.equal(x[:n], y) and torch.equal(x[n:], upper)
