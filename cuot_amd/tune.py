@@ -12,7 +12,7 @@ speed.
 Stages and knobs:
   * "qc"  -- quasi-cyclic encode of one party at n COTs: FFT layers per upper
              pass (qc_radix 4..7) and, for n > 2^24, columns per tile (qc_cols
-             1, 2, 4, 8);
+             1, 2, 4, 8), one setting of each that launch the same;
              features (log2 n, m, radix, log2 cols);
   * "ggm" -- GGM expansion of t trees of depth h: the built-in rule (ggm_dfs 0,
              which gives a few deep trees several workgroups each) or per-lane
@@ -164,8 +164,25 @@ def qc_log_len(n: int) -> int:
     return m
 
 
+def qc_passes(n: int, radix: int):
+    """Layers of each upper pass of the transform for 2^12 < n <= 2^24."""
+    layers = min((n - 1).bit_length() + 1 - 5, 15) - 8
+    return tuple(min(radix, layers - i) for i in range(0, layers, radix))
+
+
+def qc_space(n: int):
+    """One setting per distinct launch sequence of an encode of n: the matrix cores
+    have no such knob, the transform for 2^12 < n <= 2^24 has fixed columns and at
+    most seven upper layers, the one on packed chunks takes both."""
+    if 17 <= n <= _lib.load().cuot_qc_mfma_crossover():
+        return [dict(qc_radix=7, qc_cols=0)]
+    if (1 << 12) < n <= (1 << 24):
+        return list({qc_passes(n, r): dict(qc_radix=r, qc_cols=0) for r in (4, 5, 6, 7)}.values())
+    return QC_SPACE if qc_log_len(n) > 7 else [dict(qc_radix=7, qc_cols=0)]
+
+
 def qc_features(n: int, knobs: dict):
-    return [math.log2(n), qc_log_len(n), knobs["qc_radix"], math.log2(knobs["qc_cols"])]
+    return [math.log2(n), qc_log_len(n), knobs["qc_radix"], math.log2(max(1, knobs["qc_cols"]))]
 
 
 def ggm_features(t: int, h: int, knobs: dict):
@@ -251,7 +268,7 @@ class Autotuner:
 
     def collect_qc(self, sizes, space=None):
         for n in sizes:
-            for k in space or QC_SPACE:
+            for k in space or qc_space(n):
                 self.add("qc", qc_features(n, k), self.measure_qc(n, k))
 
     def collect_ggm(self, shapes):
@@ -264,8 +281,9 @@ class Autotuner:
         return self.models[stage].fit(np.array(x), np.array(t), epochs=epochs, lr=lr)
 
     def choose_qc(self, n: int) -> dict:
-        feats = np.array([qc_features(n, k) for k in QC_SPACE])
-        return QC_SPACE[int(np.argmin(self.models["qc"].predict(feats)))]
+        space = qc_space(n)
+        feats = np.array([qc_features(n, k) for k in space])
+        return space[int(np.argmin(self.models["qc"].predict(feats)))]
 
     def choose_ggm(self, t: int, h: int) -> dict:
         space = ggm_space(h)
@@ -275,6 +293,7 @@ class Autotuner:
     def exhaustive_qc(self, n: int):
         """(best knobs, best ms, all ms, seconds spent measuring)"""
         t0 = time.perf_counter()
-        ms = [self.measure_qc(n, k) for k in QC_SPACE]
+        space = qc_space(n)
+        ms = [self.measure_qc(n, k) for k in space]
         i = int(np.argmin(ms))
-        return QC_SPACE[i], ms[i], ms, time.perf_counter() - t0
+        return space[i], ms[i], ms, time.perf_counter() - t0

@@ -89,11 +89,26 @@ static int check_ggm_dfs() {
   return 0;
 }
 
+// upper passes of an encode, there and back, and the one that joins them
+static int print_passes(int64_t n, int radix) {
+  cuot_ctx* ctx = nullptr;
+  REQUIRE(cuot_init(0, &ctx) == CUOT_OK);
+  const cuot_knob_values k = {radix, 0, 0, 0, -1, 0};
+  REQUIRE(cuot_set_knobs(&k) == CUOT_OK);
+  REQUIRE(cuot_qc_encode(ctx, n, (uint32_t*)buf, (cuot_block*)buf, (cuot_block*)buf, buf, nullptr) == CUOT_OK);
+  int passes = 0;
+  for (const Launch& l : g_launches) passes += l.kernel.find("fa_pass32") != std::string::npos;
+  printf("passes %d\n", passes);
+  REQUIRE(cuot_destroy(ctx) == CUOT_OK);
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   int rc = 2;
   if (what == "devices") rc = check_devices();
   if (what == "ggm_dfs") rc = check_ggm_dfs();
+  if (what == "passes" && argc > 3) rc = print_passes(atoll(argv[2]), atoi(argv[3]));
   if (!rc) printf("%s ok\n", what.c_str());
   return rc;
 }

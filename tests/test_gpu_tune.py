@@ -40,3 +40,25 @@ def test_tuned_qc_knobs_near_exhaustive(ctx):
         assert tuned <= 1.15 * best_ms
         assert tuned <= 1.05 * default
     print(f"worst tuned/best ratio {worst:.3f}", flush=True)
+
+
+def test_tuned_qc_knobs_where_the_choice_matters(ctx):
+    """Sizes past the matrix-core crossover whose settings are different launches:
+    the pick has to be near the best where a wrong one is far from it."""
+    from cuot_amd.tune import Autotuner, qc_space
+
+    tu = Autotuner(ctx, reps=7)
+    print("collecting QC timings", flush=True)
+    tu.collect_qc([150001, 1 << 18, 300001, 1 << 19, 600000, 1 << 20, 3 << 19, 1 << 21])
+    tu.train("qc", epochs=1500)
+    wrong = 0.0
+    for n in [400001, 700001, 5 << 18]:
+        assert len(qc_space(n)) == 4
+        k = tu.choose_qc(n)
+        best_k, best_ms, all_ms, _ = tu.exhaustive_qc(n)
+        tuned = tu.measure_qc(n, k)
+        print(f"n={n}: tuned {k} {tuned:.3f} ms | exhaustive {best_k} {best_ms:.3f} | all {np.round(all_ms, 3)}",
+              flush=True)
+        assert tuned <= 1.05 * best_ms
+        wrong = max(wrong, max(all_ms) / best_ms)
+    assert wrong > 1.05
