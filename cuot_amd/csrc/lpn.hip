@@ -265,9 +265,18 @@ bool fill_args(const LpnLaunch& l, LpnKArgs& a) {
 // the index AES twice (0.4 ms at n = 10,168,320, both roles) and pays from
 // about 11 MB on: k = 262,144 (8 MB) 1.03 ms whole, 1.07 in two; 327,680 (10 MB)
 // 1.14 / 1.13; 393,216 (12 MB) 1.24 / 1.16; 452,160 (14 MB) 1.32 / 1.22;
-// three slices lose everywhere (1.58 at 452,160).
+// three slices lose everywhere (1.58 at 452,160).  An L2 has to see its share of the
+// table again and again: with few rows per k the second pass costs what it is
+// (whole / two slices, us; one role: k = 730,000, n = 11,406 20 / 39, 365,000 56 / 62,
+// 730,000 110 / 102, 2,190,000 264 / 240; k = 1,600,000, n = k 273 / 290, 2k 490 / 476;
+// both: k = 452,160, n = 2k 141 / 145, 4k 280 / 271, 10k 607 / 574; k = 800,000
+// (26 MB), n = 6k 751 / 786, 10k 1234 / 1210; k = 1,600,000 (51 MB), n = 10k 2771 / 2881).
 int lpn_slices(const LpnKArgs& a) {
-  return a.cnt && (int64_t)a.cnt * 16 * a.nroles > (11ll << 20) ? 2 : 1;
+  const int64_t bytes = (int64_t)a.cnt * 16 * a.nroles;
+  if (bytes <= (11ll << 20)) return 1;
+  if (a.nroles == 1) return a.n >= 2 * a.k ? 2 : 1;
+  if (bytes > (32ll << 20)) return 1;
+  return a.n >= (bytes > (16ll << 20) ? 10 : 4) * a.k ? 2 : 1;
 }
 
 }  // namespace

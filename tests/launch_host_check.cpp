@@ -89,6 +89,30 @@ static int check_ggm_dfs() {
   return 0;
 }
 
+// A table above 11 MB takes two launches only where the rows pay for the second.
+static int check_lpn_slices() {
+  cuot_ctx* ctx = nullptr;
+  REQUIRE(cuot_init(0, &ctx) == CUOT_OK);
+  const struct {
+    int64_t n, k;
+    size_t launches;
+  } rows[] = {{4000000, 720896, 1}, {65536, 720897, 1}, {2 * 720897 - 1, 720897, 1}, {2 * 720897, 720897, 2}};
+  for (const auto& r : rows) {
+    cuot_lpn_params p;
+    memset(&p, 0, sizeof(p));
+    p.n = r.n;
+    p.k = r.k;
+    p.d = 10;
+    p.ntasks = 1;
+    g_launches.clear();
+    REQUIRE(cuot_lpn(ctx, &p, (cuot_block*)buf, (cuot_block*)buf, (cuot_block*)buf, nullptr) == CUOT_OK);
+    if (g_launches.size() != r.launches) printf("n = %ld, k = %ld: %zu launches\n", r.n, r.k, g_launches.size());
+    REQUIRE(g_launches.size() == r.launches);
+  }
+  REQUIRE(cuot_destroy(ctx) == CUOT_OK);
+  return 0;
+}
+
 // upper passes of an encode, there and back, and the one that joins them
 static int print_passes(int64_t n, int radix) {
   cuot_ctx* ctx = nullptr;
@@ -108,6 +132,7 @@ int main(int argc, char** argv) {
   int rc = 2;
   if (what == "devices") rc = check_devices();
   if (what == "ggm_dfs") rc = check_ggm_dfs();
+  if (what == "lpn_slices") rc = check_lpn_slices();
   if (what == "passes" && argc > 3) rc = print_passes(atoll(argv[2]), atoi(argv[3]));
   if (!rc) printf("%s ok\n", what.c_str());
   return rc;

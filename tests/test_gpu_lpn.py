@@ -62,3 +62,37 @@ def test_lpn_table_slices_both_roles(ctx):
     os_, or_, _ = po.ferret_run(n, k, t, h, seed, ntasks=3, nthreads=4)
     assert np.array_equal(to_np(s), os_)
     assert np.array_equal(to_np(w), or_)
+
+
+# two slices need rows enough as well as a table above 11 MB: at the least rows
+# that take them, and one short of it
+@pytest.mark.parametrize("n", [2 * 720897 - 1, 2 * 720897])
+def test_lpn_table_slices_many_rows(ctx, n):
+    k = 720897
+    print(f"lpn slices n={n} k={k}", flush=True)
+    r = rng(n + k)
+    seed = rand_blocks(r, 1)[0]
+    noise, kk = rand_blocks(r, n), rand_blocks(r, k)
+    ref = po.ferret_lpn(noise, kk, seed, ntasks=3, nthreads=8)
+    a = to_dev(noise)
+    ctx.lpn(_p(n, k, seed, 3), a, to_dev(kk), a)
+    assert np.array_equal(to_np(a)[:n], ref)
+
+
+@pytest.mark.parametrize("n", [4 * 360449 - 1, 4 * 360449])
+def test_lpn_table_slices_many_rows_both_roles(ctx, n):
+    import torch
+
+    import cuot_amd
+
+    k, h = 360449, 13
+    t = -(-n >> h)
+    print(f"lpn slices both roles n={n} k={k}", flush=True)
+    seed = np.array([79, 80], dtype=np.uint64)
+    cfg = cuot_amd.FerretConfig(n=n, k=k, t=t, h=h, ntasks=1, seed=cuot_amd.to_block(seed))
+    ws = torch.empty(ctx.ferret_workspace_bytes(cfg), dtype=torch.uint8, device="cuda")
+    s, w = dev_blocks(n), dev_blocks(n)
+    ctx.ferret_run(cfg, ws, s, w)
+    os_, or_, _ = po.ferret_run(n, k, t, h, seed, nthreads=8)
+    assert np.array_equal(to_np(s), os_)
+    assert np.array_equal(to_np(w), or_)

@@ -36,6 +36,10 @@ def test_ggm_knob_without_a_split_is_the_rule(check):
     check("ggm_dfs")
 
 
+def test_lpn_slices_need_rows(check):
+    check("lpn_slices")
+
+
 def test_tuner_can_choose_the_ggm_rule():
     from cuot_amd import tune
 
