@@ -99,7 +99,7 @@ CUOT_DEV void lpn_unit(const AesLds& aes, const LpnKArgs& a, int64_t u, int par)
   // locate the task and the unit inside it
   int64_t task = 0;
   if (a.ntasks > 1) {
-    task = u / a.units_per_task;
+    task = a.units_total >> 32 ? u / a.units_per_task : (int64_t)((uint32_t)u / (uint32_t)a.units_per_task);
     if (task >= a.ntasks) task = a.ntasks - 1;
   }
   const int64_t start = task * a.width;
@@ -279,16 +279,24 @@ int lpn_slices(const LpnKArgs& a) {
   return a.n >= (bytes > (16ll << 20) ? 10 : 4) * a.k ? 2 : 1;
 }
 
+// Workgroups: one wave of them, two a CU, so that each fills its AES table once
+// (2048 -> 512, us; one role / both: n = 1,048,576 65 / 71 -> 56 / 65, 3,145,728 160 / 214 ->
+// 152 / 200, 10,168,320 both 1179 -> 1147, 20,000,000 both 3190 -> 2900), but for one role
+// with many rows, where it loses (20,000,000 1853 -> 1928).
+int64_t lpn_grid(const LpnKArgs& a) {
+  const int64_t g = (a.units_total + LPN_UNITS - 1) / LPN_UNITS;
+  const int knob = cuot_knobs().lpn_wgs;
+  const int64_t cap = knob > 0 ? knob : a.nroles == 1 && a.units_total > (1 << 20) ? 2048 : 512;
+  return g > cap ? cap : g < 1 ? 1 : g;
+}
+
 }  // namespace
 
 hipError_t cuot_launch_lpn(const LpnLaunch& l, hipStream_t st) {
   if (l.n <= 0) return hipSuccess;
   LpnKArgs a;
   if (!fill_args(l, a)) return hipErrorInvalidValue;
-  int64_t g = (a.units_total + LPN_UNITS - 1) / LPN_UNITS;
-  const int64_t cap = cuot_knobs().lpn_wgs > 0 ? cuot_knobs().lpn_wgs : 2048;
-  if (g > cap) g = cap;
-  if (g < 1) g = 1;
+  const int64_t g = lpn_grid(a);
   // algorithmic bytes per role and row: noise in, d gathers, row out
   cuot_rec_begin(st, "lpn_kernel", 16.0 * (D + 2) * (double)l.n * l.nroles);
   const int ns = lpn_slices(a);
