@@ -113,6 +113,22 @@ static int check_lpn_slices() {
   return 0;
 }
 
+// Whole words of 2^25 bits and more fill the chip with a lane per two words.
+static int check_sparse() {
+  cuot_ctx* ctx = nullptr;
+  REQUIRE(cuot_init(0, &ctx) == CUOT_OK);
+  const int64_t m = (int64_t)1 << 25;
+  for (int64_t n : {m - 32, m - 1, m, m + 1, m + 32, 2 * m}) {
+    g_launches.clear();
+    REQUIRE(cuot_qc_sparse(ctx, n, (uint8_t*)buf, (int64_t*)buf, 16, (uint8_t*)buf, nullptr) == CUOT_OK);
+    REQUIRE(g_launches.size() == 1);
+    const bool wide = g_launches[0].kernel.find("sparse_encode_wide") != std::string::npos;
+    REQUIRE(wide == (n >= m && n % 32 == 0));
+  }
+  REQUIRE(cuot_destroy(ctx) == CUOT_OK);
+  return 0;
+}
+
 // upper passes of an encode, there and back, and the one that joins them
 static int print_passes(int64_t n, int radix) {
   cuot_ctx* ctx = nullptr;
@@ -133,6 +149,7 @@ int main(int argc, char** argv) {
   if (what == "devices") rc = check_devices();
   if (what == "ggm_dfs") rc = check_ggm_dfs();
   if (what == "lpn_slices") rc = check_lpn_slices();
+  if (what == "sparse") rc = check_sparse();
   if (what == "passes" && argc > 3) rc = print_passes(atoll(argv[2]), atoi(argv[3]));
   if (!rc) printf("%s ok\n", what.c_str());
   return rc;

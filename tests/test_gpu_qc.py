@@ -291,3 +291,18 @@ def test_qc_encode_in_place(ctx, knob_mfma, n, mfma):
     upper = x[n:].clone()
     ctx.qc_encode(n, ahat, x, x, scratch)
     assert torch.equal(x[:n], y) and torch.equal(x[n:], upper)
+
+
+# whole words of 2^25 bits and more take all positions in one lane, others share
+# them out; positions at the ends, and ones to be ignored
+@pytest.mark.parametrize("n", [(1 << 25) - 32, (1 << 25) - 1, 1 << 25, (1 << 25) + 1, (1 << 25) + 32])
+def test_sparse_wide(ctx, n):
+    import torch
+
+    print(f"sparse wide n={n}", flush=True)
+    r = rng(n)
+    a = rand_bits(r, n)
+    pos = np.array([-1, 0, 77, n - 1, n, n + 1, n + 63, 2 * n - 1, 2 * n, 2 * n + 5], dtype=np.int64)
+    out = torch.full((((n + 31) // 32) * 4,), 0xA5, dtype=torch.uint8, device="cuda")
+    ctx.qc_sparse(n, dev_bits(a, n), torch.from_numpy(pos).cuda(), out)
+    assert np.array_equal(out.cpu().numpy()[: (n + 7) // 8], po.qc_sparse(pos, a, n))

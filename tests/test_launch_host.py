@@ -40,6 +40,10 @@ def test_lpn_slices_need_rows(check):
     check("lpn_slices")
 
 
+def test_sparse_product_of_many_words(check):
+    check("sparse")
+
+
 def test_tuner_can_choose_the_ggm_rule():
     from cuot_amd import tune
 
