@@ -58,8 +58,9 @@ constexpr int FFT_LD = 16;  // 16-byte loads in flight per lane (tile staging)
 
 constexpr int FFT_WGS = 512;  // FFT pass grid: two resident WGs on each of the 256 CUs
 constexpr int CR_LD = 8;    // same for the bit-row conversion tiles
-// the row-layout conversion handles strings of 2^5 .. 2^20 coefficients (128 KB, padded 144 KB, of LDS)
-constexpr int ROW_MP_MIN = 5, ROW_MP_MAX = 20;
+// the row-layout conversion handles strings of 2^5 .. 2^16 coefficients: up to 2^8
+// here (n <= 2^12), 2^13 up for the transform of qc_fa.hip
+constexpr int ROW_MP_MIN = 5, ROW_MP_MAX = 16;
 
 struct Beta {
   uint32_t v[32];
@@ -243,14 +244,12 @@ struct BarrierSync {
 };
 
 // PAD (strings of >= 2^10 coefficients): the string sits in LDS with four pad
-// words after every 32, and levels 9..0 run per 1024-bit block in registers.
-// MULTI (PAD, strings shorter than 2^20): a workgroup converts S = 1024 /
-// (blocks per string) strings side by side, one lane per block, so that short
-// strings still occupy every lane (the same LDS footprint for every length:
-// 1024 padded blocks).  Its per-lane LDS base costs registers, so there the
-// in-word levels (the first inverse and the last forward step) ride on the
-// copies between global memory and LDS (INW); a single string keeps them in
-// the register blocks, which measured faster.
+// words after every 32, and levels 9..0 run per 1024-bit block in registers.  A
+// workgroup converts S = 1024 / (blocks per string) strings side by side, one
+// lane per block, so that short strings still occupy every lane (the same LDS
+// footprint for every length: 1024 padded blocks).  The per-lane LDS base costs
+// registers, so the in-word levels (the first inverse and the last forward
+// step) ride on the copies between global memory and LDS (INW).
 CUOT_DEV uint4 inword4(uint4 v, bool inv) {
   v.x = cbt_word_all(v.x, inv);
   v.y = cbt_word_all(v.y, inv);
@@ -298,21 +297,17 @@ __device__ __forceinline__ void rows_store(uint32_t* g, const uint32_t* sw, int6
   }
 }
 
-template <bool PAD, bool INV, bool MULTI>
+template <bool PAD, bool INV>
 __global__ __launch_bounds__(1024) void qc_conv_rows(uint32_t* __restrict__ Bw, int64_t tile_words, int64_t ntiles,
                                                      int64_t tiles_per_inst, int64_t inst_words, int mp) {
-  static_assert(PAD || !MULTI, "several strings per workgroup need the blocked form");
   extern __shared__ uint32_t sw_all[];
-  if constexpr (!MULTI) {
+  if constexpr (!PAD) {
     for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
       uint32_t* g = Bw + (tile / tiles_per_inst) * inst_words + (tile % tiles_per_inst) * tile_words;
-      rows_load<PAD, false>(g, sw_all, tile_words, threadIdx.x, blockDim.x);
+      rows_load<false, false>(g, sw_all, tile_words, threadIdx.x, blockDim.x);
       __syncthreads();
-      if constexpr (PAD)
-        cbp_convert<true, INV>(sw_all, 0, mp, threadIdx.x, blockDim.x, BarrierSync());
-      else
-        cbt_convert(sw_all, mp, INV, threadIdx.x, blockDim.x, BarrierSync());
-      rows_store<PAD, false>(g, sw_all, tile_words, threadIdx.x, blockDim.x);
+      cbt_convert(sw_all, mp, INV, threadIdx.x, blockDim.x, BarrierSync());
+      rows_store<false, false>(g, sw_all, tile_words, threadIdx.x, blockDim.x);
       __syncthreads();
     }
   } else {
@@ -346,39 +341,21 @@ __global__ __launch_bounds__(1024) void qc_conv_rows(uint32_t* __restrict__ Bw, 
 
 // the blocked, padded form needs 1024-bit blocks: strings of >= 2^10 coefficients
 bool row_pad(int mp) { return mp >= 10; }
-// LDS of one workgroup: one string, or 1024 / (blocks per string) padded strings
+// LDS of one workgroup: one string, or 1024 / (blocks per string) padded strings (144 KB)
 size_t row_lds_bytes(int64_t tile_words, int mp) {
   return row_pad(mp) ? (size_t)cbp_words(32 * 1024, true) * 4 : (size_t)tile_words * 4;
 }
 
 hipError_t launch_conv_rows(unsigned cap, hipStream_t st, uint32_t* Bw, int64_t tile_words, int64_t ntiles,
                             int64_t tpi, int64_t inst_words, int mp, int inverse) {
-  if (row_pad(mp) && (tile_words < 32 || tile_words > 32 * 1024)) return hipErrorInvalidValue;
+  if (mp < ROW_MP_MIN || mp > ROW_MP_MAX || tile_words != ((int64_t)1 << mp) / 32) return hipErrorInvalidValue;
   const size_t lds = row_lds_bytes(tile_words, mp);
-  const bool multi = row_pad(mp) && tile_words < 32 * 1024;
-  const int64_t per_wg = multi ? 1024 / (tile_words >> 5) : 1;  // strings per workgroup
+  const int64_t per_wg = row_pad(mp) ? 1024 / (tile_words >> 5) : 1;  // strings per workgroup
   const int64_t need = (ntiles + per_wg - 1) / per_wg;
   const unsigned grid = (unsigned)(need < (int64_t)cap ? (need < 1 ? 1 : need) : cap);
-#define CONV_ROWS_LAUNCH(PAD, INV, MULTI)                                                                    \
-  hipLaunchKernelGGL((qc_conv_rows<PAD, INV, MULTI>), dim3(grid), dim3(1024), lds, st, Bw, tile_words, ntiles, \
-                     tpi, inst_words, mp)
-  if (multi) {
-    if (inverse)
-      CONV_ROWS_LAUNCH(true, true, true);
-    else
-      CONV_ROWS_LAUNCH(true, false, true);
-  } else if (row_pad(mp)) {
-    if (inverse)
-      CONV_ROWS_LAUNCH(true, true, false);
-    else
-      CONV_ROWS_LAUNCH(true, false, false);
-  } else {
-    if (inverse)
-      CONV_ROWS_LAUNCH(false, true, false);
-    else
-      CONV_ROWS_LAUNCH(false, false, false);
-  }
-#undef CONV_ROWS_LAUNCH
+  const auto kernel = row_pad(mp) ? (inverse ? qc_conv_rows<true, true> : qc_conv_rows<true, false>)
+                                  : (inverse ? qc_conv_rows<false, true> : qc_conv_rows<false, false>);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(1024), lds, st, Bw, tile_words, ntiles, tpi, inst_words, mp);
   return hipGetLastError();
 }
 
@@ -826,7 +803,7 @@ __global__ void qcs_fft_layer(const QcPrep* __restrict__ pr, QcPrep pr1, int64_t
 // The whole preparation of one polynomial in one workgroup's LDS when its
 // 2^m words fit (small codes): the same pack, conversion levels and FFT layers
 // as the kernels above, separated by barriers instead of launches.
-constexpr int PREP_LDS_MMAX = 15;  // 2^15 words = 128 KB
+constexpr int PREP_LDS_MMAX = 9;  // the largest of n <= 2^12 (2 KB)
 
 __global__ __launch_bounds__(1024) void qcs_prepare_lds(const QcPrep* __restrict__ pr, QcPrep pr1, int m) {
   extern __shared__ uint32_t L[];
@@ -1028,21 +1005,9 @@ hipError_t allow_lds() {
   e = hipFuncSetAttribute((const void*)qc_fft_pass<16>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (ftc_max<16>() * fstride<16>() + CTAB_WORDS) * 4);
   if (e != hipSuccess) return e;
-  e = hipFuncSetAttribute((const void*)qcs_prepare_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          ((int64_t)1 << PREP_LDS_MMAX) * 4);
-  if (e != hipSuccess) return e;
-  {
-    const void* fns[6] = {(const void*)qc_conv_rows<false, false, false>,
-                          (const void*)qc_conv_rows<false, true, false>,
-                          (const void*)qc_conv_rows<true, false, false>,
-                          (const void*)qc_conv_rows<true, true, false>,
-                          (const void*)qc_conv_rows<true, false, true>,
-                          (const void*)qc_conv_rows<true, true, true>};
-    for (int i = 0; i < 6; i++) {
-      e = hipFuncSetAttribute(fns[i], hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)row_lds_bytes(((int64_t)1 << ROW_MP_MAX) / 32, ROW_MP_MAX));
-      if (e != hipSuccess) return e;
-    }
+  for (const void* f : {(const void*)qc_conv_rows<true, false>, (const void*)qc_conv_rows<true, true>}) {
+    e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)row_lds_bytes(0, ROW_MP_MAX));
+    if (e != hipSuccess) return e;
   }
   e = hipFuncSetAttribute((const void*)qc_conv_lds<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (1 << CONV_B) * 16);
@@ -1351,7 +1316,7 @@ hipError_t encode_batch(const QcIo* io, QcIo io1, const uint32_t* ahat1, const u
                         void* scratch, hipStream_t st, hipEvent_t ready = nullptr) {
   hipError_t e = configure_lds();
   if (e != hipSuccess) return e;
-  if (B > 1 && !row_path(m - 1)) return hipErrorInvalidValue;
+  if (B > 1 && !cuot_qc_batchable(m)) return hipErrorInvalidValue;
   if (cuot_qc_fa_selected(((int64_t)1 << (m + 2)) + 1))
     return cuot_launch_qc_fa_encode(io, io1, ahat1, ahats, B, m + 4, io ? (int64_t)1 << (m + 3) : io1.n, scratch, st,
                                     ready);
@@ -1449,7 +1414,9 @@ int cuot_qc_log_len(int64_t n) {
 
 size_t cuot_qc_scratch_bytes_for(int64_t n) { return cuot_qc_batch_scratch_bytes(cuot_qc_log_len(n), 1); }
 
-bool cuot_qc_batchable(int m) { return row_path(m - 1); }
+// the orbits' transform, or the conversion of rows (n > 2^24 and n <= 2^8 convert
+// elements, one instance at a time)
+bool cuot_qc_batchable(int m) { return cuot_qc_fa_selected(((int64_t)1 << (m + 2)) + 1) || row_path(m - 1); }
 
 hipError_t cuot_qc_configure() {
   hipError_t e = configure_lds();
