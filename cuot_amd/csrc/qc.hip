@@ -91,22 +91,22 @@ CUOT_DEV uint32_t chunk_const(const uint32_t* beta, uint64_t g) {
   return c;
 }
 
-// C(g) from three 256-entry tables of the low 24 bits of g (tab[256*q + v] =
-// C(v << 8q)); g < 2^24 for every transform length handled here (m <= 24)
-constexpr int CTAB_WORDS = 3 * 256;
+// C(g) from tables of g's bytes (tab[256*q + v] = C(v << 8q)); g < 2^29 for the
+// longest transform (m = 30), so the last one has 32 entries
+constexpr int CTAB_WORDS = 3 * 256 + 32;
 
 CUOT_DEV void ctab_fill(uint32_t* tab, int tid, int nth) {
   for (int i = tid; i < CTAB_WORDS; i += nth) {
     const int q = i >> 8, v = i & 255;
     uint32_t c = 0;
-    for (int b = 0; b < 8; b++)
+    for (int b = 0; b < (q < 3 ? 8 : 5); b++)
       if ((v >> b) & 1) c ^= c_beta.v[8 * q + b + 1];
     tab[i] = c;
   }
 }
 
 CUOT_DEV uint32_t ctab_const(const uint32_t* tab, uint32_t g) {
-  return tab[g & 255] ^ tab[256 + ((g >> 8) & 255)] ^ tab[512 + ((g >> 16) & 255)];
+  return tab[g & 255] ^ tab[256 + ((g >> 8) & 255)] ^ tab[512 + ((g >> 16) & 255)] ^ tab[768 + (g >> 24)];
 }
 
 CUOT_DEV uint4 x4(uint4 a, uint4 b) { return make_uint4(a.x ^ b.x, a.y ^ b.y, a.z ^ b.z, a.w ^ b.w); }

@@ -306,3 +306,14 @@ def test_sparse_wide(ctx, n):
     out = torch.full((((n + 31) // 32) * 4,), 0xA5, dtype=torch.uint8, device="cuda")
     ctx.qc_sparse(n, dev_bits(a, n), torch.from_numpy(pos).cuda(), out)
     assert np.array_equal(out.cpu().numpy()[: (n + 7) // 8], po.qc_sparse(pos, a, n))
+
+
+# 2^26 elements: butterflies with more than 24 bits above them (about 95 GB in all)
+def test_qc_longest_product_rotations(ctx):
+    import torch
+
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 110e9:
+        pytest.skip("needs 110 GB of device memory")
+    test_qc_orbit_product_rotations(ctx, lambda v: None, (1 << 28) + 1)
+    torch.cuda.empty_cache()
