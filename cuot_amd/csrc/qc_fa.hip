@@ -200,7 +200,9 @@ CUOT_DEV int fa_insert(int P, int b, int r) { return ((P >> b) << (b + 1)) | (r 
 // ---- basis conversion in registers ----------------------------------------------------
 // Between the monomial basis and the novel one, every split of the index bits at
 // r = 16, 8, 4, 2, 1 is an expansion in powers of s_r = x^(2^r) + x, followed by
-// the same for the bits above the split (X = s_r) and below it.  s_r^(2^i) has
+// the same for the bits above the split (X = s_r) and below it (the conversion of
+// Lin, Al-Naffouri, Han and Yang, 2016, after Gao and Mateer's Taylor expansions,
+// 2010; the columns in registers below are this file's).  s_r^(2^i) has
 // one lower term, so the level of bit b = r + i takes, with half = 2^b and e =
 // 2^i, q = hi with its first e coefficients corrected by its last ones, and
 // lo_j ^= q_{j-e} (backwards the same with the two steps exchanged): 32 such
